@@ -111,8 +111,8 @@ static int check_dtypes(int p_dtype, int g_dtype) {
 // Completes prefix and pivots of a launch batch and launches it.  Args is FusedArgs
 // or SmallArgs; `chunks` is the batch's total chunk count.
 template <typename Args>
-static void finish_prefix(Args &a) {
-  for (int i = a.ntensors; i < Args::kPivots * 8; ++i) a.first_chunk[i] = 0x7fffffffu;
+static void finish_prefix(Args &a, int ntensors) {
+  for (int i = ntensors; i < Args::kPivots * 8; ++i) a.first_chunk[i] = 0x7fffffffu;
   for (int k = 0; k < Args::kPivots; ++k) a.pivot[k] = a.first_chunk[k * 8];
 }
 
@@ -126,6 +126,7 @@ static void finish_prefix(Args &a) {
 // fused kernels pad their grids to one).
 constexpr uint64_t kMaxChunksPerLaunch = 0x7ffffff0ull;   // per batch
 constexpr uint64_t kHipWorkItemsPerGrid = 0xffffffffull;
+constexpr uint64_t kMaxStatWorkgroups = 1ull << 23;        // rank-1 row-scale and commit launches: one grid
 constexpr int64_t kMaxInterchangeElements = 1ll << 40;     // q4adamw_quantize / q4adamw_dequantize
 static std::atomic<uint64_t> g_grid_limit_override{0};    // q4adamw_set_grid_limit (tests)
 
@@ -148,7 +149,7 @@ static int for_each_grid(uint64_t chunks, unsigned threads, F launch) {
 
 static int launch_fused_batch(FusedArgs &a, uint64_t chunks, void (*kernel)(const FusedArgs),
                               hipStream_t stream) {
-  finish_prefix(a);
+  finish_prefix(a, a.ntensors);
   return for_each_grid(chunks, kThreads, [&](uint64_t base, uint64_t count) -> int {
     a.chunk_base = (uint32_t)base;
     a.nchunks = (uint32_t)(base + count);
@@ -161,7 +162,7 @@ static int launch_fused_batch(FusedArgs &a, uint64_t chunks, void (*kernel)(cons
 
 static int launch_small_batch(SmallArgs &a, uint64_t chunks, void (*kernel)(const SmallArgs),
                               hipStream_t stream) {
-  finish_prefix(a);
+  finish_prefix(a, a.ntensors);
   return for_each_grid(chunks, 256, [&](uint64_t base, uint64_t count) -> int {
     a.chunk_base = (uint32_t)base;
     hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(256), 0, stream, a);
@@ -216,35 +217,52 @@ static uint64_t rank1_chunks(const q4adamw_rank1_tensor &t, int64_t tile_elems) 
   return ((uint64_t)t.rows * (uint64_t)t.cols + chunk_elems - 1) / chunk_elems;
 }
 
-template <bool EXT>
-static Rank1StatKernel pick_rank1_stats_ext(int g_dtype) {
-  if (g_dtype == Q4ADAMW_BF16) return rank1_stats_kernel<Q4ADAMW_BF16, EXT>;
-  if (g_dtype == Q4ADAMW_FP16) return rank1_stats_kernel<Q4ADAMW_FP16, EXT>;
-  return rank1_stats_kernel<Q4ADAMW_FP32, EXT>;
+// Which statistics kernel a matrix takes.  Flat: fewer columns than a wave of the wide form's
+// lanes could share (below that a lane per column or per 8 columns leaves lanes without work: of a
+// 786432 x 3 matrix 3 of 256, which took 260 us; of a 4096 x 16 one 2 of 64).  Wide: 8 columns per lane; rows that are no
+// multiple of 8 long take the variant that finds their codes at either nibble.  Lead: as flat, for
+// tensors with several leading dimensions.
+enum Rank1StatForm { kStatFlat = 0, kStatLead = 1, kStatWide = 2, kStatWideAny = 3, kStatForms = 4 };
+
+static bool rank1_has_leads(const q4adamw_rank1_tensor &t) { return t.lead_dims >= 2; }
+
+static Rank1StatForm rank1_stat_form(const q4adamw_rank1_tensor &t) {
+  if (t.cols <= (int64_t)kFlatMaxCols) return rank1_has_leads(t) ? kStatLead : kStatFlat;
+  return t.cols % 8 == 0 ? kStatWide : kStatWideAny;
 }
 
-static Rank1StatKernel pick_rank1_stats(int g_dtype, bool ext) {
-  return ext ? pick_rank1_stats_ext<true>(g_dtype) : pick_rank1_stats_ext<false>(g_dtype);
+template <int GT, bool EXT>
+static Rank1StatKernel pick_rank1_stats_form(Rank1StatForm form) {
+  if (form == kStatFlat) return rank1_stats_flat_kernel<GT, EXT>;
+  if (form == kStatLead) return rank1_stats_lead_kernel<GT, EXT>;
+  return form == kStatWide ? rank1_stats_kernel<GT, EXT, false> : rank1_stats_kernel<GT, EXT, true>;
 }
 
-template <bool EXT>
-static Rank1StatKernel pick_rank1_stats_any_ext(int g_dtype) {
-  if (g_dtype == Q4ADAMW_BF16) return rank1_stats_any_kernel<Q4ADAMW_BF16, EXT>;
-  if (g_dtype == Q4ADAMW_FP16) return rank1_stats_any_kernel<Q4ADAMW_FP16, EXT>;
-  return rank1_stats_any_kernel<Q4ADAMW_FP32, EXT>;
+static Rank1StatKernel pick_rank1_stats(Rank1StatForm form, int g_dtype, bool ext) {
+  if (g_dtype == Q4ADAMW_BF16) return ext ? pick_rank1_stats_form<Q4ADAMW_BF16, true>(form) : pick_rank1_stats_form<Q4ADAMW_BF16, false>(form);
+  if (g_dtype == Q4ADAMW_FP16) return ext ? pick_rank1_stats_form<Q4ADAMW_FP16, true>(form) : pick_rank1_stats_form<Q4ADAMW_FP16, false>(form);
+  return ext ? pick_rank1_stats_form<Q4ADAMW_FP32, true>(form) : pick_rank1_stats_form<Q4ADAMW_FP32, false>(form);
 }
 
-static Rank1StatKernel pick_rank1_stats_any(int g_dtype, bool ext) {
-  return ext ? pick_rank1_stats_any_ext<true>(g_dtype) : pick_rank1_stats_any_ext<false>(g_dtype);
+// Rows of a wide form's tile in a launch over `elements` elements: 256 if that makes four
+// workgroups per CU, else as few as 32.
+static uint32_t rank1_stat_rows(uint64_t elements) {
+  uint32_t rows = kStatRows;
+  while (rows > 32u && elements / ((uint64_t)rows * kStatCols) < 1024u) rows /= 2u;
+  return rows;
 }
 
-// tiles of the statistics launch of a matrix, by the form its rows allow
-static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t *col_groups) {
-  const bool any = t.cols % 8 != 0 || t.cols < 16;
-  const int64_t tile_rows = any ? kAnyStatRows : kStatRows, tile_cols = any ? kAnyStatCols : kStatCols;
-  const uint64_t groups = (uint64_t)((t.cols + tile_cols - 1) / tile_cols);
-  if (col_groups) *col_groups = (uint32_t)groups;
-  return (uint64_t)((t.rows + tile_rows - 1) / tile_rows) * groups;
+// tiles of the statistics launch of a matrix
+static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_rows) {
+  if (rank1_stat_form(t) == kStatFlat) {
+    const uint64_t tile_rows = flat_tile_rows((uint32_t)t.cols);
+    return ((uint64_t)t.rows + tile_rows - 1) / tile_rows;
+  }
+  if (rank1_stat_form(t) == kStatLead) {
+    const uint32_t outer = (uint32_t)t.lead_shape[0];
+    return (uint64_t)((outer + kLeadOuter - 1) / kLeadOuter) * lead_tiles((uint32_t)t.rows, outer, (uint32_t)t.cols).inner;
+  }
+  return (((uint64_t)t.rows + stat_rows - 1) / stat_rows) * (uint64_t)((t.cols + kStatCols - 1) / kStatCols);
 }
 
 // Fills the kernels' view of the caller's gradient options; returns whether the
@@ -509,25 +527,26 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       }
       if (prod != t.rows) return fail(Q4ADAMW_ERR_ARG, "rows must be the product of the leading dimensions");
     }
-    const uint64_t stat_chunks = rank1_stat_chunks(t, nullptr);
+    const uint64_t stat_chunks = rank1_stat_chunks(t, 32u);   // at most
     if (rank1_chunks(t, chunk_elems / kWaves) > kMaxChunksPerLaunch || stat_chunks > kMaxChunksPerLaunch)
       return fail(Q4ADAMW_ERR_TOO_LARGE, "tensor too large: more than 2^31 - 16 chunks");
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t tile_elems = chunk_elems / kWaves;
   const bool exact = exact_update(update_form, p_dtype, sr, true);
-  FoldArgs fa;   // the batch's tensors with several leading dimensions
-  fa.go = a.go;
-  fa.ntensors = 0;
+  RowScaleArgs ra;   // the batch's tensors with several leading dimensions
+  ra.go = a.go;
+  CommitArgs ca;
+  ca.go = a.go;
+  int leads = 0;
   Rank1Kernel kernel = nullptr;
   Rank1StatKernel stat_kernel = nullptr;
   a.ntensors = 0;
-  uint64_t chunks = 0, stat_chunks = 0;
-  // statistics of every tensor of the batch, then the update, then the commit
+  uint64_t chunks = 0, stat_chunks = 0, scale_chunks = 0, commit_chunks = 0;
+  // statistics of every tensor of the batch (and its rows' scales, with several leading
+  // dimensions), then the update, then the commit
   auto launch = [&]() -> int {
-    sa.ntensors = a.ntensors;
-    finish_prefix(sa);
-    sa.nchunks = (uint32_t)stat_chunks;
+    finish_prefix(sa, a.ntensors);
     if (int rc = for_each_grid(stat_chunks, kThreads, [&](uint64_t base, uint64_t count) -> int {
           sa.chunk_base = (uint32_t)base;
           hipLaunchKernelGGL(stat_kernel, dim3((unsigned)count), dim3(kThreads), 0, s, sa);
@@ -535,12 +554,12 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
           return 0;
         }))
       return rc;
-    if (fa.ntensors > 0) {   // rows' maxima -> leading statistics -> rows' scales
-      hipLaunchKernelGGL(rank1_fold_kernel<0>, dim3(64, (unsigned)fa.ntensors), dim3(256), 0, s, fa);
-      hipLaunchKernelGGL(rank1_fold_kernel<1>, dim3(64, (unsigned)fa.ntensors), dim3(256), 0, s, fa);
+    if (leads > 0) {   // leading statistics -> rows' scales
+      finish_prefix(ra, leads);
+      hipLaunchKernelGGL(rank1_row_scale_kernel, dim3((unsigned)scale_chunks), dim3(256), 0, s, ra);
       Q4_HIP(hipGetLastError());
     }
-    finish_prefix(a);
+    finish_prefix(a, a.ntensors);
     if (int rc = for_each_grid(chunks, kThreads, [&](uint64_t base, uint64_t count) -> int {
           a.chunk_base = (uint32_t)base;
           a.nchunks = (uint32_t)(base + count);
@@ -550,48 +569,52 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
           return 0;
         }))
       return rc;
-    hipLaunchKernelGGL(rank1_commit_kernel, dim3(64, (unsigned)a.ntensors), dim3(256), 0, s, a);
+    finish_prefix(ca, a.ntensors);
+    hipLaunchKernelGGL(rank1_commit_kernel, dim3((unsigned)commit_chunks), dim3(256), 0, s, ca);
     Q4_HIP(hipGetLastError());
-    if (fa.ntensors > 0) {
-      hipLaunchKernelGGL(rank1_fold_kernel<2>, dim3(8, (unsigned)fa.ntensors), dim3(256), 0, s, fa);
-      Q4_HIP(hipGetLastError());
-      fa.ntensors = 0;
-    }
-    a.ntensors = 0;
-    chunks = 0;
-    stat_chunks = 0;
+    a.ntensors = leads = 0;
+    chunks = stat_chunks = scale_chunks = commit_chunks = 0;
     return 0;
   };
-  // three passes: matrices whose rows are whole tiles take the kernel whose workgroups share
-  // the columns' maxima of four rows; other matrices with rows of at least a tile the one
-  // that finds a tile's row on the scalar unit; narrower ones the one whose lanes find their own
-  for (int shape = kShapeRows; shape <= kShapeAny; ++shape) {
-    kernel = shape == kShapeRows     ? pick_rank1_rows(p_dtype, g_dtype, ext, sr, exact)
-             : shape == kShapeWide   ? pick_rank1_wide(p_dtype, g_dtype, ext, sr, exact)
-             : shape == kShapeNarrow ? pick_rank1_narrow(p_dtype, g_dtype, ext, sr, exact)
-                                     : pick_rank1_any(p_dtype, g_dtype, ext, sr, exact);
-    stat_kernel = shape == kShapeAny ? pick_rank1_stats_any(g_dtype, ext) : pick_rank1_stats(g_dtype, ext);
+  // a pass per update kernel and statistics kernel: matrices whose rows are whole tiles take the
+  // update kernel whose workgroups share the columns' maxima of four rows; other matrices with
+  // rows of at least a tile the one that finds a tile's row on the scalar unit; narrower ones
+  // the one whose lanes find their own; rows of any length the one whose elements do
+  for (int pass = 0; pass < 4 * kStatForms; ++pass) {
+    const int shape = pass / kStatForms;
+    const Rank1StatForm form = (Rank1StatForm)(pass % kStatForms);
+    auto in_pass = [&](const q4adamw_rank1_tensor &t) {
+      return t.rows != 0 && t.cols != 0 && rank1_shape(t, tile_elems) == shape && rank1_stat_form(t) == form;
+    };
+    uint64_t pass_elements = 0;
     for (int i = 0; i < count; ++i) {
+      if (in_pass(tensors[i])) pass_elements += (uint64_t)(tensors[i].rows * tensors[i].cols);
+    }
+    sa.stat_rows = rank1_stat_rows(pass_elements);
+    kernel = nullptr;
+    for (int i = 0; i < count && pass_elements != 0; ++i) {
       const q4adamw_rank1_tensor &t = tensors[i];
-      if (t.rows == 0 || t.cols == 0 || rank1_shape(t, tile_elems) != shape) continue;
-      const int64_t numel = t.rows * t.cols;
-      const uint64_t c = rank1_chunks(t, tile_elems);
-      uint32_t groups = 0;
-      const uint64_t sc_ = rank1_stat_chunks(t, &groups);
-      if (a.ntensors == kMaxRank1Tensors || chunks + c > kMaxChunksPerLaunch ||
-          stat_chunks + sc_ > kMaxChunksPerLaunch || (t.lead_dims >= 2 && fa.ntensors == kMaxFoldTensors)) {
-        if (int rc = launch()) return rc;
+      if (!in_pass(t)) continue;
+      if (!kernel) {
+        kernel = shape == kShapeRows     ? pick_rank1_rows(p_dtype, g_dtype, ext, sr, exact)
+                 : shape == kShapeWide   ? pick_rank1_wide(p_dtype, g_dtype, ext, sr, exact)
+                 : shape == kShapeNarrow ? pick_rank1_narrow(p_dtype, g_dtype, ext, sr, exact)
+                                         : pick_rank1_any(p_dtype, g_dtype, ext, sr, exact);
+        stat_kernel = pick_rank1_stats(form, g_dtype, ext);
       }
-      if (t.lead_dims >= 2) {
-        FoldDesc &f = fa.desc[fa.ntensors++];
-        f.row_next = t.row_max_next;
-        f.rows = t.rows;
-        f.dims = t.lead_dims;
-        for (int j = 0; j < 3; ++j) {
-          f.shape[j] = j < t.lead_dims ? t.lead_shape[j] : 1;
-          f.cur[j] = j < t.lead_dims ? t.lead_max[j] : nullptr;
-          f.next[j] = j < t.lead_dims ? t.lead_max_next[j] : nullptr;
-        }
+      const int64_t numel = t.rows * t.cols;
+      const uint64_t c = rank1_chunks(t, tile_elems), sc_ = rank1_stat_chunks(t, sa.stat_rows);
+      auto commit_chunks_of = [](int64_t size) { return ((uint64_t)size + kCommitChunk - 1) / kCommitChunk; };
+      uint64_t cc = commit_chunks_of(t.rows) + commit_chunks_of(t.cols);
+      if (rank1_has_leads(t)) {
+        for (int j = 0; j < t.lead_dims; ++j) cc += commit_chunks_of(t.lead_shape[j]);
+      }
+      const uint64_t rc_ = ((uint64_t)t.rows + kRowScaleChunk - 1) / kRowScaleChunk;
+      // the row-scale and commit launches stay within one grid (one tensor's rows and columns
+      // are fewer than 2^32, 2^21 chunks)
+      if (a.ntensors == kMaxRank1Tensors || chunks + c > kMaxChunksPerLaunch || stat_chunks + sc_ > kMaxChunksPerLaunch ||
+          commit_chunks + cc > kMaxStatWorkgroups || scale_chunks + rc_ > kMaxStatWorkgroups) {
+        if (int rc = launch()) return rc;
       }
       Rank1Desc &d = a.desc[a.ntensors];
       d.p = t.p;
@@ -622,13 +645,42 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       sd.cmax = t.col_max;
       sd.rmax_next = t.row_max_next;
       sd.cmax_next = t.col_max_next;
-      sd.rows = t.rows;
-      sd.cols = t.cols;
+      sd.lead_dims = rank1_has_leads(t) ? (uint32_t)t.lead_dims : 0u;
+      sd.rows = (uint32_t)t.rows;
+      sd.cols = (uint32_t)t.cols;
       sa.first_chunk[a.ntensors] = (uint32_t)stat_chunks;
-      sa.col_groups[a.ntensors] = groups;
+      CommitArgs::Desc &cd = ca.desc[a.ntensors];
+      cd.cur[0] = t.row_max;
+      cd.next[0] = t.row_max_next;
+      cd.size[0] = sd.rows;
+      cd.cur[1] = t.col_max;
+      cd.next[1] = t.col_max_next;
+      cd.size[1] = sd.cols;
+      for (int j = 0; j < 3; ++j) {
+        const bool there = j < (int)sd.lead_dims;
+        sd.lead_next[j] = cd.next[2 + j] = there ? t.lead_max_next[j] : nullptr;
+        cd.cur[2 + j] = there ? t.lead_max[j] : nullptr;
+        sd.lead_shape[j] = there ? (uint32_t)t.lead_shape[j] : 1u;
+        cd.size[2 + j] = there ? (uint32_t)t.lead_shape[j] : 0u;
+      }
+      ca.first_chunk[a.ntensors] = (uint32_t)commit_chunks;
+      if (sd.lead_dims != 0u) {
+        RowScaleArgs::Desc &rd = ra.desc[leads];
+        rd.row_next = t.row_max_next;
+        rd.lead_dims = sd.lead_dims;
+        rd.rows = sd.rows;
+        for (int j = 0; j < 3; ++j) {
+          rd.lead_next[j] = sd.lead_next[j];
+          rd.lead_shape[j] = sd.lead_shape[j];
+        }
+        ra.first_chunk[leads] = (uint32_t)scale_chunks;
+        ++leads;
+        scale_chunks += rc_;
+      }
       ++a.ntensors;
       chunks += c;
       stat_chunks += sc_;
+      commit_chunks += cc;
     }
     if (a.ntensors > 0) {
       if (int rc = launch()) return rc;
@@ -699,7 +751,7 @@ static int grad_norm_impl(const q4adamw_grad *grads, int count, int g_dtype, flo
   a.ntensors = 0;
   uint64_t chunks = 0;
   auto launch = [&]() -> int {
-    finish_prefix(a);
+    finish_prefix(a, a.ntensors);
     a.nchunks = (uint32_t)chunks;
     if (g_dtype == Q4ADAMW_BF16) hipLaunchKernelGGL(grad_sumsq_kernel<Q4ADAMW_BF16>, dim3(kNormPartials), dim3(256), 0, s, a);
     else if (g_dtype == Q4ADAMW_FP16) hipLaunchKernelGGL(grad_sumsq_kernel<Q4ADAMW_FP16>, dim3(kNormPartials), dim3(256), 0, s, a);

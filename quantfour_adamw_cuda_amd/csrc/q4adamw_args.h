@@ -152,8 +152,7 @@ static FastDiv make_fast_div(uint32_t d) {  // d >= 2
 constexpr int kMaxRank1Tensors = 32;
 
 // Kernel arguments of the rank-1 launches.  The update kernel indexes chunks of
-// kChunk flat elements like FusedArgs; the statistics kernel indexes tiles of
-// kStatRows rows x kStatCols columns (stat_first_chunk, stat_col_groups).
+// kChunk flat elements like FusedArgs.
 struct Rank1Args {
   static constexpr int kCapacity = kMaxRank1Tensors;
   static constexpr int kPivots = (kMaxRank1Tensors + 7) / 8;
@@ -170,49 +169,71 @@ struct Rank1Args {
   Rank1Desc desc[kMaxRank1Tensors];
 };
 
+// The statistics kernels index tiles of a matrix (rank1_stat_chunks).  A tensor with two or
+// three leading dimensions is the matrix [their product, last dimension]; its rows' maxima go
+// straight into one statistic per leading dimension (lead_next) and `rmax_next` is left alone.
+// Row and column counts fit 32 bits (2^35 - 1 elements, at least 16 columns above 2^32).
 struct Rank1StatArgs {
   static constexpr int kCapacity = kMaxRank1Tensors;
   static constexpr int kPivots = (kMaxRank1Tensors + 7) / 8;
   float b2, r2;
   GradOps go;
-  int ntensors;
   uint32_t chunk_base;     // this grid's first tile (workgroup 0)
-  uint32_t nchunks;
+  uint32_t stat_rows;      // rows of a tile of the wide forms: four times the rows a wave walks
   uint32_t pivot[kPivots];
   uint32_t first_chunk[kPivots * 8];
-  uint32_t col_groups[kMaxRank1Tensors];   // column groups per row group of tensor t
-  struct Desc {
+  struct Desc {  // 96 bytes
     const void *g;
     const uint8_t *v;
     const float *rmax;
     const float *cmax;
     float *rmax_next;
     float *cmax_next;
-    int64_t rows;
-    int64_t cols;
+    float *lead_next[3];
+    uint32_t lead_shape[3];
+    uint32_t lead_dims;    // 0, 2 or 3
+    uint32_t rows;
+    uint32_t cols;
   } desc[kMaxRank1Tensors];
 };
 
-// Rank-1 scaling of a tensor with two or three leading dimensions (its rows are their
-// product): the statistics kernel leaves every flattened row's own maximum, these kernels
-// reduce them to one statistic per leading dimension and hand the update kernel the rows'
-// scales, the minimum over a row's leading statistics.
-constexpr int kMaxFoldTensors = 16;
+// Between statistics and update of tensors with several leading dimensions: the rows' new
+// scales, each the minimum over its leading statistics.  Chunks of kRowScaleChunk rows.
+constexpr int kRowScaleChunk = 2048;
 
-struct FoldDesc {  // 104 bytes
-  float *row_next;   // in: the rows' own new maxima; out: the rows' new scales
-  int64_t rows;
-  int32_t dims;      // 2 or 3 leading dimensions
-  int32_t pad_;
-  int64_t shape[3];
-  float *cur[3];     // current statistic of each leading dimension
-  float *next[3];    // the step's new statistics (all zero between steps)
+struct RowScaleArgs {
+  static constexpr int kCapacity = kMaxRank1Tensors;
+  static constexpr int kPivots = (kMaxRank1Tensors + 7) / 8;
+  GradOps go;
+  uint32_t pivot[kPivots];
+  uint32_t first_chunk[kPivots * 8];
+  struct Desc {  // 64 bytes
+    float *row_next;
+    const float *lead_next[3];
+    uint32_t lead_shape[3];
+    uint32_t lead_dims;
+    uint32_t rows;
+    uint32_t pad_;
+  } desc[kMaxRank1Tensors];
 };
 
-struct FoldArgs {
+// After the update: every new statistic (rows, columns, leading dimensions) becomes the current
+// one and its buffer returns to zero.  Chunks of kCommitChunk floats, each in one of a tensor's
+// vectors.
+constexpr int kCommitChunk = 2048;
+
+struct CommitArgs {
+  static constexpr int kCapacity = kMaxRank1Tensors;
+  static constexpr int kPivots = (kMaxRank1Tensors + 7) / 8;
   GradOps go;
-  int ntensors;
-  FoldDesc desc[kMaxFoldTensors];
+  uint32_t pivot[kPivots];
+  uint32_t first_chunk[kPivots * 8];
+  struct Desc {  // 104 bytes
+    float *cur[5];    // rows, columns, leading dimensions (unused ones have size 0)
+    float *next[5];
+    uint32_t size[5];
+    uint32_t pad_;
+  } desc[kMaxRank1Tensors];
 };
 
 // Gradient-norm launch: every workgroup walks chunks of 32 KiB with a grid stride.
@@ -239,7 +260,8 @@ struct NormArgs {
 
 static_assert(sizeof(StepConsts) <= Q4ADAMW_STEP_CONSTS_BYTES, "the device copy of a step's scalars");
 static_assert(sizeof(FusedArgs) <= 4096 && sizeof(SmallArgs) <= 4096 && sizeof(NormArgs) <= 4096 &&
-                  sizeof(Rank1Args) <= 4096 && sizeof(Rank1StatArgs) <= 4096 && sizeof(FoldArgs) <= 4096,
+                  sizeof(Rank1Args) <= 4096 && sizeof(Rank1StatArgs) <= 4096 && sizeof(RowScaleArgs) <= 4096 &&
+                  sizeof(CommitArgs) <= 4096,
               "kernel arguments are limited to 4 KiB");
 
 // the first-moment bucket table (see q4adamw_tables.h), copied into LDS by every

@@ -1,24 +1,88 @@
 // Rank-1 scaling of the second moment, the launches around the update kernels of
-// q4adamw_step.h: statistics (new second moments reduced to row and column maxima), commit,
-// and the folds for tensors with several leading dimensions.
+// q4adamw_step.h: statistics (new second moments reduced to row and column maxima, or to one
+// statistic per dimension for tensors with several leading dimensions), those tensors' row
+// scales, and the commit.
 #pragma once
 #include "q4adamw_device.h"
 
 namespace q4 {
 
-constexpr int kStatRowsPerWave = 64;     // rows a wave walks
-constexpr int kStatRows = kStatRowsPerWave * kWaves;   // rows per workgroup of the statistics kernel
+// Raises a statistic to u (a non-negative float's bits).  Maxima settle early, so most calls
+// find the statistic already there: a value read too early is only too small, and then the
+// atomic decides.  Unconditional atomics on statistics that many workgroups share are what such
+// a launch waits for: 786432 rows x 3 leading statistics one by one took 4.6 ms.
+__device__ __forceinline__ void raise_max(float *addr, uint32_t u) {
+  unsigned int *const a = reinterpret_cast<unsigned int *>(addr);
+  if (u > __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(a, u);
+}
+
+// A workgroup's share of the leading statistics: rows [row0, row0 + n) with their maxima in
+// row_bits.  The rows are consecutive, so dimension j meets at most min(shape[j], n / stride + 2)
+// of its indices: one LDS slot for each of them, all dimensions side by side (at most 2 n + 4
+// words), then one update per slot, all of them in flight together.
+template <typename Desc>
+__device__ __forceinline__ void fold_rows(const Desc &T, uint32_t row0, uint32_t n, const uint32_t *row_bits,
+                                          uint32_t *slots) {
+  uint32_t first[3], count[3];   // per dimension: index of slot 0 (before the wrap at shape), slots
+  uint32_t stride = 1, total = 0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {  // from the last leading dimension to the first
+    const int j = (int)T.lead_dims - 1 - k;
+    const uint32_t shape = j >= 0 ? T.lead_shape[j] : 1u;
+    first[k] = row0 / stride;
+    const uint32_t span = (row0 + n - 1) / stride - first[k] + 1;
+    count[k] = j < 0 ? 0u : span < shape ? span : shape;
+    total += count[k];
+    stride *= shape;
+  }
+  for (uint32_t i = threadIdx.x; i < total; i += kThreads) slots[i] = 0u;
+  __syncthreads();
+  for (uint32_t r = threadIdx.x; r < n; r += kThreads) {
+    const uint32_t u = row_bits[r];
+    uint32_t q = row0 + r, base = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      if (count[k] != 0u) {
+        uint32_t slot = q - first[k];
+        const uint32_t shape = T.lead_shape[(int)T.lead_dims - 1 - k], next = q / shape;
+        if (count[k] == shape) slot %= shape;
+        if (u > slots[base + slot]) atomicMax(&slots[base + slot], u);
+        base += count[k];
+        q = next;
+      }
+    }
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < total; i += kThreads) {
+    uint32_t slot = i;
+    int k = 0;
+    if (slot >= count[0]) { slot -= count[0]; k = 1; }
+    if (k == 1 && slot >= count[1]) { slot -= count[1]; k = 2; }
+    const int j = (int)T.lead_dims - 1 - k;
+    const uint32_t base = k == 0 ? first[0] : k == 1 ? first[1] : first[2];
+    if (slots[i] != 0u) raise_max(T.lead_next[j] + (base + slot) % T.lead_shape[j], slots[i]);
+  }
+}
+
+constexpr int kStatRowsPerWave = 64;     // rows a wave walks, at most
+constexpr int kStatRows = kStatRowsPerWave * kWaves;   // rows per workgroup of the statistics kernel, at most
 constexpr int kStatCols = 512;           // columns per workgroup: 8 per lane
 
-// New second moments of a tile of kStatRows x kStatCols elements, reduced to row and
+// New second moments of a tile of stat_rows x kStatCols elements, reduced to row and
 // column maxima (get_variance_tensor_statistics, adamw_fourbit_triton.py:738-746).  The
 // arithmetic is the update kernel's, operation for operation, so the maxima are maxima
 // of exactly the values that kernel quantizes.  The four waves of a workgroup share the
 // columns and split the rows: every lane keeps 8 columns over its wave's rows, the waves'
 // column maxima meet in LDS, and the tile issues one atomic per column and one per row
 // (atomics on the column vector are what this kernel's time depends on most: a tile of
-// 64 rows with four times as many of them took 1.25 to 2 times as long).
-template <int GT, bool EXT>
+// 64 rows with four times as many of them took 1.25 to 2 times as long).  A wave walks 64 rows
+// where the launch has workgroups enough for the chip (args.stat_rows = 256) and fewer in a
+// small launch, which would otherwise wait for one wave's 16 rounds of loads (one 1000 x 512
+// matrix: 30 us with 64 rows per wave).
+// ANY: rows of any length (at least 8).  A row may then start at either nibble of a byte of the
+// codes, and the lane that would run past the row's end works on the row's last 8 columns
+// instead: maxima do not mind columns seen twice.
+template <int GT, bool EXT, bool ANY>
 __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatArgs args) {
   constexpr int kAhead = 4;  // rows whose loads are in flight together
   __shared__ uint32_t row_bits[4][kStatRows];       // row maxima of each 16-lane quarter of the row's wave
@@ -29,23 +93,31 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
   const int t = find_tensor(args, chunk);
   const auto &T = args.desc[t];
   const uint32_t local = chunk - args.first_chunk[t];
-  const uint32_t groups = args.col_groups[t];
+  const uint32_t groups = (T.cols + kStatCols - 1) / kStatCols;
   const uint32_t rg = local / groups, cg = local - rg * groups;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t col = (int64_t)cg * kStatCols + lane * 8;
-  const bool active = col < T.cols;  // cols is a multiple of 8: all 8 columns or none
-  const int64_t tile_row0 = (int64_t)rg * kStatRows;
-  const int tile_rows = (int)(tile_row0 + kStatRows < T.rows ? kStatRows : T.rows - tile_row0);
-  const int wave_row0 = wave * kStatRowsPerWave;                         // within the tile
+  const bool active = cg * kStatCols + (uint32_t)lane * 8u < T.cols;
+  // the tile's first column, and the lane's counted from there: all 8 of the lane's are in the row
+  uint32_t col0 = cg * kStatCols, lane_elem = (uint32_t)lane * 8u;
+  if (ANY) {
+    col0 = col0 < T.cols - 8u ? col0 : T.cols - 8u;
+    const uint32_t last = T.cols - 8u - col0;
+    lane_elem = lane_elem < last ? lane_elem : last;
+  }
+  const uint32_t stat_rows = args.stat_rows;
+  const uint32_t tile_row0 = rg * stat_rows;
+  const int tile_rows = (int)(T.rows - tile_row0 < stat_rows ? T.rows - tile_row0 : stat_rows);
+  const int rows_per_wave = (int)(stat_rows / kWaves);
+  const int wave_row0 = wave * rows_per_wave;                            // within the tile
   int nrows = tile_rows - wave_row0;                                      // rows of this wave
-  nrows = nrows < 0 ? 0 : (nrows > kStatRowsPerWave ? kStatRowsPerWave : nrows);
+  nrows = nrows < 0 ? 0 : (nrows > rows_per_wave ? rows_per_wave : nrows);
   // lanes past the last column work on zeros: code 0 under a zero scale and a zero
   // gradient give a zero second moment, which leaves every maximum alone
   float c_old[8], c_max[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    c_old[k] = active ? as_global<const float>(T.cmax)[col + k] : 0.0f;
+    c_old[k] = active ? as_global<const float>(T.cmax)[col0 + lane_elem + k] : 0.0f;
     c_max[k] = 0.0f;
   }
   const uint32_t quarter = (uint32_t)lane >> 4;
@@ -57,18 +129,25 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
       const int r = r0 + i < nrows ? r0 + i : nrows - 1;
-      const int64_t row = tile_row0 + wave_row0 + r;
+      const uint32_t row = tile_row0 + wave_row0 + r;
       r_old[i] = as_global<const float>(T.rmax)[row];
       // row bases are uniform; the lane's column is a 32-bit offset
-      const int64_t row_first = row * T.cols + (int64_t)cg * kStatCols;
-      const uint32_t lane_elem = (uint32_t)lane * 8u;
+      const int64_t row_first = (int64_t)row * T.cols + col0;
       const void *g_row = static_cast<const char *>(T.g) + row_first * (GT ? 2 : 4);
       const void *v_row = T.v + (row_first >> 1);
       vw[i] = 0u;
 #pragma unroll
       for (int h = 0; h < (GT ? 1 : 2); ++h) gw[i][h] = u32x4{0u, 0u, 0u, 0u};
       if (active) {
-        vw[i] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(v_row), lane_elem >> 1, 0, kNtReadOnly);
+        if (ANY) {
+          // eight codes from either nibble of a byte on: four bytes, or four and the low nibble of a fifth
+          const uint32_t nibble = ((uint32_t)row_first & 1u) + lane_elem;
+          vw[i] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(v_row), nibble >> 1, 0, kNtReadOnly);
+          if (nibble & 1u)
+            vw[i] = (vw[i] >> 4) | (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(tile_rsrc(v_row), (nibble >> 1) + 4u, 0, kNtReadOnly) << 28;
+        } else {
+          vw[i] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(v_row), lane_elem >> 1, 0, kNtReadOnly);
+        }
         if (GT) {
           gw[i][0] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_row), lane_elem * 2u, 0, kNtReadOnly);
         } else {
@@ -113,135 +192,299 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
 #pragma unroll
   for (int k = 0; k < 8; ++k) col_bits[wave][lane * 8 + k] = f2bits(c_max[k]);
   __syncthreads();
-  // one atomic per column and per row of the tile
+  // one update per column of the tile, and one per row or per leading index of its rows
 #pragma unroll
   for (int h = 0; h < kStatCols / kThreads; ++h) {
-    const int c = tid + h * kThreads;
+    const uint32_t c = (uint32_t)(tid + h * kThreads);
     uint32_t u = col_bits[0][c];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) u = u > col_bits[w][c] ? u : col_bits[w][c];
-    const int64_t cc = (int64_t)cg * kStatCols + c;
-    if (cc < T.cols && u != 0u) atomic_max_nonneg(T.cmax_next + cc, bits2f(u));
-  }
-#pragma unroll
-  for (int h = 0; h < kStatRows / kThreads; ++h) {
-    const int r = tid + h * kThreads;
-    if (r < tile_rows) {
-      uint32_t u = row_bits[0][r];
-#pragma unroll
-      for (int qi = 1; qi < 4; ++qi) u = u > row_bits[qi][r] ? u : row_bits[qi][r];
-      if (u != 0u) atomic_max_nonneg(T.rmax_next + tile_row0 + r, bits2f(u));
+    const bool there = cg * kStatCols + (ANY ? c & ~7u : c) < T.cols;
+    uint32_t cc = cg * kStatCols + c;
+    if (ANY) {   // the column that slot c's lane worked on
+      const uint32_t first = c & ~7u, last = T.cols - 8u - col0;
+      cc = col0 + (first < last ? first : last) + (c & 7u);
     }
+    if (there && u != 0u) raise_max(T.cmax_next + cc, u);
   }
+  static_assert(kStatRows == kThreads, "one row per thread below");
+  uint32_t u = row_bits[0][tid];
+#pragma unroll
+  for (int qi = 1; qi < 4; ++qi) u = u > row_bits[qi][tid] ? u : row_bits[qi][tid];
+  if (T.lead_dims == 0u) {
+    if (tid < tile_rows && u != 0u) raise_max(T.rmax_next + tile_row0 + tid, u);
+    return;
+  }
+  __syncthreads();          // every thread has read its row's quarters
+  row_bits[0][tid] = u;
+  __syncthreads();
+  fold_rows(T, tile_row0, (uint32_t)tile_rows, row_bits[0], row_bits[1]);
 }
 
-// The same statistics for rows of any length (not a multiple of 8, or shorter than 16), where a
-// row starts at any element of the packed codes: a workgroup takes kAnyStatRows rows x 256
-// columns, a thread one column, element by element; the rows' maxima meet in LDS, then one
-// atomic per row and per column.  Same arithmetic, operation for operation.
-constexpr int kAnyStatRows = 64;
-constexpr int kAnyStatCols = 256;
+// The same statistics for matrices of fewer than kFlatMaxCols columns: a workgroup takes
+// as many whole rows as fit a tile of kFlatWords elements (an odd row pitch, so that a walk
+// along rows and one across them meet all banks) and reads them as one run of consecutive
+// elements: thread t's elements are t, t + k * cols, t + 2 * k * cols, ... (k rows a time), all of
+// one column, whose maximum stays in a register.  The second moments meet the rows in LDS:
+// a thread per row, or several where the tile has fewer than 256 rows.  A row lies in one
+// workgroup, so its maximum is stored without an atomic.
+// The forms it replaces here gave a lane to every column or to every 8th of them: with 3 columns
+// (the last dimension of a 3x3 convolution kernel) 3 of 256 threads had work.
+// Same arithmetic, operation for operation.
+constexpr uint32_t kFlatMaxCols = 256;
+constexpr uint32_t kFlatWords = 4096;
+constexpr uint32_t kFlatMaxRows = kFlatWords / 3;     // 2 and 3 columns: a pitch of 3 words
+
+__host__ __device__ __forceinline__ uint32_t flat_tile_rows(uint32_t cols) { return kFlatWords / (cols | 1u); }
 
 template <int GT, bool EXT>
-__global__ __launch_bounds__(kThreads) void rank1_stats_any_kernel(const Rank1StatArgs args) {
-  __shared__ uint32_t row_bits[kAnyStatRows];
+__global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1StatArgs args) {
+  constexpr int kAhead = 8;   // elements of a thread whose loads are in flight together
+  __shared__ float tile[kFlatWords];
+  __shared__ uint32_t row_bits[kFlatMaxRows];
+  __shared__ uint32_t col_bits[kFlatMaxCols];
   const uint32_t chunk = args.chunk_base + blockIdx.x;
   float gscale = 1.0f;
   if (EXT && !grad_ops_begin(args.go, gscale)) return;
   const int t = find_tensor(args, chunk);
   const auto &T = args.desc[t];
-  const uint32_t local = chunk - args.first_chunk[t];
-  const uint32_t groups = args.col_groups[t];
-  const uint32_t rg = local / groups, cg = local - rg * groups;
-  const int tid = threadIdx.x;
-  const int64_t col = (int64_t)cg * kAnyStatCols + tid;
-  const bool active = col < T.cols;
-  const int64_t row0 = (int64_t)rg * kAnyStatRows;
-  const int nrows = (int)(row0 + kAnyStatRows < T.rows ? kAnyStatRows : T.rows - row0);
-  if (tid < kAnyStatRows) row_bits[tid] = 0u;
-  __syncthreads();
-  const float c_old = active ? as_global<const float>(T.cmax)[col] : 0.0f;
+  const uint32_t tid = threadIdx.x, cols = T.cols, pitch = cols | 1u;
+  const uint32_t row0 = (chunk - args.first_chunk[t]) * flat_tile_rows(cols);
+  const uint32_t n = T.rows - row0 < flat_tile_rows(cols) ? T.rows - row0 : flat_tile_rows(cols);
+  const uint32_t parts = n >= (uint32_t)kThreads ? 1u : (uint32_t)kThreads / n;   // threads per row
+  if (tid < cols) col_bits[tid] = 0u;
+  if (parts > 1u && tid < n) row_bits[tid] = 0u;
+
+  const uint32_t rows_per_pass = (uint32_t)kThreads / cols;
+  const uint32_t r_first = tid / cols, col = tid - r_first * cols;
+  const bool active = r_first < rows_per_pass && r_first < n;
+  const int64_t first = (int64_t)row0 * cols;                 // the tile's first element
+  const void *g_tile = static_cast<const char *>(T.g) + first * (GT ? 2 : 4);
+  const uint8_t *v_tile = T.v + (first >> 1);
+  const uint32_t odd = (uint32_t)first & 1u;
   float c_max = 0.0f;
-  for (int r = 0; r < nrows; ++r) {
-    float v = 0.0f;     // lanes past the last column leave every maximum alone
-    if (active) {
-      const int64_t e = (row0 + r) * T.cols + col;
-      float g = load_scalar<GT>(T.g, e);
-      if (EXT) g *= gscale;
-      const uint32_t code = ((uint32_t)as_global<const uint8_t>(T.v)[e >> 1] >> (4 * (int)(e & 1))) & 15u;
-      const float code_value = __builtin_fmaf((float)code, 0.0625f, 0.0625f);  // (code + 1) / 16, exact
-      const float v_old = code_value * min_nonneg(as_global<const float>(T.rmax)[row0 + r], c_old);
-      v = args.b2 * v_old + args.r2 * (g * g);
-    }
-    // fmaxf drops a NaN: a NaN never becomes a maximum, as in the update kernel's scales
-    c_max = __builtin_fmaxf(c_max, v);
-    uint32_t u = f2bits(__builtin_fmaxf(v, 0.0f));
+  if (active) {
+    const float c_old = as_global<const float>(T.cmax)[col];
+    for (uint32_t r0 = r_first; r0 < n; r0 += kAhead * rows_per_pass) {
+      float g[kAhead], r_old[kAhead];
+      uint32_t byte[kAhead];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const uint32_t o = (uint32_t)__shfl_xor((int)u, off, 64);
-      u = u > o ? u : o;
+      for (int i = 0; i < kAhead; ++i) {
+        uint32_t r = r0 + (uint32_t)i * rows_per_pass;
+        r = r < n ? r : r0;                                  // past the tile: a row seen already
+        const uint32_t e = r * cols + col;
+        g[i] = load_scalar<GT>(g_tile, e);
+        byte[i] = as_global<const uint8_t>(v_tile)[(e + odd) >> 1];
+        r_old[i] = as_global<const float>(T.rmax)[row0 + r];
+      }
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        uint32_t r = r0 + (uint32_t)i * rows_per_pass;
+        r = r < n ? r : r0;
+        const float gi = EXT ? g[i] * gscale : g[i];
+        const uint32_t code = (byte[i] >> (4u * ((r * cols + col + odd) & 1u))) & 15u;
+        const float code_value = __builtin_fmaf((float)code, 0.0625f, 0.0625f);  // (code + 1) / 16, exact
+        const float v_old = code_value * min_nonneg(r_old[i], c_old);
+        const float v = __builtin_fmaxf(args.b2 * v_old + args.r2 * (gi * gi), 0.0f);   // a NaN never becomes a maximum
+        c_max = __builtin_fmaxf(c_max, v);
+        tile[r * pitch + col] = v;
+      }
     }
-    if ((tid & 63) == 0 && u != 0u) atomicMax(&row_bits[r], u);
   }
-  if (active && c_max != 0.0f) atomic_max_nonneg(T.cmax_next + col, c_max);
   __syncthreads();
-  if (tid < nrows && row_bits[tid] != 0u) atomic_max_nonneg(T.rmax_next + row0 + tid, bits2f(row_bits[tid]));
+  if (active && c_max != 0.0f) atomicMax(&col_bits[col], f2bits(c_max));
+  for (uint32_t i = tid; i < n * parts; i += kThreads) {
+    const uint32_t r = i / parts, part = i - r * parts;
+    float r_max = 0.0f;
+    for (uint32_t c = part; c < cols; c += parts) r_max = __builtin_fmaxf(r_max, tile[r * pitch + c]);
+    if (parts == 1u) row_bits[r] = f2bits(r_max);
+    else if (r_max != 0.0f) atomicMax(&row_bits[r], f2bits(r_max));
+  }
+  __syncthreads();
+  if (tid < cols && col_bits[tid] != 0u) raise_max(T.cmax_next + tid, col_bits[tid]);
+  for (uint32_t r = tid; r < n; r += kThreads) as_global<uint32_t>(T.rmax_next)[row0 + r] = row_bits[r];
+}
+
+// The same for tensors with several leading dimensions and fewer than kFlatMaxCols columns (a
+// stack of 3x3 convolution kernels: [out, in, 3, 3]), straight to one statistic per dimension.
+// What bounds such a kernel is not its bytes but the updates of statistics that every
+// workgroup shares, which the memory side takes one after another: tiles of consecutive rows meet
+// nearly all of the second dimension each (on 20 such stacks, 11 million elements, a kernel
+// with those tiles took 23 us without its updates and 64 us with them).  So a tile is
+// two-dimensional: kLeadOuter indices of the first dimension times a run of at most 256
+// consecutive elements below it (whole rows), which meets 16 indices of the first dimension and
+// a few dozen of the second: 30 to 37 us, against 5.7 ms for statistics and folds before.
+// A thread keeps one element of the run over the first dimension's indices.
+constexpr uint32_t kLeadOuter = 16;
+
+struct LeadTiles {
+  uint32_t inner_rows;   // rows below one index of the first dimension
+  uint32_t rows;         // of them in a tile
+  uint32_t inner;        // tiles along them
+};
+
+__host__ __device__ __forceinline__ LeadTiles lead_tiles(uint32_t rows, uint32_t outer, uint32_t cols) {
+  LeadTiles l;
+  l.inner_rows = rows / outer;
+  const uint32_t most = 256u / cols;
+  l.inner = (l.inner_rows + most - 1u) / most;
+  l.rows = (l.inner_rows + l.inner - 1u) / l.inner;   // evenly
+  return l;
+}
+
+template <int GT, bool EXT>
+__global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1StatArgs args) {
+  constexpr int kAhead = 8;   // elements of a thread whose loads are in flight together
+  __shared__ uint32_t outer_bits[kThreads / 16][kLeadOuter];   // first dimension: each 16 lanes' maxima
+  __shared__ uint32_t slots[3][256];                           // second and third dimension, columns
+  const uint32_t chunk = args.chunk_base + blockIdx.x;
+  float gscale = 1.0f;
+  if (EXT && !grad_ops_begin(args.go, gscale)) return;
+  const int t = find_tensor(args, chunk);
+  const auto &T = args.desc[t];
+  const uint32_t tid = threadIdx.x, cols = T.cols, outer = T.lead_shape[0];
+  const LeadTiles L = lead_tiles(T.rows, outer, cols);
+  const uint32_t local = chunk - args.first_chunk[t], ot = local / L.inner, it = local - ot * L.inner;
+  const uint32_t o0 = ot * kLeadOuter, r0 = it * L.rows;
+  const uint32_t no = outer - o0 < kLeadOuter ? outer - o0 : kLeadOuter;
+  // the even split may leave its last tiles with fewer rows, or none
+  const uint32_t nr = r0 >= L.inner_rows ? 0u : L.inner_rows - r0 < L.rows ? L.inner_rows - r0 : L.rows;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) slots[k][tid] = 0u;
+
+  // this thread's element of the run, the same under every index of the first dimension
+  const uint32_t row = tid / cols, col = tid - row * cols;
+  const bool active = row < nr;
+  const int64_t below = (int64_t)L.inner_rows * cols;          // elements below one index
+  const int64_t first = (int64_t)o0 * below + (int64_t)r0 * cols;
+  float x_max = 0.0f;
+  const float c_old = active ? as_global<const float>(T.cmax)[col] : 0.0f;
+#pragma unroll
+  for (uint32_t base = 0; base < kLeadOuter; base += kAhead) {
+    float g[kAhead], r_old[kAhead];
+    uint32_t byte[kAhead];
+    if (base < no) {
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        // past the first dimension's end: its last index once more (maxima do not mind)
+        const uint32_t o = base + i < no ? base + i : no - 1u;
+        const int64_t e = first + (int64_t)o * below;          // uniform
+        g[i] = r_old[i] = 0.0f;
+        byte[i] = 0u;
+        if (active) {
+          g[i] = load_scalar<GT>(static_cast<const char *>(T.g) + e * (GT ? 2 : 4), tid);
+          byte[i] = as_global<const uint8_t>(T.v + (e >> 1))[(((uint32_t)e & 1u) + tid) >> 1];
+          r_old[i] = as_global<const float>(T.rmax)[(o0 + o) * L.inner_rows + r0 + row];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const uint32_t o = base + i < no ? base + i : no - 1u;
+        const uint32_t odd = (uint32_t)(first + (int64_t)o * below) & 1u;
+        const float gi = EXT ? g[i] * gscale : g[i];
+        const uint32_t code = (byte[i] >> (4u * ((tid + odd) & 1u))) & 15u;
+        const float code_value = __builtin_fmaf((float)code, 0.0625f, 0.0625f);  // (code + 1) / 16, exact
+        const float v_old = code_value * min_nonneg(r_old[i], c_old);
+        const float v = __builtin_fmaxf(args.b2 * v_old + args.r2 * (gi * gi), 0.0f);   // a NaN never becomes a maximum
+        x_max = __builtin_fmaxf(x_max, v);
+        const float quarter_max = row_max16(v);
+        if ((tid & 15u) == 0u) outer_bits[tid >> 4][base + i] = f2bits(quarter_max);
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t shape2 = T.lead_dims == 3u ? T.lead_shape[2] : 1u;
+  const uint32_t first1 = r0 / shape2;                          // the tile's first index of the second dimension
+  if (active && x_max != 0.0f) {
+    const uint32_t q = (r0 + row) / shape2;
+    atomicMax(&slots[0][q - first1], f2bits(x_max));
+    if (T.lead_dims == 3u) {
+      // the third dimension's indices of consecutive rows, folded into 256 slots: a tile has at
+      // most 128 rows, so rows that share a slot share the index
+      const uint32_t i2 = r0 + row - q * shape2;
+      atomicMax(&slots[1][shape2 <= 256u ? i2 : row], f2bits(x_max));
+    }
+    atomicMax(&slots[2][col], f2bits(x_max));
+  }
+  __syncthreads();
+  if (tid < no) {
+    uint32_t u = outer_bits[0][tid];
+#pragma unroll
+    for (int k = 1; k < kThreads / 16; ++k) u = u > outer_bits[k][tid] ? u : outer_bits[k][tid];
+    if (u != 0u) raise_max(T.lead_next[0] + o0 + tid, u);
+  }
+  if (slots[0][tid] != 0u) raise_max(T.lead_next[1] + first1 + tid, slots[0][tid]);
+  if (slots[1][tid] != 0u) raise_max(T.lead_next[2] + (shape2 <= 256u ? tid : (r0 + tid) % shape2), slots[1][tid]);
+  if (slots[2][tid] != 0u) raise_max(T.cmax_next + tid, slots[2][tid]);
+}
+
+// Tensors with several leading dimensions, between statistics and update: every row's new scale
+// is the minimum over its leading statistics.  A thread takes four consecutive rows a time: one
+// division per dimension for the first, the others by counting on.
+__global__ __launch_bounds__(256) void rank1_row_scale_kernel(const RowScaleArgs args) {
+  float gscale;
+  if (!grad_ops_begin(args.go, gscale)) return;
+  const int t = find_tensor(args, blockIdx.x);
+  const auto &T = args.desc[t];
+  const uint32_t row0 = (blockIdx.x - args.first_chunk[t]) * kRowScaleChunk;
+  const uint32_t n = T.rows - row0 < (uint32_t)kRowScaleChunk ? T.rows - row0 : (uint32_t)kRowScaleChunk;
+  const gptr<float> out = as_global<float>(T.row_next) + row0;
+  // the last two leading dimensions, and the first of three (or a dimension of one index)
+  const uint32_t d = T.lead_dims, s2 = T.lead_shape[d - 1], s1 = T.lead_shape[d - 2], s0 = d == 3u ? T.lead_shape[0] : 1u;
+  const gptr<const float> x2 = as_global<const float>(T.lead_next[d - 1]), x1 = as_global<const float>(T.lead_next[d - 2]);
+  const gptr<const float> x0 = as_global<const float>(d == 3u ? T.lead_next[0] : T.lead_next[d - 2]);
+#pragma unroll
+  for (int pass = 0; pass < kRowScaleChunk / 1024; ++pass) {
+    const uint32_t r = (uint32_t)pass * 1024u + threadIdx.x * 4u;
+    if (r >= n) return;
+    uint32_t q = row0 + r, i2, i1, i0;
+    i2 = q % s2; q /= s2;
+    i1 = q % s1; i0 = q / s1;
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v[k] = min_nonneg(x2[i2], x1[i1]);
+      if (d == 3u) v[k] = min_nonneg(v[k], x0[i0]);
+      if (++i2 == s2) {
+        i2 = 0u;
+        if (++i1 == s1) { i1 = 0u; i0 = i0 + 1u < s0 ? i0 + 1u : i0; }   // past the last row: stay in bounds
+      }
+    }
+    if (r + 4u <= n) {
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4{f2bits(v[0]), f2bits(v[1]), f2bits(v[2]), f2bits(v[3])},
+                                             tile_rsrc(T.row_next + row0), r * 4u, 0, 0);
+    } else {
+      for (uint32_t k = 0; r + k < n; ++k) out[r + k] = k == 0u ? v[0] : k == 1u ? v[1] : v[2];
+    }
+  }
 }
 
 // After the update: the new statistics become the current ones and the buffers that
-// received them go back to zero for the next step's maxima.  One workgroup column per
-// tensor (blockIdx.y), grid-stride over rows + cols floats.
-__global__ __launch_bounds__(256) void rank1_commit_kernel(const Rank1Args args) {
+// received them go back to zero for the next step's maxima.  A workgroup's chunk lies in one of
+// the tensor's vectors (rows, columns, leading dimensions); all its loads are in flight
+// together.
+__global__ __launch_bounds__(256) void rank1_commit_kernel(const CommitArgs args) {
+  constexpr int kPer = kCommitChunk / 256;
   float gscale;
   if (!grad_ops_begin(args.go, gscale)) return;
-  const Rank1Desc &T = args.desc[blockIdx.y];
-  const int64_t total = T.rows + T.cols;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
-    const bool is_row = i < T.rows;
-    const gptr<float> cur = as_global<float>(is_row ? T.rmax : T.cmax) + (is_row ? i : i - T.rows);
-    const gptr<float> next = as_global<float>(is_row ? T.rmax_next : T.cmax_next) + (is_row ? i : i - T.rows);
-    *cur = *next;
-    *next = 0.0f;
+  const int t = find_tensor(args, blockIdx.x);
+  const auto &T = args.desc[t];
+  uint32_t local = blockIdx.x - args.first_chunk[t];
+  int k = 0;
+  while (k < 4 && local >= (T.size[k] + kCommitChunk - 1) / kCommitChunk) {
+    local -= (T.size[k] + kCommitChunk - 1) / kCommitChunk;
+    ++k;
   }
-}
-
-// Tensors with several leading dimensions, between statistics and update: row -> its
-// index in leading dimension j (row-major).
-__device__ __forceinline__ int64_t lead_index(const FoldDesc &T, int64_t row, int j) {
-  int64_t stride = 1;
-  for (int k = T.dims - 1; k > j; --k) stride *= T.shape[k];
-  return (row / stride) % T.shape[j];
-}
-
-// mode 0: every leading dimension's new statistic = maximum over the rows that share the index
-// mode 1: every row's new scale = minimum over its leading statistics (after mode 0 is complete)
-// mode 2: after the update, new statistics become current, their buffers return to zero
-// One workgroup column per tensor (blockIdx.y), grid-stride over its rows.
-template <int MODE>
-__global__ __launch_bounds__(256) void rank1_fold_kernel(const FoldArgs args) {
-  float gscale;
-  if (!grad_ops_begin(args.go, gscale)) return;
-  const FoldDesc &T = args.desc[blockIdx.y];
-  const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
-  if (MODE == 2) {
-    for (int j = 0; j < T.dims; ++j) {
-      for (int64_t i = first; i < T.shape[j]; i += stride) {
-        as_global<float>(T.cur[j])[i] = as_global<float>(T.next[j])[i];
-        as_global<float>(T.next[j])[i] = 0.0f;
-      }
-    }
-    return;
-  }
-  for (int64_t row = first; row < T.rows; row += stride) {
-    if (MODE == 0) {
-      const float r = as_global<const float>(T.row_next)[row];
-      if (r != 0.0f) {
-        for (int j = 0; j < T.dims; ++j) atomic_max_nonneg(T.next[j] + lead_index(T, row, j), r);
-      }
-    } else {
-      float s = as_global<const float>(T.next[0])[lead_index(T, row, 0)];
-      for (int j = 1; j < T.dims; ++j) s = min_nonneg(s, as_global<const float>(T.next[j])[lead_index(T, row, j)]);
-      as_global<float>(T.row_next)[row] = s;
+  const uint32_t i0 = local * kCommitChunk + threadIdx.x, size = T.size[k];
+  const gptr<float> cur = as_global<float>(T.cur[k]), next = as_global<float>(T.next[k]);
+  float x[kPer];
+#pragma unroll
+  for (int h = 0; h < kPer; ++h) x[h] = i0 + h * 256u < size ? next[i0 + h * 256u] : 0.0f;
+#pragma unroll
+  for (int h = 0; h < kPer; ++h) {
+    if (i0 + h * 256u < size) {
+      cur[i0 + h * 256u] = x[h];
+      next[i0 + h * 256u] = 0.0f;
     }
   }
 }
