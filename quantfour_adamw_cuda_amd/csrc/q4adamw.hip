@@ -234,7 +234,9 @@ static Rank1StatForm rank1_stat_form(const q4adamw_rank1_tensor &t) {
 template <int GT, bool EXT>
 static Rank1StatKernel pick_rank1_stats_form(Rank1StatForm form) {
   if (form == kStatFlat) return rank1_stats_flat_kernel<GT, EXT>;
-  if (form == kStatLead) return rank1_stats_lead_kernel<GT, EXT>;
+  if constexpr (GT != kAbsValues) {
+    if (form == kStatLead) return rank1_stats_lead_kernel<GT, EXT>;
+  }
   return form == kStatWide ? rank1_stats_kernel<GT, EXT, false> : rank1_stats_kernel<GT, EXT, true>;
 }
 
@@ -933,13 +935,13 @@ int q4adamw_quantize(const float *x, int64_t numel, int which, uint8_t *codes, f
   if (numel == 0) return 0;
   if (!x || !codes || !scales) return fail(Q4ADAMW_ERR_ARG, "null tensor pointer");
   if (!aligned(x, 4) || !aligned(scales, 4)) return fail(Q4ADAMW_ERR_ALIGN, "fp32 buffers must be 4-byte aligned");
-  const uint64_t blocks = ((uint64_t)numel + Q4ADAMW_BLOCK - 1) / Q4ADAMW_BLOCK;
-  const uint64_t groups = (blocks + 3) / 4;
+  const uint64_t groups = ((uint64_t)numel + kEncodeChunk - 1) / kEncodeChunk;
+  const bool even = aligned(codes, 2);
   if (numel > kMaxInterchangeElements) return fail(Q4ADAMW_ERR_TOO_LARGE, "more than 2^40 elements");
   hipStream_t s = static_cast<hipStream_t>(stream);
   return for_each_grid(groups, 256, [&](uint64_t base, uint64_t count) -> int {
-    if (which) hipLaunchKernelGGL(quantize_kernel<true>, dim3((unsigned)count), dim3(256), 0, s, x, numel, codes, scales, (int64_t)base);
-    else hipLaunchKernelGGL(quantize_kernel<false>, dim3((unsigned)count), dim3(256), 0, s, x, numel, codes, scales, (int64_t)base);
+    if (which) hipLaunchKernelGGL(quantize_kernel<true>, dim3((unsigned)count), dim3(256), 0, s, x, numel, codes, scales, (int64_t)base, even);
+    else hipLaunchKernelGGL(quantize_kernel<false>, dim3((unsigned)count), dim3(256), 0, s, x, numel, codes, scales, (int64_t)base, even);
     Q4_HIP(hipGetLastError());
     return 0;
   });
@@ -952,6 +954,19 @@ static int check_rank1_shape(int64_t rows, int64_t cols) {
   return 0;
 }
 
+static int launch_quantize_rank1(const float *x, int64_t rows, int64_t cols, uint8_t *codes, const float *row_max,
+                                 const float *col_max, hipStream_t s) {
+  const uint64_t numel = (uint64_t)rows * (uint64_t)cols;
+  const bool big = numel > 0xffffffffull || cols < 2, even = aligned(codes, 2);
+  const FastDiv div = big ? FastDiv{0u, 0u} : make_fast_div((uint32_t)cols);
+  return for_each_grid((numel + kEncodeChunk - 1) / kEncodeChunk, kThreads, [&](uint64_t base, uint64_t count) -> int {
+    hipLaunchKernelGGL(big ? quantize_rank1_kernel<true> : quantize_rank1_kernel<false>, dim3((unsigned)count),
+                       dim3(kThreads), 0, s, x, rows, cols, div, row_max, col_max, codes, (int64_t)base, even);
+    Q4_HIP(hipGetLastError());
+    return 0;
+  });
+}
+
 int q4adamw_quantize_rank1(const float *x, int64_t rows, int64_t cols, uint8_t *codes,
                            float *row_max, float *col_max, void *stream) {
   if (int rc = check_rank1_shape(rows, cols)) return rc;
@@ -959,19 +974,30 @@ int q4adamw_quantize_rank1(const float *x, int64_t rows, int64_t cols, uint8_t *
   if (!x || !codes || !row_max || !col_max) return fail(Q4ADAMW_ERR_ARG, "null tensor pointer");
   if (!aligned(x, 4) || !aligned(row_max, 4) || !aligned(col_max, 4))
     return fail(Q4ADAMW_ERR_ALIGN, "fp32 buffers must be 4-byte aligned");
-  const dim3 tiles((unsigned)((cols + 255) / 256), (unsigned)((rows + 63) / 64));
-  if (tiles.y > 65535u) return fail(Q4ADAMW_ERR_TOO_LARGE, "more than 4194240 rows");
+  if (rows > 4194240) return fail(Q4ADAMW_ERR_TOO_LARGE, "more than 4194240 rows");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(fill_zero_kernel, dim3(64), dim3(256), 0, s, row_max, rows);
-  hipLaunchKernelGGL(fill_zero_kernel, dim3(64), dim3(256), 0, s, col_max, cols);
-  hipLaunchKernelGGL(rank1_absmax_kernel, tiles, dim3(256), 0, s, x, rows, cols, row_max, col_max);
-  const uint64_t groups = (((uint64_t)rows * cols + 1) / 2 + 255) / 256;
-  return for_each_grid(groups, 256, [&](uint64_t base, uint64_t count) -> int {
-    hipLaunchKernelGGL(quantize_rank1_kernel, dim3((unsigned)count), dim3(256), 0, s, x, rows, cols,
-                       static_cast<const float *>(row_max), static_cast<const float *>(col_max), codes, (int64_t)base);
-    Q4_HIP(hipGetLastError());
-    return 0;
-  });
+  q4adamw_rank1_tensor t = {};
+  t.rows = rows;
+  t.cols = cols;
+  Rank1StatArgs sa = {};
+  const Rank1StatForm form = rank1_stat_form(t);
+  sa.stat_rows = rank1_stat_rows((uint64_t)rows * (uint64_t)cols);
+  sa.desc[0].g = x;
+  sa.desc[0].rmax_next = row_max;
+  sa.desc[0].cmax_next = col_max;
+  sa.desc[0].rows = (uint32_t)rows;
+  sa.desc[0].cols = (uint32_t)cols;
+  finish_prefix(sa, 1);
+  hipLaunchKernelGGL(fill_zero_kernel, dim3(64), dim3(256), 0, s, row_max, rows, col_max, cols);
+  const Rank1StatKernel kernel = pick_rank1_stats_form<kAbsValues, false>(form);
+  if (int rc = for_each_grid(rank1_stat_chunks(t, sa.stat_rows), kThreads, [&](uint64_t base, uint64_t count) -> int {
+        sa.chunk_base = (uint32_t)base;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(kThreads), 0, s, sa);
+        Q4_HIP(hipGetLastError());
+        return 0;
+      }))
+    return rc;
+  return launch_quantize_rank1(x, rows, cols, codes, row_max, col_max, s);
 }
 
 int q4adamw_quantize_rank1_scaled(const float *x, int64_t rows, int64_t cols, const float *row_scale,
@@ -981,13 +1007,7 @@ int q4adamw_quantize_rank1_scaled(const float *x, int64_t rows, int64_t cols, co
   if (!x || !codes || !row_scale || !col_max) return fail(Q4ADAMW_ERR_ARG, "null tensor pointer");
   if (!aligned(x, 4) || !aligned(row_scale, 4) || !aligned(col_max, 4))
     return fail(Q4ADAMW_ERR_ALIGN, "fp32 buffers must be 4-byte aligned");
-  const uint64_t groups = (((uint64_t)rows * cols + 1) / 2 + 255) / 256;
-  return for_each_grid(groups, 256, [&](uint64_t base, uint64_t count) -> int {
-    hipLaunchKernelGGL(quantize_rank1_kernel, dim3((unsigned)count), dim3(256), 0, static_cast<hipStream_t>(stream), x,
-                       rows, cols, row_scale, col_max, codes, (int64_t)base);
-    Q4_HIP(hipGetLastError());
-    return 0;
-  });
+  return launch_quantize_rank1(x, rows, cols, codes, row_scale, col_max, static_cast<hipStream_t>(stream));
 }
 
 int q4adamw_dequantize_rank1(const uint8_t *codes, const float *row_max, const float *col_max,
@@ -997,10 +1017,13 @@ int q4adamw_dequantize_rank1(const uint8_t *codes, const float *row_max, const f
   if (!codes || !row_max || !col_max || !out) return fail(Q4ADAMW_ERR_ARG, "null tensor pointer");
   if (!aligned(out, 4) || !aligned(row_max, 4) || !aligned(col_max, 4))
     return fail(Q4ADAMW_ERR_ALIGN, "fp32 buffers must be 4-byte aligned");
-  const uint64_t groups = (((uint64_t)rows * cols + 1) / 2 + 255) / 256;
-  return for_each_grid(groups, 256, [&](uint64_t base, uint64_t count) -> int {
-    hipLaunchKernelGGL(dequantize_rank1_kernel, dim3((unsigned)count), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), codes, row_max, col_max, rows, cols, out, (int64_t)base);
+  const uint64_t numel = (uint64_t)rows * (uint64_t)cols;
+  const bool big = numel > 0xffffffffull || cols < 2, even = aligned(codes, 2);
+  const FastDiv div = big ? FastDiv{0u, 0u} : make_fast_div((uint32_t)cols);
+  return for_each_grid((numel + kDecodeChunk - 1) / kDecodeChunk, kThreads, [&](uint64_t base, uint64_t count) -> int {
+    hipLaunchKernelGGL(big ? dequantize_rank1_kernel<true> : dequantize_rank1_kernel<false>, dim3((unsigned)count),
+                       dim3(kThreads), 0, static_cast<hipStream_t>(stream), codes, row_max, col_max, rows, cols, div, out,
+                       (int64_t)base, even);
     Q4_HIP(hipGetLastError());
     return 0;
   });
@@ -1012,12 +1035,13 @@ int q4adamw_dequantize(const uint8_t *codes, const float *scales, int64_t numel,
   if (numel == 0) return 0;
   if (!out || !codes || !scales) return fail(Q4ADAMW_ERR_ARG, "null tensor pointer");
   if (!aligned(out, 4) || !aligned(scales, 4)) return fail(Q4ADAMW_ERR_ALIGN, "fp32 buffers must be 4-byte aligned");
-  const uint64_t groups = (((uint64_t)numel + 1) / 2 + 255) / 256;
+  const uint64_t groups = ((uint64_t)numel + kDecodeChunk - 1) / kDecodeChunk;
+  const bool even = aligned(codes, 2);
   if (numel > kMaxInterchangeElements) return fail(Q4ADAMW_ERR_TOO_LARGE, "more than 2^40 elements");
   hipStream_t s = static_cast<hipStream_t>(stream);
   return for_each_grid(groups, 256, [&](uint64_t base, uint64_t count) -> int {
-    if (which) hipLaunchKernelGGL(dequantize_kernel<true>, dim3((unsigned)count), dim3(256), 0, s, codes, scales, numel, out, (int64_t)base);
-    else hipLaunchKernelGGL(dequantize_kernel<false>, dim3((unsigned)count), dim3(256), 0, s, codes, scales, numel, out, (int64_t)base);
+    if (which) hipLaunchKernelGGL(dequantize_kernel<true>, dim3((unsigned)count), dim3(256), 0, s, codes, scales, numel, out, (int64_t)base, even);
+    else hipLaunchKernelGGL(dequantize_kernel<false>, dim3((unsigned)count), dim3(256), 0, s, codes, scales, numel, out, (int64_t)base, even);
     Q4_HIP(hipGetLastError());
     return 0;
   });

@@ -231,136 +231,289 @@ __global__ __launch_bounds__(256) void grad_norm_finish_kernel(const double *par
 }
 
 // ---------------------------------------------------------------------------
-// stand-alone quantize / dequantize of one moment (checkpoint interchange)
+// stand-alone quantize / dequantize of moments (checkpoint interchange)
 // ---------------------------------------------------------------------------
-// One wave per 128-element block, two elements (one packed byte) per lane.  These run
-// once per checkpoint, so they take the exact route only: IEEE division and the
-// 15-compare count (optim/adamw_fourbit_triton.py:618-630, cuda_adamw_kernels.cu:167-194).
+// fp32 on one side and 4-bit codes on the other: 4.03 bytes per element one way and 0.5 the
+// other, so these are streams, bound by HBM.  A wave takes two (encoding) or four (decoding)
+// tiles of 256 consecutive elements, a lane four elements of each: one 16-byte access on the
+// fp32 side and one 2-byte access on the codes' per tile, all tiles' loads in flight together.
+// Tiles per wave measured on 14336 x 4096 elements, first / second moment, us: encoding one
+// 53 / 51, two 41.8 / 40.0, four 42.2 / 42.6, eight 44.0 / 44.4; decoding one 64 / 53, two
+// 49 / 46, four 45.8 / 44.0, eight 48.6 / 49.6.
+constexpr int kEncodeTiles = 2, kDecodeTiles = 4;
+constexpr int64_t kEncodeChunk = 256 * kEncodeTiles * kWaves, kDecodeChunk = 256 * kDecodeTiles * kWaves;   // elements per workgroup
+
+__device__ __forceinline__ int wave_number() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+
+// Four consecutive elements from e on (e a multiple of 4) of x, and how many of them exist.
+__device__ __forceinline__ int load_four(const float *x, int64_t e, int64_t numel, float (&v)[4]) {
+  const int64_t rem = numel - e;
+  if (rem >= 4) {
+    const f32x4 w = __builtin_nontemporal_load((gptr<const f32x4u>)(uintptr_t)(x + e));
+    v[0] = w.x; v[1] = w.y; v[2] = w.z; v[3] = w.w;
+    return 4;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = j < rem ? as_global<const float>(x)[e + j] : 0.0f;
+  return rem > 0 ? (int)rem : 0;
+}
+
+// The codes of n of four elements from e on, a nibble each.
+__device__ __forceinline__ void store_four_codes(uint8_t *codes, int64_t e, int n, uint32_t word, bool even) {
+  const gptr<uint8_t> out = as_global<uint8_t>(codes) + (e >> 1);
+  if (n == 4 && even) {
+    __builtin_nontemporal_store((uint16_t)word, (gptr<uint16_t>)(uintptr_t)(codes + (e >> 1)));
+    return;
+  }
+  word &= (1u << (4 * n)) - 1u;          // an odd element count: the last byte's high nibble stays 0
+  if (n > 0) out[0] = (uint8_t)word;
+  if (n > 2) out[1] = (uint8_t)(word >> 8);
+}
+
+__device__ __forceinline__ uint32_t load_four_codes(const uint8_t *codes, int64_t e, int64_t numel, bool even) {
+  const int64_t rem = numel - e;
+  if (rem >= 4 && even) return __builtin_nontemporal_load((gptr<const uint16_t>)(uintptr_t)(codes + (e >> 1)));
+  uint32_t word = 0;
+  if (rem > 0) word = as_global<const uint8_t>(codes)[e >> 1];
+  if (rem > 2) word |= (uint32_t)as_global<const uint8_t>(codes)[(e >> 1) + 1] << 8;
+  return word;
+}
+
+// v to the four elements of the lane in the tile (uniform) at tile0.  The streamed stores' policy
+// (kNt) measures 2 to 4 % faster here than the non-temporal hint alone.
+__device__ __forceinline__ void store_four(float *out, int64_t tile0, int64_t numel, const float (&v)[4]) {
+  const uint32_t lane4 = (threadIdx.x & 63u) * 4u;
+  const int64_t e = tile0 + lane4, rem = numel - e;
+  if (rem >= 4) {
+    store_b128<kNt>(u32x4{f2bits(v[0]), f2bits(v[1]), f2bits(v[2]), f2bits(v[3])}, out + tile0, lane4 * 4u);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    if (j < rem) as_global<float>(out)[e + j] = v[j];
+  }
+}
+
+// Second moment: the codes of four values under scales whose 16 / scale are inv16; the step's fast path
+// (q4adamw_step.h) for values of either sign.  near: raised where a quotient is within the guard
+// band of a threshold.
+__device__ __forceinline__ uint32_t fast_codes_v(const float (&x)[4], const float (&inv16)[4], float &near) {
+  uint32_t word = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float t = __builtin_fmaxf(__builtin_fmaf(x[j], inv16[j], kVGuard - 0.5f), 0.0f);   // a NaN: code 0
+    t = __builtin_fminf(t, 15.5f);         // scales may be given, and smaller than the values
+    near = __builtin_fminf(near, t == 0.0f ? 1.0f : __builtin_amdgcn_fractf(t));
+    word |= (uint32_t)(int)t << (4 * j);
+  }
+  return word;
+}
+
+// Per-128 abs-max and nearest codes (optim/adamw_fourbit_triton.py:618-630,
+// cuda_adamw_kernels.cu:167-194).  The quotients are the step kernel's: a refined reciprocal, the
+// half-indexed bucket table for the first moment, one multiply-add for the second; blocks
+// whose scale is out of range and values within the guard band of a threshold take IEEE
+// division and the 15-compare count.  even: codes starts at an even address.
+// 14336 x 4096 elements: 123 us (one wave per block, 8 bytes per lane, every quotient divided)
+// -> 41 us = 6.5 TB/s.
 template <bool SECOND>
-__global__ __launch_bounds__(256) void quantize_kernel(const float *__restrict__ x_, int64_t numel,
-                                                       uint8_t *__restrict__ codes_,
-                                                       float *__restrict__ scale_, int64_t group0) {
-  const gptr<const float> x = as_global<const float>(x_);
-  const int lane = threadIdx.x & 63;
-  const int64_t blk = (group0 + blockIdx.x) * 4 + (threadIdx.x >> 6);   // group0: this grid's first workgroup
-  const int64_t nblk = (numel + Q4ADAMW_BLOCK - 1) / Q4ADAMW_BLOCK;
-  if (blk >= nblk) return;
-  const int64_t e = blk * Q4ADAMW_BLOCK + lane * 2;
-  const float a = e < numel ? x[e] : 0.0f;
-  const float b = e + 1 < numel ? x[e + 1] : 0.0f;
-  // fmaxf drops a NaN next to a number; two NaN count as 0: a NaN never becomes the scale
-  const float lane_max = __builtin_fmaxf(__builtin_fabsf(a), __builtin_fabsf(b));
-  uint32_t u = lane_max == lane_max ? f2bits(lane_max) : 0u;
+__global__ __launch_bounds__(kThreads) void quantize_kernel(const float *__restrict__ x_, int64_t numel,
+                                                            uint8_t *__restrict__ codes_,
+                                                            float *__restrict__ scale_, int64_t group0, bool even) {
+  __shared__ uint2 table[SECOND ? 1 : kHalfTableEntries];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t wave0 = ((group0 + blockIdx.x) * kWaves + wave_number()) * (256 * kEncodeTiles);
+  float x[kEncodeTiles][4];
+  int n[kEncodeTiles];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const uint32_t o = (uint32_t)__shfl_xor((int)u, off, 64);
-    u = u > o ? u : o;
+  for (int k = 0; k < kEncodeTiles; ++k) n[k] = load_four(x_, wave0 + k * 256 + lane * 4, numel, x[k]);
+  if (!SECOND) {
+    const MtabEntry e = kHalfTable.e[tid];
+    table[tid] = make_uint2(e.lo, e.hi);
+    __syncthreads();
   }
-  const float s = bits2f(u);
-  if (lane == 0) as_global<float>(scale_)[blk] = s;
-  if (e < numel) {
-    uint32_t byte = 0;
-    const float q0 = a / s, q1 = b / s;
 #pragma unroll
-    for (int k = 0; k < 15; ++k) {
-      const float t = SECOND ? qmid_v(k) : bits2f(kQmidMBits[k]);
-      byte += (t < q0) ? 1u : 0u;
-      byte += (e + 1 < numel && t < q1) ? 16u : 0u;
+  for (int k = 0; k < kEncodeTiles; ++k) {
+    const int64_t e = wave0 + k * 256 + lane * 4;
+    // fmaxf drops a NaN next to a number; from 0 on a NaN never becomes the scale
+    float am = 0.0f, unused = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) am = __builtin_fmaxf(am, __builtin_fabsf(x[k][j]));
+    block_max32_pair(am, unused);
+    if (n[k] > 0 && (lane & 31) == 0) as_global<float>(scale_)[e / Q4ADAMW_BLOCK] = am;
+    const bool safe = am >= kScaleLo && am <= kScaleHi;
+    const float r = safe ? refined_rcp(am) : 0.0f;
+    bool redo = !safe && am != 0.0f;
+    uint32_t word = 0;
+    if (SECOND) {
+      const float inv = r * 16.0f, inv16[4] = {inv, inv, inv, inv};
+      float near = 1.0f;
+      word = fast_codes_v(x[k], inv16, near);
+      redo |= near < 2.0f * kVGuard;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        const float q0 = x[k][j] * r, q1 = x[k][j + 1] * r;
+        const uint32_t halves = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(q0, q1));
+        const uint2 e0 = table[(halves >> 8) & 255u], e1 = table[halves >> 24];
+        const bool hi0 = q0 > bits2f(e0.y), hi1 = q1 > bits2f(e1.y);
+        redo |= hi0 != (q0 > bits2f(e0.x));
+        redo |= hi1 != (q1 > bits2f(e1.x));
+        word = __builtin_amdgcn_alignbit(e0.x + (hi0 ? 1u : 0u), word, 4);
+        word = __builtin_amdgcn_alignbit(e1.x + (hi1 ? 1u : 0u), word, 4);
+      }
+      word >>= 16;
     }
-    as_global<uint8_t>(codes_)[e >> 1] = (uint8_t)byte;
-  }
-}
-
-// Rank-1 forms for the second moment of a rows x cols matrix (run once per
-// checkpoint).  Statistics: a workgroup takes 64 rows x 256 columns, a thread one
-// column; row maxima meet in LDS, then one atomic per row and per column.
-__global__ __launch_bounds__(256) void fill_zero_kernel(float *x_, int64_t n) {
-  const gptr<float> x = as_global<float>(x_);
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) x[i] = 0.0f;
-}
-
-__global__ __launch_bounds__(256) void rank1_absmax_kernel(const float *x_, int64_t rows, int64_t cols,
-                                                           float *row_max, float *col_max) {
-  __shared__ uint32_t row_bits[64];
-  const gptr<const float> x = as_global<const float>(x_);
-  const int tid = threadIdx.x;
-  const int64_t col = (int64_t)blockIdx.x * 256 + tid;
-  const int64_t row0 = (int64_t)blockIdx.y * 64;
-  const int nrows = (int)(row0 + 64 < rows ? 64 : rows - row0);
-  if (tid < 64) row_bits[tid] = 0u;
-  __syncthreads();
-  float c_max = 0.0f;
-  for (int r = 0; r < nrows; ++r) {
-    float a = col < cols ? __builtin_fabsf(x[(row0 + r) * cols + col]) : 0.0f;
-    a = a == a ? a : 0.0f;  // a NaN never becomes a maximum
-    c_max = __builtin_fmaxf(c_max, a);
-    uint32_t u = f2bits(a);
+    if (__builtin_expect(redo, 0)) {
+      Vals<4> v;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const uint32_t o = (uint32_t)__shfl_xor((int)u, off, 64);
-      u = u > o ? u : o;
+      for (int j = 0; j < 4; ++j) v.x[j] = x[k][j];
+      word = quantize_exact<SECOND, 4>(v, am);
     }
-    if ((tid & 63) == 0 && u != 0u) atomicMax(&row_bits[r], u);
-  }
-  if (col < cols && c_max != 0.0f) atomic_max_nonneg(col_max + col, c_max);
-  __syncthreads();
-  if (tid < nrows && row_bits[tid] != 0u) atomic_max_nonneg(row_max + row0 + tid, bits2f(row_bits[tid]));
-}
-
-// one thread per packed byte: x / min(row maximum, column maximum), IEEE division, the
-// 15-compare count (optim/adamw_fourbit_triton.py:834-863).  Rows may have any length, so the
-// byte's two elements find their rows and columns separately.
-__global__ __launch_bounds__(256) void quantize_rank1_kernel(const float *x_, int64_t rows, int64_t cols,
-                                                             const float *row_max, const float *col_max,
-                                                             uint8_t *codes_, int64_t group0) {
-  const int64_t e = ((group0 + blockIdx.x) * 256 + threadIdx.x) * 2;
-  const int64_t numel = rows * cols;
-  if (e >= numel) return;
-  uint32_t byte = 0;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    if (e + h >= numel) break;     // an odd element count: the last byte's high nibble stays 0
-    const int64_t i = (e + h) / cols, j = (e + h) - i * cols;
-    const float q = as_global<const float>(x_)[e + h] /
-                    __builtin_fminf(as_global<const float>(row_max)[i], as_global<const float>(col_max)[j]);
-#pragma unroll
-    for (int k = 0; k < 15; ++k) byte += (qmid_v(k) < q) ? (1u << (4 * h)) : 0u;
-  }
-  as_global<uint8_t>(codes_)[e >> 1] = (uint8_t)byte;
-}
-
-// optim/adamw_fourbit_triton.py:520-527: code-book entry times min(row, column maximum)
-__global__ __launch_bounds__(256) void dequantize_rank1_kernel(const uint8_t *codes_, const float *row_max,
-                                                               const float *col_max, int64_t rows,
-                                                               int64_t cols, float *out_, int64_t group0) {
-  const int64_t e = ((group0 + blockIdx.x) * 256 + threadIdx.x) * 2;
-  const int64_t numel = rows * cols;
-  if (e >= numel) return;
-  const uint32_t byte = as_global<const uint8_t>(codes_)[e >> 1];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    if (e + h >= numel) break;
-    const int64_t i = (e + h) / cols, j = (e + h) - i * cols;
-    as_global<float>(out_)[e + h] = qmap_v((int)((byte >> (4 * h)) & 15u)) *
-                                    __builtin_fminf(as_global<const float>(row_max)[i], as_global<const float>(col_max)[j]);
+    if (am == 0.0f) word = 0;     // 0/0: code 0 for the whole block
+    store_four_codes(codes_, e, n[k], word, even);
   }
 }
 
 // cuda_adamw_kernels.cu:329-343: code -> code-book entry * block scale
+// 14336 x 4096 elements: 116 us for a first, 87 us for a second moment (one byte of codes per
+// thread) -> 43 us = 6.1 TB/s.
 template <bool SECOND>
-__global__ __launch_bounds__(256) void dequantize_kernel(const uint8_t *__restrict__ codes_,
-                                                         const float *__restrict__ scale_,
-                                                         int64_t numel, float *__restrict__ out_, int64_t group0) {
-  const int64_t e = ((group0 + blockIdx.x) * 256 + threadIdx.x) * 2;
-  if (e >= numel) return;
-  const uint32_t byte = as_global<const uint8_t>(codes_)[e >> 1];
-  const float s = as_global<const float>(scale_)[e / Q4ADAMW_BLOCK];
-  const uint32_t c0 = byte & 15u, c1 = byte >> 4;
-  const float v0 = (SECOND ? qmap_v((int)c0) : bits2f(kQmapMDev[c0])) * s;
-  as_global<float>(out_)[e] = v0;
-  if (e + 1 < numel) {
-    const float v1 = (SECOND ? qmap_v((int)c1) : bits2f(kQmapMDev[c1])) * s;
-    as_global<float>(out_)[e + 1] = v1;
+__global__ __launch_bounds__(kThreads) void dequantize_kernel(const uint8_t *__restrict__ codes_,
+                                                              const float *__restrict__ scale_,
+                                                              int64_t numel, float *__restrict__ out_, int64_t group0,
+                                                              bool even) {
+  __shared__ float book[16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t wave0 = ((group0 + blockIdx.x) * kWaves + wave_number()) * (256 * kDecodeTiles);
+  uint32_t word[kDecodeTiles];
+  float s[kDecodeTiles];
+#pragma unroll
+  for (int k = 0; k < kDecodeTiles; ++k) {
+    const int64_t e = wave0 + k * 256 + lane * 4;
+    word[k] = load_four_codes(codes_, e, numel, even);
+    s[k] = e < numel ? as_global<const float>(scale_)[e / Q4ADAMW_BLOCK] : 0.0f;
+  }
+  if (!SECOND) {
+    if (tid < 16) book[tid] = bits2f(kQmapMDev[tid]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < kDecodeTiles; ++k) {
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t c = (word[k] >> (4 * j)) & 15u;
+      v[j] = (SECOND ? qmap_v((int)c) : book[c]) * s[k];
+    }
+    store_four(out_, wave0 + k * 256, numel, v);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// rank-1 forms for the second moment of a rows x cols matrix
+// ---------------------------------------------------------------------------
+// Zeros over two vectors (a matrix's row and column maxima before their statistics launch).
+__global__ __launch_bounds__(256) void fill_zero_kernel(float *x_, int64_t nx, float *y_, int64_t ny) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nx + ny; i += (int64_t)gridDim.x * 256) {
+    if (i < nx) as_global<float>(x_)[i] = 0.0f;
+    else as_global<float>(y_)[i - nx] = 0.0f;
+  }
+}
+
+// The scales min(row maximum, column maximum) of four consecutive elements from e on (those
+// past the matrix's end get the last row's).  div: by cols, where the matrix has fewer than
+// 2^32 elements and two columns or more (BIG, everything else: a 64-bit division, one per lane).
+template <bool BIG>
+__device__ __forceinline__ void four_scales(int64_t e, int64_t rows, int64_t cols, FastDiv div, const float *row_max,
+                                            const float *col_max, float (&s)[4]) {
+  const gptr<const float> rm = as_global<const float>(row_max), cm = as_global<const float>(col_max);
+  int64_t i, j;
+  if (BIG) {
+    i = e / cols;
+    j = e - i * cols;
+  } else {
+    const uint32_t q = fast_div((uint32_t)e, div.magic, div.shift);
+    i = q;
+    j = (uint32_t)e - q * (uint32_t)cols;
+  }
+  if (j + 4 <= cols) {
+    const float r = rm[i];
+    const f32x4 c = *(gptr<const f32x4u>)(uintptr_t)(col_max + j);
+    s[0] = min_nonneg(r, c.x); s[1] = min_nonneg(r, c.y); s[2] = min_nonneg(r, c.z); s[3] = min_nonneg(r, c.w);
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    s[k] = min_nonneg(rm[i], cm[j]);
+    if (++j == cols) {
+      j = 0;
+      i = i + 1 < rows ? i + 1 : i;
+    }
+  }
+}
+
+// x / min(row maximum, column maximum), nearest code (optim/adamw_fourbit_triton.py:834-863).
+// As quantize_kernel, the scales from the (cached) statistics; an element whose scale is out of
+// the reciprocal's range sends its lane to the exact path unless it is a zero (code 0 both ways).
+template <bool BIG>
+__global__ __launch_bounds__(kThreads) void quantize_rank1_kernel(const float *x_, int64_t rows, int64_t cols, FastDiv div,
+                                                                  const float *row_max, const float *col_max,
+                                                                  uint8_t *codes_, int64_t group0, bool even) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t numel = rows * cols;
+  const int64_t wave0 = ((group0 + blockIdx.x) * kWaves + wave_number()) * (256 * kEncodeTiles);
+  float x[kEncodeTiles][4];
+  int n[kEncodeTiles];
+#pragma unroll
+  for (int k = 0; k < kEncodeTiles; ++k) n[k] = load_four(x_, wave0 + k * 256 + lane * 4, numel, x[k]);
+#pragma unroll
+  for (int k = 0; k < kEncodeTiles; ++k) {
+    const int64_t e = wave0 + k * 256 + lane * 4;
+    if (e >= numel) return;
+    float s[4], inv16[4], near = 1.0f;
+    four_scales<BIG>(e, rows, cols, div, row_max, col_max, s);
+    bool redo = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      redo |= !(s[j] >= kScaleLo && s[j] <= kScaleHi) && x[k][j] != 0.0f;
+      inv16[j] = refined_rcp(max_nonneg(s[j], kScaleLo)) * 16.0f;
+    }
+    uint32_t word = fast_codes_v(x[k], inv16, near);
+    redo |= near < 2.0f * kVGuard;
+    if (__builtin_expect(redo, 0)) {
+      Vals<4> v, sc;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v.x[j] = x[k][j];
+        sc.x[j] = s[j];
+      }
+      word = quantize_exact_scales<4>(v, sc);
+    }
+    store_four_codes(codes_, e, n[k], word, even);
+  }
+}
+
+// optim/adamw_fourbit_triton.py:520-527: code-book entry times min(row, column maximum)
+template <bool BIG>
+__global__ __launch_bounds__(kThreads) void dequantize_rank1_kernel(const uint8_t *codes_, const float *row_max,
+                                                                    const float *col_max, int64_t rows, int64_t cols,
+                                                                    FastDiv div, float *out_, int64_t group0, bool even) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t numel = rows * cols;
+  const int64_t wave0 = ((group0 + blockIdx.x) * kWaves + wave_number()) * (256 * kDecodeTiles);
+  uint32_t word[kDecodeTiles];
+#pragma unroll
+  for (int k = 0; k < kDecodeTiles; ++k) word[k] = load_four_codes(codes_, wave0 + k * 256 + lane * 4, numel, even);
+#pragma unroll
+  for (int k = 0; k < kDecodeTiles; ++k) {
+    const int64_t e = wave0 + k * 256 + lane * 4;
+    if (e >= numel) return;
+    float s[4], v[4];
+    four_scales<BIG>(e, rows, cols, div, row_max, col_max, s);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = qmap_v((int)((word[k] >> (4 * j)) & 15u)) * s[j];
+    store_four(out_, wave0 + k * 256, numel, v);
   }
 }
 

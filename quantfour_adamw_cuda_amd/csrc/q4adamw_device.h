@@ -17,6 +17,7 @@ using gptr = __attribute__((address_space(1))) T *;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4u __attribute__((aligned(4)));   // in memory, at any element's address
 
 template <typename T>
 __device__ __forceinline__ gptr<T> as_global(const void *p) {

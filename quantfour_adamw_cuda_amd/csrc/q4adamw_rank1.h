@@ -64,6 +64,10 @@ __device__ __forceinline__ void fold_rows(const Desc &T, uint32_t row0, uint32_t
   }
 }
 
+// GT = kAbsValues: the statistics of |g| itself (fp32, no codes): what the checkpoint quantizer
+// needs of a second moment it is handed.
+constexpr int kAbsValues = 3;
+
 constexpr int kStatRowsPerWave = 64;     // rows a wave walks, at most
 constexpr int kStatRows = kStatRowsPerWave * kWaves;   // rows per workgroup of the statistics kernel, at most
 constexpr int kStatCols = 512;           // columns per workgroup: 8 per lane
@@ -82,8 +86,10 @@ constexpr int kStatCols = 512;           // columns per workgroup: 8 per lane
 // ANY: rows of any length (at least 8).  A row may then start at either nibble of a byte of the
 // codes, and the lane that would run past the row's end works on the row's last 8 columns
 // instead: maxima do not mind columns seen twice.
-template <int GT, bool EXT, bool ANY>
+template <int GT_, bool EXT, bool ANY>
 __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatArgs args) {
+  constexpr bool kAbs = GT_ == kAbsValues;
+  constexpr int GT = kAbs ? Q4ADAMW_FP32 : GT_;
   constexpr int kAhead = 4;  // rows whose loads are in flight together
   __shared__ uint32_t row_bits[4][kStatRows];       // row maxima of each 16-lane quarter of the row's wave
   __shared__ uint32_t col_bits[kWaves][kStatCols];  // column maxima of each wave
@@ -117,7 +123,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
   float c_old[8], c_max[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    c_old[k] = active ? as_global<const float>(T.cmax)[col0 + lane_elem + k] : 0.0f;
+    c_old[k] = active && !kAbs ? as_global<const float>(T.cmax)[col0 + lane_elem + k] : 0.0f;
     c_max[k] = 0.0f;
   }
   const uint32_t quarter = (uint32_t)lane >> 4;
@@ -130,7 +136,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
     for (int i = 0; i < kAhead; ++i) {
       const int r = r0 + i < nrows ? r0 + i : nrows - 1;
       const uint32_t row = tile_row0 + wave_row0 + r;
-      r_old[i] = as_global<const float>(T.rmax)[row];
+      r_old[i] = kAbs ? 0.0f : as_global<const float>(T.rmax)[row];
       // row bases are uniform; the lane's column is a 32-bit offset
       const int64_t row_first = (int64_t)row * T.cols + col0;
       const void *g_row = static_cast<const char *>(T.g) + row_first * (GT ? 2 : 4);
@@ -139,7 +145,9 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
 #pragma unroll
       for (int h = 0; h < (GT ? 1 : 2); ++h) gw[i][h] = u32x4{0u, 0u, 0u, 0u};
       if (active) {
-        if (ANY) {
+        if (kAbs) {
+          // no codes
+        } else if (ANY) {
           // eight codes from either nibble of a byte on: four bytes, or four and the low nibble of a fifth
           const uint32_t nibble = ((uint32_t)row_first & 1u) + lane_elem;
           vw[i] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(v_row), nibble >> 1, 0, kNtReadOnly);
@@ -177,7 +185,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
         const uint32_t code = ((k & 1 ? odd : even) >> (8 * (k >> 1))) & 0xffu;
         const float code_value = __builtin_fmaf((float)code, 0.0625f, 0.0625f);  // (code + 1) / 16, exact
         const float v_old = code_value * min_nonneg(r_old[i], c_old[k]);
-        const float v = args.b2 * v_old + args.r2 * (gk * gk);
+        const float v = kAbs ? __builtin_fabsf(gk) : args.b2 * v_old + args.r2 * (gk * gk);
         c_max[k] = __builtin_fmaxf(c_max[k], v);
         r_max = __builtin_fmaxf(r_max, v);
       }
@@ -233,12 +241,14 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
 // Same arithmetic, operation for operation.
 constexpr uint32_t kFlatMaxCols = 256;
 constexpr uint32_t kFlatWords = 4096;
-constexpr uint32_t kFlatMaxRows = kFlatWords / 3;     // 2 and 3 columns: a pitch of 3 words
+constexpr uint32_t kFlatMaxRows = kFlatWords / 3;     // up to 3 columns: a pitch of 3 words
 
-__host__ __device__ __forceinline__ uint32_t flat_tile_rows(uint32_t cols) { return kFlatWords / (cols | 1u); }
+__host__ __device__ __forceinline__ uint32_t flat_tile_rows(uint32_t cols) { return cols < 3u ? kFlatMaxRows : kFlatWords / (cols | 1u); }
 
-template <int GT, bool EXT>
+template <int GT_, bool EXT>
 __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1StatArgs args) {
+  constexpr bool kAbs = GT_ == kAbsValues;
+  constexpr int GT = kAbs ? Q4ADAMW_FP32 : GT_;
   constexpr int kAhead = 8;   // elements of a thread whose loads are in flight together
   __shared__ float tile[kFlatWords];
   __shared__ uint32_t row_bits[kFlatMaxRows];
@@ -264,7 +274,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1S
   const uint32_t odd = (uint32_t)first & 1u;
   float c_max = 0.0f;
   if (active) {
-    const float c_old = as_global<const float>(T.cmax)[col];
+    const float c_old = kAbs ? 0.0f : as_global<const float>(T.cmax)[col];
     for (uint32_t r0 = r_first; r0 < n; r0 += kAhead * rows_per_pass) {
       float g[kAhead], r_old[kAhead];
       uint32_t byte[kAhead];
@@ -274,8 +284,8 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1S
         r = r < n ? r : r0;                                  // past the tile: a row seen already
         const uint32_t e = r * cols + col;
         g[i] = load_scalar<GT>(g_tile, e);
-        byte[i] = as_global<const uint8_t>(v_tile)[(e + odd) >> 1];
-        r_old[i] = as_global<const float>(T.rmax)[row0 + r];
+        byte[i] = kAbs ? 0u : as_global<const uint8_t>(v_tile)[(e + odd) >> 1];
+        r_old[i] = kAbs ? 0.0f : as_global<const float>(T.rmax)[row0 + r];
       }
 #pragma unroll
       for (int i = 0; i < kAhead; ++i) {
@@ -285,7 +295,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1S
         const uint32_t code = (byte[i] >> (4u * ((r * cols + col + odd) & 1u))) & 15u;
         const float code_value = __builtin_fmaf((float)code, 0.0625f, 0.0625f);  // (code + 1) / 16, exact
         const float v_old = code_value * min_nonneg(r_old[i], c_old);
-        const float v = __builtin_fmaxf(args.b2 * v_old + args.r2 * (gi * gi), 0.0f);   // a NaN never becomes a maximum
+        const float v = __builtin_fmaxf(kAbs ? __builtin_fabsf(gi) : args.b2 * v_old + args.r2 * (gi * gi), 0.0f);   // a NaN never becomes a maximum
         c_max = __builtin_fmaxf(c_max, v);
         tile[r * pitch + col] = v;
       }
