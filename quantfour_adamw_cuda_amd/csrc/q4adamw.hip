@@ -29,7 +29,7 @@
 //             a workgroup finds its tensor with two scalar loads from the kernarg
 //             segment and nothing is staged in device memory.  Workgroup ids are
 //             dealt round-robin to the 8 XCDs; the kernel maps id -> chunk so that
-//             each XCD walks one contiguous eighth of the chunk space, which keeps
+//             runs of consecutive chunks go to one XCD (ChunkRuns), which keeps
 //             neighbouring blocks' scales (4 bytes per block) in one L2.
 // Per element the kernel reads p, g and one nibble of each moment, and writes p
 // and one nibble of each moment; per block it reads and writes two fp32 scales.
@@ -122,8 +122,8 @@ static void finish_prefix(Args &a, int ntensors) {
 // 2^24 - 1 workgroups of 256 threads, which 1.7e10 fp32 elements exceed -- a flat FSDP
 // parameter fits 288 GB several times over.  So a batch's chunks are dealt to as many grids as
 // it takes, each with the number of its first chunk in the arguments (chunk_base); a tensor
-// larger than a grid simply spans grids.  The grid size is rounded down to a multiple of 8 (the
-// fused kernels pad their grids to one).
+// larger than a grid simply spans grids.  The grid size is rounded down to a multiple of 8, so
+// that every grid begins on the same XCD.
 constexpr uint64_t kMaxChunksPerLaunch = 0x7ffffff0ull;   // per batch
 constexpr uint64_t kHipWorkItemsPerGrid = 0xffffffffull;
 constexpr uint64_t kMaxStatWorkgroups = 1ull << 23;        // rank-1 row-scale and commit launches: one grid
@@ -152,9 +152,8 @@ static int launch_fused_batch(FusedArgs &a, uint64_t chunks, void (*kernel)(cons
   finish_prefix(a, a.ntensors);
   return for_each_grid(chunks, kThreads, [&](uint64_t base, uint64_t count) -> int {
     a.chunk_base = (uint32_t)base;
-    a.nchunks = (uint32_t)(base + count);
-    a.chunks_per_xcd = (uint32_t)((count + 7) / 8);
-    hipLaunchKernelGGL(kernel, dim3(a.chunks_per_xcd * 8u), dim3(kThreads), 0, stream, a);
+    a.runs = make_chunk_runs((uint32_t)count);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(kThreads), 0, stream, a);
     Q4_HIP(hipGetLastError());
     return 0;
   });
@@ -564,9 +563,8 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
     finish_prefix(a, a.ntensors);
     if (int rc = for_each_grid(chunks, kThreads, [&](uint64_t base, uint64_t count) -> int {
           a.chunk_base = (uint32_t)base;
-          a.nchunks = (uint32_t)(base + count);
-          a.chunks_per_xcd = (uint32_t)((count + 7) / 8);
-          hipLaunchKernelGGL(kernel, dim3(a.chunks_per_xcd * 8u), dim3(kThreads), 0, s, a);
+          a.runs = make_chunk_runs((uint32_t)count);
+          hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(kThreads), 0, s, a);
           Q4_HIP(hipGetLastError());
           return 0;
         }))

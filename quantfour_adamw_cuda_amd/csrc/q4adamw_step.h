@@ -512,8 +512,7 @@ __global__ __launch_bounds__(kThreads) void fused_4bit_kernel(const FusedArgs ar
   __shared__ uint2 lds[kLdsEntries];
   const int tid = threadIdx.x;
   const TableSlot slot = request_table_slot<SR>(tid);
-  const uint32_t chunk = args.chunk_base + (blockIdx.x & 7u) * args.chunks_per_xcd + (blockIdx.x >> 3);
-  if (chunk >= args.nchunks) return;  // whole workgroup: the grid is padded to a multiple of 8
+  const uint32_t chunk = args.chunk_base + run_chunk(args.runs, blockIdx.x);
   float gscale = 1.0f;
   const bool cancelled = EXT && !grad_ops_begin(args.go, gscale);  // whole grid
   const bool zero_g = EXT && args.go.zero != 0u;
@@ -551,8 +550,7 @@ __global__ __launch_bounds__(kThreads) void fused_4bit_rank1_kernel(const Rank1A
   __shared__ uint2 lds[kLdsEntries];
   const int tid = threadIdx.x;
   const TableSlot slot = request_table_slot<SR>(tid);
-  const uint32_t chunk = args.chunk_base + (blockIdx.x & 7u) * args.chunks_per_xcd + (blockIdx.x >> 3);
-  if (chunk >= args.nchunks) return;
+  const uint32_t chunk = args.chunk_base + run_chunk(args.runs, blockIdx.x);
   float gscale = 1.0f;
   const bool cancelled = EXT && !grad_ops_begin(args.go, gscale);
   const bool zero_g = EXT && args.go.zero != 0u;
@@ -591,8 +589,7 @@ __global__ __launch_bounds__(kThreads) void fused_4bit_rank1_rows_kernel(const R
   __shared__ __attribute__((aligned(16))) float columns[3 * G::kTile];
   const int tid = threadIdx.x;
   const TableSlot slot = request_table_slot<SR>(tid);
-  const uint32_t chunk = args.chunk_base + (blockIdx.x & 7u) * args.chunks_per_xcd + (blockIdx.x >> 3);
-  if (chunk >= args.nchunks) return;
+  const uint32_t chunk = args.chunk_base + run_chunk(args.runs, blockIdx.x);
   float gscale = 1.0f;
   const bool cancelled = EXT && !grad_ops_begin(args.go, gscale);
   const bool zero_g = EXT && args.go.zero != 0u;

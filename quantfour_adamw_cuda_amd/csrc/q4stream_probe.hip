@@ -12,7 +12,7 @@
 //                 which shows what these small streams cost the large ones.
 //
 // All three use the step's launch shape (one tile per wave64, four waves per workgroup,
-// workgroups dealt to the XCDs so that each walks a contiguous eighth), its buffer
+// runs of consecutive workgroups' chunks per XCD), its buffer
 // instructions and its cache policy (q4adamw_device.h), so a difference between the step and
 // its probe is the step's arithmetic and tables, not its addressing.
 //
@@ -31,12 +31,11 @@ struct ProbeArgs {
   uint8_t *m, *v;     // step streams: packed codes
   float *sm, *sv;     // step streams: block scales
   uint64_t units;     // copy / read: 16-byte units; step streams: elements
-  uint32_t nchunks;
-  uint32_t chunks_per_xcd;
+  ChunkRuns runs;
 };
 
 __device__ __forceinline__ uint32_t probe_chunk(const ProbeArgs &a) {
-  return (blockIdx.x & 7u) * a.chunks_per_xcd + (blockIdx.x >> 3);
+  return run_chunk(a.runs, blockIdx.x);
 }
 
 // mode 0: copy, mode 1: read only (the sink is written by no lane in practice: the test
@@ -44,7 +43,6 @@ __device__ __forceinline__ uint32_t probe_chunk(const ProbeArgs &a) {
 template <int MODE>
 __global__ __launch_bounds__(kThreads) void probe_move_kernel(const ProbeArgs a) {
   const uint32_t chunk = probe_chunk(a);
-  if (chunk >= a.nchunks) return;
   const uint64_t unit0 = (uint64_t)chunk * kThreads;   // first 16-byte unit of the workgroup
   const uint32_t tid = threadIdx.x;
   if (unit0 + tid >= a.units) return;
@@ -68,7 +66,6 @@ __global__ __launch_bounds__(kThreads) void probe_step_streams_kernel(const Prob
   constexpr int kLanesPerBlock = Q4ADAMW_BLOCK / N;
   constexpr int kBlocksPerTile = kTile / Q4ADAMW_BLOCK;
   const uint32_t chunk = probe_chunk(a);
-  if (chunk >= a.nchunks) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t tile = (int64_t)chunk * kWaves + wave;
@@ -136,9 +133,8 @@ __global__ __launch_bounds__(kThreads) void probe_step_streams_kernel(const Prob
 static int probe_launch(ProbeArgs &a, uint64_t chunks, void (*kernel)(const ProbeArgs), void *stream) {
   if (chunks == 0) return 0;
   if (chunks > 0x7ffffff0ull) return Q4PROBE_ERR_ARG;
-  a.nchunks = (uint32_t)chunks;
-  a.chunks_per_xcd = (uint32_t)((chunks + 7) / 8);
-  hipLaunchKernelGGL(kernel, dim3(a.chunks_per_xcd * 8u), dim3(kThreads), 0, static_cast<hipStream_t>(stream), a);
+  a.runs = make_chunk_runs((uint32_t)chunks);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)chunks), dim3(kThreads), 0, static_cast<hipStream_t>(stream), a);
   return (int)hipGetLastError();
 }
 
