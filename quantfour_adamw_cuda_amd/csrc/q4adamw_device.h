@@ -314,15 +314,6 @@ __device__ __forceinline__ uint32_t quantize_exact_scales(const Vals<N> &v, cons
   return word;
 }
 
-// Adds element j's code to a lane's word of 4-bit codes.  Four elements per lane: the code
-// (0..15 and no other bits) goes to its place.  Eight: every code enters at the top and
-// moves down four bits per later element.
-template <int N>
-__device__ __forceinline__ uint32_t append_code(uint32_t word, uint32_t code, int j) {
-  if (N == 4) return j == 0 ? code : ((code << (4 * j)) | word);
-  return __builtin_amdgcn_alignbit(code, word, 4);
-}
-
 // A 32-bit integer mixer (two multiply-xorshift rounds) for the rounding noise.
 __host__ __device__ __forceinline__ uint32_t lowbias32(uint32_t x) {
   x ^= x >> 16;
@@ -334,9 +325,9 @@ __host__ __device__ __forceinline__ uint32_t lowbias32(uint32_t x) {
 }
 
 // lowbias32 without its last step: lowbias32(x) == y ^ (y >> 16) for y = lowbias32_open(x).
-// The step kernel takes the two 16-bit halves of the hash as floats and lets the conversions
-// do that step: the high half of y ^ (y >> 16) is y's own, the low half is y's two halves
-// xor-ed, and both selections ride on the instructions' operand selectors.
+// The rounding noise of the two moments is the hash's two 16-bit halves: the high half of
+// y ^ (y >> 16) is y's own, the low half is y's two halves xor-ed, and both selections ride on
+// the instructions' operand selectors.
 __device__ __forceinline__ uint32_t lowbias32_open(uint32_t x) {
   x ^= x >> 16;
   x *= 0x7FEB352Du;
@@ -345,16 +336,12 @@ __device__ __forceinline__ uint32_t lowbias32_open(uint32_t x) {
   return x;
 }
 
-__device__ __forceinline__ float hash_high_half_as_float(uint32_t y) {
-  float r;
-  asm("v_cvt_f32_u32_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1" : "=v"(r) : "v"(y));
-  return r;
-}
+__device__ __forceinline__ uint32_t hash_high_half(uint32_t y) { return y >> 16; }
 
-__device__ __forceinline__ float hash_low_half_as_float(uint32_t y) {
+__device__ __forceinline__ uint32_t hash_low_half(uint32_t y) {
   uint32_t lo;
   asm("v_xor_b32_sdwa %0, %1, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1 src1_sel:WORD_0" : "=v"(lo) : "v"(y));
-  return (float)lo;
+  return lo;
 }
 
 // halves' high 16 bits if q >= thr, else its low 16 bits (a NaN on either side: the low half).
@@ -374,55 +361,92 @@ __device__ __forceinline__ uint32_t high_half_if_ge(float q, float thr, uint32_t
   return r;
 }
 
-// noise in (0, 1) from a 16-bit number (as a float): (2 n + 1) / 2^17, exact
+// noise in (0, 1) from a 16-bit number: (2 n + 1) / 2^17, exact
 constexpr float kNoiseStep = 1.52587890625e-05f;     // 2^-16
-__device__ __forceinline__ float sr_noise_value(float n16) {
-  return __builtin_fmaf(n16, kNoiseStep, 0.5f * kNoiseStep);
+__device__ __forceinline__ float sr_noise_value(uint32_t n16) {
+  return __builtin_fmaf((float)n16, kNoiseStep, 0.5f * kNoiseStep);
 }
 
-// Stochastic rounding, exact form (the closed form of quantize_bsearch<STOCHASTIC>,
-// optim/adamw_fourbit_triton.py:1050-1075, without its division): IEEE quotient, its
-// interval [Q[k], Q[k+1]) among the code-book entries, upper code iff
-// noise * (Q[k+1] - Q[k]) < q - Q[k].  0/0 is NaN and gets code 0.
-template <bool SECOND>
-__device__ __forceinline__ uint32_t sr_code_exact(float q, float noise) {
-  uint32_t k_raw = 0;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const float t = SECOND ? qmap_v(k) : bits2f(kQmapMBits[k]);
-    k_raw += (t <= q) ? 1u : 0u;
-  }
-  float lower, width;
-  if (SECOND) {
-    lower = k_raw == 0u ? -3.4028234663852886e38f : (float)k_raw * 0.0625f;
-    width = k_raw == 0u ? 0.0f : (k_raw == 16u ? __builtin_inff() : 0.0625f);
-  } else {
-    const SrInterval iv = kSrIntervals.e[k_raw];
-    lower = iv.lower;
-    width = iv.width;
-  }
-  const bool up = noise * width < q - lower;
-  int c = (int)k_raw - 1 + (up ? 1 : 0);
-  c = c < 0 ? 0 : (c > 15 ? 15 : c);
-  return (uint32_t)c;
+// ---------------------------------------------------------------------------
+// Codes in fixed point.  Nearest rounding of the second moment gives the code floor(y) with
+// y = 16 q - 1/2, stochastic rounding floor(y - noise) with y the value's position among the
+// code-book entries (16 q for the second moment, interval number plus position in the interval
+// for the first), noise = (n + 1/2) / 2^16 for a 16-bit number n; below 0 the code is 0.  One fma
+// leaves z = 160 - y as a float in [128, 256), where a unit in the last place is 2^-16: its bits
+// are a fixed-point number G with 16 bits of fraction, to which the noise is added as the
+// integer it is, and whose upper half holds 15 - code in its low four bits.
+//   * The upper halves of two elements share a register (one v_perm_b32), one packed minimum
+//     with 0x431f (159.99) clamps what lies above 160 -- y below 0, and a NaN of either sign,
+//     which gets code 0 -- and the nibbles are collected eight (or four) at a time.
+//   * G's low half says how near y is to a threshold; its minimum over the elements (one
+//     v_min3_u16 for two) decides whether the lane takes the exact path.
+// In units of 2^-16, with e the error of z besides its own rounding (at most 1/2):
+// nearest: |G - Z| <= 1/2 + e < 1, so only G = 0 (mod 2^16) is undecided; e <= 0.31 (the scale's
+// reciprocal within two ulps, rank-1; the block scale's is refined, 0.13; z's quotient against
+// the IEEE one).  Stochastic: z carries one unit more than it should, so that the noise's half
+// makes it Z in [G - 1 - e, G + e], and G = 0, 1 (mod 2^16) are undecided for every e < 1; first
+// moment e <= 0.65: the rounded constant of the affine form 1/2, the quotient 3 * 2^-24 relative
+// times less than 9, the rounded slope 2^-24 times less than 9.
+// Before, a coordinate took a conversion of the noise, a fract, a conversion to integer and a
+// shift into the word: 7.5 vector instructions more per element with stochastic rounding, 1.4
+// with nearest.
+// ---------------------------------------------------------------------------
+constexpr float kCodeTop = 160.0f;
+constexpr uint32_t kNearRn = 1u, kNearSr = 2u;    // low halves below this are undecided
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// The least of the low halves of least, a and b, in the low half (the upper half holds nothing).
+__device__ __forceinline__ void min_low_halves(uint32_t &least, uint32_t a, uint32_t b) {
+  asm("v_min3_u16 %0, %0, %1, %2" : "+v"(least) : "v"(a), "v"(b));
 }
 
-template <bool SECOND, int N>
-__device__ __forceinline__ uint32_t quantize_exact_sr(const Vals<N> &v, float scale, const Vals<N> &noise) {
-  uint32_t word = 0;
-#pragma unroll
-  for (int j = 0; j < N; ++j) word |= sr_code_exact<SECOND>(v.x[j] / scale, noise.x[j]) << (4 * j);
-  return word;
+// The upper halves of a and b, clamped, side by side.
+__device__ __forceinline__ uint32_t clamped_halves(uint32_t a, uint32_t b) {
+  const u16x2 h = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(b, a, 0x07060302u));
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(h, u16x2{0x431f, 0x431f}));
 }
 
-// The same for the second moment with a scale per element (rank-1 scaling).
+// The lane's word of codes from its N elements' fixed-point numbers (N = 4: upper half zero).
 template <int N>
-__device__ __forceinline__ uint32_t quantize_exact_sr_scales(const Vals<N> &v, const Vals<N> &scale,
-                                                             const Vals<N> &noise) {
-  uint32_t word = 0;
-#pragma unroll
-  for (int j = 0; j < N; ++j) word |= sr_code_exact<true>(v.x[j] / scale.x[j], noise.x[j]) << (4 * j);
-  return word;
+__device__ __forceinline__ uint32_t collect_codes(const uint32_t (&g)[N]) {
+  const uint32_t a = clamped_halves(g[0], g[2]), b = clamped_halves(g[1], g[3]);
+  if constexpr (N == 4) {
+    const uint32_t w = (a & 0x000f000fu) | ((b << 4) & ~0x000f000fu);
+    return ~__builtin_amdgcn_perm(w, w, 0x0d0d0200u);   // selector 0x0d: a byte of ones
+  } else {
+    const uint32_t c = clamped_halves(g[4], g[6]), d = clamped_halves(g[5], g[7]);
+    const uint32_t even = __builtin_amdgcn_perm(c, a, 0x06040200u), odd = __builtin_amdgcn_perm(d, b, 0x06040200u);
+    return ~((even & 0x0f0f0f0fu) | ((odd << 4) & 0xf0f0f0f0u));
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The exact path of the step's quantizers: IEEE quotients, which are at most 1 because the
+// scale is a maximum over the values, or NaN (0/0, a NaN value), which gets code 0.
+// ---------------------------------------------------------------------------
+// second moment, nearest: the number of thresholds (k + 1/2) / 16, k = 1..15, strictly below q;
+// 16 q - 1/2 is exact wherever it is positive
+__device__ __forceinline__ uint32_t exact_code_v(float q) {
+  const float c = __builtin_ceilf(16.0f * q - 0.5f) - 1.0f;
+  return (uint32_t)(int)__builtin_fmaxf(c, 0.0f);
+}
+
+// Stochastic (the closed form of quantize_bsearch<STOCHASTIC>,
+// optim/adamw_fourbit_triton.py:1050-1075, without its division): the interval [Q[k], Q[k+1]) among
+// the code-book entries, upper code iff noise * (Q[k+1] - Q[k]) < q - Q[k].
+// second moment: entries (k + 1) / 16, everything exact in units of 1/16
+__device__ __forceinline__ uint32_t exact_sr_code_v(float q, float noise) {
+  const float x = 16.0f * q, k = __builtin_floorf(x);
+  const int c = (int)k - 1 + (noise < x - k ? 1 : 0);
+  return (uint32_t)(c < 0 ? 0 : c);
+}
+
+// first moment: bucket_offset is 8 * (number of entries <= q), 0..16 entries (1 for a NaN)
+__device__ __forceinline__ uint32_t exact_sr_code_m(float q, float noise, uint32_t bucket_offset) {
+  const SrInterval iv = kSrIntervals.e[bucket_offset >> 3];
+  const int c = (int)(bucket_offset >> 3) - 1 + (noise * iv.width < q - iv.lower ? 1 : 0);
+  return (uint32_t)(c < 0 ? 0 : c > 15 ? 15 : c);
 }
 
 // (x & mask) | base as one v_and_or_b32: the mask travels in a scalar register (the
@@ -531,8 +555,7 @@ constexpr float kScaleHi = 1.2676506002282294e+30f;  // 2^100
 // 16 / scale at or above this (2^103.5) means a scale at the lower end of the range or below
 // it (16 / kScaleLo is 2^104 give or take the reciprocal's ulp)
 constexpr float kInvScaleLo16 = 1.4340386889e+31f;
-constexpr float kVGuard = 7.62939453125e-06f;        // 2^-17, in units of 16*q
-static_assert(kVGuard == 0.5f * kNoiseStep, "the fast path lets the noise's offset cancel the guard band");
+constexpr float kVGuard = 7.62939453125e-06f;        // 2^-17, in units of 16*q (stand-alone quantizers)
 
 // Uniform search of the launch's tensor list: the last tensor whose first chunk is
 // <= chunk.  first_chunk[0] is 0, so the result is never negative.  Chunk indices and
@@ -578,7 +601,7 @@ __device__ __forceinline__ TableSlot request_table_slot(int tid) {
   if (SR) {
     const SrSlot e = kSrHalfTable.e[tid];
     s.entry = make_uint2(e.thr, e.offsets);
-    const SrAffine af = kSrAffine.e[tid < 17 ? tid : 0];
+    const SrAffine af = kSrFixed.e[tid < 17 ? tid : 0];
     s.interval = make_uint2(f2bits(af.a), f2bits(af.c));
   } else {
     const MtabEntry e = kHalfTable.e[tid];

@@ -319,18 +319,16 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     }
   }
 
-  // fast quantization: multiply by a refined reciprocal, decide every code whose
-  // quotient is clear of all thresholds, flag the rest
+  // fast quantization: multiply by a refined reciprocal, decide every code whose quotient is
+  // clear of all thresholds, flag the rest -- each moment for itself, since the exact path of one
+  // leaves the other's codes alone
   const bool safe_m = am >= kScaleLo && am <= kScaleHi;
   const bool safe_v = RANK1 || (av >= kScaleLo && av <= kScaleHi);
   const float rm = safe_m ? refined_rcp(am) : 0.0f;
   const float rv16 = (safe_v && !RANK1) ? refined_rcp(av) * 16.0f : 0.0f;  // exact scaling
-  bool redo = (!safe_m && am != 0.0f) || (!safe_v && av != 0.0f);
-  // smallest fractional part of a code coordinate shifted up by the guard band: second
-  // moment 16 q - 1/2 (nearest), both moments' coordinate minus noise (stochastic)
-  float vfrac = 1.0f;
+  bool redo_m = !safe_m && am != 0.0f, redo_v = !safe_v && av != 0.0f;
   // rank-1: the new scale of every element and 16 / scale.  The hardware reciprocal's
-  // one ulp is well inside the second moment's guard band (2^-17 in units of 16 q), so
+  // one ulp is well inside what the fixed-point codes' guard allows (q4adamw_device.h), so
   // it goes unrefined.  Scales below the safe range are clamped for the reciprocal: a
   // zero value under a zero scale then still gets code 0; any other value under such a
   // scale sends the lane to the exact path.
@@ -348,7 +346,7 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
       inv16.x[j] = max_nonneg(row_inv16, c_new.x[j]);
       inv_max = max_nonneg(inv_max, inv16.x[j]);
     }
-    redo |= r_new > kScaleHi || (inv_max >= kInvScaleLo16 && v_lane_max != 0.0f);
+    redo_v |= r_new > kScaleHi || (inv_max >= kInvScaleLo16 && v_lane_max != 0.0f);
   } else if constexpr (RANK1 && SHAPE == kTileAny) {
     float s_least = rn.x[0], s_most = 0.0f;
 #pragma unroll
@@ -359,7 +357,7 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
       s_most = max_nonneg(s_most, sj);
       inv16.x[j] = __builtin_amdgcn_rcpf(max_nonneg(sj, kScaleLo)) * 16.0f;
     }
-    redo |= s_most > kScaleHi || (s_least < kScaleLo && v_lane_max != 0.0f);
+    redo_v |= s_most > kScaleHi || (s_least < kScaleLo && v_lane_max != 0.0f);
   } else if constexpr (RANK1) {
     float c_min = c_new.x[0];
 #pragma unroll
@@ -370,13 +368,10 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
       inv16.x[j] = __builtin_amdgcn_rcpf(max_nonneg(sj, kScaleLo)) * 16.0f;
     }
     // every scale is at most r_new and at least min(r_new, c_min)
-    redo |= r_new > kScaleHi || (min_nonneg(r_new, c_min) < kScaleLo && v_lane_max != 0.0f);
+    redo_v |= r_new > kScaleHi || (min_nonneg(r_new, c_min) < kScaleLo && v_lane_max != 0.0f);
   }
   uint32_t mword = 0, vword = 0;
-  // stochastic rounding: the elements' 16-bit noise numbers n as floats; the noise itself is
-  // (2 n + 1) / 2^17 = n * kNoiseStep + kVGuard, and the fast path works with code
-  // coordinates shifted up by the guard band, so the two halves of a step cancel there
-  Vals<N> um, uv;
+  uint32_t noise[N] = {};   // stochastic rounding: the elements' hashes (without the mixer's last step)
   if constexpr (SR) {
     // key = low half of the element index, xor the salt, xor the mixed high half
     const uint32_t tile_salt = salt ^ ((uint32_t)((uint64_t)tb >> 32) * 0x9E3779B9u);
@@ -385,12 +380,10 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     // element is a multiple of N, so element j's key is the first one's with j in its low bits
     const uint32_t key0 = ((uint32_t)tb + e0) ^ tile_salt;
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-      const uint32_t y = lowbias32_open(key0 ^ (uint32_t)j);   // the hash is y ^ (y >> 16)
-      um.x[j] = hash_high_half_as_float(y);
-      uv.x[j] = hash_low_half_as_float(y);
-    }
+    for (int j = 0; j < N; ++j) noise[j] = lowbias32_open(key0 ^ (uint32_t)j);
   }
+  uint32_t mg[N], vg[N];   // the codes in fixed point (first moment: stochastic rounding only)
+  uint32_t m_near = 0xffffu, v_near = 0xffffu;   // in the low halves
 #pragma unroll
   for (int j = 0; j < N; j += 2) {
     // first moment: the quotients' bucket entries, two quotients per conversion
@@ -399,57 +392,60 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     const uint2 ent0 = *reinterpret_cast<const uint2 *>(lds_bytes + kLdsBuckets * 8u + byte_shifted<1>(halves, three));
     const uint2 ent1 = *reinterpret_cast<const uint2 *>(lds_bytes + kLdsBuckets * 8u + byte_shifted<3>(halves, three));
     if constexpr (SR) {
-      // interval among the code-book entries; inside it the code is floor(k + position -
-      // noise), an affine function of the quotient.  Computed shifted up by the guard band
-      // (coordinate - n * kNoiseStep): a fractional part below twice the band then marks a
-      // value within the band of an integer on either side, which goes to the exact path,
-      // and every other value truncates to its code.  Error budget in units of one code: the
-      // quotient is within 2^-22 relative of the exact one and |q| / width < 9 (2.25 *
-      // 2^-20), the map's two roundings and the two operations here add 2^-21 each: 0.54 of
-      // the band.  The value is never negative, and below 16 outside the band.
+      // the interval among the code-book entries; inside it the position is an affine function of
+      // the quotient
       const float qq[2] = {q0, q1};
       const uint2 ent[2] = {ent0, ent1};
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const uint32_t interval = high_half_if_ge(qq[h], bits2f(ent[h].x), ent[h].y);   // byte offset into the affine table
         const float2 af = *reinterpret_cast<const float2 *>(lds_bytes + kLdsIntervals * 8u + interval);
-        const float y = __builtin_fmaf(um.x[j + h], -kNoiseStep, __builtin_fmaf(qq[h], af.x, af.y));
-        vfrac = __builtin_fminf(vfrac, __builtin_amdgcn_fractf(y));
-        mword = append_code<N>(mword, (uint32_t)(int)y, j + h);
+        mg[j + h] = f2bits(__builtin_fmaf(qq[h], af.x, af.y)) + hash_high_half(noise[j + h]);
       }
+      min_low_halves(m_near, mg[j], mg[j + 1]);
     } else {
       const bool hi0 = q0 > bits2f(ent0.y), hi1 = q1 > bits2f(ent1.y);
-      redo |= hi0 != (q0 > bits2f(ent0.x));
-      redo |= hi1 != (q1 > bits2f(ent1.x));
+      redo_m |= hi0 != (q0 > bits2f(ent0.x));
+      redo_m |= hi1 != (q1 > bits2f(ent1.x));
       // base code in the entry's low nibble, plus one above the threshold; every
       // code enters the word at the top and moves down four bits per later element
       mword = __builtin_amdgcn_alignbit(ent0.x + (hi0 ? 1u : 0u), mword, 4);
       mword = __builtin_amdgcn_alignbit(ent1.x + (hi1 ? 1u : 0u), mword, 4);
     }
 
-    // second moment: thresholds at 16q = k + 0.5, k = 1..15
+    // second moment: thresholds at 16 q = k + 1/2, k = 1..15 (nearest), entries at 16 q = 1..16
+    // (stochastic)
 #pragma unroll
     for (int k = j; k < j + 2; ++k) {
-      if constexpr (SR) {
-        // code-book entries at 16 q = 1..16: interval number floor(16 q), position in it
-        // fract(16 q), up iff noise < position, i.e. code = floor(16 q - noise) wherever
-        // that difference is clear of an integer; shifted up by the guard band as for the
-        // first moment.  The shifted value is above -1 (truncation gives 0 below 0) and,
-        // outside the band, below 16.
-        const float y = __builtin_fmaf(vn.x[k], RANK1 ? inv16.x[k] : rv16, uv.x[k] * -kNoiseStep);
-        vfrac = __builtin_fminf(vfrac, __builtin_amdgcn_fractf(y));
-        vword = append_code<N>(vword, (uint32_t)(int)y, k);
-      } else {
-        const float t = __builtin_fmaf(vn.x[k], RANK1 ? inv16.x[k] : rv16, kVGuard - 0.5f);
-        vfrac = __builtin_fminf(vfrac, __builtin_amdgcn_fractf(t));
-        // t > -1, so truncation gives 0 for t < 0
-        vword = append_code<N>(vword, (uint32_t)(int)t, k);
+      const float inv = RANK1 ? inv16.x[k] : rv16;
+      if constexpr (SR) vg[k] = f2bits(__builtin_fmaf(-vn.x[k], inv, kCodeTop + kNoiseStep)) + hash_low_half(noise[k]);
+      else vg[k] = f2bits(__builtin_fmaf(-vn.x[k], inv, kCodeTop + 0.5f));
+    }
+    min_low_halves(v_near, vg[j], vg[j + 1]);
+  }
+  if constexpr (SR) {
+    mword = collect_codes<N>(mg);
+    redo_m |= (uint16_t)m_near < kNearSr;
+  } else if (N == 4) {
+    mword >>= 16;   // four codes entered at the top
+  }
+  vword = collect_codes<N>(vg);
+  redo_v |= (uint16_t)v_near < (SR ? kNearSr : kNearRn);
+  if (__builtin_expect(redo_m, 0)) {
+    if constexpr (SR) {
+      mword = 0;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const float q = mn.x[j] / am;
+        const uint32_t half = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(q, q));
+        const uint2 ent = *reinterpret_cast<const uint2 *>(lds_bytes + kLdsBuckets * 8u + byte_shifted<1>(half, three));
+        mword |= exact_sr_code_m(q, sr_noise_value(hash_high_half(noise[j])), high_half_if_ge(q, bits2f(ent.x), ent.y)) << (4 * j);
       }
+    } else {
+      mword = quantize_exact<false, N>(mn, am);
     }
   }
-  if (N == 4 && !SR) mword >>= 16;   // four codes entered at the top
-  redo |= vfrac < 2.0f * kVGuard;
-  if (__builtin_expect(redo, 0)) {
+  if (__builtin_expect(redo_v, 0)) {
     if constexpr (RANK1 && kRows) {
       // the scales themselves: the new column maxima are the third array of the staging area
 #pragma unroll
@@ -461,19 +457,12 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
         s_new.x[k + 3] = min_nonneg(r_new, c.w);
       }
     }
-    if constexpr (SR) {
+    vword = 0;
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
-        um.x[j] = sr_noise_value(um.x[j]);
-        uv.x[j] = sr_noise_value(uv.x[j]);
-      }
-      mword = quantize_exact_sr<false, N>(mn, am, um);
-      if constexpr (RANK1) vword = quantize_exact_sr_scales<N>(vn, s_new, uv);
-      else vword = quantize_exact_sr<true, N>(vn, av, uv);
-    } else {
-      mword = quantize_exact<false, N>(mn, am);
-      if constexpr (RANK1) vword = quantize_exact_scales<N>(vn, s_new);
-      else vword = quantize_exact<true, N>(vn, av);
+    for (int j = 0; j < N; ++j) {
+      const float q = vn.x[j] / (RANK1 ? s_new.x[j] : av);
+      const uint32_t c = SR ? exact_sr_code_v(q, sr_noise_value(hash_low_half(noise[j]))) : exact_code_v(q);
+      vword |= c << (4 * j);
     }
   }
   if (am == 0.0f) mword = 0;  // 0/0: code 0 for the whole block

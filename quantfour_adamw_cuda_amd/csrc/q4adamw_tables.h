@@ -262,11 +262,32 @@ struct SrAffineTable {
   SrAffine e[17];
 };
 
-constexpr SrAffineTable make_sr_affine_table() {
+// The same for 160 + 2^-16 - y (y the position above; q4adamw_device.h, codes in fixed point),
+// the constant again from the exact interval and rounded once: it lies in [128, 256), so
+// that rounding is at most 2^-17.
+constexpr double kSrFixedTop = 160.0 + 1.0 / 65536.0;
+
+Q4_HD constexpr SrAffine sr_fixed_m(uint32_t k_raw) {  // k_raw 0..16
+  if (k_raw == 0u) return SrAffine{0.0f, (float)(kSrFixedTop - 1.0)};
+  if (k_raw == 16u) return SrAffine{0.0f, (float)(kSrFixedTop - 16.0)};
+  const double lower = (double)bits2f(kQmapMBits[k_raw - 1u]);
+  const double width = (double)bits2f(kQmapMBits[k_raw]) - lower;
+  return SrAffine{(float)(-1.0 / width), (float)(kSrFixedTop - ((double)k_raw - lower / width))};
+}
+
+constexpr SrAffineTable make_sr_fixed_table() {
   SrAffineTable t{};
-  for (uint32_t k = 0; k < 17; ++k) t.e[k] = sr_affine_m(k);
+  for (uint32_t k = 0; k < 17; ++k) t.e[k] = sr_fixed_m(k);
   return t;
 }
+
+constexpr bool sr_fixed_in_binade() {
+  for (uint32_t k = 0; k < 17; ++k) {
+    if (sr_fixed_m(k).c < 144.0f || sr_fixed_m(k).c >= 160.0f) return false;
+  }
+  return true;
+}
+static_assert(sr_fixed_in_binade(), "a constant's rounding must be that of [128, 256)");
 
 // The error of the affine form, in units of one code, is the quotient's relative error
 // times |q| / width: the guard band of the fast path is sized for a ratio below 9.
