@@ -378,8 +378,8 @@ __device__ __forceinline__ float sr_noise_value(uint32_t n16) {
 //   * The upper halves of two elements share a register (one v_perm_b32), one packed minimum
 //     with 0x431f (159.99) clamps what lies above 160 -- y below 0, and a NaN of either sign,
 //     which gets code 0 -- and the nibbles are collected eight (or four) at a time.
-//   * G's low half says how near y is to a threshold; its minimum over the elements (one
-//     v_min3_u16 for two) decides whether the lane takes the exact path.
+//   * G's low half says how near y is to a threshold; its minimum over the elements decides
+//     whether the lane takes the exact path.
 // In units of 2^-16, with e the error of z besides its own rounding (at most 1/2):
 // nearest: |G - Z| <= 1/2 + e < 1, so only G = 0 (mod 2^16) is undecided; e <= 0.31 (the scale's
 // reciprocal within two ulps, rank-1; the block scale's is refined, 0.13; z's quotient against
@@ -391,14 +391,23 @@ __device__ __forceinline__ float sr_noise_value(uint32_t n16) {
 // shift into the word: 7.5 vector instructions more per element with stochastic rounding, 1.4
 // with nearest.
 // ---------------------------------------------------------------------------
-constexpr float kCodeTop = 160.0f;
 constexpr uint32_t kNearRn = 1u, kNearSr = 2u;    // low halves below this are undecided
 
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
-// The least of the low halves of least, a and b, in the low half (the upper half holds nothing).
-__device__ __forceinline__ void min_low_halves(uint32_t &least, uint32_t a, uint32_t b) {
-  asm("v_min3_u16 %0, %0, %1, %2" : "+v"(least) : "v"(a), "v"(b));
+// 160.5 + v * neg_inv16 (nearest) or 160 + 2^-16 + v * neg_inv16 (stochastic): an fma whose third
+// operand is a literal issues in 2 cycles, one of three registers in 4.
+template <bool SR>
+__device__ __forceinline__ uint32_t fixed_code_v(float v, float neg_inv16) {
+  uint32_t g;
+  if (SR) asm("v_fmaak_f32 %0, %1, %2, 0x43200001" : "=v"(g) : "v"(v), "v"(neg_inv16));
+  else asm("v_fmaak_f32 %0, %1, %2, 0x43208000" : "=v"(g) : "v"(v), "v"(neg_inv16));
+  return g;
+}
+
+// The lesser of the low halves of least and g, in the low half (2 cycles each; v_min3_u16 takes 8).
+__device__ __forceinline__ void min_low_half(uint32_t &least, uint32_t g) {
+  asm("v_min_u16 %0, %0, %1" : "+v"(least) : "v"(g));
 }
 
 // The upper halves of a and b, clamped, side by side.
@@ -447,6 +456,15 @@ __device__ __forceinline__ uint32_t exact_sr_code_m(float q, float noise, uint32
   const SrInterval iv = kSrIntervals.e[bucket_offset >> 3];
   const int c = (int)(bucket_offset >> 3) - 1 + (noise * iv.width < q - iv.lower ? 1 : 0);
   return (uint32_t)(c < 0 ? 0 : c > 15 ? 15 : c);
+}
+
+// A uniform value in a vector register: a multiplication or an addition of vector registers issues
+// in 2 cycles, one with a scalar operand in 4 (a wave64 instruction on this GPU, 8 waves per
+// SIMD).  Pays for itself from three uses on.
+__device__ __forceinline__ float in_vgpr(float s) {
+  float v;
+  asm("v_mov_b32 %0, %1" : "=v"(v) : "s"(s));
+  return v;
 }
 
 // (x & mask) | base as one v_and_or_b32: the mask travels in a scalar register (the

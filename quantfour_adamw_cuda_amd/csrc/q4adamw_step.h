@@ -47,7 +47,7 @@ constexpr int kTileWide = 0, kTileNarrow = 1, kTileRows = 2, kTileRowsLast = 3, 
 // What a wave of the kTileRows form knows beyond its tile number: its row, the tile's first
 // column, and this thread's share of the workgroup's fetch of the columns' maxima (old and
 // new; kTile / 256 consecutive columns per thread), which goes to `columns` in LDS:
-// [0, kTile) old, [kTile, 2 kTile) 16 / max(new, kScaleLo) -- the reciprocal every element of
+// [0, kTile) old, [kTile, 2 kTile) -16 / max(new, kScaleLo) -- the reciprocal every element of
 // the column would otherwise take for itself -- and [2 kTile, 3 kTile) new, which only the
 // exact path reads.
 struct RowsTile {
@@ -61,13 +61,13 @@ struct RowsTile {
 // Writes a thread's share of the columns' maxima into LDS (before the workgroup's barrier).
 template <int N>
 __device__ __forceinline__ void stage_columns(const RowsTile &rt, int tid) {
-  const float inv_x = __builtin_amdgcn_rcpf(max_nonneg(rt.share_new.x, kScaleLo)) * 16.0f;
+  const float inv_x = __builtin_amdgcn_rcpf(max_nonneg(rt.share_new.x, kScaleLo)) * -16.0f;
   if (N == 4) {
     rt.columns[tid] = rt.share_old.x;
     rt.columns[64 * N + tid] = inv_x;
     rt.columns[128 * N + tid] = rt.share_new.x;
   } else {
-    const float inv_y = __builtin_amdgcn_rcpf(max_nonneg(rt.share_new.y, kScaleLo)) * 16.0f;
+    const float inv_y = __builtin_amdgcn_rcpf(max_nonneg(rt.share_new.y, kScaleLo)) * -16.0f;
     *reinterpret_cast<float2 *>(rt.columns + 2 * tid) = rt.share_old;
     *reinterpret_cast<float2 *>(rt.columns + 64 * N + 2 * tid) = make_float2(inv_x, inv_y);
     *reinterpret_cast<float2 *>(rt.columns + 128 * N + 2 * tid) = rt.share_new;
@@ -179,8 +179,9 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     load_elems<GT, N, FULL>(g_tile, e0, nv, g);
   }
   if (EXT) {
+    const float gscale_v = in_vgpr(gscale);
 #pragma unroll
-    for (int j = 0; j < N; ++j) g[j] *= gscale;
+    for (int j = 0; j < N; ++j) g[j] *= gscale_v;
     if (zero_g && lane_on) zero_elems<GT, N, FULL>(const_cast<void *>(g_tile), e0, nv);
   }
   uint32_t mw = 0, vw = 0;
@@ -240,7 +241,7 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
   if constexpr (RANK1 && kRows) {
 #pragma unroll
     for (int k = 0; k < N; k += 4) {
-      // c_new: 16 / max(new column maximum, kScaleLo) in this form, not the maximum itself
+      // c_new: -16 / max(new column maximum, kScaleLo) in this form, not the maximum itself
       const float4 a = *reinterpret_cast<const float4 *>(rt->columns + e0 + k);
       const float4 b = *reinterpret_cast<const float4 *>(rt->columns + 64 * N + e0 + k);
       c_old.x[k] = a.x; c_old.x[k + 1] = a.y; c_old.x[k + 2] = a.z; c_old.x[k + 3] = a.w;
@@ -255,6 +256,9 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
   const uint32_t v_even = and_or(vw, 0x0F0F0F0Fu, cb_bytes), v_odd = and_or(vw >> 4, 0x0F0F0F0Fu, cb_bytes);
 
   // dequantize, update moments and parameter (cuda_adamw_kernels.cu:334-351)
+  const float r1 = in_vgpr(sc.r1), r2 = in_vgpr(sc.r2), wdu = in_vgpr(sc.wdu);
+  const float b2 = RANK1 ? in_vgpr(sc.b2) : 0.0f;
+  const float c2s_rcp = EXACT ? in_vgpr(sc.c2s_rcp) : 0.0f, eps = EXACT ? in_vgpr(sc.eps) : 0.0f, ss = EXACT ? in_vgpr(sc.ss) : 0.0f;
   Vals<N> mn, vn;
   float am = 0.0f, av = 0.0f;
   float m_least = kExactHi, v_least = kExactVHi;   // EXACT: the lane's smallest |m| and v
@@ -265,23 +269,23 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     const uint32_t vo = entry_offset(j & 1 ? v_odd : v_even, j >> 1, two);
     const float m_old = *reinterpret_cast<const float *>(lds_bytes + mo);
     float v_old = *reinterpret_cast<const float *>(lds_bytes + vo + kLdsSecondMoment * 4u);
-    if constexpr (RANK1) v_old = sc.b2 * (v_old * min_nonneg(SHAPE == kTileAny ? ro.x[j] : r_old, c_old.x[j]));  // adamw_fourbit_triton.py:520-527
+    if constexpr (RANK1) v_old = b2 * (v_old * min_nonneg(SHAPE == kTileAny ? ro.x[j] : r_old, c_old.x[j]));  // adamw_fourbit_triton.py:520-527
     const float gj = g[j];
-    float m = m_old + sc.r1 * gj;                 // m_old, v_old: beta times the old moment
-    float v = v_old + sc.r2 * (gj * gj);
+    float m = m_old + r1 * gj;                 // m_old, v_old: beta times the old moment
+    float v = v_old + r2 * (gj * gj);
     if (!FULL && j >= nv) { m = 0.0f; v = 0.0f; }
     if constexpr (EXACT) {
       // the reference's seven operations, each rounded as IEEE 754 rounds it
       // (cuda_adamw_kernels.cu:334,351), valid inside the ranges checked below
-      const float den = div_by_reciprocal(sqrt_rn(v), sc.c2s, sc.c2s_rcp) + sc.eps;
-      p_new[j] = p[j] * sc.wdu - sc.ss * div_rn(m, den);
+      const float den = div_by_reciprocal(sqrt_rn(v), sc.c2s, c2s_rcp) + eps;
+      p_new[j] = p[j] * wdu - ss * div_rn(m, den);
       m_least = __builtin_fminf(m_least, __builtin_fabsf(m));
       v_least = __builtin_fminf(v_least, v);
     } else {
       // folded form: the hardware's 1-ulp square root and a reciprocal in place of the
       // divisions; the parameters then agree with the reference's to a tolerance only
       const float den = __builtin_fmaf(__builtin_amdgcn_sqrtf(v), sc.den_scale, sc.den_eps);
-      p_new[j] = __builtin_fmaf(-m, __builtin_amdgcn_rcpf(den), p[j] * sc.wdu);
+      p_new[j] = __builtin_fmaf(-m, __builtin_amdgcn_rcpf(den), p[j] * wdu);
     }
     mn.x[j] = m;
     vn.x[j] = v;
@@ -325,28 +329,28 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
   const bool safe_m = am >= kScaleLo && am <= kScaleHi;
   const bool safe_v = RANK1 || (av >= kScaleLo && av <= kScaleHi);
   const float rm = safe_m ? refined_rcp(am) : 0.0f;
-  const float rv16 = (safe_v && !RANK1) ? refined_rcp(av) * 16.0f : 0.0f;  // exact scaling
+  const float neg_rv16 = (safe_v && !RANK1) ? refined_rcp(av) * -16.0f : 0.0f;  // exact scaling
   bool redo_m = !safe_m && am != 0.0f, redo_v = !safe_v && av != 0.0f;
-  // rank-1: the new scale of every element and 16 / scale.  The hardware reciprocal's
+  // rank-1: the new scale of every element and -16 / scale.  The hardware reciprocal's
   // one ulp is well inside what the fixed-point codes' guard allows (q4adamw_device.h), so
   // it goes unrefined.  Scales below the safe range are clamped for the reciprocal: a
   // zero value under a zero scale then still gets code 0; any other value under such a
   // scale sends the lane to the exact path.
-  Vals<N> s_new, inv16;
+  Vals<N> s_new, neg_inv16;
   if constexpr (RANK1 && kRows) {
     // 16 / min(row maximum, column maximum) is the larger of the two reciprocals, the row's
     // taken once per lane and the columns' once per workgroup (stage_columns): one
     // instruction per element.  (Where the hardware reciprocal is not monotonic the other
     // one is within an ulp of it, which the guard band covers all the same.)  A clamped
     // scale shows as the reciprocal of the clamp.
-    const float row_inv16 = __builtin_amdgcn_rcpf(max_nonneg(r_new, kScaleLo)) * 16.0f;
-    float inv_max = 0.0f;
+    const float row_inv = __builtin_amdgcn_rcpf(max_nonneg(r_new, kScaleLo)) * -16.0f;
+    float inv_max = -0.0f;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      inv16.x[j] = max_nonneg(row_inv16, c_new.x[j]);
-      inv_max = max_nonneg(inv_max, inv16.x[j]);
+      neg_inv16.x[j] = max_nonneg(row_inv, c_new.x[j]);   // both negative: the one of larger magnitude
+      inv_max = max_nonneg(inv_max, neg_inv16.x[j]);
     }
-    redo_v |= r_new > kScaleHi || (inv_max >= kInvScaleLo16 && v_lane_max != 0.0f);
+    redo_v |= r_new > kScaleHi || (inv_max <= -kInvScaleLo16 && v_lane_max != 0.0f);
   } else if constexpr (RANK1 && SHAPE == kTileAny) {
     float s_least = rn.x[0], s_most = 0.0f;
 #pragma unroll
@@ -355,7 +359,7 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
       s_new.x[j] = sj;
       s_least = min_nonneg(s_least, sj);
       s_most = max_nonneg(s_most, sj);
-      inv16.x[j] = __builtin_amdgcn_rcpf(max_nonneg(sj, kScaleLo)) * 16.0f;
+      neg_inv16.x[j] = __builtin_amdgcn_rcpf(max_nonneg(sj, kScaleLo)) * -16.0f;
     }
     redo_v |= s_most > kScaleHi || (s_least < kScaleLo && v_lane_max != 0.0f);
   } else if constexpr (RANK1) {
@@ -365,7 +369,7 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
       const float sj = min_nonneg(r_new, c_new.x[j]);        // adamw_fourbit_triton.py:749-755
       s_new.x[j] = sj;
       c_min = min_nonneg(c_min, c_new.x[j]);
-      inv16.x[j] = __builtin_amdgcn_rcpf(max_nonneg(sj, kScaleLo)) * 16.0f;
+      neg_inv16.x[j] = __builtin_amdgcn_rcpf(max_nonneg(sj, kScaleLo)) * -16.0f;
     }
     // every scale is at most r_new and at least min(r_new, c_min)
     redo_v |= r_new > kScaleHi || (min_nonneg(r_new, c_min) < kScaleLo && v_lane_max != 0.0f);
@@ -401,8 +405,8 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
         const uint32_t interval = high_half_if_ge(qq[h], bits2f(ent[h].x), ent[h].y);   // byte offset into the affine table
         const float2 af = *reinterpret_cast<const float2 *>(lds_bytes + kLdsIntervals * 8u + interval);
         mg[j + h] = f2bits(__builtin_fmaf(qq[h], af.x, af.y)) + hash_high_half(noise[j + h]);
+        min_low_half(m_near, mg[j + h]);
       }
-      min_low_halves(m_near, mg[j], mg[j + 1]);
     } else {
       const bool hi0 = q0 > bits2f(ent0.y), hi1 = q1 > bits2f(ent1.y);
       redo_m |= hi0 != (q0 > bits2f(ent0.x));
@@ -417,11 +421,11 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     // (stochastic)
 #pragma unroll
     for (int k = j; k < j + 2; ++k) {
-      const float inv = RANK1 ? inv16.x[k] : rv16;
-      if constexpr (SR) vg[k] = f2bits(__builtin_fmaf(-vn.x[k], inv, kCodeTop + kNoiseStep)) + hash_low_half(noise[k]);
-      else vg[k] = f2bits(__builtin_fmaf(-vn.x[k], inv, kCodeTop + 0.5f));
+      const float inv = RANK1 ? neg_inv16.x[k] : neg_rv16;
+      vg[k] = fixed_code_v<SR>(vn.x[k], inv);
+      if constexpr (SR) vg[k] += hash_low_half(noise[k]);
+      min_low_half(v_near, vg[k]);
     }
-    min_low_halves(v_near, vg[j], vg[j + 1]);
   }
   if constexpr (SR) {
     mword = collect_codes<N>(mg);
