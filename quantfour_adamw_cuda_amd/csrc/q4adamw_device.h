@@ -559,6 +559,7 @@ __device__ __forceinline__ float div_rn(float m, float d) {
 constexpr float kExactLo = 8.673617379884035e-19f;   // 2^-60
 constexpr float kExactHi = 1.152921504606847e+18f;   // 2^60
 constexpr float kExactVLo = 1.262177448353619e-29f;  // 2^-96
+constexpr float kStepSizeHi = 3.4028234663852886e38f;  // the largest finite float
 constexpr float kExactVHi = 1.2379400392853803e+27f; // 2^90
 
 // The update as the reference writes it; `sqrtf` and `/` are the compiler's general
