@@ -16,6 +16,13 @@ __device__ __forceinline__ void raise_max(float *addr, uint32_t u) {
   if (u > __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(a, u);
 }
 
+// The same without the look.  Where a statistic meets no more than a few hundred workgroups the
+// atomic, for which nothing waits, costs less than the load that every workgroup would end with:
+// statistics of 218 million elements (fp32 gradients, one layer's matrices) 179 us against 189.
+__device__ __forceinline__ void atomic_max_bits(float *addr, uint32_t u) {
+  atomicMax(reinterpret_cast<unsigned int *>(addr), u);
+}
+
 // A workgroup's share of the leading statistics: rows [row0, row0 + n) with their maxima in
 // row_bits.  The rows are consecutive, so dimension j meets at most min(shape[j], n / stride + 2)
 // of its indices: one LDS slot for each of them, all dimensions side by side (at most 2 n + 4
@@ -213,14 +220,14 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
       const uint32_t first = c & ~7u, last = T.cols - 8u - col0;
       cc = col0 + (first < last ? first : last) + (c & 7u);
     }
-    if (there && u != 0u) raise_max(T.cmax_next + cc, u);
+    if (there && u != 0u) atomic_max_bits(T.cmax_next + cc, u);
   }
   static_assert(kStatRows == kThreads, "one row per thread below");
   uint32_t u = row_bits[0][tid];
 #pragma unroll
   for (int qi = 1; qi < 4; ++qi) u = u > row_bits[qi][tid] ? u : row_bits[qi][tid];
   if (T.lead_dims == 0u) {
-    if (tid < tile_rows && u != 0u) raise_max(T.rmax_next + tile_row0 + tid, u);
+    if (tid < tile_rows && u != 0u) atomic_max_bits(T.rmax_next + tile_row0 + tid, u);
     return;
   }
   __syncthreads();          // every thread has read its row's quarters
