@@ -162,6 +162,9 @@ static int launch_fused_batch(FusedArgs &a, uint64_t chunks, void (*kernel)(cons
 static int launch_small_batch(SmallArgs &a, uint64_t chunks, void (*kernel)(const SmallArgs),
                               hipStream_t stream) {
   finish_prefix(a, a.ntensors);
+  // where the last tensor ends; larger than every chunk of the batch, so the search is none the wiser
+  a.first_chunk[a.ntensors] = (uint32_t)chunks;
+  if (a.ntensors % 8 == 0) a.pivot[a.ntensors / 8] = (uint32_t)chunks;
   return for_each_grid(chunks, 256, [&](uint64_t base, uint64_t count) -> int {
     a.chunk_base = (uint32_t)base;
     hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(256), 0, stream, a);
@@ -860,7 +863,7 @@ int q4adamw_fused_single_tensor_multi_ex(const q4adamw_small_tensor *tensors, in
     d.g = t.g;
     d.m = t.exp_avg;
     d.v = t.exp_avg_sq;
-    d.numel = t.numel;
+    a.last[a.ntensors] = (uint16_t)((uint64_t)t.numel - (c - 1) * (uint64_t)kSmallChunk);
     a.first_chunk[a.ntensors] = (uint32_t)chunks;
     ++a.ntensors;
     chunks += c;

@@ -18,7 +18,7 @@ __global__ __launch_bounds__(256) void single_tensor_kernel(const SmallArgs args
   const SmallDesc &T = args.desc[t];
   const StepConsts sc = EXT ? step_consts(args.sc, args.go) : args.sc;
   const int64_t base = (int64_t)(chunk - args.first_chunk[t]) * kSmallChunk;
-  const int64_t end = base + kSmallChunk < T.numel ? base + kSmallChunk : T.numel;
+  const int64_t end = base + (chunk + 1u == args.first_chunk[t + 1] ? args.last[t] : kSmallChunk);
   if (cancelled) {  // a cancelled step still clears the gradients it was asked to clear
     for (int64_t i = base + threadIdx.x; i < end; i += 256) {
       store_scalar<GT>(const_cast<void *>(T.g), i, 0.0f);
