@@ -56,8 +56,14 @@ def check_unquantized(p, g, exp_avg, exp_avg_sq):
         assert t.device == p.device and t.is_contiguous(), "state must be contiguous on the param's device"
 
 
+# The current stream's handle without a Stream object around it (2.0 us a launch against 0.1).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 class _OnDevice:
@@ -92,7 +98,7 @@ def fused_4bit(p, g, exp, sq, exp_scale, sq_scale, beta1, beta2, lr, weight_deca
                                 weight_decay, eps, step, update_form=update_form)
     L = _lib.load()
     check_quantized(p, g, exp, sq, exp_scale, sq_scale)
-    with torch.cuda.device(p.device):
+    with _on(p.device):
         rc = L.q4adamw_fused_4bit(p.data_ptr(), g.data_ptr(), exp.data_ptr(), sq.data_ptr(),
                                   exp_scale.data_ptr(), sq_scale.data_ptr(), p.numel(),
                                   _tag(p, "param"), _tag(g, "grad"), beta1, beta2, lr,
@@ -104,7 +110,7 @@ def fused_single_tensor(p, g, exp_avg, exp_avg_sq, beta1, beta2, lr, weight_deca
     """optim/cuda_fused_interface.cc:49-64."""
     L = _lib.load()
     check_unquantized(p, g, exp_avg, exp_avg_sq)
-    with torch.cuda.device(p.device):
+    with _on(p.device):
         rc = L.q4adamw_fused_single_tensor(p.data_ptr(), g.data_ptr(), exp_avg.data_ptr(),
                                            exp_avg_sq.data_ptr(), p.numel(), _tag(p, "param"),
                                            _tag(g, "grad"), beta1, beta2, lr, weight_decay, eps,
@@ -209,7 +215,7 @@ def device_step(step, table, consts, beta1, beta2, lr, weight_decay, eps, lr_dev
     assert consts.device == device and consts.numel() * consts.element_size() >= _lib.STEP_CONSTS_BYTES
     lr_ptr = None if lr_dev is None else _device_scalar(lr_dev, device, "lr_dev")
     skip = None if found_inf is None else _device_scalar(found_inf, device, "found_inf")
-    with torch.cuda.device(device):
+    with _on(device):
         rc = L.q4adamw_device_step(step.data_ptr(), table.data_ptr(), 1, table.shape[0], lr_ptr, beta1, beta2,
                                    float(lr), weight_decay, eps, skip, consts.data_ptr(), _stream(device))
     _lib.check(rc, "device_step")
@@ -445,7 +451,7 @@ def grad_norm_table(arr, device, g_tag, out3, workspace, grad_scale=1.0, grad_sc
     assert out3.dtype == torch.float32 and out3.numel() >= 3 and out3.device == device
     assert workspace.device == device and workspace.numel() * workspace.element_size() >= _lib.NORM_WORKSPACE_BYTES
     dev_ptr = None if grad_scale_dev is None else _device_scalar(grad_scale_dev, device, "grad_scale_dev")
-    with torch.cuda.device(device):
+    with _on(device):
         rc = L.q4adamw_grad_norm(arr, len(arr), g_tag, float(grad_scale), dev_ptr, float(max_norm),
                                  workspace.data_ptr(), workspace.numel() * workspace.element_size(),
                                  out3.data_ptr(), _stream(device))
@@ -479,7 +485,7 @@ def quantize_state(x, which):
     nbytes, nblk = state_sizes(x.numel())
     codes = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
     scales = torch.empty(nblk, dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = L.q4adamw_quantize(x.data_ptr(), x.numel(), int(which), codes.data_ptr(),
                                 scales.data_ptr(), _stream(x.device))
     _lib.check(rc, "quantize")
@@ -495,7 +501,7 @@ def dequantize_state(codes, scales, numel, which):
     assert codes.dtype == torch.uint8 and codes.numel() == nbytes and codes.is_contiguous()
     assert scales.dtype == torch.float32 and scales.numel() == nblk and scales.is_contiguous()
     out = torch.empty(numel, dtype=torch.float32, device=codes.device)
-    with torch.cuda.device(codes.device):
+    with _on(codes.device):
         rc = L.q4adamw_dequantize(codes.data_ptr(), scales.data_ptr(), numel, int(which),
                                   out.data_ptr(), _stream(codes.device))
     _lib.check(rc, "dequantize")
@@ -513,7 +519,7 @@ def quantize_state_rank1(x):
     codes = torch.empty((rows * cols + 1) // 2, dtype=torch.uint8, device=x.device)
     row_max = torch.empty(rows, dtype=torch.float32, device=x.device)
     col_max = torch.empty(cols, dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = L.q4adamw_quantize_rank1(x.data_ptr(), rows, cols, codes.data_ptr(), row_max.data_ptr(),
                                       col_max.data_ptr(), _stream(x.device))
     _lib.check(rc, "quantize_rank1")
@@ -531,7 +537,7 @@ def quantize_state_rank1_scaled(x, row_scale, col_max):
     for t, n in ((row_scale, rows), (col_max, cols)):
         assert t.dtype == torch.float32 and t.numel() == n and t.device == x.device and t.is_contiguous()
     codes = torch.empty((rows * cols + 1) // 2, dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = L.q4adamw_quantize_rank1_scaled(x.data_ptr(), rows, cols, row_scale.data_ptr(), col_max.data_ptr(),
                                              codes.data_ptr(), _stream(x.device))
     _lib.check(rc, "quantize_rank1_scaled")
@@ -547,7 +553,7 @@ def dequantize_state_rank1(codes, row_max, col_max):
     for t in (row_max, col_max):
         assert t.dtype == torch.float32 and t.device == codes.device and t.is_contiguous()
     out = torch.empty(rows, cols, dtype=torch.float32, device=codes.device)
-    with torch.cuda.device(codes.device):
+    with _on(codes.device):
         rc = L.q4adamw_dequantize_rank1(codes.data_ptr(), row_max.data_ptr(), col_max.data_ptr(), rows, cols,
                                         out.data_ptr(), _stream(codes.device))
     _lib.check(rc, "dequantize_rank1")
