@@ -4,7 +4,7 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload llama3-8b]
 
 One "step" is one `optimizer.step()` over the whole synthetic parameter set: one
-multi-tensor launch of the fused 4-bit kernel per batch of 48 tensors plus one launch of
+multi-tensor launch of the fused 4-bit kernel per batch of 61 tensors plus one launch of
 the non-quantized kernel for the tensors of at most 4096 elements.  Inputs are resident in
 HBM before the timed region starts.  Prints ONE JSON line:
 
@@ -234,15 +234,15 @@ def run_config(torch, params, grad_sets, p_dtype_s, g_dtype_s, steps, warmup, va
     elapsed = time.perf_counter() - t0
     kernel_timing, opt.kernel_timing = opt.kernel_timing, None
 
-    # one entry per step: the step's fused launches (one kernel per batch of up to 48
+    # one entry per step: the step's fused launches (one kernel per batch of up to 61
     # tensors, back to back on the stream) between two events
     fused_ms = [s.elapsed_time(e) for kind, s, e in kernel_timing if kind.startswith("fused_4bit")]
     avg_kernel_s = sum(fused_ms) / steps / 1e3
     rank1 = [p for p in params if opt.state[p]["variance_qstate"]["overhead"].get("max_dims") is not None]
     grouped = sum(1 for p in params if p.numel() > 4096) - len(rank1)
-    # kernels per step: one per batch of 48 block-scaled tensors; statistics + update +
+    # kernels per step: one per batch of 61 block-scaled tensors; statistics + update +
     # commit per batch of 32 rank-1 tensors
-    launches_per_step = -(-grouped // 48) + 3 * -(-len(rank1) // 32)
+    launches_per_step = -(-grouped // 61) + 3 * -(-len(rank1) // 32)
 
     # Host time of step(): a burst of a few more steps issued into the drained queue, without
     # the timing events (the first two of them untimed: the first launch after an idle
@@ -252,7 +252,7 @@ def run_config(torch, params, grad_sets, p_dtype_s, g_dtype_s, steps, warmup, va
     host_ms_per_step = None
     if host_burst:
         small = sum(1 for p in params if p.numel() <= 4096)
-        burst = max(2, min(steps, 16, 192 // (launches_per_step + -(-small // 80)) - 2))
+        burst = max(2, min(steps, 16, 192 // (launches_per_step + -(-small // 103)) - 2))
         for i in range(2 + burst):
             if i == 2:
                 host_s[0] = 0.0

@@ -163,7 +163,7 @@ int q4adamw_fused_4bit(void *p, const void *g, uint8_t *exp_avg, uint8_t *exp_av
                        float weight_decay, float eps, float step, void *stream);
 
 /*
- * The same step over many tensors: one launch per batch of up to 48 tensors.  All
+ * The same step over many tensors: one launch per batch of up to 61 tensors.  All
  * tensors share dtypes, hyper-parameters and step.  `tensors` is a host array that
  * is read before the call returns.  Replaces the reference's per-parameter Python
  * loop around fused_4bit (optim/fused_quantfour.py:171-292).
@@ -279,7 +279,7 @@ int q4adamw_fused_single_tensor(void *p, const void *g, float *exp_avg, float *e
                                 float beta2, float lr, float weight_decay, float eps,
                                 float step, void *stream);
 
-/* Many non-quantized tensors, one launch per batch of up to 80 (`tensors` is a host array). */
+/* Many non-quantized tensors, one launch per batch of up to 103 (`tensors` is a host array). */
 int q4adamw_fused_single_tensor_multi(const q4adamw_small_tensor *tensors, int count,
                                       int p_dtype, int g_dtype, float beta1, float beta2,
                                       float lr, float weight_decay, float eps, float step,

@@ -289,6 +289,16 @@ constexpr bool sr_fixed_in_binade() {
 }
 static_assert(sr_fixed_in_binade(), "a constant's rounding must be that of [128, 256)");
 
+// the same map as sr_affine_m, negated and shifted: equal slopes, constants within both roundings
+constexpr bool sr_fixed_matches() {
+  for (uint32_t k = 0; k < 17; ++k) {
+    const double d = (double)sr_fixed_m(k).c - (kSrFixedTop - (double)sr_affine_m(k).c);
+    if (sr_fixed_m(k).a != -sr_affine_m(k).a || d > 8.2e-6 || d < -8.2e-6) return false;   // 2^-17 + 2^-21
+  }
+  return true;
+}
+static_assert(sr_fixed_matches(), "two forms of one table");
+
 // The error of the affine form, in units of one code, is the quotient's relative error
 // times |q| / width: the guard band of the fast path is sized for a ratio below 9.
 constexpr bool sr_affine_ratio_ok() {
