@@ -329,10 +329,11 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1S
 // nearly all of the second dimension each (on 20 such stacks, 11 million elements, a kernel
 // with those tiles took 23 us without its updates and 64 us with them).  So a tile is
 // two-dimensional: kLeadOuter indices of the first dimension times a run of at most 256
-// consecutive elements below it (whole rows), which meets 16 indices of the first dimension and
-// a few dozen of the second: 30 to 37 us, against 5.7 ms for statistics and folds before.
+// consecutive elements below it (whole rows), which meets 32 indices of the first dimension and
+// a few dozen of the second, 16 elements of a thread in flight: 26 to 30 us (16 indices 31 to 38,
+// 8 indices 42 to 49, 64 indices 34 to 44), against 5.7 ms for statistics and folds before.
 // A thread keeps one element of the run over the first dimension's indices.
-constexpr uint32_t kLeadOuter = 16;
+constexpr uint32_t kLeadOuter = 32;
 
 struct LeadTiles {
   uint32_t inner_rows;   // rows below one index of the first dimension
@@ -351,7 +352,7 @@ __host__ __device__ __forceinline__ LeadTiles lead_tiles(uint32_t rows, uint32_t
 
 template <int GT, bool EXT>
 __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1StatArgs args) {
-  constexpr int kAhead = 8;   // elements of a thread whose loads are in flight together
+  constexpr int kAhead = 16;   // elements of a thread whose loads are in flight together
   __shared__ uint32_t outer_bits[kThreads / 16][kLeadOuter];   // first dimension: each 16 lanes' maxima
   __shared__ uint32_t slots[3][256];                           // second and third dimension, columns
   const uint32_t chunk = args.chunk_base + blockIdx.x;
