@@ -71,7 +71,8 @@ struct ChunkRuns {
 
 // Runs of 1024 chunks in grids where every XCD gets 64 of them, otherwise of 64 or, in grids too small
 // for 64 of those, the longest that leave every XCD 64.  Against 64 (and four of them at least)
-// everywhere, medians on one box: the Llama-3-8B set 15.58 -> 15.53 ms (one eighth of the grid per XCD: 15.60), its
+// everywhere, medians on one box: the Llama-3-8B set 15.58 -> 15.53 ms (one eighth of the grid per XCD: 15.60; in
+// two other jobs, in which it was up to 0.8 % the faster, 15.53 and 15.72 against 15.64 and 15.79), its
 // layers and tables with rank-1 scaling 4504 -> 4475 us, Llama-2-13B layers with stochastic rounding
 // 2171 -> 2159, the 4096 x 4096 tensor (runs of 32) 38.2 -> 36.5 to 38.4; GPT-2-small keeps 64
 // (353; 128 357, 512 354).
