@@ -405,6 +405,11 @@ __device__ __forceinline__ uint32_t fixed_code_v(float v, float neg_inv16) {
   return g;
 }
 
+// g with a 16-bit noise number added.  A number's sum stays below 0x43210002; a NaN whose upper half is
+// all ones would leave the 32 bits and come back as a small number (code 15), so the sum saturates:
+// 0xffffffff is a NaN still.
+__device__ __forceinline__ uint32_t add_noise(uint32_t g, uint32_t n16) { return __builtin_elementwise_add_sat(g, n16); }
+
 // The lesser of the low halves of least and g, in the low half (2 cycles each; v_min3_u16 takes 8).
 __device__ __forceinline__ void min_low_half(uint32_t &least, uint32_t g) {
   asm("v_min_u16 %0, %0, %1" : "+v"(least) : "v"(g));

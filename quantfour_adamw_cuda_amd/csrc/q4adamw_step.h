@@ -448,7 +448,7 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
       for (int h = 0; h < 2; ++h) {
         const uint32_t interval = high_half_if_ge(qq[h], bits2f(ent[h].x), ent[h].y);   // byte offset into the affine table
         const float2 af = *reinterpret_cast<const float2 *>(lds_bytes + kLdsIntervals * 8u + interval);
-        mg[j + h] = f2bits(__builtin_fmaf(qq[h], af.x, af.y)) + hash_high_half(noise[j + h]);
+        mg[j + h] = add_noise(f2bits(__builtin_fmaf(qq[h], af.x, af.y)), hash_high_half(noise[j + h]));
         min_low_half(m_near, mg[j + h]);
       }
     } else {
@@ -467,7 +467,7 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     for (int k = j; k < j + 2; ++k) {
       const float inv = RANK1 ? neg_inv16.x[k] : neg_rv16;
       vg[k] = fixed_code_v<SR>(vn.x[k], inv);
-      if constexpr (SR) vg[k] += hash_low_half(noise[k]);
+      if constexpr (SR) vg[k] = add_noise(vg[k], hash_low_half(noise[k]));
       min_low_half(v_near, vg[k]);
     }
   }

@@ -7,6 +7,7 @@ import torch
 
 import quantfour_adamw_cuda_amd as q4
 from oracle import q4_oracle as oc
+from oracle import q4_oracle_torch as ot
 from tests.q4_testlib import HP, DeviceTensor, OracleTensor, assert_state_equal, bits
 
 pytestmark = pytest.mark.gpu
@@ -94,3 +95,50 @@ def test_nan_payloads(cuda, pattern, grads):
     ref.step(g.float(), 1)
     assert np.array_equal(dev.m.cpu().numpy(), ref.m) and np.array_equal(dev.v.cpu().numpy(), ref.v)
     assert np.array_equal(bits(dev.sm.cpu().numpy()), bits(ref.sm)) and np.array_equal(bits(dev.sv.cpu().numpy()), bits(ref.sv))
+
+
+# every payload whose upper half is all ones reaches the noise's addition at the top of the 32-bit range
+ONES = {"float32": (torch.int32, torch.float32, [0xFFFFFFFF, 0xFFFF8001, 0x7FFFFFFF, 0xFFC00001]),
+        "bfloat16": (torch.int16, torch.bfloat16, [0xFFFF]), "float16": (torch.int16, torch.float16, [0xFFFF, 0x7FFF])}
+
+
+@pytest.mark.parametrize("rank1", [False, True])
+@pytest.mark.parametrize("p_dt", ["float32", "float16"])
+@pytest.mark.parametrize("g_dt,pattern", [(k, x) for k, v in ONES.items() for x in v[2]])
+def test_nan_payloads_stochastic(cuda, g_dt, pattern, p_dt, rank1):
+    """stochastic rounding: code 0 for a NaN moment, single elements, half a row and whole blocks of them"""
+    ints, dt, _ = ONES[g_dt]
+    rows, cols, seed = 96, 768, 0x1234_5678_9ABC
+    gen = torch.Generator().manual_seed(pattern & 0xFFFF)
+    p = (torch.randn(rows, cols, generator=gen) * 0.02).to(getattr(torch, p_dt))
+    g = (torch.randn(rows, cols, generator=gen) * 1e-3).to(dt)
+    bits_ = g.view(ints)
+    value = pattern - (1 << (32 if ints is torch.int32 else 16)) if pattern >> (31 if ints is torch.int32 else 15) else pattern
+    bits_[torch.rand(rows, cols, generator=gen) < 0.02] = value
+    bits_[5, :384] = value
+    bits_[40:42] = value
+    n = rows * cols
+    zeros = lambda k, d=torch.float32: torch.zeros(k, dtype=d)
+    nbytes, nblk = oc.state_sizes(n)
+    m, v, sm = zeros(nbytes, torch.uint8), zeros(nbytes, torch.uint8), zeros(nblk)
+    hpa = (HP["beta1"], HP["beta2"], HP["lr"], HP["weight_decay"], HP["eps"], 1)
+    g32 = torch.where(torch.isnan(g.float()), torch.nan, g.float())
+    with np.errstate(invalid="ignore"):
+        if rank1:
+            want = ot.step_quant_rank1_sr(p, g32, m, v, sm, zeros(rows), zeros(cols), step=1, seed=seed, tensor_salt=0, **HP)[1:]
+        else:
+            want = ot.step_quant_sr(p.view(-1), g32.view(-1), m, v, sm, zeros(nblk), step=1, seed=seed, tensor_salt=0, **HP)[1:]
+    d = lambda t: t.clone().to(cuda)
+    if rank1:
+        got = [d(m), d(v), d(sm), d(zeros(rows)), d(zeros(cols))]
+        q4.quantfour_hip.fused_4bit_rank1_multi([d(p)], [d(g)], *[[t] for t in got], [d(zeros(rows))], [d(zeros(cols))], *hpa, seed=seed)
+    else:
+        got = [d(m), d(v), d(sm), d(zeros(nblk))]
+        q4.quantfour_hip.fused_4bit_multi_sr([d(p).view(-1)], [d(g).view(-1)], *[[t] for t in got], *hpa, seed)
+    names = ("m codes", "v codes", "m scales", "v scales or rows", "columns")
+    for name, a, b in zip(names, got, want):
+        a, b = a.cpu(), b.reshape(-1)
+        if a.dtype == torch.float32:
+            a, b = a.view(torch.int32), b.contiguous().view(torch.int32)
+        bad = torch.nonzero(a != b).reshape(-1)
+        assert bad.numel() == 0, f"{name}: {bad.numel()} differ, first {bad[:4].tolist()}: {a[bad[:4]].tolist()} for {b[bad[:4]].tolist()}"
