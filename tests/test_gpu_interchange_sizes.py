@@ -68,3 +68,27 @@ def test_matrices(cuda, rows, cols):
     back = q.dequantize_state_rank1(codes, rmax, cmax)
     want = ot.dequantize_rank1(rc, rr, rcm)
     assert torch.equal(back.cpu().reshape(-1).view(torch.int32), want.reshape(-1).view(torch.int32))
+
+
+@pytest.mark.parametrize("rows,cols", [(64, 40), (33, 7), (9, 1030)])
+def test_statistics_that_are_no_maxima(cuda, rows, cols):
+    """A caller's row and column scales are taken as numbers: the lesser of the two is the scale also
+    where one of them is negative or -0.0, and a NaN beside a number gives way to it."""
+    gen = torch.Generator().manual_seed(rows)
+    x = grads_config1(gen, rows * cols).square().view(rows, cols)
+    r, c = torch.rand(rows, generator=gen) * 1e-2 + 1e-3, torch.rand(cols, generator=gen) * 1e-2 + 1e-3
+    r[3], r[5], r[7] = -0.0, -1e-3, float("nan")
+    c[2], c[4], c[6] = -0.0, -2e-3, float("nan")
+    scale = torch.fmin(r[:, None].expand(rows, cols), c[None, :].expand(rows, cols))
+    codes = torch.randint(0, 256, ((rows * cols + 1) // 2,), dtype=torch.uint8, generator=gen)
+    if rows * cols % 2:
+        codes[-1] &= 15
+    nibbles = torch.stack((codes & 15, codes >> 4), 1).reshape(-1)[:rows * cols].long()
+    want = (ot.QMAP[1][nibbles] * scale.reshape(-1)).view(rows, cols)
+    got = q.dequantize_state_rank1(codes.to(cuda), r.to(cuda), c.to(cuda)).cpu()
+    number = ~torch.isnan(want)
+    assert torch.equal(torch.isnan(got), ~number)
+    assert torch.equal(got[number].view(torch.int32), want[number].view(torch.int32))
+    want = torch.bucketize(torch.nan_to_num(x.div(scale), nan=-2.0, posinf=float("inf")), ot.QMID[1], right=False)
+    got = q.quantize_state_rank1_scaled(x.to(cuda), r.to(cuda), c.to(cuda)).cpu()
+    assert torch.equal(got, ot.pack(want.reshape(-1), rows * cols))
