@@ -316,15 +316,19 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     // the embedding's rows never touched took 3870 us a step instead of 3700.
     const bool in_range = m_least >= kExactLo && am <= kExactHi && v_least >= kExactVLo && av <= kExactVHi;
     if (__builtin_expect(!(sc.exact_short != 0u && in_range), 0)) {
-      // exact_short and a finite step size: eps and c2s keep every denominator positive and finite
-      bool general = sc.exact_short == 0u || !(sc.ss <= kStepSizeHi), nonzero = false;
+      // exact_short and a finite step size: eps and c2s keep every denominator positive and finite.
+      // A lane outside the ranges without a first moment of zero needs no look at its elements:
+      // gradients of 1e-25 (5e7 fp32 elements: 137 us with the look, 128 without)
+      bool general = sc.exact_short == 0u || !(sc.ss <= kStepSizeHi) || m_least > 0.0f, nonzero = m_least > 0.0f;
+      if (!nonzero) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
-        const float m = mn.x[j], v = vn.x[j], size = __builtin_fabsf(m);
-        const bool zero = m == 0.0f && v >= 0.0f && v <= kExactVHi;
-        general |= !zero && !(size >= kExactLo && size <= kExactHi && v >= kExactVLo && v <= kExactVHi);
-        nonzero |= !(m == 0.0f && v == 0.0f);
-        if (zero) p_new[j] = p[j] * wdu - m;
+        for (int j = 0; j < N; ++j) {
+          const float m = mn.x[j], v = vn.x[j], size = __builtin_fabsf(m);
+          const bool zero = m == 0.0f && v >= 0.0f && v <= kExactVHi;
+          general |= !zero && !(size >= kExactLo && size <= kExactHi && v >= kExactVLo && v <= kExactVHi);
+          nonzero |= !(m == 0.0f && v == 0.0f);
+          if (zero) p_new[j] = p[j] * wdu - m;
+        }
       }
       if (general) {
 #pragma unroll

@@ -97,6 +97,19 @@ def test_nan_payloads(cuda, pattern, grads):
     assert np.array_equal(bits(dev.sm.cpu().numpy()), bits(ref.sm)) and np.array_equal(bits(dev.sv.cpu().numpy()), bits(ref.sv))
 
 
+@pytest.mark.parametrize("value", [1e-44, 1e-38, 1e-25, 1e-20, 1e18, 1e19])
+@pytest.mark.parametrize("zeros", [0.0, 0.1])
+def test_moments_out_of_range(cuda, value, zeros):
+    """lanes all of whose moments lie outside the short sequences' ranges, with and without zeros among them"""
+    n = 4096 + 37
+    gen = torch.Generator().manual_seed(6)
+    dev, ref = _pair(n, gen, cuda)
+    for step in (1, 2, 3):
+        g = (torch.rand(n, generator=gen) + 0.5) * value * torch.sign(torch.randn(n, generator=gen))
+        g[torch.rand(n, generator=gen) < zeros] = 0.0
+        _step(dev, ref, g, cuda, step, f"{value}, step {step}")
+
+
 # every payload whose upper half is all ones reaches the noise's addition at the top of the 32-bit range
 ONES = {"float32": (torch.int32, torch.float32, [0xFFFFFFFF, 0xFFFF8001, 0x7FFFFFFF, 0xFFC00001]),
         "bfloat16": (torch.int16, torch.bfloat16, [0xFFFF]), "float16": (torch.int16, torch.float16, [0xFFFF, 0x7FFF])}
