@@ -219,17 +219,21 @@ static uint64_t rank1_chunks(const q4adamw_rank1_tensor &t, int64_t tile_elems) 
   return ((uint64_t)t.rows * (uint64_t)t.cols + chunk_elems - 1) / chunk_elems;
 }
 
-// Which statistics kernel a matrix takes.  Flat: fewer columns than a wave of the wide form's
-// lanes could share (below that a lane per column or per 8 columns leaves lanes without work: of a
-// 786432 x 3 matrix 3 of 256, which took 260 us; of a 4096 x 16 one 2 of 64).  Wide: 8 columns per lane; rows that are no
-// multiple of 8 long take the variant that finds their codes at either nibble.  Lead: as flat, for
-// tensors with several leading dimensions.
+// Which statistics kernel a matrix takes.  Flat: rows too short for the wide forms' lanes of 8 columns
+// each (of a 786432 x 3 matrix a lane per column left 3 of 256 with work, which took 260 us; of a 4096 x 16
+// one 2 of 64).  Wide: rows of 8 columns per lane from 96 columns on, where its 16-byte loads and larger tiles
+// outweigh the idle lanes: statistics of 100000 and 1000000 fp32 rows, us, flat / wide, 64 columns 26 / 34 and
+// 91 / 127, 80 columns 34 / 33 and 112 / 130, 96 columns 38 / 33 and 130 / 135, 128 columns 39 / 34 and
+// 151 / 146, 192 columns 60 / 34 and 239 / 188.  Rows that are no
+// multiple of 8 long take the variant that finds their codes at either nibble, above 256 columns.  Lead: as
+// flat, for tensors with several leading dimensions.
 enum Rank1StatForm { kStatFlat = 0, kStatLead = 1, kStatWide = 2, kStatWideAny = 3, kStatForms = 4 };
 
 static bool rank1_has_leads(const q4adamw_rank1_tensor &t) { return t.lead_dims >= 2; }
 
 static Rank1StatForm rank1_stat_form(const q4adamw_rank1_tensor &t) {
-  if (t.cols <= (int64_t)kFlatMaxCols) return rank1_has_leads(t) ? kStatLead : kStatFlat;
+  if (rank1_has_leads(t) && t.cols <= (int64_t)kFlatMaxCols) return kStatLead;
+  if (t.cols <= (int64_t)(t.cols % 8 == 0 ? kFlatMaxCols8 : kFlatMaxCols)) return kStatFlat;
   return t.cols % 8 == 0 ? kStatWide : kStatWideAny;
 }
 
@@ -248,19 +252,27 @@ static Rank1StatKernel pick_rank1_stats(Rank1StatForm form, int g_dtype, bool ex
   return ext ? pick_rank1_stats_form<Q4ADAMW_FP32, true>(form) : pick_rank1_stats_form<Q4ADAMW_FP32, false>(form);
 }
 
-// Rows of a wide form's tile in a launch over `elements` elements: 256 if that makes four
-// workgroups per CU, else as few as 32.
-static uint32_t rank1_stat_rows(uint64_t elements) {
-  uint32_t rows = kStatRows;
-  while (rows > 32u && elements / ((uint64_t)rows * kStatCols) < 1024u) rows /= 2u;
+// Rows whose statistics one workgroup takes together, in a launch over `elements` elements of matrices
+// of at most `tallest` rows.  Two costs meet.  A wave walks a quarter of the rows, four at a time with
+// nothing else in flight, about 0.09 us a row: 6 us with 32 rows, 26 with 256, which a launch with workgroups to
+// spare hides.  And every workgroup updates the statistic of every column it meets; updates of one address
+// are taken one after another, 20 ns each.  So 256 where that makes four workgroups per CU, else as few
+// as 32, but no fewer than a sixth of the rows' square root calls for, where the two costs balance.
+// Statistics of one fp32 matrix with 32, 64, 128, 256 rows, us: 4000 x 512 8.6, 10.9, 17.4, 29.1;
+// 16000 x 264 15.4, 13.4, 16.8, 28.4; 50257 x 264 38.6, 30.4, 23.8, 29.7; 100000 x 264 68.1, 45.6, 41.6, 35.6;
+// 300000 x 264 187, 112, 87, 85.
+static uint32_t rank1_stat_rows(uint64_t elements, uint64_t tallest) {
+  uint32_t rows = kStatRows, least = 32u;
+  while (least < (uint32_t)kStatRows && tallest > 6ull * least * least) least *= 2u;
+  while (rows > least && elements / ((uint64_t)rows * kStatCols) < 1024u) rows /= 2u;
   return rows;
 }
 
 // tiles of the statistics launch of a matrix
 static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_rows) {
   if (rank1_stat_form(t) == kStatFlat) {
-    const uint64_t tile_rows = flat_tile_rows((uint32_t)t.cols);
-    return ((uint64_t)t.rows + tile_rows - 1) / tile_rows;
+    const uint64_t rows = (uint64_t)flat_tile_rows((uint32_t)t.cols) * flat_tiles((uint32_t)t.cols, stat_rows);
+    return ((uint64_t)t.rows + rows - 1) / rows;
   }
   if (rank1_stat_form(t) == kStatLead) {
     const uint32_t outer = (uint32_t)t.lead_shape[0];
@@ -589,11 +601,13 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
     auto in_pass = [&](const q4adamw_rank1_tensor &t) {
       return t.rows != 0 && t.cols != 0 && rank1_shape(t, tile_elems) == shape && rank1_stat_form(t) == form;
     };
-    uint64_t pass_elements = 0;
+    uint64_t pass_elements = 0, tallest = 0;
     for (int i = 0; i < count; ++i) {
-      if (in_pass(tensors[i])) pass_elements += (uint64_t)(tensors[i].rows * tensors[i].cols);
+      if (!in_pass(tensors[i])) continue;
+      pass_elements += (uint64_t)(tensors[i].rows * tensors[i].cols);
+      tallest = (uint64_t)tensors[i].rows > tallest ? (uint64_t)tensors[i].rows : tallest;
     }
-    sa.stat_rows = rank1_stat_rows(pass_elements);
+    sa.stat_rows = rank1_stat_rows(pass_elements, tallest);
     kernel = nullptr;
     for (int i = 0; i < count && pass_elements != 0; ++i) {
       const q4adamw_rank1_tensor &t = tensors[i];
@@ -982,7 +996,7 @@ int q4adamw_quantize_rank1(const float *x, int64_t rows, int64_t cols, uint8_t *
   t.cols = cols;
   Rank1StatArgs sa = {};
   const Rank1StatForm form = rank1_stat_form(t);
-  sa.stat_rows = rank1_stat_rows((uint64_t)rows * (uint64_t)cols);
+  sa.stat_rows = rank1_stat_rows((uint64_t)rows * (uint64_t)cols, (uint64_t)rows);
   sa.desc[0].g = x;
   sa.desc[0].rmax_next = row_max;
   sa.desc[0].cmax_next = col_max;

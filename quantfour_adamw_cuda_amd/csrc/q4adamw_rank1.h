@@ -89,7 +89,7 @@ constexpr int kStatCols = 512;           // columns per workgroup: 8 per lane
 // 64 rows with four times as many of them took 1.25 to 2 times as long).  A wave walks 64 rows
 // where the launch has workgroups enough for the chip (args.stat_rows = 256) and fewer in a
 // small launch, which would otherwise wait for one wave's 16 rounds of loads (one 1000 x 512
-// matrix: 30 us with 64 rows per wave).
+// matrix: 30 us with 64 rows per wave); how many rows, and why, is said where the launch decides.
 // ANY: rows of any length (at least 8).  A row may then start at either nibble of a byte of the
 // codes, and the lane that would run past the row's end works on the row's last 8 columns
 // instead: maxima do not mind columns seen twice.
@@ -236,21 +236,31 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
   fold_rows(T, tile_row0, (uint32_t)tile_rows, row_bits[0], row_bits[1]);
 }
 
-// The same statistics for matrices of fewer than kFlatMaxCols columns: a workgroup takes
-// as many whole rows as fit a tile of kFlatWords elements (an odd row pitch, so that a walk
-// along rows and one across them meet all banks) and reads them as one run of consecutive
-// elements: thread t's elements are t, t + k * cols, t + 2 * k * cols, ... (k rows a time), all of
+// The same statistics for matrices of up to kFlatMaxCols columns: a tile is as many whole rows as fit
+// kFlatWords elements (an odd row pitch, so that a walk along rows and one across them meet all
+// banks), read as one run of consecutive elements: thread t's elements are t, t + k * cols,
+// t + 2 * k * cols, ... (k rows a time), all of
 // one column, whose maximum stays in a register.  The second moments meet the rows in LDS:
 // a thread per row, or several where the tile has fewer than 256 rows.  A row lies in one
 // workgroup, so its maximum is stored without an atomic.
 // The forms it replaces here gave a lane to every column or to every 8th of them: with 3 columns
 // (the last dimension of a 3x3 convolution kernel) 3 of 256 threads had work.
+// In tall matrices a workgroup takes one tile after another until it has the rows of a wide form's tile
+// (stat_rows), for the same reason, the updates of the columns' statistics: of an fp32 matrix of 100000 x 64
+// 41 us with one tile, 26 with four; of four of 50000 x 64 75 and 38; of one of 1000000 x 100 154 and 143.
 // Same arithmetic, operation for operation.
-constexpr uint32_t kFlatMaxCols = 256;
+constexpr uint32_t kFlatMaxCols = 256, kFlatMaxCols8 = 88;   // the latter for multiples of 8
 constexpr uint32_t kFlatWords = 4096;
 constexpr uint32_t kFlatMaxRows = kFlatWords / 3;     // up to 3 columns: a pitch of 3 words
 
 __host__ __device__ __forceinline__ uint32_t flat_tile_rows(uint32_t cols) { return cols < 3u ? kFlatMaxRows : kFlatWords / (cols | 1u); }
+
+// tiles of a workgroup (one in short matrices, where they would only wait for each other: 1000 x 255 7.2 us
+// with one, 9.8 with two)
+__host__ __device__ __forceinline__ uint32_t flat_tiles(uint32_t cols, uint32_t stat_rows) {
+  const uint32_t tiles = stat_rows / flat_tile_rows(cols);
+  return stat_rows > 32u && tiles > 1u ? tiles : 1u;
+}
 
 template <int GT_, bool EXT>
 __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1StatArgs args) {
@@ -265,61 +275,66 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1S
   if (EXT && !grad_ops_begin(args.go, gscale)) return;
   const int t = find_tensor(args, chunk);
   const auto &T = args.desc[t];
-  const uint32_t tid = threadIdx.x, cols = T.cols, pitch = cols | 1u;
-  const uint32_t row0 = (chunk - args.first_chunk[t]) * flat_tile_rows(cols);
-  const uint32_t n = T.rows - row0 < flat_tile_rows(cols) ? T.rows - row0 : flat_tile_rows(cols);
-  const uint32_t parts = n >= (uint32_t)kThreads ? 1u : (uint32_t)kThreads / n;   // threads per row
+  const uint32_t tid = threadIdx.x, cols = T.cols, pitch = cols | 1u, tile_rows = flat_tile_rows(cols);
+  const uint32_t tiles = flat_tiles(cols, args.stat_rows), tile0 = (chunk - args.first_chunk[t]) * tiles;
   if (tid < cols) col_bits[tid] = 0u;
-  if (parts > 1u && tid < n) row_bits[tid] = 0u;
 
   const uint32_t rows_per_pass = (uint32_t)kThreads / cols;
   const uint32_t r_first = tid / cols, col = tid - r_first * cols;
-  const bool active = r_first < rows_per_pass && r_first < n;
-  const int64_t first = (int64_t)row0 * cols;                 // the tile's first element
-  const void *g_tile = static_cast<const char *>(T.g) + first * (GT ? 2 : 4);
-  const uint8_t *v_tile = T.v + (first >> 1);
-  const uint32_t odd = (uint32_t)first & 1u;
   float c_max = 0.0f;
-  if (active) {
-    const float c_old = kAbs ? 0.0f : as_global<const float>(T.cmax)[col];
-    for (uint32_t r0 = r_first; r0 < n; r0 += kAhead * rows_per_pass) {
-      float g[kAhead], r_old[kAhead];
-      uint32_t byte[kAhead];
+  const float c_old = kAbs ? 0.0f : as_global<const float>(T.cmax)[col];
+  for (uint32_t k = 0; k < tiles; ++k) {
+    const uint32_t row0 = (tile0 + k) * tile_rows;
+    if (row0 >= T.rows) break;                                // the first tile is always there
+    const uint32_t n = T.rows - row0 < tile_rows ? T.rows - row0 : tile_rows;
+    const uint32_t parts = n >= (uint32_t)kThreads ? 1u : (uint32_t)kThreads / n;   // threads per row
+    if (k != 0u) __syncthreads();                             // the last tile's row maxima have been read
+    if (parts > 1u && tid < n) row_bits[tid] = 0u;
+    const int64_t first = (int64_t)row0 * cols;               // the tile's first element
+    const void *g_tile = static_cast<const char *>(T.g) + first * (GT ? 2 : 4);
+    const uint8_t *v_tile = T.v + (first >> 1);
+    const uint32_t odd = (uint32_t)first & 1u;
+    if (r_first < rows_per_pass) {
+      for (uint32_t r0 = r_first; r0 < n; r0 += kAhead * rows_per_pass) {
+        float g[kAhead], r_old[kAhead];
+        uint32_t byte[kAhead];
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        uint32_t r = r0 + (uint32_t)i * rows_per_pass;
-        r = r < n ? r : r0;                                  // past the tile: a row seen already
-        const uint32_t e = r * cols + col;
-        g[i] = load_scalar<GT>(g_tile, e);
-        byte[i] = kAbs ? 0u : as_global<const uint8_t>(v_tile)[(e + odd) >> 1];
-        r_old[i] = kAbs ? 0.0f : as_global<const float>(T.rmax)[row0 + r];
-      }
+        for (int i = 0; i < kAhead; ++i) {
+          uint32_t r = r0 + (uint32_t)i * rows_per_pass;
+          r = r < n ? r : r0;                                  // past the tile: a row seen already
+          const uint32_t e = r * cols + col;
+          g[i] = load_scalar<GT>(g_tile, e);
+          byte[i] = kAbs ? 0u : as_global<const uint8_t>(v_tile)[(e + odd) >> 1];
+          r_old[i] = kAbs ? 0.0f : as_global<const float>(T.rmax)[row0 + r];
+        }
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        uint32_t r = r0 + (uint32_t)i * rows_per_pass;
-        r = r < n ? r : r0;
-        const float gi = EXT ? g[i] * gscale : g[i];
-        const uint32_t code = (byte[i] >> (4u * ((r * cols + col + odd) & 1u))) & 15u;
-        const float code_value = __builtin_fmaf((float)code, 0.0625f, 0.0625f);  // (code + 1) / 16, exact
-        const float v_old = code_value * min_nonneg(r_old[i], c_old);
-        const float v = __builtin_fmaxf(kAbs ? __builtin_fabsf(gi) : args.b2 * v_old + args.r2 * (gi * gi), 0.0f);   // a NaN never becomes a maximum
-        c_max = __builtin_fmaxf(c_max, v);
-        tile[r * pitch + col] = v;
+        for (int i = 0; i < kAhead; ++i) {
+          uint32_t r = r0 + (uint32_t)i * rows_per_pass;
+          r = r < n ? r : r0;
+          const float gi = EXT ? g[i] * gscale : g[i];
+          const uint32_t code = (byte[i] >> (4u * ((r * cols + col + odd) & 1u))) & 15u;
+          const float code_value = __builtin_fmaf((float)code, 0.0625f, 0.0625f);  // (code + 1) / 16, exact
+          const float v_old = code_value * min_nonneg(r_old[i], c_old);
+          const float v = __builtin_fmaxf(kAbs ? __builtin_fabsf(gi) : args.b2 * v_old + args.r2 * (gi * gi), 0.0f);   // a NaN never becomes a maximum
+          c_max = __builtin_fmaxf(c_max, v);
+          tile[r * pitch + col] = v;
+        }
       }
     }
+    __syncthreads();
+    for (uint32_t i = tid; i < n * parts; i += kThreads) {
+      const uint32_t r = i / parts, part = i - r * parts;
+      float r_max = 0.0f;
+      for (uint32_t c = part; c < cols; c += parts) r_max = __builtin_fmaxf(r_max, tile[r * pitch + c]);
+      if (parts == 1u) row_bits[r] = f2bits(r_max);
+      else if (r_max != 0.0f) atomicMax(&row_bits[r], f2bits(r_max));
+    }
+    __syncthreads();
+    for (uint32_t r = tid; r < n; r += kThreads) as_global<uint32_t>(T.rmax_next)[row0 + r] = row_bits[r];
   }
-  __syncthreads();
-  if (active && c_max != 0.0f) atomicMax(&col_bits[col], f2bits(c_max));
-  for (uint32_t i = tid; i < n * parts; i += kThreads) {
-    const uint32_t r = i / parts, part = i - r * parts;
-    float r_max = 0.0f;
-    for (uint32_t c = part; c < cols; c += parts) r_max = __builtin_fmaxf(r_max, tile[r * pitch + c]);
-    if (parts == 1u) row_bits[r] = f2bits(r_max);
-    else if (r_max != 0.0f) atomicMax(&row_bits[r], f2bits(r_max));
-  }
+  if (r_first < rows_per_pass && c_max != 0.0f) atomicMax(&col_bits[col], f2bits(c_max));
   __syncthreads();
   if (tid < cols && col_bits[tid] != 0u) raise_max(T.cmax_next + tid, col_bits[tid]);
-  for (uint32_t r = tid; r < n; r += kThreads) as_global<uint32_t>(T.rmax_next)[row0 + r] = row_bits[r];
 }
 
 // The same for tensors with several leading dimensions and fewer than kFlatMaxCols columns (a
