@@ -3,8 +3,12 @@ flat form up to 256 columns, or 88 where they are a multiple of 8 (a tile is 409
 the wide forms above it, and the leading statistics of tensors with several
 leading dimensions, whose rows fill part of a tile, one tile or several."""
 import pytest
+import torch
 
+from oracle import q4_oracle_torch as ot
+from quantfour_adamw_cuda_amd import quantfour_hip as q
 from tests import test_gpu_rank1 as base
+from tests.q4_testlib import HP, grads_config1
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +39,44 @@ def test_statistics_of_a_tall_matrix(cuda, shape, p_dt, g_dt):
 @pytest.mark.parametrize("shape", TENSORS)
 def test_statistics_of_several_dimensions(cuda, shape, p_dt, g_dt):
     base.test_rank1_more_than_two_dimensions_against_oracle(cuda, shape, p_dt, g_dt, False)
+
+
+@pytest.mark.parametrize("p_dt,g_dt", [("fp32", "bf16"), ("bf16", "bf16")])
+@pytest.mark.parametrize("copies", [1, 9])
+def test_one_list_of_every_form(cuda, copies, p_dt, g_dt):
+    """Matrices and tensors of every statistics kernel side by side in one call, several kinds to a batch, in
+    one batch of an update kernel and in more: each equals the oracle's, and the steps are the same as one by one."""
+    shapes = [(40, 64), (3, 5, 64), (36, 400), (33, 77), (30, 301), (4, 6, 7), (66, 1024), (20, 520), (2, 9, 264), (5, 3, 3, 3)] * copies
+    gen = torch.Generator().manual_seed(copies)
+    z = lambda n, dt=torch.float32: torch.zeros(n, dtype=dt, device=cuda)
+
+    def state(p):
+        n, cols = p.numel(), p.shape[-1]
+        lead = [z(d) for d in p.shape[:-1]] if p.dim() > 2 else None
+        return dict(p=p.clone().to(cuda), m=z((n + 1) // 2, torch.uint8), v=z((n + 1) // 2, torch.uint8), sm=z((n + 127) // 128),
+                    r=z(n // cols), c=z(cols), rn=z(n // cols), cn=z(cols), lead=lead and (lead, [torch.zeros_like(x) for x in lead]))
+
+    def call(ss, gs, step):
+        pick = lambda k: [s[k] for s in ss]
+        q.fused_4bit_rank1_multi(pick("p"), [g.clone() for g in gs], pick("m"), pick("v"), pick("sm"), pick("r"), pick("c"), pick("rn"),
+                                 pick("cn"), *base.HPA, step, leads=pick("lead"))
+
+    ps = [(torch.randn(s, generator=gen) * 0.05).to(base.DT[p_dt]) for s in shapes]
+    together, alone = [state(p) for p in ps], [state(p) for p in ps]
+    refs = [(p, z((p.numel() + 1) // 2, torch.uint8).cpu(), z((p.numel() + 1) // 2, torch.uint8).cpu(), z((p.numel() + 127) // 128).cpu(),
+             [torch.zeros([p.shape[j] if d == j else 1 for d in range(p.dim())]) for j in range(p.dim())]) for p in ps]
+    for step in (1, 2):
+        gs = [grads_config1(gen, p.numel()).view(p.shape).to(base.DT[g_dt]) for p in ps]
+        dev = [g.to(cuda) for g in gs]
+        call(together, dev, step)
+        for i, s in enumerate(alone):
+            call([s], [dev[i]], step)
+            refs[i] = ot.step_quant_rank1_nd(refs[i][0], gs[i], *refs[i][1:], step=step, **HP)
+            t = together[i]
+            for k in ("p", "m", "v", "sm", "r", "c"):
+                assert torch.equal(s[k].view(torch.uint8), t[k].view(torch.uint8)), f"{shapes[i]} step {step}: {k} alone and together"
+            assert torch.equal(t["m"].cpu(), refs[i][1]) and torch.equal(t["v"].cpu(), refs[i][2]), f"{shapes[i]} step {step}: codes"
+            stats = (t["lead"][0] if t["lead"] else [t["r"]]) + [t["c"]]
+            for have, want in zip(stats, refs[i][4]):
+                assert torch.equal(have.cpu().view(torch.int32), want.reshape(-1).view(torch.int32)), f"{shapes[i]} step {step}: statistics"
+            assert not t["rn"].any() and not t["cn"].any()
