@@ -43,8 +43,8 @@ ROOT = os.path.dirname(_HERE)
 DEFAULT_PATH = os.path.join(ROOT, "profiles", "hbm_traffic.json")
 COPY_KERNEL = "probe_move_kernel<0>"
 COPY_BYTES = 4 << 30
-STEP_KERNELS = ("fused_4bit_kernel", "fused_4bit_rank1", "rank1_stats_kernel", "rank1_stats_flat_kernel", "rank1_commit_kernel",
-                "rank1_row_scale_kernel", "single_tensor_kernel")
+# parts of the names of the kernels a step consists of
+STEP_KERNELS = ("fused_4bit_", "rank1_stats_", "rank1_commit_kernel", "rank1_row_scale_kernel", "single_tensor_kernel")
 
 
 def source_hash():

@@ -127,6 +127,21 @@ def test_source_hash_covers_the_kernel_sources_only(tmp_path, monkeypatch):
     assert ht.source_hash() != h2
 
 
+def test_every_kernel_of_a_step_is_counted():
+    """a kernel of csrc/q4adamw_*.h either belongs to a step, and its bytes to the record, or is one of those around it"""
+    import glob
+    import re
+    others = {"quantize_kernel", "dequantize_kernel", "quantize_rank1_kernel", "dequantize_rank1_kernel", "fill_zero_kernel",
+              "rounding_selfcheck_kernel", "device_step_kernel", "grad_sumsq_kernel", "grad_norm_finish_kernel"}
+    names = set()
+    for path in glob.glob(os.path.join(ht._HERE, "csrc", "q4adamw*")):
+        if path.endswith((".h", ".hip")):
+            names |= set(re.findall(r"__global__[^;{]*?void\s+(\w+)\(", open(path).read()))
+    assert {"fused_4bit_kernel", "rank1_stats_lead_kernel"} | others <= names
+    counted = {n for n in names if any(part in f"void q4::{n}<0>(q4::Args)" for part in ht.STEP_KERNELS)}
+    assert counted == names - others
+
+
 def test_committed_record_is_well_formed():
     with open(ht.DEFAULT_PATH) as f:
         doc = json.load(f)
