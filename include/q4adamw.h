@@ -432,7 +432,8 @@ int q4adamw_mtable_half_bucket(uint32_t half_index);
  * the whole bucket; k = out2[1] + (q >= value) is the number of code-book values <= q.
  * q4adamw_sr_affine_entry: entry k (0..16) of the table that turns a normalised value
  * into its code coordinate, out2 = {slope, offset}: floor(slope * q + offset - noise) is
- * the code wherever that value is clear of an integer.  For tests.
+ * the code wherever that value is clear of an integer (the kernels hold the same map
+ * negated and shifted).  For tests.
  */
 int q4adamw_sr_bucket_entry(uint32_t half_index, uint32_t *out2);
 int q4adamw_sr_affine_entry(uint32_t k, float *out2);
