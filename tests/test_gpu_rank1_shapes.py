@@ -80,3 +80,44 @@ def test_one_list_of_every_form(cuda, copies, p_dt, g_dt):
             for have, want in zip(stats, refs[i][4]):
                 assert torch.equal(have.cpu().view(torch.int32), want.reshape(-1).view(torch.int32)), f"{shapes[i]} step {step}: statistics"
             assert not t["rn"].any() and not t["cn"].any()
+
+
+@pytest.mark.parametrize("stochastic", [False, True])
+@pytest.mark.parametrize("g_dt", ["fp32", "bf16", "fp16"])
+@pytest.mark.parametrize("shape", [(300, 3), (77, 50), (1000, 88), (6200, 41), (64, 264), (33, 301),
+                                   (5, 40, 3, 3), (33, 7, 5), (20, 3, 64), (3, 9, 264), (2, 5, 300), (2, 3, 300, 3), (3, 2, 270, 40)])
+def test_multiplier_and_non_finite_gradients(cuda, shape, g_dt, stochastic):
+    """Every statistics kernel with a device multiplier (gradients scaled up by it, so that the product is
+    exact) and cleared gradients; NaN and infinities in the second step: maxima are taken over the
+    non-NaN values, a finite value under an infinite scale and a NaN get code 0."""
+    gen = torch.Generator().manual_seed(sum(shape))
+    n, cols, k = int(torch.Size(shape).numel()), shape[-1], len(shape) - 1
+    rows = n // cols
+    z = lambda m, dt=torch.float32: torch.zeros(m, dtype=dt, device=cuda)
+    p0 = torch.randn(shape, generator=gen) * 0.05
+    p, m, v, sm = p0.clone().to(cuda), z((n + 1) // 2, torch.uint8), z((n + 1) // 2, torch.uint8), z((n + 127) // 128)
+    r, rn, c, cn = z(rows), z(rows), z(cols), z(cols)
+    lead = ([z(d) for d in shape[:-1]], [z(d) for d in shape[:-1]]) if k > 1 else None
+    ref = (p0, m.cpu(), v.cpu(), sm.cpu(), [torch.zeros([shape[j] if d == j else 1 for d in range(k + 1)]) for j in range(k + 1)])
+    scale = torch.tensor([0.0625], device=cuda)
+    sr = dict(seed=0xABCD_1234_5678, tensor_salt=2) if stochastic else {}
+    for step in (1, 2, 3):
+        g = grads_config1(gen, n).view(shape)
+        if step == 2:
+            flat = g.view(-1)
+            flat[n // 3], flat[n // 2], flat[n // 2 + 1], flat[n - 1] = float("inf"), float("nan"), float("-inf"), float("nan")
+            g.view(rows, cols)[rows // 4] = float("nan")
+        g = g.to(base.DT[g_dt]) * 16          # a power of two: the multiplier takes it back exactly
+        with torch.no_grad():
+            ref = ot.step_quant_rank1_nd(ref[0], g.float() * 0.0625, *ref[1:], step=step, **sr, **HP)
+        dg = g.to(cuda)
+        q.fused_4bit_rank1_multi([p], [dg], [m], [v], [sm], [r], [c], [rn], [cn], *base.HPA, step, grad_scale_dev=scale, zero_grad=True,
+                                 leads=[lead], **(dict(seed=sr["seed"], salts=[2]) if stochastic else {}))
+        what = f"{shape} {g_dt} step {step}"
+        assert not dg.any(), f"{what}: gradients not cleared"
+        assert torch.equal(m.cpu(), ref[1]), f"{what}: m codes"
+        assert torch.equal(sm.cpu().view(torch.int32), ref[3].view(torch.int32)), f"{what}: m scales"
+        for have, want in zip((lead[0] if lead else [r]) + [c], ref[4]):
+            assert torch.equal(have.cpu().view(torch.int32), want.reshape(-1).view(torch.int32)), f"{what}: statistics"
+        assert torch.equal(v.cpu(), ref[2]), f"{what}: v codes"
+        assert not rn.any() and not cn.any(), f"{what}: scratch"
