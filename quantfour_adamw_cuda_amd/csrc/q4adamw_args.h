@@ -69,13 +69,17 @@ struct ChunkRuns {
   uint32_t grouped;   // a multiple of 8 << shift
 };
 
-// Runs of 1024 chunks in grids where every XCD gets 64 of them, otherwise of 64 or, in grids too small
-// for 64 of those, the longest that leave every XCD 64.  Against 64 (and four of them at least)
-// everywhere, medians on one box: the Llama-3-8B set 15.58 -> 15.53 ms (one eighth of the grid per XCD: 15.60; in
-// two other jobs, in which it was up to 0.8 % the faster, 15.53 and 15.72 against 15.64 and 15.79), its
-// layers and tables with rank-1 scaling 4504 -> 4475 us, Llama-2-13B layers with stochastic rounding
-// 2171 -> 2159, the 4096 x 4096 tensor (runs of 32) 38.2 -> 36.5 to 38.4; GPT-2-small keeps 64
-// (353; 128 357, 512 354).
+// Runs of 1024 chunks in grids where every XCD gets 64 of them (2^19 chunks), otherwise of 64 or, in grids too
+// small for 64 of those, the longest that leave every XCD 64.  Both sides of the line, medians of ten rounds in
+// turn in one process, the range over four cards, us a step with runs of 64 / 1024 / one eighth of the grid per
+// XCD; fp32 parameters and bf16 gradients, Llama-3-8B's layers:
+//     426000 chunks   838-854      841-856      847-855
+//     852000 chunks   1694-1718    1686-1710    1694-1711
+//    1704000 chunks   3407-3453    3373-3439    3391-3438
+//    7842048 chunks   15744-16004  15642-15871  15719-15904   (the whole set)
+// i.e. 0.5 to 0.8 % on the whole set, on every card.  All in fp32 or in bf16 the line could lie higher: 852000
+// chunks 1888-1909 / 1897-1909 / 1926-1935 and 2189-2200 / 2206-2210 / 2250-2269.  The 4096 x 4096 tensor in
+// fp32 (runs of 32): 38.5, 38.3 with runs of 64, 37.9 with 256, 41.5 with one eighth.
 __host__ inline ChunkRuns make_chunk_runs(uint32_t count) {
   ChunkRuns r = {(count >> 13) >= 64u ? 10u : 6u, 0u};
   while (r.shift > 0u && (count >> (r.shift + 3u)) < 64u) --r.shift;
@@ -99,7 +103,7 @@ struct TensorDesc {  // 56 bytes
   int64_t numel;
 };
 
-// Kernel arguments of one fused launch (about 3 KiB, passed by value).
+// Kernel arguments of one fused launch (nearly 4 KiB, passed by value).
 // first_chunk[i] = index of tensor i's first chunk; entries past ntensors hold
 // 0x7fffffff (more than any chunk index).  pivot[k] = first_chunk[8k] lets a workgroup find its tensor with two
 // wide scalar loads.
