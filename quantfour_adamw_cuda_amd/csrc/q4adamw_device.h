@@ -696,10 +696,4 @@ __device__ __forceinline__ float max_nonneg(float a, float b) {
   return bits2f(x > y ? x : y);
 }
 
-// Atomic maximum of non-negative floats through their bit patterns.
-__device__ __forceinline__ void atomic_max_nonneg(const float *addr, float x) {
-  // non-negative floats order like their bit patterns
-  atomicMax(reinterpret_cast<unsigned int *>(const_cast<float *>(addr)), f2bits(x));
-}
-
 }  // namespace q4

@@ -16,9 +16,10 @@ __device__ __forceinline__ void raise_max(float *addr, uint32_t u) {
   if (u > __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(a, u);
 }
 
-// The same without the look.  Where a statistic meets no more than a few hundred workgroups the
-// atomic, for which nothing waits, costs less than the load that every workgroup would end with:
-// statistics of 218 million elements (fp32 gradients, one layer's matrices) 179 us against 189.
+// The same without the look.  In the wide statistics form the atomic, for which nothing waits, costs less
+// than the load that every workgroup would end with, from 16 workgroups for a column's statistic (4096 x
+// 14336 fp32, four of them: 191 us against 195; 4000 x 512: 8.6 against 11.0) to 3906 (1000000 x 264: 253
+// against 270).
 __device__ __forceinline__ void atomic_max_bits(float *addr, uint32_t u) {
   atomicMax(reinterpret_cast<unsigned int *>(addr), u);
 }

@@ -1,6 +1,6 @@
 """Every chunk of a grid is taken exactly once, whatever the length of the runs of chunks that go
-to one XCD: grids around the sizes where the run length changes (32 << k chunks) and grids
-with a remainder beyond whole rounds of runs.  A chunk taken twice would step twice, one left
+to one XCD: grids around powers of two, where the run length doubles from 512 << k on (up to runs of 64,
+from 2^19 chunks on of 1024), and grids with a remainder beyond whole rounds of runs.  A chunk taken twice would step twice, one left
 out not at all."""
 import pytest
 import torch

@@ -1,6 +1,6 @@
-"""Checkpoint quantize / dequantize where their tiles end: a workgroup takes 4096 elements, a
-wave four tiles of 256, a lane four elements of each; code buffers at odd addresses; matrices
-whose rows end inside a lane's four elements."""
+"""Checkpoint quantize / dequantize where their tiles end: a workgroup takes 2048 elements to encode and
+4096 to decode, a wave two and four tiles of 256, a lane four elements of each; code buffers at odd
+addresses; matrices whose rows end inside a lane's four elements."""
 import numpy as np
 import pytest
 import torch
