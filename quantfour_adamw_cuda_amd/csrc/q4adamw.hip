@@ -5,7 +5,7 @@
 //   q4adamw_device.h  device helpers
 //   q4adamw_step.h    the fused step (block-scaled, stochastic rounding, rank-1); its kernels are
 //                     instantiated in q4adamw_pick_*.hip (q4adamw_pick.h)
-//   q4adamw_rank1.h   rank-1 scaling: statistics, commit, folds
+//   q4adamw_rank1.h   rank-1 scaling: statistics, row scales, commit
 //   q4adamw_aux.h     small-tensor step, gradient norm, quantize / dequantize
 //
 // Build (quantfour_adamw_cuda_amd/build.py): every q4adamw*.hip is compiled by itself with
@@ -1009,6 +1009,7 @@ int q4adamw_quantize_rank1(const float *x, int64_t rows, int64_t cols, uint8_t *
   if (!x || !codes || !row_max || !col_max) return fail(Q4ADAMW_ERR_ARG, "null tensor pointer");
   if (!aligned(x, 4) || !aligned(row_max, 4) || !aligned(col_max, 4))
     return fail(Q4ADAMW_ERR_ALIGN, "fp32 buffers must be 4-byte aligned");
+  // a limit of this entry point, not of its kernels: 65535 groups of 64 rows
   if (rows > 4194240) return fail(Q4ADAMW_ERR_TOO_LARGE, "more than 4194240 rows");
   hipStream_t s = static_cast<hipStream_t>(stream);
   q4adamw_rank1_tensor t = {};
