@@ -463,15 +463,6 @@ __device__ __forceinline__ uint32_t exact_sr_code_m(float q, float noise, uint32
   return (uint32_t)(c < 0 ? 0 : c > 15 ? 15 : c);
 }
 
-// A uniform value in a vector register: a multiplication or an addition of vector registers issues
-// in 2 cycles, one with a scalar operand in 4 (a wave64 instruction on this GPU, 8 waves per
-// SIMD).  Pays for itself from three uses on.
-__device__ __forceinline__ float in_vgpr(float s) {
-  float v;
-  asm("v_mov_b32 %0, %1" : "=v"(v) : "s"(s));
-  return v;
-}
-
 // (x & mask) | base as one v_and_or_b32: the mask travels in a scalar register (the
 // compiler splits the operation when the mask is a literal, which a VOP3 encoding
 // cannot hold).
