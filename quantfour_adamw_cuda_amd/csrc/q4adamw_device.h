@@ -575,16 +575,22 @@ constexpr float kVGuard = 7.62939453125e-06f;        // 2^-17, in units of 16*q 
 // Uniform search of the launch's tensor list: the last tensor whose first chunk is
 // <= chunk.  first_chunk[0] is 0, so the result is never negative.  Chunk indices and
 // table entries are below 2^31, so bit 31 of (x - chunk - 1) says x <= chunk: plain
-// integer arithmetic that stays on the scalar unit.
+// integer arithmetic that stays on the scalar unit.  The masks take nothing away; they tell the compiler
+// how small the sums are, which keeps the index and the addresses made from it in 32 bits.  Every workgroup
+// waits for this chain before its first load: without them, and with eight pivots instead of six since a
+// launch holds 61 tensors, Llama-3-8B's step (fp32 / bf16, exact update) took 15.56 ms, with them 15.51.
 template <typename Args>
 __device__ __forceinline__ int find_tensor(const Args &a, uint32_t chunk) {
+  constexpr uint32_t kGroupMask = Args::kPivots <= 4 ? 3u : Args::kPivots <= 8 ? 7u : Args::kPivots <= 16 ? 15u : 31u;
+  static_assert(Args::kPivots <= 32, "the widest mask");
   uint32_t group = 0;
 #pragma unroll
   for (int k = 1; k < Args::kPivots; ++k) group += (a.pivot[k] - chunk - 1u) >> 31;
+  group &= kGroupMask;
   uint32_t within = 0;
 #pragma unroll
   for (int k = 0; k < 8; ++k) within += (a.first_chunk[group * 8 + k] - chunk - 1u) >> 31;
-  return (int)(group * 8 + within) - 1;
+  return (int)((group * 8 + within - 1u) & (8u * kGroupMask + 7u));
 }
 
 // LDS of a workgroup, one array of 8-byte entries:
