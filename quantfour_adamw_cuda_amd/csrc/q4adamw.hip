@@ -257,7 +257,7 @@ static Rank1StatKernel pick_rank1_stats(Rank1StatForm form, int g_dtype, bool ex
 // nothing else in flight, about 0.09 us a row: 6 us with 32 rows, 26 with 256, which a launch with workgroups to
 // spare hides.  And every workgroup updates the statistic of every column it meets; updates of one address
 // are taken one after another, 20 ns each.  So 256 where that makes four workgroups per CU, else as few
-// as 32, but no fewer than a sixth of the rows' square root calls for, where the two costs balance.
+// as 32, but in matrices of more than 6 r^2 rows more than r, which is about where the two costs balance.
 // Statistics of one fp32 matrix with 32, 64, 128, 256 rows, us: 4000 x 512 8.6, 10.9, 17.4, 29.1;
 // 16000 x 264 15.4, 13.4, 16.8, 28.4; 50257 x 264 38.6, 30.4, 23.8, 29.7; 100000 x 264 68.1, 45.6, 41.6, 35.6;
 // 300000 x 264 187, 112, 87, 85.
