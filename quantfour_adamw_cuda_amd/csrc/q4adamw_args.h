@@ -220,6 +220,7 @@ struct Rank1StatArgs {
   float b2, r2;
   GradOps go;
   uint32_t chunk_base;     // this grid's first tile (workgroup 0)
+  ChunkRuns runs;          // wide forms: which tile a workgroup takes
   uint32_t stat_rows;      // rows of a workgroup (flat form: at most, but for one tile): 32, 64, 128 or 256
   uint32_t pivot[kPivots];
   uint32_t first_chunk[kPivots * 8];

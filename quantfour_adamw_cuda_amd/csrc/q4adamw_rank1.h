@@ -80,6 +80,18 @@ constexpr int kStatRowsPerWave = 64;     // rows a wave walks, at most
 constexpr int kStatRows = kStatRowsPerWave * kWaves;   // rows per workgroup of the statistics kernel, at most
 constexpr int kStatCols = 512;           // columns per workgroup: 8 per lane
 
+// The packed codes of PER (4 or 8) consecutive elements from element `elem` of a run whose first code is at
+// the low (odd = 0) or high nibble of byte 0.  ANY: elem + odd may be odd, and the codes end in one byte more.
+template <uint32_t PER, bool ANY>
+__device__ __forceinline__ uint32_t load_part_codes(const void *run, uint32_t odd, uint32_t elem) {
+  const uint32_t nibble = ANY ? odd + elem : elem;
+  uint32_t w = PER == 8 ? __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(run), nibble >> 1, 0, kNtReadOnly)
+                        : (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(tile_rsrc(run), nibble >> 1, 0, kNtReadOnly);
+  if (ANY && (nibble & 1u) != 0u)
+    w = (w >> 4) | (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(tile_rsrc(run), (nibble >> 1) + PER / 2, 0, kNtReadOnly) << (4 * PER - 4);
+  return w;
+}
+
 // New second moments of a tile of stat_rows x kStatCols elements, reduced to row and
 // column maxima (get_variance_tensor_statistics, adamw_fourbit_triton.py:738-746).  The
 // arithmetic is the update kernel's, operation for operation, so the maxima are maxima
@@ -99,9 +111,15 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
   constexpr bool kAbs = GT_ == kAbsValues;
   constexpr int GT = kAbs ? Q4ADAMW_FP32 : GT_;
   constexpr int kAhead = 4;  // rows whose loads are in flight together
+  // A lane's 8 columns.  Of 16-bit gradients they are consecutive, one 16-byte access; of fp32 ones two parts of 4
+  // columns half a tile apart, so that a wave's access is one run of bytes: with 8 consecutive columns, two
+  // accesses of every other 16 bytes, GPT-2-small in fp32 took 412 us a step against 391, a 4-bit encoding of
+  // 14336 x 4096 elements 133 against 128, a step of 8000 x 9001 elements 327 against 314.
+  constexpr int kParts = GT ? 1 : 2;
+  constexpr uint32_t kPer = 8 / kParts;
   __shared__ uint32_t row_bits[4][kStatRows];       // row maxima of each 16-lane quarter of the row's wave
   __shared__ uint32_t col_bits[kWaves][kStatCols];  // column maxima of each wave
-  const uint32_t chunk = args.chunk_base + blockIdx.x;
+  const uint32_t chunk = args.chunk_base + run_chunk(args.runs, blockIdx.x);
   float gscale = 1.0f;
   if (EXT && !grad_ops_begin(args.go, gscale)) return;
   const int t = find_tensor(args, chunk);
@@ -111,13 +129,19 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
   const uint32_t rg = local / groups, cg = local - rg * groups;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool active = cg * kStatCols + (uint32_t)lane * 8u < T.cols;
-  // the tile's first column, and the lane's counted from there: all 8 of the lane's are in the row
-  uint32_t col0 = cg * kStatCols, lane_elem = (uint32_t)lane * 8u;
+  // the tile's first column, and the lane's parts counted from there: all columns of a part are in the row
+  uint32_t col0 = cg * kStatCols, part_elem[kParts];
+  bool active[kParts];
+#pragma unroll
+  for (int h = 0; h < kParts; ++h) {
+    part_elem[h] = (uint32_t)(h * (kStatCols / kParts) + lane * kPer);
+    active[h] = col0 + part_elem[h] < T.cols;
+  }
   if (ANY) {
-    col0 = col0 < T.cols - 8u ? col0 : T.cols - 8u;
-    const uint32_t last = T.cols - 8u - col0;
-    lane_elem = lane_elem < last ? lane_elem : last;
+    col0 = col0 < T.cols - kPer ? col0 : T.cols - kPer;
+    const uint32_t last = T.cols - kPer - col0;
+#pragma unroll
+    for (int h = 0; h < kParts; ++h) part_elem[h] = part_elem[h] < last ? part_elem[h] : last;
   }
   const uint32_t stat_rows = args.stat_rows;
   const uint32_t tile_row0 = rg * stat_rows;
@@ -131,14 +155,14 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
   float c_old[8], c_max[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    c_old[k] = active && !kAbs ? as_global<const float>(T.cmax)[col0 + lane_elem + k] : 0.0f;
+    c_old[k] = active[k / kPer] && !kAbs ? as_global<const float>(T.cmax)[col0 + part_elem[k / kPer] + k % kPer] : 0.0f;
     c_max[k] = 0.0f;
   }
   const uint32_t quarter = (uint32_t)lane >> 4;
   for (int r0 = 0; r0 < nrows; r0 += kAhead) {
     // a group past the wave's last row repeats that row: maxima do not mind
-    u32x4 gw[kAhead][GT ? 1 : 2];
-    uint32_t vw[kAhead];
+    u32x4 gw[kAhead][kParts];
+    uint32_t vw[kAhead][kParts];
     float r_old[kAhead];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
@@ -149,49 +173,39 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
       const int64_t row_first = (int64_t)row * T.cols + col0;
       const void *g_row = static_cast<const char *>(T.g) + row_first * (GT ? 2 : 4);
       const void *v_row = T.v + (row_first >> 1);
-      vw[i] = 0u;
 #pragma unroll
-      for (int h = 0; h < (GT ? 1 : 2); ++h) gw[i][h] = u32x4{0u, 0u, 0u, 0u};
-      if (active) {
-        if (kAbs) {
-          // no codes
-        } else if (ANY) {
-          // eight codes from either nibble of a byte on: four bytes, or four and the low nibble of a fifth
-          const uint32_t nibble = ((uint32_t)row_first & 1u) + lane_elem;
-          vw[i] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(v_row), nibble >> 1, 0, kNtReadOnly);
-          if (nibble & 1u)
-            vw[i] = (vw[i] >> 4) | (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(tile_rsrc(v_row), (nibble >> 1) + 4u, 0, kNtReadOnly) << 28;
-        } else {
-          vw[i] = __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(v_row), lane_elem >> 1, 0, kNtReadOnly);
-        }
-        if (GT) {
-          gw[i][0] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_row), lane_elem * 2u, 0, kNtReadOnly);
-        } else {
-          gw[i][0] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_row), lane_elem * 4u, 0, kNtReadOnly);
-          gw[i][GT ? 0 : 1] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_row), lane_elem * 4u + 16u, 0, kNtReadOnly);
+      for (int h = 0; h < kParts; ++h) {
+        vw[i][h] = 0u;
+        gw[i][h] = u32x4{0u, 0u, 0u, 0u};
+        if (active[h]) {
+          if (!kAbs) vw[i][h] = load_part_codes<kPer, ANY>(v_row, (uint32_t)row_first & 1u, part_elem[h]);
+          gw[i][h] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_row), part_elem[h] * (GT ? 2u : 4u), 0, kNtReadOnly);
         }
       }
     }
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
-      float g[8];
-      if constexpr (GT != 0) {
-        widen_pair<GT>(gw[i][0].x, g[0], g[1]);
-        widen_pair<GT>(gw[i][0].y, g[2], g[3]);
-        widen_pair<GT>(gw[i][0].z, g[4], g[5]);
-        widen_pair<GT>(gw[i][0].w, g[6], g[7]);
-      } else {
-        const u32x4 lo = gw[i][0], hi = gw[i][GT ? 0 : 1];
-        g[0] = bits2f(lo.x); g[1] = bits2f(lo.y); g[2] = bits2f(lo.z); g[3] = bits2f(lo.w);
-        g[4] = bits2f(hi.x); g[5] = bits2f(hi.y); g[6] = bits2f(hi.z); g[7] = bits2f(hi.w);
+      float g[8], code[8];   // codes as numbers, 0 .. 15
+#pragma unroll
+      for (int h = 0; h < kParts; ++h) {
+        const u32x4 w = gw[i][h];
+        if constexpr (GT != 0) {
+          widen_pair<GT>(w.x, g[0], g[1]);
+          widen_pair<GT>(w.y, g[2], g[3]);
+          widen_pair<GT>(w.z, g[4], g[5]);
+          widen_pair<GT>(w.w, g[6], g[7]);
+        } else {
+          g[4 * h] = bits2f(w.x); g[4 * h + 1] = bits2f(w.y); g[4 * h + 2] = bits2f(w.z); g[4 * h + 3] = bits2f(w.w);
+        }
+        const uint32_t even = vw[i][h] & 0x0F0F0F0Fu, odd = (vw[i][h] >> 4) & 0x0F0F0F0Fu;  // one code per byte
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; ++k) code[kPer * h + k] = (float)(((k & 1 ? odd : even) >> (8 * (k >> 1))) & 0xffu);
       }
-      const uint32_t even = vw[i] & 0x0F0F0F0Fu, odd = (vw[i] >> 4) & 0x0F0F0F0Fu;  // one code per byte
       float r_max = 0.0f;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const float gk = EXT ? g[k] * gscale : g[k];
-        const uint32_t code = ((k & 1 ? odd : even) >> (8 * (k >> 1))) & 0xffu;
-        const float code_value = __builtin_fmaf((float)code, 0.0625f, 0.0625f);  // (code + 1) / 16, exact
+        const float code_value = __builtin_fmaf(code[k], 0.0625f, 0.0625f);  // (code + 1) / 16, exact
         const float v_old = code_value * min_nonneg(r_old[i], c_old[k]);
         const float v = kAbs ? __builtin_fabsf(gk) : args.b2 * v_old + args.r2 * (gk * gk);
         c_max[k] = __builtin_fmaxf(c_max[k], v);
@@ -206,7 +220,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
     }
   }
 #pragma unroll
-  for (int k = 0; k < 8; ++k) col_bits[wave][lane * 8 + k] = f2bits(c_max[k]);
+  for (int k = 0; k < 8; ++k) col_bits[wave][k / kPer * (kStatCols / kParts) + lane * kPer + k % kPer] = f2bits(c_max[k]);
   __syncthreads();
   // one update per column of the tile, and one per row or per leading index of its rows
 #pragma unroll
@@ -215,11 +229,11 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
     uint32_t u = col_bits[0][c];
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) u = u > col_bits[w][c] ? u : col_bits[w][c];
-    const bool there = cg * kStatCols + (ANY ? c & ~7u : c) < T.cols;
+    const bool there = cg * kStatCols + (ANY ? c & ~(kPer - 1u) : c) < T.cols;
     uint32_t cc = cg * kStatCols + c;
     if (ANY) {   // the column that slot c's lane worked on
-      const uint32_t first = c & ~7u, last = T.cols - 8u - col0;
-      cc = col0 + (first < last ? first : last) + (c & 7u);
+      const uint32_t first = c & ~(kPer - 1u), last = T.cols - kPer - col0;
+      cc = col0 + (first < last ? first : last) + (c & (kPer - 1u));
     }
     if (there && u != 0u) atomic_max_bits(T.cmax_next + cc, u);
   }

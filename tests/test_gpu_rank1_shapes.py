@@ -20,12 +20,22 @@ MATRICES = [(1365, 3), (1366, 2), (4100, 3), (240, 16), (241, 16), (31, 128), (6
 # where a workgroup's rows double (6144, 24576 and 98304 rows): several tiles of the flat form, more rows of the
 # wide ones; the last workgroup with all of its tiles, with some, with part of one
 TALL = [(6145, 50), (6144 + 63 * 5, 64), (6200, 255), (24577, 33), (24640, 88), (98305, 24), (98304 + 500, 41), (6150, 96), (24600, 104), (98310, 96), (6200, 257)]
+# the wide forms' lanes have two parts of 4 columns each under fp32 gradients, 256 columns apart: rows that end in
+# either part, on its first and last columns and between them; 130 and 136 tiles, of which 128 are dealt in runs of 8
+PARTS = [(37, 258), (37, 259), (40, 260), (37, 261), (40, 504), (37, 507), (40, 508), (37, 510), (40, 512), (37, 515), (40, 520), (37, 767),
+         (37, 770), (2080, 520), (1088, 1541)]
 TENSORS = [(5, 300, 3, 3), (2, 700, 3), (1400, 1, 2), (300, 2, 7), (16, 16, 16), (3, 100, 260), (2, 130, 4, 257), (64, 3, 7, 7)]
 
 
 @pytest.mark.parametrize("p_dt,g_dt", [("fp32", "fp32"), ("bf16", "bf16"), ("fp32", "fp16")])
 @pytest.mark.parametrize("shape", MATRICES)
 def test_statistics_of_a_matrix(cuda, shape, p_dt, g_dt):
+    base.test_rank1_against_oracle(cuda, p_dt, g_dt, shape)
+
+
+@pytest.mark.parametrize("p_dt,g_dt", [("fp32", "fp32"), ("bf16", "fp32"), ("bf16", "bf16")])
+@pytest.mark.parametrize("shape", PARTS)
+def test_statistics_of_rows_that_end_anywhere_in_a_tile(cuda, shape, p_dt, g_dt):
     base.test_rank1_against_oracle(cuda, p_dt, g_dt, shape)
 
 
