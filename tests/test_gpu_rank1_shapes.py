@@ -39,6 +39,16 @@ def test_statistics_of_rows_that_end_anywhere_in_a_tile(cuda, shape, p_dt, g_dt)
     base.test_rank1_against_oracle(cuda, p_dt, g_dt, shape)
 
 
+# the update of rows of any length: rows shorter than a lane's elements, rows that begin at each of a lane's
+# elements, a matrix that ends with a row's first element in a lane, and rows of a tile and a little more or less
+@pytest.mark.parametrize("stochastic", [False, True])
+@pytest.mark.parametrize("p_dt,g_dt", [("fp32", "fp32"), ("bf16", "bf16")])
+@pytest.mark.parametrize("shape", [(41, c) for c in (2, 3, 5, 6, 7, 9, 10, 11, 12, 13, 14, 15, 17, 255, 257, 261, 511, 513, 514, 515)])
+def test_update_of_rows_that_begin_anywhere_in_a_lane(cuda, shape, p_dt, g_dt, stochastic):
+    test = base.test_rank1_stochastic_rounding_against_oracle if stochastic else base.test_rank1_against_oracle
+    test(cuda, p_dt, g_dt, shape)
+
+
 @pytest.mark.parametrize("p_dt,g_dt", [("fp32", "fp32"), ("bf16", "bf16")])
 @pytest.mark.parametrize("shape", TALL)
 def test_statistics_of_a_tall_matrix(cuda, shape, p_dt, g_dt):
