@@ -208,6 +208,21 @@ static Rank1Shape rank1_shape(const q4adamw_rank1_tensor &t, int64_t tile_elems)
   return kShapeWide;
 }
 
+static bool rank1_has_leads(const q4adamw_rank1_tensor &t) { return t.lead_dims >= 2; }
+
+// Tensors with several leading dimensions whose elements would gather their scales one by one (kShapeAny) take a
+// kernel of their own if their rows are short, so that rows' scales are a good part of their bytes: it makes
+// them from the leading statistics, and no launches make and copy them around it.  us a step of [256, n, c], 41
+// million elements, in fp32 / in bf16, without and with it: c = 5 255 / 251 and 219 / 198, 8 239 / 188 and 209 / 188; the
+// form for multiples of 8 is the better one in bf16 from 16 columns on (213 / 168 and 208 / 185 at 16, 210 / 164 and 210 / 185
+// at 32).
+constexpr int kRouteShort = 4, kRoutes = 5;   // the others: Rank1Shape
+
+static int rank1_route(const q4adamw_rank1_tensor &t, int64_t tile_elems) {
+  const Rank1Shape shape = rank1_shape(t, tile_elems);
+  return shape == kShapeAny && rank1_has_leads(t) && t.cols <= (int64_t)kShortMaxCols ? kRouteShort : (int)shape;
+}
+
 static uint64_t rank1_tiles_per_row(const q4adamw_rank1_tensor &t, int64_t tile_elems) {
   return (uint64_t)((t.cols + tile_elems - 1) / tile_elems);
 }
@@ -228,8 +243,6 @@ static uint64_t rank1_chunks(const q4adamw_rank1_tensor &t, int64_t tile_elems) 
 // multiple of 8 long take the variant that finds their codes at either nibble, above 256 columns.  Lead: as
 // flat, for tensors with several leading dimensions.
 enum Rank1StatForm { kStatFlat = 0, kStatLead = 1, kStatWide = 2, kStatWideAny = 3, kStatForms = 4 };
-
-static bool rank1_has_leads(const q4adamw_rank1_tensor &t) { return t.lead_dims >= 2; }
 
 static Rank1StatForm rank1_stat_form(const q4adamw_rank1_tensor &t) {
   if (rank1_has_leads(t) && t.cols <= (int64_t)kFlatMaxCols) return kStatLead;
@@ -289,6 +302,41 @@ static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_r
     return (uint64_t)((outer + kLeadOuter - 1) / kLeadOuter) * lead_tiles((uint32_t)t.rows, outer, (uint32_t)t.cols).inner;
   }
   return (((uint64_t)t.rows + stat_rows - 1) / stat_rows) * (uint64_t)((t.cols + kStatCols - 1) / kStatCols);
+}
+
+static FastDiv make_fast_div_any(uint32_t d) { return d == 1u ? FastDiv{0u, 0u} : make_fast_div(d); }
+
+static ShortDesc short_desc(const q4adamw_rank1_tensor &t) {
+  ShortDesc d = {};
+  d.p = t.p;
+  d.g = t.g;
+  d.m = t.exp_avg;
+  d.v = t.exp_avg_sq;
+  d.sm = t.exp_avg_scale;
+  d.rmax = t.row_max;
+  d.cmax = t.col_max;
+  d.cmax_next = t.col_max_next;
+  d.numel = (uint32_t)(t.rows * t.cols);
+  d.cols = (uint16_t)t.cols;
+  const FastDiv by_cols = make_fast_div((uint32_t)t.cols);
+  d.cols_magic = by_cols.magic;
+  d.cols_shift = (uint8_t)by_cols.shift;
+  const int n = t.lead_dims;
+  d.lead_dims = (uint8_t)n;
+  d.last = t.lead_max[n - 1];
+  d.last_next = t.lead_max_next[n - 1];
+  d.before = t.lead_max[n - 2];
+  d.before_next = t.lead_max_next[n - 2];
+  d.outer = t.lead_max[0];
+  d.outer_next = t.lead_max_next[0];
+  d.last_size = (uint32_t)t.lead_shape[n - 1];
+  d.before_size = (uint32_t)t.lead_shape[n - 2];
+  const FastDiv by_last = make_fast_div_any(d.last_size), by_before = make_fast_div_any(d.before_size);
+  d.last_magic = by_last.magic;
+  d.last_shift = (uint8_t)by_last.shift;
+  d.before_magic = by_before.magic;
+  d.before_shift = (uint8_t)by_before.shift;
+  return d;
 }
 
 // Fills the kernels' view of the caller's gradient options; returns whether the
@@ -560,12 +608,18 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t tile_elems = chunk_elems / kWaves;
   const bool exact = exact_update(update_form, p_dtype, sr, true);
+  ShortArgs ha;      // the batch, if it takes the kernel for short rows
+  ha.sc = a.sc;
+  ha.go = a.go;
+  ha.seed_lo = a.seed_lo;
+  ha.seed_hi = a.seed_hi;
   RowScaleArgs ra;   // the batch's tensors with several leading dimensions
   ra.go = a.go;
   CommitArgs ca;
   ca.go = a.go;
-  int leads = 0;
+  int leads = 0, route = 0;
   Rank1Kernel kernel = nullptr;
+  ShortKernel short_kernel = nullptr;
   const q4adamw_rank1_tensor *batch[kMaxRank1Tensors];
   a.ntensors = 0;
   uint64_t chunks = 0, stat_chunks = 0, scale_chunks = 0, commit_chunks = 0;   // stat_chunks: an upper bound
@@ -624,15 +678,17 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       hipLaunchKernelGGL(rank1_row_scale_kernel, dim3((unsigned)scale_chunks), dim3(256), 0, s, ra);
       Q4_HIP(hipGetLastError());
     }
-    finish_prefix(a, a.ntensors);
-    if (int rc = for_each_grid(chunks, kThreads, [&](uint64_t base, uint64_t count) -> int {
-          a.chunk_base = (uint32_t)base;
-          a.runs = make_chunk_runs((uint32_t)count);
-          hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(kThreads), 0, s, a);
-          Q4_HIP(hipGetLastError());
-          return 0;
-        }))
-      return rc;
+    auto launch_update = [&](auto &args, auto update) -> int {
+      finish_prefix(args, a.ntensors);
+      return for_each_grid(chunks, kThreads, [&](uint64_t base, uint64_t count) -> int {
+        args.chunk_base = (uint32_t)base;
+        args.runs = make_chunk_runs((uint32_t)count);
+        hipLaunchKernelGGL(update, dim3((unsigned)count), dim3(kThreads), 0, s, args);
+        Q4_HIP(hipGetLastError());
+        return 0;
+      });
+    };
+    if (int rc = route == kRouteShort ? launch_update(ha, short_kernel) : launch_update(a, kernel)) return rc;
     finish_prefix(ca, a.ntensors);
     hipLaunchKernelGGL(rank1_commit_kernel, dim3((unsigned)commit_chunks), dim3(256), 0, s, ca);
     Q4_HIP(hipGetLastError());
@@ -646,62 +702,75 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
   // the one whose lanes find their own; rows of any length the one whose elements do.  Tensors of one
   // statistics kernel after another, and a batch may hold several kinds: a batch for each would repeat
   // update and commit (bf16 matrices of 1000 x 64 and 1000 x 400: a step of 29 us, 34 with two batches)
-  auto pass_of = [&](const q4adamw_rank1_tensor &t) { return rank1_shape(t, tile_elems) * kStatForms + rank1_stat_form(t); };
+  auto pass_of = [&](const q4adamw_rank1_tensor &t) { return rank1_route(t, tile_elems) * kStatForms + rank1_stat_form(t); };
   uint32_t present = 0u;   // a bit per pass
   for (int i = 0; i < count; ++i) {
     if (tensors[i].rows != 0 && tensors[i].cols != 0) present |= 1u << pass_of(tensors[i]);
   }
-  for (int pass = 0; pass < 4 * kStatForms; ++pass) {
-    const int shape = pass / kStatForms;
-    kernel = shape == kShapeRows     ? pick_rank1_rows(p_dtype, g_dtype, ext, sr, exact)
-             : shape == kShapeWide   ? pick_rank1_wide(p_dtype, g_dtype, ext, sr, exact)
-             : shape == kShapeNarrow ? pick_rank1_narrow(p_dtype, g_dtype, ext, sr, exact)
-                                     : pick_rank1_any(p_dtype, g_dtype, ext, sr, exact);
+  for (int pass = 0; pass < kRoutes * kStatForms; ++pass) {
+    route = pass / kStatForms;
+    if (route == kRouteShort) short_kernel = pick_rank1_short(p_dtype, g_dtype, ext, sr, exact);
+    else
+      kernel = route == kShapeRows     ? pick_rank1_rows(p_dtype, g_dtype, ext, sr, exact)
+               : route == kShapeWide   ? pick_rank1_wide(p_dtype, g_dtype, ext, sr, exact)
+               : route == kShapeNarrow ? pick_rank1_narrow(p_dtype, g_dtype, ext, sr, exact)
+                                       : pick_rank1_any(p_dtype, g_dtype, ext, sr, exact);
+    const int capacity = route == kRouteShort ? kMaxShortTensors : kMaxRank1Tensors;
     for (int i = 0; i < count && (present >> pass & 1u) != 0u; ++i) {
       const q4adamw_rank1_tensor &t = tensors[i];
       if (t.rows == 0 || t.cols == 0 || pass_of(t) != pass) continue;
       const int64_t numel = t.rows * t.cols;
       const uint64_t c = rank1_chunks(t, tile_elems), sc_ = rank1_stat_chunks(t, 32u);
       auto commit_chunks_of = [](int64_t size) { return ((uint64_t)size + kCommitChunk - 1) / kCommitChunk; };
-      uint64_t cc = commit_chunks_of(t.rows) + commit_chunks_of(t.cols);
+      // the kernel for short rows writes the rows' scales itself
+      const bool rows_follow = route == kRouteShort;
+      uint64_t cc = (rows_follow ? 0 : commit_chunks_of(t.rows)) + commit_chunks_of(t.cols);
       if (rank1_has_leads(t)) {
         for (int j = 0; j < t.lead_dims; ++j) cc += commit_chunks_of(t.lead_shape[j]);
       }
       const uint64_t rc_ = ((uint64_t)t.rows + kRowScaleChunk - 1) / kRowScaleChunk;
       // the row-scale and commit launches stay within one grid (one tensor's rows and columns
       // are fewer than 2^32, 2^21 chunks)
-      if (a.ntensors == kMaxRank1Tensors || chunks + c > kMaxChunksPerLaunch || stat_chunks + sc_ > kMaxChunksPerLaunch ||
+      if (a.ntensors == capacity || chunks + c > kMaxChunksPerLaunch || stat_chunks + sc_ > kMaxChunksPerLaunch ||
           commit_chunks + cc > kMaxStatWorkgroups || scale_chunks + rc_ > kMaxStatWorkgroups) {
         if (int rc = launch()) return rc;
       }
-      Rank1Desc &d = a.desc[a.ntensors];
-      d.p = t.p;
-      d.g = t.g;
-      d.m = t.exp_avg;
-      d.v = t.exp_avg_sq;
-      d.sm = t.exp_avg_scale;
-      d.rmax = t.row_max;
-      d.cmax = t.col_max;
-      d.rmax_next = t.row_max_next;
-      d.cmax_next = t.col_max_next;
-      d.numel = numel;
-      d.rows = t.rows;
-      d.cols = t.cols;
-      // the divisor the tensor's kernel needs: tiles per row, cols, or cols / 8
-      const FastDiv fd = make_fast_div(shape == kShapeRows  ? (uint32_t)rank1_tiles_per_row(t, tile_elems)
-                                       : shape == kShapeAny ? (uint32_t)t.cols
-                                                            : (uint32_t)(t.cols >> 3));
-      d.div_magic = fd.magic;
-      d.div_shift = fd.shift;
-      a.sr_salt[a.ntensors] = !sr ? 0u : a.go.sc_dev ? lowbias32(salts ? salts[i] : (uint32_t)i)
-                                                     : q4adamw_sr_tensor_salt(seed, step, salts ? salts[i] : (uint32_t)i);
-      a.first_chunk[a.ntensors] = (uint32_t)chunks;
+      const uint32_t salt = !sr ? 0u : a.go.sc_dev ? lowbias32(salts ? salts[i] : (uint32_t)i)
+                                                   : q4adamw_sr_tensor_salt(seed, step, salts ? salts[i] : (uint32_t)i);
+      if (route == kRouteShort) {
+        ShortDesc &d = ha.desc[a.ntensors];
+        d = short_desc(t);
+        ha.sr_salt[a.ntensors] = salt;
+        ha.first_chunk[a.ntensors] = (uint32_t)chunks;
+      } else {
+        Rank1Desc &d = a.desc[a.ntensors];
+        d.p = t.p;
+        d.g = t.g;
+        d.m = t.exp_avg;
+        d.v = t.exp_avg_sq;
+        d.sm = t.exp_avg_scale;
+        d.rmax = t.row_max;
+        d.cmax = t.col_max;
+        d.rmax_next = t.row_max_next;
+        d.cmax_next = t.col_max_next;
+        d.numel = numel;
+        d.rows = t.rows;
+        d.cols = t.cols;
+        // the divisor the tensor's kernel needs: tiles per row, cols, or cols / 8
+        const FastDiv fd = make_fast_div(route == kShapeRows  ? (uint32_t)rank1_tiles_per_row(t, tile_elems)
+                                         : route == kShapeAny ? (uint32_t)t.cols
+                                                              : (uint32_t)(t.cols >> 3));
+        d.div_magic = fd.magic;
+        d.div_shift = fd.shift;
+        a.sr_salt[a.ntensors] = salt;
+        a.first_chunk[a.ntensors] = (uint32_t)chunks;
+      }
       batch[a.ntensors] = &t;
       const int lead_dims = rank1_has_leads(t) ? t.lead_dims : 0;
       CommitArgs::Desc &cd = ca.desc[a.ntensors];
       cd.cur[0] = t.row_max;
       cd.next[0] = t.row_max_next;
-      cd.size[0] = (uint32_t)t.rows;
+      cd.size[0] = rows_follow ? 0u : (uint32_t)t.rows;
       cd.cur[1] = t.col_max;
       cd.next[1] = t.col_max_next;
       cd.size[1] = (uint32_t)t.cols;
@@ -712,7 +781,7 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
         cd.size[2 + j] = there ? (uint32_t)t.lead_shape[j] : 0u;
       }
       ca.first_chunk[a.ntensors] = (uint32_t)commit_chunks;
-      if (lead_dims != 0) {
+      if (lead_dims != 0 && !rows_follow) {
         RowScaleArgs::Desc &rd = ra.desc[leads];
         rd.row_next = t.row_max_next;
         rd.lead_dims = (uint32_t)lead_dims;

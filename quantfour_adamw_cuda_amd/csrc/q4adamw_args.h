@@ -182,6 +182,11 @@ __host__ __device__ __forceinline__ uint32_t fast_div(uint32_t n, uint32_t magic
   return (t + ((n - t) >> 1)) >> shift;
 }
 
+// divisors from 1 on (a size of 1 has the magic number 0, which no other has)
+__host__ __device__ __forceinline__ uint32_t fast_div_any(uint32_t n, uint32_t magic, uint32_t shift) {
+  return magic == 0u ? n : fast_div(n, magic, shift);
+}
+
 static FastDiv make_fast_div(uint32_t d) {  // d >= 2
   uint32_t l = 0;
   while ((1ull << l) < d) ++l;                     // ceil(log2 d) >= 1
@@ -208,6 +213,46 @@ struct Rank1Args {
   uint32_t sr_salt[kMaxRank1Tensors];   // stochastic rounding: as FusedArgs::sr_salt
   uint32_t seed_lo, seed_hi;
   Rank1Desc desc[kMaxRank1Tensors];
+};
+
+// The same for tensors with several leading dimensions and short rows, of fewer than 2^32 elements, whose update
+// reads the leading dimensions' statistics themselves.
+constexpr int kMaxShortTensors = 25;
+constexpr uint32_t kShortMaxCols = 64;
+
+struct ShortDesc {  // 144 bytes
+  void *p;
+  const void *g;
+  uint8_t *m;
+  uint8_t *v;
+  float *sm;
+  float *rmax;              // rows' scales, written
+  const float *cmax;
+  const float *cmax_next;
+  // statistics of the last leading dimension, the one before it and the first of three (of two: the first again)
+  const float *last, *before, *outer;
+  const float *last_next, *before_next, *outer_next;
+  uint32_t numel;
+  uint32_t last_size, before_size;
+  uint32_t cols_magic, last_magic, before_magic;   // divisions by cols and by the two sizes (fast_div)
+  uint16_t cols;
+  uint8_t cols_shift, last_shift, before_shift;
+  uint8_t lead_dims;        // 2 or 3
+};
+
+struct ShortArgs {
+  static constexpr int kCapacity = kMaxShortTensors;
+  static constexpr int kPivots = (kMaxShortTensors + 7) / 8;
+  StepConsts sc;
+  GradOps go;
+  int ntensors;
+  uint32_t chunk_base;     // as FusedArgs
+  ChunkRuns runs;
+  uint32_t pivot[kPivots];
+  uint32_t first_chunk[kPivots * 8];
+  uint32_t sr_salt[kMaxShortTensors];
+  uint32_t seed_lo, seed_hi;
+  ShortDesc desc[kMaxShortTensors];
 };
 
 // The statistics kernels index tiles of a matrix (rank1_stat_chunks).  A tensor with two or
@@ -302,7 +347,7 @@ struct NormArgs {
 
 static_assert(sizeof(StepConsts) <= Q4ADAMW_STEP_CONSTS_BYTES, "the device copy of a step's scalars");
 static_assert(sizeof(FusedArgs) <= 4096 && sizeof(SmallArgs) <= 4096 && sizeof(NormArgs) <= 4096 &&
-                  sizeof(Rank1Args) <= 4096 && sizeof(Rank1StatArgs) <= 4096 && sizeof(RowScaleArgs) <= 4096 &&
+                  sizeof(Rank1Args) <= 4096 && sizeof(ShortDesc) == 144 && sizeof(ShortArgs) <= 4096 && sizeof(Rank1StatArgs) <= 4096 && sizeof(RowScaleArgs) <= 4096 &&
                   sizeof(CommitArgs) <= 4096,
               "kernel arguments are limited to 4 KiB");
 

@@ -9,6 +9,7 @@ namespace q4 {
 typedef void (*FusedKernel)(const FusedArgs);
 typedef void (*SmallKernel)(const SmallArgs);
 typedef void (*Rank1Kernel)(const Rank1Args);
+typedef void (*ShortKernel)(const ShortArgs);
 typedef void (*Rank1StatKernel)(const Rank1StatArgs);
 
 // Kernel of a family for the (parameter, gradient) element types of a call: the tags
@@ -31,10 +32,12 @@ typedef void (*Rank1StatKernel)(const Rank1StatArgs);
 FusedKernel pick_fused(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 // the rank-1 update kernels: tiles anywhere in a matrix of rows at least a tile long
 // (pick_rank1_wide), matrices narrower than a tile (pick_rank1_narrow), tiles aligned to the
-// rows of a matrix (pick_rank1_rows), rows of any length (pick_rank1_any)
+// rows of a matrix (pick_rank1_rows), rows of any length (pick_rank1_any), rows shorter than a tile in tensors
+// of fewer than 2^32 elements (pick_rank1_short)
 Rank1Kernel pick_rank1_wide(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 Rank1Kernel pick_rank1_narrow(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 Rank1Kernel pick_rank1_rows(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 Rank1Kernel pick_rank1_any(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
+ShortKernel pick_rank1_short(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 
 }  // namespace q4

@@ -42,7 +42,9 @@ struct Geometry {
 // lanes of the others load nothing, work on zeros and store nothing.  kTileAny: rows of any
 // length (not a multiple of 8, or shorter than 16): every element finds its own row and column
 // (matrices of fewer than 2^32 elements).
-constexpr int kTileWide = 0, kTileNarrow = 1, kTileRows = 2, kTileRowsLast = 3, kTileAny = 4;
+// kTileShort: short rows of a tensor with several leading dimensions; a workgroup's tiles are consecutive, and it lays
+// the scales of the rows they meet and those of all columns out in LDS (ShortTile).
+constexpr int kTileWide = 0, kTileNarrow = 1, kTileRows = 2, kTileRowsLast = 3, kTileAny = 4, kTileShort = 5;
 
 // What a wave of the kTileRows form knows beyond its tile number: its row, the tile's first
 // column, and this thread's share of the workgroup's fetch of the columns' maxima (old and
@@ -74,6 +76,86 @@ __device__ __forceinline__ void stage_columns(const RowsTile &rt, int tid) {
   }
 }
 
+// A workgroup of the kTileShort form lays out in LDS, of the rows that its kChunk consecutive elements meet and of all
+// columns, the old maximum and -16 / max(new one, kScaleLo) -- or a NaN, as a pattern larger than any other of them,
+// where the new maximum is above kScaleHi.  A thread requests its share of the maxima before the tile's own loads and
+// lays it out after them (stage).
+template <int N>
+struct ShortTile {
+  static constexpr int kChunk = 64 * N * kWaves, kRows = N == 4 ? 2 : 3;   // enough for rows of 3 elements
+  float2 *rows, *columns;      // LDS
+  const ShortDesc &T;
+  uint32_t first, row0, nrows, last_row;
+  float old_row[kRows][3], new_row[kRows][3];
+  float old_col, new_col;
+
+  __device__ __forceinline__ ShortTile(const ShortDesc &T_, uint32_t local, float2 *rows_, float2 *columns_)
+      : rows(rows_), columns(columns_), T(T_) {
+    first = local * (uint32_t)kChunk;    // fewer than 2^32 elements
+    row0 = fast_div(first, T.cols_magic, T.cols_shift);
+    last_row = fast_div(T.numel - 1u, T.cols_magic, T.cols_shift);
+    nrows = fast_div(first + (uint32_t)kChunk - 1u, T.cols_magic, T.cols_shift) - row0 + 1u;
+  }
+  // The statistics whose least is the scale of a row, old and new ones: of its last leading dimension, of the one
+  // before it and of the first of three.  Without branches, behind which the compiler would wait for the loads: of
+  // two dimensions the first is looked up twice.
+  __device__ __forceinline__ void look_up(uint32_t row, float (&old_max)[3], float (&new_max)[3]) const {
+    const uint32_t q = fast_div_any(row, T.last_magic, T.last_shift), k3 = fast_div_any(q, T.before_magic, T.before_shift);
+    const uint32_t i = row - q * T.last_size, j = T.lead_dims == 2u ? q : q - k3 * T.before_size, k = T.lead_dims == 2u ? q : k3;
+    old_max[0] = as_global<const float>(T.last)[i];
+    old_max[1] = as_global<const float>(T.before)[j];
+    old_max[2] = as_global<const float>(T.outer)[k];
+    new_max[0] = as_global<const float>(T.last_next)[i];
+    new_max[1] = as_global<const float>(T.before_next)[j];
+    new_max[2] = as_global<const float>(T.outer_next)[k];
+  }
+  static __device__ __forceinline__ float least(const float (&x)[3]) { return min_nonneg(min_nonneg(x[0], x[1]), x[2]); }
+  static __device__ __forceinline__ float2 old_and_inverse(float old_max, float new_max) {
+    const float inv = __builtin_amdgcn_rcpf(max_nonneg(new_max, kScaleLo)) * -16.0f;
+    return make_float2(old_max, new_max > kScaleHi ? bits2f(0xffc00000u) : inv);
+  }
+  __device__ __forceinline__ void request() {   // lanes without a row or column of their own take another's
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+      const uint32_t r = threadIdx.x + (uint32_t)h * kThreads, row = row0 + r;
+      look_up(row < last_row ? row : last_row, old_row[h], new_row[h]);
+    }
+    const uint32_t c = threadIdx.x < T.cols ? threadIdx.x : 0u;
+    old_col = as_global<const float>(T.cmax)[c];
+    new_col = as_global<const float>(T.cmax_next)[c];
+  }
+  // f(j, row, column) for a lane's N elements, the first at (row, column)
+  template <typename F>
+  __device__ __forceinline__ void walk(uint32_t row, uint32_t col, F f) const {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      f(j, row, col);
+      const bool ends = ++col == T.cols;
+      col = ends ? 0u : col;
+      row += ends ? 1u : 0u;
+    }
+  }
+  __device__ __forceinline__ void put_row(uint32_t r, const float (&old_max)[3], const float (&new_max)[3]) const {
+    const float fresh = least(new_max);
+    rows[r] = old_and_inverse(least(old_max), fresh);
+    // written by the workgroup where the row begins; nothing reads them while the step runs
+    if (row0 + r <= last_row && (uint64_t)(row0 + r) * T.cols >= first) as_global<float>(T.rmax)[row0 + r] = fresh;
+  }
+  __device__ __forceinline__ void stage() const {
+#pragma unroll
+    for (int h = 0; h < kRows; ++h) {
+      const uint32_t r = threadIdx.x + (uint32_t)h * kThreads;
+      if (r < nrows) put_row(r, old_row[h], new_row[h]);
+    }
+    for (uint32_t r = threadIdx.x + kRows * kThreads; r < nrows; r += kThreads) {   // rows of two elements
+      float old_max[3], new_max[3];
+      look_up(row0 + r < last_row ? row0 + r : last_row, old_max, new_max);
+      put_row(r, old_max, new_max);
+    }
+    if (threadIdx.x < T.cols) columns[threadIdx.x] = old_and_inverse(old_col, new_col);
+  }
+};
+
 // A lane's codes of both moments in a full tile.
 template <int N>
 __device__ __forceinline__ void store_codes(uint32_t mword, uint32_t vword, const uint8_t *m_tile, const uint8_t *v_tile, uint32_t offset) {
@@ -90,7 +172,7 @@ template <int PT, int GT, bool FULL, bool EXT, bool RANK1, bool SR, int SHAPE, b
 __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane, int wave, int tid,
                                              const StepConsts &sc, uint2 *lds, const TableSlot &slot,
                                              float gscale, bool zero_g, uint32_t salt,
-                                             const RowsTile *rt = nullptr) {
+                                             const RowsTile *rt = nullptr, const ShortTile<Geometry<PT, GT>::kEpl> *st = nullptr) {
   using G = Geometry<PT, GT>;
   constexpr int N = G::kEpl;
   constexpr bool kRows = SHAPE == kTileRows || SHAPE == kTileRowsLast;
@@ -121,7 +203,10 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
   float r_old = 0.0f, r_new = 0.0f;
   Vals<N> c_old, c_new;
   Vals<N> ro, rn;   // kTileAny: the row maxima of every element
-  if constexpr (RANK1 && SHAPE == kTileAny) {
+  uint32_t short_row = 0, short_col = 0;   // kTileShort: the lane's first element
+  if constexpr (SHAPE == kTileShort) {
+    // through LDS, further down
+  } else if constexpr (RANK1 && SHAPE == kTileAny) {
     // T.div_magic / div_shift divide by cols; rows of elements past the end are clamped.  A lane whose elements
     // lie in one row, nearly every one of a matrix of hundreds of columns, takes one maximum of the row and the
     // columns' with 16-byte loads (at any element's address), old and new: 4 or 6 loads.  One of each kind per element
@@ -271,6 +356,7 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     entry[kLdsSecondMoment] = v_entry;
   }
   if constexpr (RANK1 && kRows) stage_columns<N>(*rt, tid);
+  if constexpr (SHAPE == kTileShort) st->stage();
   setup_tables<SR>(lds, tid, slot);
   if constexpr (RANK1 && kRows) {
 #pragma unroll
@@ -281,6 +367,16 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
       c_old.x[k] = a.x; c_old.x[k + 1] = a.y; c_old.x[k + 2] = a.z; c_old.x[k + 3] = a.w;
       c_new.x[k] = b.x; c_new.x[k + 1] = b.y; c_new.x[k + 2] = b.z; c_new.x[k + 3] = b.w;
     }
+  }
+  if constexpr (SHAPE == kTileShort) {
+    // c_old: the elements' old scales, c_new: the reciprocals of their new ones (the larger of row's and column's)
+    short_row = fast_div((uint32_t)tb + e0, T.cols_magic, T.cols_shift);
+    short_col = (uint32_t)tb + e0 - short_row * T.cols;
+    st->walk(short_row - st->row0, short_col, [&](int j, uint32_t row, uint32_t col) {
+      const float2 r = st->rows[row], c = st->columns[col];
+      c_old.x[j] = min_nonneg(r.x, c.x);
+      c_new.x[j] = max_nonneg(r.y, c.y);
+    });
   }
 
   // entry numbers of the lane's codes, one per byte: even elements, odd elements
@@ -304,7 +400,7 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     const uint32_t vo = entry_offset(j & 1 ? v_odd : v_even, j >> 1, two);
     const float m_old = *reinterpret_cast<const float *>(lds_bytes + mo);
     float v_old = *reinterpret_cast<const float *>(lds_bytes + vo + kLdsSecondMoment * 4u);
-    if constexpr (RANK1) v_old = sc.b2 * (v_old * min_nonneg(SHAPE == kTileAny ? ro.x[j] : r_old, c_old.x[j]));  // adamw_fourbit_triton.py:520-527
+    if constexpr (RANK1) v_old = sc.b2 * (v_old * (SHAPE == kTileShort ? c_old.x[j] : min_nonneg(SHAPE == kTileAny ? ro.x[j] : r_old, c_old.x[j])));  // adamw_fourbit_triton.py:520-527
     const float gj = g[j];
     float m = m_old + sc.r1 * gj;                 // m_old, v_old: beta times the old moment
     float v = v_old + sc.r2 * (gj * gj);
@@ -422,6 +518,15 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
       inv_max = max_nonneg(inv_max, neg_inv16.x[j]);
     }
     redo_v |= r_new > kScaleHi || (inv_max <= -kInvScaleLo16 && v_lane_max != 0.0f);
+  } else if constexpr (SHAPE == kTileShort) {
+    // a NaN, and the reciprocal of a clamped scale, as patterns are at least the limit's
+    uint32_t inv_max = 0u;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      neg_inv16.x[j] = c_new.x[j];
+      inv_max = f2bits(c_new.x[j]) > inv_max ? f2bits(c_new.x[j]) : inv_max;
+    }
+    redo_v |= inv_max >= f2bits(-kInvScaleLo16) && v_lane_max != 0.0f;
   } else if constexpr (RANK1 && SHAPE == kTileAny) {
     float s_least = rn.x[0], s_most = 0.0f;
 #pragma unroll
@@ -532,6 +637,13 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
         s_new.x[k + 3] = min_nonneg(r_new, c.w);
       }
     }
+    if constexpr (SHAPE == kTileShort) {
+      st->walk(short_row, short_col, [&](int j, uint32_t row, uint32_t col) {
+        float old_max[3], new_max[3];
+        st->look_up(row < st->last_row ? row : st->last_row, old_max, new_max);
+        s_new.x[j] = min_nonneg(st->least(new_max), as_global<const float>(T.cmax_next)[col]);
+      });
+    }
     vword = 0;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
@@ -632,6 +744,50 @@ __global__ __launch_bounds__(kThreads) void fused_4bit_rank1_kernel(const Rank1A
     process_tile<PT, GT, true, EXT, true, SR, FORM, EXACT>(T, begin, lane, wave, tid, sc, lds, slot, gscale, zero_g, salt);
   else
     process_tile<PT, GT, false, EXT, true, SR, FORM, EXACT>(T, begin, lane, wave, tid, sc, lds, slot, gscale, zero_g, salt);
+}
+
+// Tensors with several leading dimensions and rows of up to kShortMaxCols elements, of any length.  A workgroup's
+// kChunk consecutive elements meet hundreds of rows, whose scales it lays out in LDS together with the columns', old
+// maxima and reciprocals of new ones (ShortTile).  The rows' come from the leading dimensions' statistics, which stay
+// in the caches; in the general form every element gathers its row's scale from vectors that a launch between
+// statistics and update makes and the commit copies, seven passes over a third as many floats as a 3x3 kernel has
+// elements.  Steps of residual networks, us, that form / this: 64 wide in fp32 106 / 88, 96 wide in bf16 238 / 174.
+// What bounds it now is latency: 88 registers in bf16 leave five waves per SIMD (six with spills: 182 us).
+template <int PT, int GT, bool EXT, bool SR, bool EXACT>
+__global__ __launch_bounds__(kThreads) void fused_4bit_rank1_short_kernel(const ShortArgs args) {
+  using G = Geometry<PT, GT>;
+  __shared__ uint2 lds[kLdsEntries];
+  __shared__ float2 rows[G::kChunk / 2 + 2], columns[kShortMaxCols];
+  const int tid = threadIdx.x;
+  const TableSlot slot = request_table_slot<SR>(tid);
+  const uint32_t chunk = args.chunk_base + run_chunk(args.runs, blockIdx.x);
+  float gscale = 1.0f;
+  const bool cancelled = EXT && !grad_ops_begin(args.go, gscale);
+  const bool zero_g = EXT && args.go.zero != 0u;
+  if (cancelled && !zero_g) return;
+  const int t = find_tensor(args, chunk);
+  const ShortDesc &T = args.desc[t];
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const uint32_t local = chunk - args.first_chunk[t];
+  const int64_t tile = (int64_t)local * kWaves + wave;
+  if (cancelled) {
+    zero_tile<GT, G::kEpl>(T.g, tile, T.numel, lane);
+    return;
+  }
+  ShortTile<G::kEpl> st(T, local, rows, columns);
+  st.request();
+  const int64_t begin = tile * G::kTile;
+  if (begin >= (int64_t)T.numel) {
+    st.stage();
+    setup_tables<SR>(lds, tid, slot);
+    return;
+  }
+  const uint32_t salt = !SR ? 0u : EXT ? step_salt(args.sr_salt[t], args.go, args.seed_lo, args.seed_hi) : args.sr_salt[t];
+  const StepConsts sc = EXT ? step_consts(args.sc, args.go) : args.sc;
+  if (begin + G::kTile <= (int64_t)T.numel)
+    process_tile<PT, GT, true, EXT, true, SR, kTileShort, EXACT>(T, begin, lane, wave, tid, sc, lds, slot, gscale, zero_g, salt, nullptr, &st);
+  else
+    process_tile<PT, GT, false, EXT, true, SR, kTileShort, EXACT>(T, begin, lane, wave, tid, sc, lds, slot, gscale, zero_g, salt, nullptr, &st);
 }
 
 // The same for matrices whose rows are a whole number of quantization blocks and at least

@@ -103,6 +103,46 @@ def test_one_list_of_every_form(cuda, copies, p_dt, g_dt):
 
 
 @pytest.mark.parametrize("stochastic", [False, True])
+@pytest.mark.parametrize("p_dt,g_dt", [("fp32", "fp32"), ("bf16", "bf16")])
+@pytest.mark.parametrize("shape", [(7, 1, 2), (1, 9, 2), (40, 60, 2), (2, 3, 400, 2), (3, 1, 50, 3), (6, 70, 1, 5), (9, 40, 3, 3), (2, 5, 7, 63),
+                                   (33, 31, 61), (5, 130, 8), (4, 11, 65)])
+def test_short_rows_of_several_dimensions(cuda, shape, p_dt, g_dt, stochastic):
+    """The kernel that makes the rows' scales from the leading statistics: rows of two elements (more of them than a
+    workgroup's threads take at once), leading dimensions of one index, the longest rows and the first
+    beyond them; gradients whose second moments lie below and above the reciprocals' range, which
+    sends elements to the division.  The rows' scales that the step leaves are the statistics' minima."""
+    gen = torch.Generator().manual_seed(sum(shape) + stochastic)
+    n, cols, k = int(torch.Size(shape).numel()), shape[-1], len(shape) - 1
+    rows = n // cols
+    z = lambda m, dt=torch.float32: torch.zeros(m, dtype=dt, device=cuda)
+    p0 = (torch.randn(shape, generator=gen) * 0.05).to(base.DT[p_dt])
+    p, m, v, sm = p0.clone().to(cuda), z((n + 1) // 2, torch.uint8), z((n + 1) // 2, torch.uint8), z((n + 127) // 128)
+    r, rn, c, cn = z(rows), z(rows), z(cols), z(cols)
+    lead = ([z(d) for d in shape[:-1]], [z(d) for d in shape[:-1]])
+    ref = (p0, m.cpu(), v.cpu(), sm.cpu(), [torch.zeros([shape[j] if d == j else 1 for d in range(k + 1)]) for j in range(k + 1)])
+    sr = dict(seed=0x1234_5678_9ABC, tensor_salt=3) if stochastic else {}
+    for step, scale in ((1, 1.0), (2, 1e-17), (3, 1e17), (4, 1.0)):
+        g = grads_config1(gen, n).view(shape) * 1e3
+        g[shape[0] // 2:] *= scale                  # half of the first dimension: scales of both kinds meet
+        g = g.to(base.DT[g_dt])
+        if step == 2:                               # the second moments are small only where no large ones are left
+            ref = (ref[0], ref[1], torch.zeros_like(ref[2]), ref[3], [torch.zeros_like(x) for x in ref[4]])
+            for x in (v, r, c, *lead[0]):
+                x.zero_()
+        with torch.no_grad():
+            ref = ot.step_quant_rank1_nd(ref[0], g, *ref[1:], step=step, **sr, **HP)
+        q.fused_4bit_rank1_multi([p], [g.to(cuda)], [m], [v], [sm], [r], [c], [rn], [cn], *base.HPA, step, leads=[lead],
+                                 **(dict(seed=sr["seed"], salts=[3]) if stochastic else {}))
+        what = f"{shape} {p_dt}/{g_dt} step {step}"
+        assert torch.equal(m.cpu(), ref[1]), f"{what}: m codes"
+        for have, want in zip(lead[0] + [c], ref[4]):
+            assert torch.equal(have.cpu().view(torch.int32), want.reshape(-1).view(torch.int32)), f"{what}: statistics"
+        assert torch.equal(v.cpu(), ref[2]), f"{what}: v codes"
+        assert torch.equal(r, q.rank1_row_scale(lead[0], shape[:-1])), f"{what}: rows' scales"
+        assert not rn.any() and not cn.any() and not any(x.any() for x in lead[1]), f"{what}: scratch"
+
+
+@pytest.mark.parametrize("stochastic", [False, True])
 @pytest.mark.parametrize("g_dt", ["fp32", "bf16", "fp16"])
 @pytest.mark.parametrize("shape", [(300, 3), (77, 50), (1000, 88), (6200, 41), (64, 264), (33, 301),
                                    (5, 40, 3, 3), (33, 7, 5), (20, 3, 64), (3, 9, 264), (2, 5, 300), (2, 3, 300, 3), (3, 2, 270, 40)])
