@@ -291,15 +291,26 @@ static ChunkRuns stat_runs(Rank1StatForm form, int g_dtype, uint32_t tiles) {
   return grouped ? ChunkRuns{3u, tiles & ~63u} : ChunkRuns{0u, 0u};
 }
 
+// Indices of the first dimension whose statistics one workgroup of the lead form takes: as many as leave the launch
+// 768 workgroups, three per CU, because every workgroup updates the other dimensions' statistics, one update of an
+// address after another.  Steps, us, with at least 512 / 768 / 2048 / any number of workgroups of 32: residual networks,
+// 64 wide in fp32, three blocks a stage 104 / 94 / 104 / 104, 96 wide in bf16 139 / 133 / 142 / 140; [256, n, c] of 41 million fp32
+// elements, c = 5 166 / 155 / 172 / 197, c = 64 145 / 157 / 184 / 215.
+static uint32_t lead_stat_outer(uint64_t elements, uint32_t run) {
+  uint32_t most = kLeadMostOuter;
+  while (most > kLeadOuter && elements / ((uint64_t)run * most) < 768u) most /= 2u;
+  return most;
+}
+
 // tiles of the statistics launch of a matrix
-static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_rows) {
+static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_rows, int g_dtype) {
   if (rank1_stat_form(t) == kStatFlat) {
     const uint64_t rows = (uint64_t)flat_tile_rows((uint32_t)t.cols) * flat_tiles((uint32_t)t.cols, stat_rows);
     return ((uint64_t)t.rows + rows - 1) / rows;
   }
   if (rank1_stat_form(t) == kStatLead) {
     const uint32_t outer = (uint32_t)t.lead_shape[0];
-    return (uint64_t)((outer + kLeadOuter - 1) / kLeadOuter) * lead_tiles((uint32_t)t.rows, outer, (uint32_t)t.cols).inner;
+    return (uint64_t)((outer + stat_rows - 1) / stat_rows) * lead_tiles((uint32_t)t.rows, outer, (uint32_t)t.cols, lead_run(g_dtype != Q4ADAMW_FP32)).inner;
   }
   return (((uint64_t)t.rows + stat_rows - 1) / stat_rows) * (uint64_t)((t.cols + kStatCols - 1) / kStatCols);
 }
@@ -601,7 +612,7 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       }
       if (prod != t.rows) return fail(Q4ADAMW_ERR_ARG, "rows must be the product of the leading dimensions");
     }
-    const uint64_t stat_chunks = rank1_stat_chunks(t, 32u);   // at most
+    const uint64_t stat_chunks = rank1_stat_chunks(t, 32u, g_dtype);   // at most
     if (rank1_chunks(t, chunk_elems / kWaves) > kMaxChunksPerLaunch || stat_chunks > kMaxChunksPerLaunch)
       return fail(Q4ADAMW_ERR_TOO_LARGE, "tensor too large: more than 2^31 - 16 chunks");
   }
@@ -633,7 +644,7 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       tallest = (uint64_t)t.rows > tallest ? (uint64_t)t.rows : tallest;
     }
     if (elements == 0) return 0;
-    sa.stat_rows = rank1_stat_rows(elements, tallest);
+    sa.stat_rows = form == kStatLead ? lead_stat_outer(elements, lead_run(g_dtype != Q4ADAMW_FP32)) : rank1_stat_rows(elements, tallest);
     int n = 0;
     for (int i = 0; i < a.ntensors; ++i) {
       const q4adamw_rank1_tensor &t = *batch[i];
@@ -651,10 +662,11 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       for (int j = 0; j < 3; ++j) {
         const bool there = j < (int)sd.lead_dims;
         sd.lead_next[j] = there ? t.lead_max_next[j] : nullptr;
+        sd.lead_old[j] = there ? t.lead_max[j] : nullptr;
         sd.lead_shape[j] = there ? (uint32_t)t.lead_shape[j] : 1u;
       }
       sa.first_chunk[n] = (uint32_t)tiles;
-      tiles += rank1_stat_chunks(t, sa.stat_rows);
+      tiles += rank1_stat_chunks(t, sa.stat_rows, g_dtype);
       ++n;
     }
     finish_prefix(sa, n);
@@ -720,7 +732,7 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       const q4adamw_rank1_tensor &t = tensors[i];
       if (t.rows == 0 || t.cols == 0 || pass_of(t) != pass) continue;
       const int64_t numel = t.rows * t.cols;
-      const uint64_t c = rank1_chunks(t, tile_elems), sc_ = rank1_stat_chunks(t, 32u);
+      const uint64_t c = rank1_chunks(t, tile_elems), sc_ = rank1_stat_chunks(t, 32u, g_dtype);
       auto commit_chunks_of = [](int64_t size) { return ((uint64_t)size + kCommitChunk - 1) / kCommitChunk; };
       // the kernel for short rows writes the rows' scales itself
       const bool rows_follow = route == kRouteShort;
@@ -1106,7 +1118,7 @@ int q4adamw_quantize_rank1(const float *x, int64_t rows, int64_t cols, uint8_t *
   finish_prefix(sa, 1);
   hipLaunchKernelGGL(fill_zero_kernel, dim3(64), dim3(256), 0, s, row_max, rows, col_max, cols);
   const Rank1StatKernel kernel = pick_rank1_stats_form<kAbsValues, false>(form);
-  if (int rc = for_each_grid(rank1_stat_chunks(t, sa.stat_rows), kThreads, [&](uint64_t base, uint64_t count) -> int {
+  if (int rc = for_each_grid(rank1_stat_chunks(t, sa.stat_rows, Q4ADAMW_FP32), kThreads, [&](uint64_t base, uint64_t count) -> int {
         sa.chunk_base = (uint32_t)base;
         sa.runs = stat_runs(form, Q4ADAMW_FP32, (uint32_t)count);
         hipLaunchKernelGGL(kernel, dim3((unsigned)count), dim3(kThreads), 0, s, sa);

@@ -266,10 +266,11 @@ struct Rank1StatArgs {
   GradOps go;
   uint32_t chunk_base;     // this grid's first tile (workgroup 0)
   ChunkRuns runs;          // wide forms: which tile a workgroup takes
-  uint32_t stat_rows;      // rows of a workgroup (flat form: at most, but for one tile): 32, 64, 128 or 256
+  // rows of a workgroup (flat form: at most, but for one tile; lead form: indices of the first dimension): 32, 64, 128 or 256
+  uint32_t stat_rows;
   uint32_t pivot[kPivots];
   uint32_t first_chunk[kPivots * 8];
-  struct Desc {  // 96 bytes
+  struct Desc {  // 120 bytes
     const void *g;
     const uint8_t *v;
     const float *rmax;
@@ -277,6 +278,7 @@ struct Rank1StatArgs {
     float *rmax_next;
     float *cmax_next;
     float *lead_next[3];
+    const float *lead_old[3];
     uint32_t lead_shape[3];
     uint32_t lead_dims;    // 0, 2 or 3
     uint32_t rows;

@@ -352,29 +352,35 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1S
   if (tid < cols && col_bits[tid] != 0u) raise_max(T.cmax_next + tid, col_bits[tid]);
 }
 
-// The same for tensors with several leading dimensions and fewer than kFlatMaxCols columns (a
+// The same for tensors with several leading dimensions and at most kFlatMaxCols columns (a
 // stack of 3x3 convolution kernels: [out, in, 3, 3]), straight to one statistic per dimension.
 // What bounds such a kernel is not its bytes but the updates of statistics that every
 // workgroup shares, which the memory side takes one after another: tiles of consecutive rows meet
 // nearly all of the second dimension each (on 20 such stacks, 11 million elements, a kernel
 // with those tiles took 23 us without its updates and 64 us with them).  So a tile is
-// two-dimensional: kLeadOuter indices of the first dimension times a run of at most 256
-// consecutive elements below it (whole rows), which meets 32 indices of the first dimension and
-// a few dozen of the second, 16 elements of a thread in flight: 26 to 30 us (16 indices 31 to 38,
-// 8 indices 42 to 49, 64 indices 34 to 44), against 5.7 ms for statistics and folds before.
-// A thread keeps one element of the run over the first dimension's indices.
-constexpr uint32_t kLeadOuter = 32;
+// two-dimensional: indices of the first dimension (args.stat_rows, 32 to 256: lead_stat_outer) times a run of whole rows
+// below it, which meets as many statistics of the first dimension and a few dozen of the second.
+// A lane keeps N consecutive elements of the run, 16 bytes of gradients, and the workgroup's waves share the first
+// dimension's indices.  Under one index after another the elements' other statistics stay the same, so a lane takes
+// their minimum once and the first dimension's is one number for the wave; the maxima stay in registers until the end.
+// With one element per lane, a load of each row's scale (4 bytes for every row of three elements) and 32 indices, steps
+// of residual networks took, us, 64 wide in fp32 88 (now 79), 96 wide in bf16 174 (133), of [256, n, 64] with 41 million
+// elements in fp32 213 (157), in bf16 166 (102).
+constexpr uint32_t kLeadOuter = 32, kLeadMostOuter = 256;    // a round's indices; the most
+
+// elements of a run, at most (16 bytes of gradients per lane)
+__host__ __device__ __forceinline__ constexpr uint32_t lead_run(bool half) { return half ? 512u : 256u; }
 
 struct LeadTiles {
   uint32_t inner_rows;   // rows below one index of the first dimension
-  uint32_t rows;         // of them in a tile
+  uint32_t rows;         // of them in a tile; the last tile begins early enough to have as many
   uint32_t inner;        // tiles along them
 };
 
-__host__ __device__ __forceinline__ LeadTiles lead_tiles(uint32_t rows, uint32_t outer, uint32_t cols) {
+__host__ __device__ __forceinline__ LeadTiles lead_tiles(uint32_t rows, uint32_t outer, uint32_t cols, uint32_t run) {
   LeadTiles l;
   l.inner_rows = rows / outer;
-  const uint32_t most = 256u / cols;
+  const uint32_t most = run / cols;
   l.inner = (l.inner_rows + most - 1u) / most;
   l.rows = (l.inner_rows + l.inner - 1u) / l.inner;   // evenly
   return l;
@@ -382,88 +388,155 @@ __host__ __device__ __forceinline__ LeadTiles lead_tiles(uint32_t rows, uint32_t
 
 template <int GT, bool EXT>
 __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1StatArgs args) {
-  constexpr int kAhead = 16;   // elements of a thread whose loads are in flight together
-  __shared__ uint32_t outer_bits[kThreads / 16][kLeadOuter];   // first dimension: each 16 lanes' maxima
-  __shared__ uint32_t slots[3][256];                           // second and third dimension, columns
+  constexpr uint32_t N = GT ? 8 : 4, kRun = lead_run(GT != 0), kSlots = 258;   // more than a run's rows, and than columns
+  constexpr int kPerWave = kLeadOuter / kWaves;                // indices of the first dimension, all in flight together
+  __shared__ uint32_t outer_bits[4][kLeadMostOuter];           // first dimension: each 16 lanes' maxima
+  __shared__ float run_max[kWaves][kRun];                      // the run's elements
+  __shared__ uint32_t slots[3][kSlots];                        // second and third dimension, columns
   const uint32_t chunk = args.chunk_base + blockIdx.x;
   float gscale = 1.0f;
   if (EXT && !grad_ops_begin(args.go, gscale)) return;
   const int t = find_tensor(args, chunk);
   const auto &T = args.desc[t];
-  const uint32_t tid = threadIdx.x, cols = T.cols, outer = T.lead_shape[0];
-  const LeadTiles L = lead_tiles(T.rows, outer, cols);
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, cols = T.cols, outer = T.lead_shape[0];
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const LeadTiles L = lead_tiles(T.rows, outer, cols, kRun);
   const uint32_t local = chunk - args.first_chunk[t], ot = local / L.inner, it = local - ot * L.inner;
-  const uint32_t o0 = ot * kLeadOuter, r0 = it * L.rows;
-  const uint32_t no = outer - o0 < kLeadOuter ? outer - o0 : kLeadOuter;
-  // the even split may leave its last tiles with fewer rows, or none
-  const uint32_t nr = r0 >= L.inner_rows ? 0u : L.inner_rows - r0 < L.rows ? L.inner_rows - r0 : L.rows;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) slots[k][tid] = 0u;
+  const uint32_t o0 = ot * args.stat_rows, no = outer - o0 < args.stat_rows ? outer - o0 : args.stat_rows;
+  // maxima do not mind rows seen twice
+  const uint32_t r0 = it * L.rows < L.inner_rows - L.rows ? it * L.rows : L.inner_rows - L.rows;
+  const uint32_t len = L.rows * cols;                          // elements of the run
+  for (uint32_t i = tid; i < kSlots; i += kThreads) slots[0][i] = slots[1][i] = slots[2][i] = 0u;
 
-  // this thread's element of the run, the same under every index of the first dimension
-  const uint32_t row = tid / cols, col = tid - row * cols;
-  const bool active = row < nr;
+  // this lane's elements, the same under every index of the first dimension: the last ones of the run for lanes
+  // that would reach past its end
+  const bool whole = len >= N;
+  const uint32_t elem = !whole ? 0u : lane * N < len - N ? lane * N : len - N;
+  const uint32_t shape2 = T.lead_dims == 3u ? T.lead_shape[2] : 1u;
+  const gptr<const float> before = as_global<const float>(T.lead_old[1]), last = as_global<const float>(T.lead_old[2]);
+  float s_old[N], x_max[N];
+  {
+    const uint32_t row = elem / cols;
+    uint32_t col = elem - row * cols, i1 = (r0 + row) / shape2, i2 = r0 + row - i1 * shape2;
+#pragma unroll
+    for (uint32_t k = 0; k < N; ++k) {
+      float s = 0.0f;
+      if (whole || k < len) {
+        s = min_nonneg(as_global<const float>(T.cmax)[col], before[i1]);
+        if (T.lead_dims == 3u) s = min_nonneg(s, last[i2]);
+      }
+      s_old[k] = s;
+      x_max[k] = 0.0f;
+      const bool row_ends = ++col == cols;
+      col = row_ends ? 0u : col;
+      i2 += row_ends ? 1u : 0u;
+      const bool wraps = i2 == shape2;
+      i2 = wraps ? 0u : i2;
+      i1 += wraps ? 1u : 0u;
+    }
+  }
   const int64_t below = (int64_t)L.inner_rows * cols;          // elements below one index
   const int64_t first = (int64_t)o0 * below + (int64_t)r0 * cols;
-  float x_max = 0.0f;
-  const float c_old = active ? as_global<const float>(T.cmax)[col] : 0.0f;
+  u32x4 gw[kPerWave];
+  uint32_t vw[kPerWave];
+  float o_old[kPerWave];
+  auto load = [&](uint32_t base, int i) {
+    // past the first dimension's end: its last index once more
+    const uint32_t mine = base + wave + (uint32_t)i * kWaves, o = mine < no ? mine : no - 1u;
+    const int64_t e = first + (int64_t)o * below;              // uniform
+    const void *g_run = static_cast<const char *>(T.g) + e * (GT ? 2 : 4);
+    const void *v_run = T.v + (e >> 1);
+    o_old[i] = as_constant<const float>(T.lead_old[0])[o0 + o];
+    if (whole) {
+      gw[i] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_run), elem * (GT ? 2u : 4u), 0, 0);
+      vw[i] = load_part_codes<N, true>(v_run, (uint32_t)e & 1u, elem);
+    } else {   // fewer elements below an index than a lane's
+      uint32_t w[4] = {0u, 0u, 0u, 0u};
+      vw[i] = 0u;
 #pragma unroll
-  for (uint32_t base = 0; base < kLeadOuter; base += kAhead) {
-    float g[kAhead], r_old[kAhead];
-    uint32_t byte[kAhead];
-    if (base < no) {
-#pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        // past the first dimension's end: its last index once more (maxima do not mind)
-        const uint32_t o = base + i < no ? base + i : no - 1u;
-        const int64_t e = first + (int64_t)o * below;          // uniform
-        g[i] = r_old[i] = 0.0f;
-        byte[i] = 0u;
-        if (active) {
-          g[i] = load_scalar<GT>(static_cast<const char *>(T.g) + e * (GT ? 2 : 4), tid);
-          byte[i] = as_global<const uint8_t>(T.v + (e >> 1))[(((uint32_t)e & 1u) + tid) >> 1];
-          r_old[i] = as_global<const float>(T.rmax)[(o0 + o) * L.inner_rows + r0 + row];
+      for (uint32_t k = 0; k < N; ++k) {
+        if (k < len) {
+          if constexpr (GT != 0) w[k / 2] |= (uint32_t)as_global<const uint16_t>(g_run)[k] << (16 * (k & 1));
+          else w[k] = as_global<const uint32_t>(g_run)[k];
+          const uint32_t nibble = ((uint32_t)e & 1u) + k;
+          vw[i] |= ((as_global<const uint8_t>(v_run)[nibble >> 1] >> (4 * (nibble & 1u))) & 15u) << (4 * k);
         }
       }
+      gw[i] = u32x4{w[0], w[1], w[2], w[3]};
+    }
+  };
+  auto reduce = [&](uint32_t base, int i) {
+    float g[8];
+    const u32x4 w = gw[i];
+    if constexpr (GT != 0) {
+      widen_pair<GT>(w.x, g[0], g[1]);
+      widen_pair<GT>(w.y, g[2], g[3]);
+      widen_pair<GT>(w.z, g[4], g[5]);
+      widen_pair<GT>(w.w, g[6], g[7]);
+    } else {
+      g[0] = bits2f(w.x); g[1] = bits2f(w.y); g[2] = bits2f(w.z); g[3] = bits2f(w.w);
+    }
+    const uint32_t even = vw[i] & 0x0F0F0F0Fu, odd = (vw[i] >> 4) & 0x0F0F0F0Fu;  // one code per byte
+    float o_max = 0.0f;
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        const uint32_t o = base + i < no ? base + i : no - 1u;
-        const uint32_t odd = (uint32_t)(first + (int64_t)o * below) & 1u;
-        const float gi = EXT ? g[i] * gscale : g[i];
-        const uint32_t code = (byte[i] >> (4u * ((tid + odd) & 1u))) & 15u;
-        const float code_value = __builtin_fmaf((float)code, 0.0625f, 0.0625f);  // (code + 1) / 16, exact
-        const float v_old = code_value * min_nonneg(r_old[i], c_old);
-        const float v = __builtin_fmaxf(args.b2 * v_old + args.r2 * (gi * gi), 0.0f);   // a NaN never becomes a maximum
-        x_max = __builtin_fmaxf(x_max, v);
-        const float quarter_max = row_max16(v);
-        if ((tid & 15u) == 0u) outer_bits[tid >> 4][base + i] = f2bits(quarter_max);
-      }
+    for (uint32_t k = 0; k < N; ++k) {
+      const float gk = EXT ? g[k] * gscale : g[k];
+      const float code_value = __builtin_fmaf((float)(((k & 1 ? odd : even) >> (8 * (k >> 1))) & 0xffu), 0.0625f, 0.0625f);  // (code + 1) / 16, exact
+      const float v_old = code_value * min_nonneg(o_old[i], s_old[k]);
+      const float v = args.b2 * v_old + args.r2 * (gk * gk);     // a NaN never becomes a maximum
+      x_max[k] = __builtin_fmaxf(x_max[k], v);
+      if (whole || k < len) o_max = __builtin_fmaxf(o_max, v);
+    }
+    o_max = row_max16(o_max);
+    const uint32_t mine = base + wave + (uint32_t)i * kWaves;
+    if ((lane & 15u) == 0u) outer_bits[lane >> 4][mine] = f2bits(o_max);
+  };
+  for (uint32_t base = 0; base < no; base += kLeadOuter) {
+    if (no - base > kLeadOuter / 2) {
+#pragma unroll
+      for (int i = 0; i < kPerWave; ++i) load(base, i);
+#pragma unroll
+      for (int i = 0; i < kPerWave; ++i) reduce(base, i);
+    } else {   // few indices are left: half as many rounds
+#pragma unroll
+      for (int i = 0; i < kPerWave / 2; ++i) load(base, i);
+#pragma unroll
+      for (int i = 0; i < kPerWave / 2; ++i) reduce(base, i);
     }
   }
-  __syncthreads();
-  const uint32_t shape2 = T.lead_dims == 3u ? T.lead_shape[2] : 1u;
-  const uint32_t first1 = r0 / shape2;                          // the tile's first index of the second dimension
-  if (active && x_max != 0.0f) {
-    const uint32_t q = (r0 + row) / shape2;
-    atomicMax(&slots[0][q - first1], f2bits(x_max));
-    if (T.lead_dims == 3u) {
-      // the third dimension's indices of consecutive rows, folded into 256 slots: a tile has at
-      // most 128 rows, so rows that share a slot share the index
-      const uint32_t i2 = r0 + row - q * shape2;
-      atomicMax(&slots[1][shape2 <= 256u ? i2 : row], f2bits(x_max));
-    }
-    atomicMax(&slots[2][col], f2bits(x_max));
+#pragma unroll
+  for (uint32_t k = 0; k < N; ++k) {
+    if (whole || k < len) run_max[wave][elem + k] = x_max[k];
   }
   __syncthreads();
+  const uint32_t first1 = r0 / shape2;                         // the tile's first index of the second dimension
+  for (uint32_t x = tid; x < len; x += kThreads) {
+    float u = run_max[0][x];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) u = __builtin_fmaxf(u, run_max[w][x]);
+    const uint32_t row = x / cols, i1 = (r0 + row) / shape2, i2 = r0 + row - i1 * shape2;
+    auto raise_slot = [&](uint32_t &slot) {
+      if (f2bits(u) > slot) atomicMax(&slot, f2bits(u));
+    };
+    raise_slot(slots[0][i1 - first1]);
+    // the third dimension's indices of consecutive rows: a run has fewer rows than slots, so rows that
+    // share a slot share the index
+    if (T.lead_dims == 3u) raise_slot(slots[1][shape2 < kSlots ? i2 : row]);
+    raise_slot(slots[2][x - row * cols]);
+  }
+  __syncthreads();
+  static_assert(kLeadMostOuter <= kThreads, "one index per thread below");
   if (tid < no) {
     uint32_t u = outer_bits[0][tid];
 #pragma unroll
-    for (int k = 1; k < kThreads / 16; ++k) u = u > outer_bits[k][tid] ? u : outer_bits[k][tid];
+    for (int k = 1; k < 4; ++k) u = u > outer_bits[k][tid] ? u : outer_bits[k][tid];
     if (u != 0u) raise_max(T.lead_next[0] + o0 + tid, u);
   }
-  if (slots[0][tid] != 0u) raise_max(T.lead_next[1] + first1 + tid, slots[0][tid]);
-  if (slots[1][tid] != 0u) raise_max(T.lead_next[2] + (shape2 <= 256u ? tid : (r0 + tid) % shape2), slots[1][tid]);
-  if (slots[2][tid] != 0u) raise_max(T.cmax_next + tid, slots[2][tid]);
+  for (uint32_t i = tid; i < kSlots; i += kThreads) {
+    if (slots[0][i] != 0u) raise_max(T.lead_next[1] + first1 + i, slots[0][i]);
+    if (slots[1][i] != 0u) raise_max(T.lead_next[2] + (shape2 < kSlots ? i : (r0 + i) % shape2), slots[1][i]);
+    if (slots[2][i] != 0u) raise_max(T.cmax_next + i, slots[2][i]);
+  }
 }
 
 // Tensors with several leading dimensions, between statistics and update: every row's new scale

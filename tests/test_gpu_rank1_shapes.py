@@ -24,7 +24,10 @@ TALL = [(6145, 50), (6144 + 63 * 5, 64), (6200, 255), (24577, 33), (24640, 88), 
 # either part, on its first and last columns and between them; 130 and 136 tiles, of which 128 are dealt in runs of 8
 PARTS = [(37, 258), (37, 259), (40, 260), (37, 261), (40, 504), (37, 507), (40, 508), (37, 510), (40, 512), (37, 515), (40, 520), (37, 767),
          (37, 770), (2080, 520), (1088, 1541)]
-TENSORS = [(5, 300, 3, 3), (2, 700, 3), (1400, 1, 2), (300, 2, 7), (16, 16, 16), (3, 100, 260), (2, 130, 4, 257), (64, 3, 7, 7)]
+TENSORS = [(5, 300, 3, 3), (2, 700, 3), (1400, 1, 2), (300, 2, 7), (16, 16, 16), (3, 100, 260), (2, 130, 4, 257), (64, 3, 7, 7),
+           # fewer elements below an index than a lane's; runs that end within a lane's; the most columns; half a round of
+           # indices, a round and one more
+           (3, 1, 2), (70, 2, 3), (700, 1, 3), (40, 1, 1, 5), (33, 90, 256), (17, 5, 2, 255), (16, 30, 3, 3), (129, 57, 3, 3), (5, 171, 3)]
 
 
 @pytest.mark.parametrize("p_dt,g_dt", [("fp32", "fp32"), ("bf16", "bf16"), ("fp32", "fp16")])
@@ -59,6 +62,27 @@ def test_statistics_of_a_tall_matrix(cuda, shape, p_dt, g_dt):
 @pytest.mark.parametrize("shape", TENSORS)
 def test_statistics_of_several_dimensions(cuda, shape, p_dt, g_dt):
     base.test_rank1_more_than_two_dimensions_against_oracle(cuda, shape, p_dt, g_dt, False)
+
+
+def test_statistics_of_many_indices_of_the_first_dimension(cuda):
+    """Enough elements that a workgroup takes 64 indices (12.6 million), the last one 8 of them; the oracle on the GPU."""
+    shape = (200, 7000, 3, 3)
+    gen = torch.Generator(device=cuda).manual_seed(5)
+    n, rows = 12_600_000, 4_200_000
+    z = lambda m, dt=torch.float32: torch.zeros(m, dtype=dt, device=cuda)
+    p0 = torch.randn(shape, generator=gen, device=cuda) * 0.05
+    p, m, v, sm = p0.clone(), z(n // 2, torch.uint8), z(n // 2, torch.uint8), z((n + 127) // 128)
+    r, rn, c, cn = z(rows), z(rows), z(3), z(3)
+    lead = ([z(d) for d in shape[:-1]], [z(d) for d in shape[:-1]])
+    ref = (p0, m.clone(), v.clone(), sm.clone(), [z(200).view(200, 1, 1, 1), z(7000).view(1, 7000, 1, 1), z(3).view(1, 1, 3, 1), z(3).view(1, 1, 1, 3)])
+    for step in (1, 2):
+        g = torch.randn(shape, generator=gen, device=cuda) * torch.rand(200, 1, 1, 1, generator=gen, device=cuda)
+        with torch.no_grad():
+            ref = ot.step_quant_rank1_nd(ref[0], g, *ref[1:], step=step, **HP)
+        q.fused_4bit_rank1_multi([p], [g], [m], [v], [sm], [r], [c], [rn], [cn], *base.HPA, step, leads=[lead])
+        for have, want in zip(lead[0] + [c], ref[4]):
+            assert torch.equal(have, want.reshape(-1)), f"step {step}: statistics"
+        assert torch.equal(m, ref[1]) and torch.equal(v, ref[2]), f"step {step}: codes"
 
 
 @pytest.mark.parametrize("p_dt,g_dt", [("fp32", "bf16"), ("bf16", "bf16")])
