@@ -122,11 +122,31 @@ EXPORTS = (
 )
 
 _lib = None
+host = None     # the module _q4host (csrc/q4host.cpp), once the library is loaded
+
+
+def _bind_host(L):
+    """Hands the native host code the library's entry points."""
+    try:
+        from . import _q4host
+    except ImportError as e:
+        raise RuntimeError(f"{os.path.join(_HERE, '_q4host.so')} is missing or does not load ({e}): build it with "
+                           "`python -m quantfour_adamw_cuda_amd.build`") from None
+    import torch
+    address = lambda name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value
+    c = torch._C
+    # without torch's two functions (a build without GPU support) every call takes the Python code's path
+    known = lambda name: getattr(c, name, None) or (lambda *a: -1)
+    _q4host.bind(*map(address, ("q4adamw_fused_4bit", "q4adamw_fused_single_tensor", "q4adamw_fused_4bit_multi_ex",
+                                "q4adamw_fused_4bit_multi_sr", "q4adamw_fused_4bit_rank1_multi", "q4adamw_fused_4bit_rank1_multi_sr",
+                                "q4adamw_fused_single_tensor_multi_ex")),
+                 known("_cuda_getCurrentRawStream"), known("_cuda_getDevice"))
+    return _q4host
 
 
 def load():
     """Returns the loaded library; raises RuntimeError when it has not been built."""
-    global _lib
+    global _lib, host
     if _lib is not None:
         return _lib
     if not os.path.exists(LIB_PATH):
@@ -204,6 +224,7 @@ def load():
     L.q4adamw_last_error.restype = ctypes.c_char_p
     L.q4adamw_version.argtypes = []
     L.q4adamw_version.restype = i
+    host = _bind_host(L)
     _lib = L
     return L
 

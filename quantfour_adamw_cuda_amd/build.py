@@ -3,7 +3,8 @@ probes) for gfx950 with hipcc (cross-compiles without a GPU).
 
 Counterpart of the reference's optim/setup.py:6-23 (a torch CUDAExtension built by
 nvcc); here the product is a plain C-ABI shared library, so no torch headers and
-no pybind11 are involved.
+no pybind11 are involved in it.  The Python side's own native part, the CPython module
+_q4host.so (csrc/q4host.cpp: host code only, built with g++), is the one that sees torch's headers.
 
 Usage:  python -m quantfour_adamw_cuda_amd.build
 """
@@ -15,6 +16,7 @@ import tempfile
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB = os.path.join(CSRC, "libq4adamw.so")
 PROBE_LIB = os.path.join(CSRC, "libq4probe.so")
+HOST_MODULE = os.path.join(os.path.dirname(CSRC), "_q4host.so")
 HOST_PASS_NOTE = "'-packed-fp32-ops' is not a recognized feature for this target (ignoring feature)"
 
 HIPCC_FLAGS = [
@@ -89,8 +91,31 @@ def compile_library(out, sources, flags=None, verbose=False, check_output=True):
     return out
 
 
+def compile_host_module(out=HOST_MODULE, verbose=False):
+    """csrc/q4host.cpp against the running interpreter's and torch's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    for path in [*include_paths(), sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", path]
+    cmd += ["-o", out, os.path.join(CSRC, "q4host.cpp")]
+    for path in library_paths():
+        cmd += ["-L" + path]
+    cmd += ["-ltorch_python", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if verbose or proc.returncode != 0:
+        print(proc.stdout)
+    if proc.returncode != 0 or proc.stdout.strip():
+        raise RuntimeError("the host module's build is kept warning-free:\n" + proc.stdout)
+    return out
+
+
 def build(verbose=False):
     """Compile unconditionally; returns the path of the step library."""
+    compile_host_module(verbose=verbose)
     compile_library(LIB, STEP_SOURCES, verbose=verbose)
     compile_library(PROBE_LIB, PROBE_SOURCES, verbose=verbose)
     return LIB

@@ -26,6 +26,7 @@ the same path through the `grad_scale` / `found_inf` attributes it sets.
 The step itself runs only in the HIP library (csrc/libq4adamw.so); without it,
 or with parameters that are not on a GPU, `step()` raises.
 """
+import ctypes
 from itertools import chain, compress
 from operator import attrgetter, is_, methodcaller
 from typing import Any, Dict, Optional
@@ -58,7 +59,14 @@ class _Bucket:
 class _Plan:
     """A param group's launches and what they rest on (see _build_plan / _refresh_plan)."""
     __slots__ = ("gi", "capturable", "stochastic", "state_obj", "params_obj", "param_ids", "all_params",
-                 "has_grad", "plannable", "params", "p_ptrs", "step_views", "grads", "buckets", "held")
+                 "has_grad", "plannable", "params", "p_ptrs", "step_views", "grads", "buckets", "held",
+                 "native", "native_held")
+
+
+# kinds of launch in the native plan, and what a failed one is called
+_KINDS = {False: 0, True: 1, "sr": 2, "rank1": 3, "rank1_sr": 4}
+_KIND_NAMES = ("fused_single_tensor_multi", "fused_4bit_multi", "fused_4bit_multi_sr", "fused_4bit_rank1_multi",
+               "fused_4bit_rank1_multi_sr")
 
 
 class AdamWFused_QuantFour(torch.optim.Optimizer):
@@ -436,6 +444,10 @@ class AdamWFused_QuantFour(torch.optim.Optimizer):
         if max_grad_norm is None:
             return host, dev
         # global norm of the multiplied gradients, per dtype on the device, combined there
+        if self.kernel_timing is None:
+            mult = self._one_norm(host, dev, float(max_grad_norm))
+            if mult is not None:
+                return 1.0, mult
         by_dtype: Dict[Any, list] = {}
         for group in self.param_groups:
             for p in group["params"]:
@@ -471,6 +483,31 @@ class AdamWFused_QuantFour(torch.optim.Optimizer):
         self.last_grad_norm = total
         mult = coef * host if dev is None else coef * host * dev
         return 1.0, mult.reshape(1)
+
+    def _one_norm(self, host, dev, max_grad_norm):
+        """The device multiplier where all gradients are dense, of one dtype and on one device, which native code
+        finds out while it fills the descriptors; None otherwise."""
+        _lib.load()
+        groups = tuple(group["params"] for group in self.param_groups)
+        size = sum(map(len, groups))
+        table = self._norm_buffers.get("table")
+        if table is None or len(table) < size:
+            table = self._norm_buffers["table"] = (_lib.Q4Grad * max(size, 1))()
+        found = _lib.host.gradients(groups, ctypes.addressof(table), len(table))
+        if found is None:
+            return None
+        count, tag, index = found
+        key = (index, tag)
+        bufs = self._norm_buffers.get(key)
+        if bufs is None:
+            device = torch.device("cuda", index)
+            out = torch.empty(3, dtype=torch.float32, device=device)
+            bufs = (device, out, torch.empty(_lib.NORM_WORKSPACE_BYTES // 8, dtype=torch.float64, device=device), out[0], out[2:3])
+            self._norm_buffers[key] = bufs
+        device, out, workspace, norm, mult = bufs
+        _q.grad_norm_table(table, device, tag, out, workspace, host, dev, max_grad_norm, count=count)
+        self.last_grad_norm = norm
+        return mult
 
     @torch.no_grad()
     def step(self, closure=None, *, grad_scale=None, found_inf=None, max_grad_norm=None,
@@ -623,9 +660,25 @@ class AdamWFused_QuantFour(torch.optim.Optimizer):
                         extra.append((variance_meta[i], key, variance_meta[i][key]))
         held = (core, extra)
         plan.held = held
+        plan.native = plan.native_held = None
         if plan.plannable:
             self._plans[gi] = plan
+            if not capturable:
+                self._make_native(plan)
         return plan
+
+    def _make_native(self, plan):
+        """The plan in native code (csrc/q4host.cpp), where it is for it: plain tensors on one device.  It borrows
+        every object that the plan holds."""
+        core, extra = plan.held
+        held = [(st, key, value) for st, *values in core for key, value in zip(("step", "exp_avg", "exp_avg_sq"), values)] + extra
+        buckets = [(_KINDS[b.kind], b.idx, ctypes.addressof(b.arr), ctypes.sizeof(b.arr._type_), b.p_tag, b.g_tag,
+                    0 if b.salts is None else ctypes.addressof(b.salts)) for b in plan.buckets]
+        buf = self._step_buffers[plan.gi][0]
+        plan.native_held = (held, buckets, buf)
+        plan.native = _lib.host.plan(plan.all_params, buf, held, buckets)
+        if plan.native is not None:
+            plan.grads = None        # native code looks at every gradient anew
 
     def _refresh_plan(self, group, plan):
         """True if the plan of the last step still describes this group -- the same parameters
@@ -636,8 +689,11 @@ class AdamWFused_QuantFour(torch.optim.Optimizer):
         params = group["params"]
         if (params is not plan.params_obj or self.state is not plan.state_obj
                 or bool(group.get("capturable", False)) != plan.capturable
-                or (group.get("round_type", "real-nearest") == "stochastic") != plan.stochastic
-                or list(map(id, params)) != plan.param_ids):
+                or (group.get("round_type", "real-nearest") == "stochastic") != plan.stochastic):
+            return False
+        if plan.native is not None:
+            return _lib.host.refresh(plan.native, params, self._step_buffers[plan.gi][0])
+        if list(map(id, params)) != plan.param_ids:
             return False
         all_grads = list(map(attrgetter("grad"), params))
         if [g is not None for g in all_grads] != plan.has_grad:
@@ -691,6 +747,18 @@ class AdamWFused_QuantFour(torch.optim.Optimizer):
         lr = 1.0 if capturable else float(group["lr"])
         weight_decay = group["weight_decay"]
         eps = group["eps"]
+        if plan.native is not None and self.kernel_timing is None:
+            options = _q.grad_options(plan.buckets[0].device, host_mult, dev_mult, found_inf, zero_grad, None,
+                                      group.get("param_update", "auto"))
+            seed = int(group["seed"]) if plan.stochastic else 0
+            done = _lib.host.run(plan.native, beta1, beta2, lr, weight_decay, eps,
+                                 0 if options is None else ctypes.addressof(options), seed)
+            if done is not None:
+                stepped.extend(plan.step_views)
+                rc, k = done
+                if rc:
+                    _lib.check(rc, _KIND_NAMES[_KINDS[plan.buckets[k].kind]])
+                return
         before = ([float(s) for s in plan.step_views]
                   if capturable and not self._has_device_steps(gi) else None)
         steps = self._advance_steps(gi, plan.params, plan.step_views)

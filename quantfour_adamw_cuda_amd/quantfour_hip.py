@@ -97,6 +97,11 @@ def fused_4bit(p, g, exp, sq, exp_scale, sq_scale, beta1, beta2, lr, weight_deca
         return fused_4bit_multi([p], [g], [exp], [sq], [exp_scale], [sq_scale], beta1, beta2, lr,
                                 weight_decay, eps, step, update_form=update_form)
     L = _lib.load()
+    rc = _lib.host.fused_4bit(p, g, exp, sq, exp_scale, sq_scale, beta1, beta2, lr, weight_decay, eps, step)
+    if rc is not None:
+        if rc:
+            _lib.check(rc, "fused_4bit")
+        return
     check_quantized(p, g, exp, sq, exp_scale, sq_scale)
     with _on(p.device):
         rc = L.q4adamw_fused_4bit(p.data_ptr(), g.data_ptr(), exp.data_ptr(), sq.data_ptr(),
@@ -109,6 +114,11 @@ def fused_4bit(p, g, exp, sq, exp_scale, sq_scale, beta1, beta2, lr, weight_deca
 def fused_single_tensor(p, g, exp_avg, exp_avg_sq, beta1, beta2, lr, weight_decay, eps, step):
     """optim/cuda_fused_interface.cc:49-64."""
     L = _lib.load()
+    rc = _lib.host.fused_single_tensor(p, g, exp_avg, exp_avg_sq, beta1, beta2, lr, weight_decay, eps, step)
+    if rc is not None:
+        if rc:
+            _lib.check(rc, "fused_single_tensor")
+        return
     check_unquantized(p, g, exp_avg, exp_avg_sq)
     with _on(p.device):
         rc = L.q4adamw_fused_single_tensor(p.data_ptr(), g.data_ptr(), exp_avg.data_ptr(),
@@ -446,13 +456,14 @@ def make_grad_table(gs):
 
 
 def grad_norm_table(arr, device, g_tag, out3, workspace, grad_scale=1.0, grad_scale_dev=None,
-                    max_norm=0.0):
+                    max_norm=0.0, count=None):
+    """count: how many of the array's descriptors, all of them by default."""
     L = _lib.load()
     assert out3.dtype == torch.float32 and out3.numel() >= 3 and out3.device == device
     assert workspace.device == device and workspace.numel() * workspace.element_size() >= _lib.NORM_WORKSPACE_BYTES
     dev_ptr = None if grad_scale_dev is None else _device_scalar(grad_scale_dev, device, "grad_scale_dev")
     with _on(device):
-        rc = L.q4adamw_grad_norm(arr, len(arr), g_tag, float(grad_scale), dev_ptr, float(max_norm),
+        rc = L.q4adamw_grad_norm(arr, len(arr) if count is None else count, g_tag, float(grad_scale), dev_ptr, float(max_norm),
                                  workspace.data_ptr(), workspace.numel() * workspace.element_size(),
                                  out3.data_ptr(), _stream(device))
     _lib.check(rc, "grad_norm")

@@ -1,0 +1,106 @@
+"""The native host code (csrc/q4host.cpp): it takes the common case and leaves everything else to the Python
+code, with the same results."""
+import ctypes
+
+import pytest
+import torch
+
+from quantfour_adamw_cuda_amd import AdamWFused_QuantFour, _lib
+from quantfour_adamw_cuda_amd import quantfour_hip as q
+
+HP = (0.9, 0.999, 1e-3, 0.01, 1e-8)
+
+
+def test_what_is_not_for_it_is_left_alone():
+    _lib.load()
+    h = _lib.host
+    p, g = torch.zeros(200), torch.zeros(200)
+    state = [torch.zeros(100, dtype=torch.uint8), torch.zeros(100, dtype=torch.uint8), torch.zeros(2), torch.zeros(2)]
+    assert h.fused_4bit(p, g, *state, *HP, 1.0) is None                    # not on a GPU
+    assert h.fused_4bit(p, None, *state, *HP, 1.0) is None and h.fused_4bit(p, g) is None
+    assert h.fused_single_tensor(p, g, p, g, *HP, 1.0) is None
+    par = torch.nn.Parameter(torch.zeros(4))
+    par.grad = torch.zeros(4)
+    table = (_lib.Q4Grad * 2)()
+    assert h.gradients(([par],), ctypes.addressof(table), 2) is None and h.gradients(([],), ctypes.addressof(table), 2) is None
+    assert h.plan((par,), torch.zeros(1), [], []) is None
+    with pytest.raises((TypeError, ValueError)):
+        h.refresh(object(), [par], torch.zeros(1))
+    with pytest.raises(TypeError):
+        h.run(1)
+
+
+def _twins(cuda, shapes, p_dt, g_dt, **kw):
+    gen = torch.Generator(device=cuda).manual_seed(3)
+    sides = []
+    base = [(torch.randn(s, generator=gen, device=cuda) * 0.05).to(p_dt) for s in shapes]
+    for native in (True, False):
+        ps = [torch.nn.Parameter(b.clone()) for b in base]
+        for p in ps:
+            if p_dt != g_dt:
+                p.grad_dtype = g_dt
+        opt = AdamWFused_QuantFour(ps, lr=1e-3, weight_decay=0.01, **kw)
+        if not native:
+            opt._make_native = lambda plan: None
+            opt._one_norm = lambda *a: None
+        sides.append((ps, opt))
+    return gen, sides
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p_dt,g_dt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("kw", [{}, dict(round_type="stochastic", seed=5), dict(variance_scale_type="rank1"),
+                                dict(variance_scale_type="rank1", round_type="stochastic", seed=2 ** 40 + 1)])
+def test_steps_equal_the_python_codes(cuda, kw, p_dt, g_dt):
+    """Every kind of launch, new gradient tensors each step, options of a step, a learning rate that changes, a
+    parameter without a gradient in one step."""
+    gen, sides = _twins(cuda, [(70, 129), (5000,), (64, 512), (100,), (3, 20, 96), (30, 16, 3, 3)], p_dt, g_dt, **kw)
+    options = [{}, dict(max_grad_norm=0.5), dict(grad_scale=0.25, zero_grad=True), dict(found_inf=torch.ones(1, device=cuda)),
+               dict(grad_scale=torch.full((1,), 2.0, device=cuda), max_grad_norm=3.0, found_inf=torch.zeros(1, device=cuda)), {}, {}]
+    for step, more in enumerate(options):
+        gs = [(torch.randn(p.shape, generator=gen, device=cuda) * 1e-2).to(g_dt) for p in sides[0][0]]
+        for ps, opt in sides:
+            opt.param_groups[0]["lr"] = 1e-3 * (1 + step)
+            for i, (p, g) in enumerate(zip(ps, gs)):
+                p.grad = None if step == 5 and i == 2 else g.clone()
+            opt.step(**more)
+        assert sides[0][1]._plans[0].native is not None and sides[1][1]._plans[0].native is None
+        for (pa, pb) in zip(sides[0][0], sides[1][0]):
+            assert torch.equal(pa.view(torch.uint8), pb.view(torch.uint8)), f"step {step}: {tuple(pa.shape)}"
+            assert pb.grad is None or torch.equal(pa.grad, pb.grad)
+        if "max_grad_norm" in more:
+            assert torch.equal(sides[0][1].last_grad_norm, sides[1][1].last_grad_norm)
+    a, b = (opt.state_dict()["state"] for _, opt in sides)
+    for i in a:
+        assert float(a[i]["step"]) == float(b[i]["step"]) == (5.0 if i == 2 else 6.0)
+        assert torch.equal(a[i]["exp_avg"], b[i]["exp_avg"]) and torch.equal(a[i]["exp_avg_sq"], b[i]["exp_avg_sq"])
+
+
+@pytest.mark.gpu
+def test_refusals_are_the_python_codes(cuda):
+    n = 5000
+    nbytes, nblk = q.state_sizes(n)
+    z = lambda k, dt=torch.float32: torch.zeros(k, dtype=dt, device=cuda)
+    p, g, m, v, sm, sv = z(n), z(n), z(nbytes, torch.uint8), z(nbytes, torch.uint8), z(nblk), z(nblk)
+    for bad, words in (((p, g[:-1], m, v, sm, sv), "grad numel"), ((p, z(2 * n)[::2], m, v, sm, sv), "grad must be contiguous"),
+                       ((p, g, m[:-1], v, sm, sv), "packed size"), ((p, g, m, v, sm, sv.double()), "scales must be float32"),
+                       ((p, g.cpu(), m, v, sm, sv), "grad must be on")):
+        with pytest.raises(AssertionError, match=words):
+            q.fused_4bit(*bad, *HP, 1)
+    with pytest.raises(TypeError, match="float32, bfloat16 or float16"):
+        q.fused_4bit(p.double(), g, m, v, sm, sv, *HP, 1)
+    with pytest.raises(RuntimeError, match="hyper-parameter"):
+        q.fused_4bit(p, g, m, v, sm, sv, 1.5, 0.999, 1e-3, 0.01, 1e-8, 1)
+    q.fused_4bit(p, g, m, v, sm, sv, *HP, torch.tensor(1.0))      # anything float() takes
+    opt = AdamWFused_QuantFour([torch.nn.Parameter(z(n))], lr=1e-3)
+    par = opt.param_groups[0]["params"][0]
+    par.grad = z(n)
+    opt.step()
+    opt.param_groups[0]["eps"] = -1.0
+    with pytest.raises(RuntimeError, match="fused_4bit_multi failed"):
+        opt.step()
+    opt.param_groups[0]["eps"] = 1e-8
+    par.grad = z(2 * n)[:n]
+    par.grad.as_strided_((n,), (2,))                              # re-strided in place: no longer dense
+    with pytest.raises(AssertionError, match="grad must be contiguous"):
+        opt.step()
