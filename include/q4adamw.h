@@ -292,6 +292,17 @@ int q4adamw_fused_single_tensor_multi_ex(const q4adamw_small_tensor *tensors, in
                                          const q4adamw_grad_options *opt, void *stream);
 
 /*
+ * One step over both kinds of tensors: q4adamw_fused_4bit_multi_ex, or _sr with `stochastic`, for `tensors` and
+ * q4adamw_fused_single_tensor_multi_ex for `small`, the same results; small models' lists, of up to 61 tensors
+ * together, in one launch.  (optim/fused_quantfour.py:171-292 makes a launch per parameter.)
+ */
+int q4adamw_fused_step_multi(const q4adamw_tensor *tensors, int count, const q4adamw_small_tensor *small,
+                             int small_count, int stochastic, const uint32_t *salts, uint64_t seed,
+                             int p_dtype, int g_dtype, float beta1, float beta2, float lr,
+                             float weight_decay, float eps, float step,
+                             const q4adamw_grad_options *opt, void *stream);
+
+/*
  * Global L2 norm of a set of gradient tensors and the clip coefficient that follows
  * from it: what torch.nn.utils.clip_grad_norm_ computes before it rescales the
  * gradients (the reference's callers clip between backward and step; the rescaling

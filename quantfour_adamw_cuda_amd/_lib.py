@@ -97,6 +97,7 @@ EXPORTS = (
     "q4adamw_fused_single_tensor",
     "q4adamw_fused_single_tensor_multi",
     "q4adamw_fused_single_tensor_multi_ex",
+    "q4adamw_fused_step_multi",
     "q4adamw_grad_norm",
     "q4adamw_grad_norm_static",
     "q4adamw_bias_table",
@@ -139,7 +140,7 @@ def _bind_host(L):
     known = lambda name: getattr(c, name, None) or (lambda *a: -1)
     _q4host.bind(*map(address, ("q4adamw_fused_4bit", "q4adamw_fused_single_tensor", "q4adamw_fused_4bit_multi_ex",
                                 "q4adamw_fused_4bit_multi_sr", "q4adamw_fused_4bit_rank1_multi", "q4adamw_fused_4bit_rank1_multi_sr",
-                                "q4adamw_fused_single_tensor_multi_ex")),
+                                "q4adamw_fused_single_tensor_multi_ex", "q4adamw_fused_step_multi")),
                  known("_cuda_getCurrentRawStream"), known("_cuda_getDevice"))
     return _q4host
 
@@ -169,6 +170,9 @@ def load():
     L.q4adamw_fused_4bit_multi_ex.restype = i
     L.q4adamw_fused_single_tensor_multi_ex.argtypes = [ctypes.POINTER(Q4SmallTensor), i, i, i] + hyper + [opt, vp]
     L.q4adamw_fused_single_tensor_multi_ex.restype = i
+    L.q4adamw_fused_step_multi.argtypes = ([ctypes.POINTER(Q4Tensor), i, ctypes.POINTER(Q4SmallTensor), i, i,
+                                            ctypes.POINTER(ctypes.c_uint32), ctypes.c_uint64, i, i] + hyper + [opt, vp])
+    L.q4adamw_fused_step_multi.restype = i
     L.q4adamw_fused_4bit_multi_sr.argtypes = ([ctypes.POINTER(Q4Tensor), i, ctypes.POINTER(ctypes.c_uint32),
                                                ctypes.c_uint64, i, i] + hyper + [opt, vp])
     L.q4adamw_fused_4bit_multi_sr.restype = i

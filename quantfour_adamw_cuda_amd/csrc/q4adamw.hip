@@ -400,7 +400,8 @@ using namespace q4;
 static int fused_4bit_multi_impl(const q4adamw_tensor *tensors, int count, int p_dtype, int g_dtype,
                                  float beta1, float beta2, float lr, float weight_decay, float eps,
                                  float step, const q4adamw_grad_options *opt, bool sr,
-                                 const uint32_t *salts, uint64_t seed, void *stream);
+                                 const uint32_t *salts, uint64_t seed, const q4adamw_small_tensor *small, int nsmall,
+                                 void *stream);
 static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int count, int p_dtype,
                                        int g_dtype, float beta1, float beta2, float lr,
                                        float weight_decay, float eps, float step,
@@ -470,7 +471,7 @@ int q4adamw_fused_4bit_multi_ex(const q4adamw_tensor *tensors, int count, int p_
                                 float beta1, float beta2, float lr, float weight_decay, float eps,
                                 float step, const q4adamw_grad_options *opt, void *stream) {
   return fused_4bit_multi_impl(tensors, count, p_dtype, g_dtype, beta1, beta2, lr, weight_decay, eps,
-                               step, opt, false, nullptr, 0, stream);
+                               step, opt, false, nullptr, 0, nullptr, 0, stream);
 }
 
 int q4adamw_fused_4bit_multi_sr(const q4adamw_tensor *tensors, int count, const uint32_t *salts,
@@ -478,7 +479,15 @@ int q4adamw_fused_4bit_multi_sr(const q4adamw_tensor *tensors, int count, const 
                                 float lr, float weight_decay, float eps, float step,
                                 const q4adamw_grad_options *opt, void *stream) {
   return fused_4bit_multi_impl(tensors, count, p_dtype, g_dtype, beta1, beta2, lr, weight_decay, eps,
-                               step, opt, true, salts, seed, stream);
+                               step, opt, true, salts, seed, nullptr, 0, stream);
+}
+
+int q4adamw_fused_step_multi(const q4adamw_tensor *tensors, int count, const q4adamw_small_tensor *small, int small_count,
+                             int stochastic, const uint32_t *salts, uint64_t seed, int p_dtype, int g_dtype, float beta1,
+                             float beta2, float lr, float weight_decay, float eps, float step,
+                             const q4adamw_grad_options *opt, void *stream) {
+  return fused_4bit_multi_impl(tensors, count, p_dtype, g_dtype, beta1, beta2, lr, weight_decay, eps,
+                               step, opt, stochastic != 0, salts, seed, small, small_count, stream);
 }
 
 uint32_t q4adamw_sr_tensor_salt(uint64_t seed, float step, uint32_t tensor_salt) {
@@ -490,23 +499,15 @@ uint32_t q4adamw_sr_tensor_salt(uint64_t seed, float step, uint32_t tensor_salt)
 
 }  // extern "C"
 
-static int fused_4bit_multi_impl(const q4adamw_tensor *tensors, int count, int p_dtype, int g_dtype,
-                                 float beta1, float beta2, float lr, float weight_decay, float eps,
-                                 float step, const q4adamw_grad_options *opt, bool sr,
-                                 const uint32_t *salts, uint64_t seed, void *stream) {
-  if (count < 0 || (count > 0 && !tensors)) return fail(Q4ADAMW_ERR_ARG, "bad tensor list");
-  if (int rc = check_dtypes(p_dtype, g_dtype)) return rc;
-  FusedArgs a;
-  bool ext = false;
-  int update_form = Q4ADAMW_UPDATE_AUTO;
-  if (int rc = make_consts(beta1, beta2, lr, weight_decay, eps, step, &a.sc)) return rc;
-  if (int rc = make_grad_ops(opt, &a.go, &ext, &update_form)) return rc;
-  a.seed_lo = (uint32_t)seed;
-  a.seed_hi = (uint32_t)(seed >> 32);
-  // a lane reads 8 consecutive elements at once when parameters and gradients are 16-bit types, else 4
+// elements of a workgroup: a lane reads 8 consecutive elements at once when parameters and gradients are 16-bit types, else 4
+static int64_t fused_chunk(int p_dtype, int g_dtype) {
+  return p_dtype != Q4ADAMW_FP32 && g_dtype != Q4ADAMW_FP32 ? Geometry<1, 1>::kChunk : Geometry<0, 0>::kChunk;
+}
+
+static int check_fused(const q4adamw_tensor *tensors, int count, int p_dtype, int g_dtype) {
   const bool p_half = p_dtype != Q4ADAMW_FP32, g_half = g_dtype != Q4ADAMW_FP32;
   const bool wide = p_half && g_half;   // 8 elements per lane
-  const int64_t chunk_elems = wide ? Geometry<1, 1>::kChunk : Geometry<0, 0>::kChunk;
+  const int64_t chunk_elems = fused_chunk(p_dtype, g_dtype);
   // Parameters and gradients need the alignment of their element type only: the 16-byte
   // accesses of the kernels are legal at any such address (the memory pipeline runs in its
   // unaligned mode under ROCm; the compiler relies on the same for amdhsa targets).  A view at
@@ -514,7 +515,6 @@ static int fused_4bit_multi_impl(const q4adamw_tensor *tensors, int count, int p
   // time on the parameter side (lines shared between waves; see kNtSharedLines).
   const uintptr_t p_align = p_half ? 2 : 4, g_align = g_half ? 2 : 4;
   const uintptr_t code_align = wide ? 4 : 2;
-  // validate everything before the first launch
   for (int i = 0; i < count; ++i) {
     const q4adamw_tensor &t = tensors[i];
     if (t.numel < 0) return fail(Q4ADAMW_ERR_ARG, "negative numel");
@@ -529,8 +529,66 @@ static int fused_4bit_multi_impl(const q4adamw_tensor *tensors, int count, int p
     if (((uint64_t)t.numel + (uint64_t)chunk_elems - 1) / (uint64_t)chunk_elems > kMaxChunksPerLaunch)
       return fail(Q4ADAMW_ERR_TOO_LARGE, "tensor too large: more than 2^31 - 16 chunks");
   }
+  return 0;
+}
+
+static int check_small(const q4adamw_small_tensor *tensors, int count, int p_dtype, int g_dtype) {
+  const uintptr_t pa = p_dtype != Q4ADAMW_FP32 ? 2 : 4, ga = g_dtype != Q4ADAMW_FP32 ? 2 : 4;
+  for (int i = 0; i < count; ++i) {
+    const q4adamw_small_tensor &t = tensors[i];
+    if (t.numel < 0) return fail(Q4ADAMW_ERR_ARG, "negative numel");
+    if (t.numel == 0) continue;
+    if (!t.p || !t.g || !t.exp_avg || !t.exp_avg_sq)
+      return fail(Q4ADAMW_ERR_ARG, "null tensor pointer");
+    if (!aligned(t.p, pa) || !aligned(t.g, ga) || !aligned(t.exp_avg, 4) || !aligned(t.exp_avg_sq, 4))
+      return fail(Q4ADAMW_ERR_ALIGN, "tensor not aligned to its element size");
+    if (((uint64_t)t.numel + (uint64_t)kSmallChunk - 1) / (uint64_t)kSmallChunk > kMaxChunksPerLaunch)
+      return fail(Q4ADAMW_ERR_TOO_LARGE, "tensor too large: more than 2^31 - 16 chunks");
+  }
+  return 0;
+}
+
+// One launch for both kinds of tensors up to this many workgroups and as many tensors as its arguments hold.  us a step
+// with two launches / one: tensors around the quantization threshold and two of 1 and 3 million elements 17.5 / 14.5, linear
+// layers 512 wide 16.9 / 14.0, 2048 wide in bf16 48.2 / 45.4, a table of 38 million elements and four layers in fp32 150.0 / 145.4; one
+// Llama-3-8B layer, beyond the limit, would gain under 1 per cent.
+constexpr uint64_t kMixedMostChunks = 1ull << 17;
+
+static int fused_4bit_multi_impl(const q4adamw_tensor *tensors, int count, int p_dtype, int g_dtype,
+                                 float beta1, float beta2, float lr, float weight_decay, float eps,
+                                 float step, const q4adamw_grad_options *opt, bool sr,
+                                 const uint32_t *salts, uint64_t seed, const q4adamw_small_tensor *small, int nsmall,
+                                 void *stream) {
+  if (count < 0 || (count > 0 && !tensors) || nsmall < 0 || (nsmall > 0 && !small)) return fail(Q4ADAMW_ERR_ARG, "bad tensor list");
+  if (int rc = check_dtypes(p_dtype, g_dtype)) return rc;
+  FusedArgs a;
+  bool ext = false;
+  int update_form = Q4ADAMW_UPDATE_AUTO;
+  if (int rc = make_consts(beta1, beta2, lr, weight_decay, eps, step, &a.sc)) return rc;
+  if (int rc = make_grad_ops(opt, &a.go, &ext, &update_form)) return rc;
+  a.seed_lo = (uint32_t)seed;
+  a.seed_hi = (uint32_t)(seed >> 32);
+  const int64_t chunk_elems = fused_chunk(p_dtype, g_dtype);
+  // validate everything before the first launch
+  if (int rc = check_fused(tensors, count, p_dtype, g_dtype)) return rc;
+  if (int rc = check_small(small, nsmall, p_dtype, g_dtype)) return rc;
+  int listed = 0;
+  uint64_t all_chunks = 0;
+  for (int i = 0; i < count; ++i) {
+    listed += tensors[i].numel != 0;
+    all_chunks += ((uint64_t)tensors[i].numel + (uint64_t)chunk_elems - 1) / (uint64_t)chunk_elems;
+  }
+  for (int i = 0; i < nsmall; ++i) {
+    listed += small[i].numel != 0;
+    all_chunks += ((uint64_t)small[i].numel + (uint64_t)chunk_elems - 1) / (uint64_t)chunk_elems;
+  }
+  const bool mixed = nsmall > 0 && count > 0 && listed <= kMaxTensors && all_chunks <= kMixedMostChunks;
+  if (nsmall > 0 && !mixed) {
+    if (int rc = q4adamw_fused_single_tensor_multi_ex(small, nsmall, p_dtype, g_dtype, beta1, beta2, lr, weight_decay, eps, step, opt, stream)) return rc;
+    nsmall = 0;
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const FusedKernel kernel = pick_fused(p_dtype, g_dtype, ext, sr, exact_update(update_form, p_dtype, sr, false));
+  const FusedKernel kernel = (mixed ? pick_mixed : pick_fused)(p_dtype, g_dtype, ext, sr, exact_update(update_form, p_dtype, sr, false));
   a.ntensors = 0;
   uint64_t chunks = 0;
   for (int i = 0; i < count; ++i) {
@@ -555,6 +613,21 @@ static int fused_4bit_multi_impl(const q4adamw_tensor *tensors, int count, int p
     a.first_chunk[a.ntensors] = (uint32_t)chunks;
     ++a.ntensors;
     chunks += c;
+  }
+  for (int i = 0; i < nsmall; ++i) {   // all of them in the one batch
+    const q4adamw_small_tensor &t = small[i];
+    if (t.numel == 0) continue;
+    TensorDesc &d = a.desc[a.ntensors];
+    d.p = t.p;
+    d.g = t.g;
+    d.m = reinterpret_cast<uint8_t *>(t.exp_avg);
+    d.v = reinterpret_cast<uint8_t *>(t.exp_avg_sq);
+    d.sm = d.sv = nullptr;
+    d.numel = t.numel;
+    a.sr_salt[a.ntensors] = 0u;
+    a.first_chunk[a.ntensors] = (uint32_t)chunks;
+    ++a.ntensors;
+    chunks += ((uint64_t)t.numel + (uint64_t)chunk_elems - 1) / (uint64_t)chunk_elems;
   }
   if (a.ntensors > 0) return launch_fused_batch(a, chunks, kernel, s);
   return 0;
@@ -959,18 +1032,7 @@ int q4adamw_fused_single_tensor_multi_ex(const q4adamw_small_tensor *tensors, in
   int update_form = Q4ADAMW_UPDATE_AUTO;   // this kernel's update is always the exact form
   if (int rc = make_consts(beta1, beta2, lr, weight_decay, eps, step, &a.sc)) return rc;
   if (int rc = make_grad_ops(opt, &a.go, &ext, &update_form)) return rc;
-  const uintptr_t pa = p_dtype != Q4ADAMW_FP32 ? 2 : 4, ga = g_dtype != Q4ADAMW_FP32 ? 2 : 4;
-  for (int i = 0; i < count; ++i) {
-    const q4adamw_small_tensor &t = tensors[i];
-    if (t.numel < 0) return fail(Q4ADAMW_ERR_ARG, "negative numel");
-    if (t.numel == 0) continue;
-    if (!t.p || !t.g || !t.exp_avg || !t.exp_avg_sq)
-      return fail(Q4ADAMW_ERR_ARG, "null tensor pointer");
-    if (!aligned(t.p, pa) || !aligned(t.g, ga) || !aligned(t.exp_avg, 4) || !aligned(t.exp_avg_sq, 4))
-      return fail(Q4ADAMW_ERR_ALIGN, "tensor not aligned to its element size");
-    if (((uint64_t)t.numel + (uint64_t)kSmallChunk - 1) / (uint64_t)kSmallChunk > kMaxChunksPerLaunch)
-      return fail(Q4ADAMW_ERR_TOO_LARGE, "tensor too large: more than 2^31 - 16 chunks");
-  }
+  if (int rc = check_small(tensors, count, p_dtype, g_dtype)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const SmallKernel kernel = pick_small(p_dtype, g_dtype, ext);
   a.ntensors = 0;
@@ -1217,6 +1279,6 @@ int q4adamw_release(void) { return 0; }
 
 const char *q4adamw_last_error(void) { return g_err.c_str(); }
 
-int q4adamw_version(void) { return 1015; }
+int q4adamw_version(void) { return 1016; }
 
 }  // extern "C"

@@ -19,32 +19,8 @@ __global__ __launch_bounds__(256) void single_tensor_kernel(const SmallArgs args
   const StepConsts sc = EXT ? step_consts(args.sc, args.go) : args.sc;
   const int64_t base = (int64_t)(chunk - args.first_chunk[t]) * kSmallChunk;
   const int64_t end = base + (chunk + 1u == args.first_chunk[t + 1] ? args.last[t] : kSmallChunk);
-  if (cancelled) {  // a cancelled step still clears the gradients it was asked to clear
-    for (int64_t i = base + threadIdx.x; i < end; i += 256) {
-      store_scalar<GT>(const_cast<void *>(T.g), i, 0.0f);
-    }
-    return;
-  }
-  for (int64_t i = base + threadIdx.x; i < end; i += 256) {
-    float gi = load_scalar<GT>(T.g, i);
-    if (EXT) {
-      gi *= gscale;
-      if (zero_g) {
-        store_scalar<GT>(const_cast<void *>(T.g), i, 0.0f);
-      }
-    }
-    const float pi = load_scalar<PT>(T.p, i);
-    const float m = sc.b1 * as_global<const float>(T.m)[i] + sc.r1 * gi;
-    const float v = sc.b2 * as_global<const float>(T.v)[i] + sc.r2 * (gi * gi);
-    as_global<float>(T.m)[i] = m;
-    as_global<float>(T.v)[i] = v;
-    // exact form here: these tensors are tiny, so the divisions cost nothing
-    const float den = __builtin_sqrtf(v) / sc.c2s + sc.eps;
-    const float pn = pi * sc.wdu - sc.ss * (m / den);
-    store_scalar<PT>(T.p, i, pn);
-  }
+  small_elements<PT, GT, EXT>(T.p, T.g, T.m, T.v, base, end, sc, gscale, zero_g, cancelled);
 }
-
 
 // ---------------------------------------------------------------------------
 // a step whose number lives on the device

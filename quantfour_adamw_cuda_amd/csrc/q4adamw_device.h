@@ -693,4 +693,32 @@ __device__ __forceinline__ float max_nonneg(float a, float b) {
   return bits2f(x > y ? x : y);
 }
 
+// Elements [base, end) of a tensor that keeps fp32 moments, by a workgroup of 256 threads (cuda_adamw_kernels.cu:100-133):
+// moments in place, the fused path's derived scalars and operation order.  A cancelled step only clears the gradients it
+// was asked to clear.
+template <int PT, int GT, bool EXT>
+__device__ __forceinline__ void small_elements(void *p, const void *g, float *m_, float *v_, int64_t base, int64_t end, const StepConsts &sc,
+                                               float gscale, bool zero_g, bool cancelled) {
+  if (EXT && cancelled) {
+    for (int64_t i = base + threadIdx.x; i < end; i += 256) store_scalar<GT>(const_cast<void *>(g), i, 0.0f);
+    return;
+  }
+  for (int64_t i = base + threadIdx.x; i < end; i += 256) {
+    float gi = load_scalar<GT>(g, i);
+    if (EXT) {
+      gi *= gscale;
+      if (zero_g) store_scalar<GT>(const_cast<void *>(g), i, 0.0f);
+    }
+    const float pi = load_scalar<PT>(p, i);
+    const float m = sc.b1 * as_global<const float>(m_)[i] + sc.r1 * gi;
+    const float v = sc.b2 * as_global<const float>(v_)[i] + sc.r2 * (gi * gi);
+    as_global<float>(m_)[i] = m;
+    as_global<float>(v_)[i] = v;
+    // exact form here: these tensors are tiny, so the divisions cost nothing
+    const float den = __builtin_sqrtf(v) / sc.c2s + sc.eps;
+    const float pn = pi * sc.wdu - sc.ss * (m / den);
+    store_scalar<PT>(p, i, pn);
+  }
+}
+
 }  // namespace q4

@@ -30,6 +30,8 @@ typedef void (*Rank1StatKernel)(const Rank1StatArgs);
 // ext: gradient options; sr: stochastic rounding; exact: the parameter update with every
 // operation rounded as IEEE 754 rounds it
 FusedKernel pick_fused(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
+// the same for lists that also hold tensors with fp32 moments
+FusedKernel pick_mixed(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 // the rank-1 update kernels: tiles anywhere in a matrix of rows at least a tile long
 // (pick_rank1_wide), matrices narrower than a tile (pick_rank1_narrow), tiles aligned to the
 // rows of a matrix (pick_rank1_rows), rows of any length (pick_rank1_any), rows shorter than a tile in tensors

@@ -8,7 +8,7 @@ namespace q4 {
 
 template <bool EXT, bool SR, bool EXACT>
 static FusedKernel pick_pg(int p_dtype, int g_dtype) {
-  Q4_PICK_PG(fused_4bit_kernel, EXT, SR, EXACT)
+  Q4_PICK_PG(fused_4bit_kernel, EXT, SR, EXACT, false)
 }
 
 template <bool EXT, bool SR>

@@ -676,7 +676,8 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
   }
 }
 
-template <int PT, int GT, bool EXT, bool SR, bool EXACT>
+// MIXED: some of the tensors (without block scales, sm null) keep fp32 moments, `m` and `v`.
+template <int PT, int GT, bool EXT, bool SR, bool EXACT, bool MIXED>
 __global__ __launch_bounds__(kThreads) void fused_4bit_kernel(const FusedArgs args) {
   using G = Geometry<PT, GT>;
   __shared__ uint2 lds[kLdsEntries];
@@ -691,6 +692,14 @@ __global__ __launch_bounds__(kThreads) void fused_4bit_kernel(const FusedArgs ar
   const TensorDesc &T = args.desc[t];
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int64_t tile = (int64_t)(chunk - args.first_chunk[t]) * kWaves + wave;
+  if constexpr (MIXED) {
+    if (T.sm == nullptr) {
+      const int64_t base = (int64_t)(chunk - args.first_chunk[t]) * G::kChunk, rem = T.numel - base;
+      small_elements<PT, GT, EXT>(T.p, T.g, reinterpret_cast<float *>(T.m), reinterpret_cast<float *>(T.v), base,
+                                  base + (rem < G::kChunk ? rem : G::kChunk), EXT ? step_consts(args.sc, args.go) : args.sc, gscale, zero_g, cancelled);
+      return;
+    }
+  }
   if (cancelled) {  // a cancelled step still clears the gradients it was asked to clear
     zero_tile<GT, G::kEpl>(T.g, tile, T.numel, lane);
     return;

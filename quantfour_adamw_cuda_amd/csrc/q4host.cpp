@@ -33,19 +33,20 @@ struct Library {
   decltype(&q4adamw_fused_4bit_rank1_multi) rank1;
   decltype(&q4adamw_fused_4bit_rank1_multi_sr) rank1_sr;
   decltype(&q4adamw_fused_single_tensor_multi_ex) small;
+  decltype(&q4adamw_fused_step_multi) both;
 };
 Library lib;
 PyObject *raw_stream_of = nullptr;     // torch._C._cuda_getCurrentRawStream
 PyObject *current_device = nullptr;    // torch._C._cuda_getDevice
 
-// bind(addresses of the seven functions above, in order, raw_stream_of, current_device)
+// bind(addresses of the eight functions above, in order, raw_stream_of, current_device)
 PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
-  if (n != 9) {
-    PyErr_SetString(PyExc_TypeError, "bind takes seven addresses and two functions");
+  if (n != 10) {
+    PyErr_SetString(PyExc_TypeError, "bind takes eight addresses and two functions");
     return nullptr;
   }
-  void *f[7];
-  for (int i = 0; i < 7; ++i) {
+  void *f[8];
+  for (int i = 0; i < 8; ++i) {
     f[i] = PyLong_AsVoidPtr(args[i]);
     if (!f[i]) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "null address");
@@ -59,10 +60,11 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
   lib.rank1 = reinterpret_cast<decltype(lib.rank1)>(f[4]);
   lib.rank1_sr = reinterpret_cast<decltype(lib.rank1_sr)>(f[5]);
   lib.small = reinterpret_cast<decltype(lib.small)>(f[6]);
-  Py_INCREF(args[7]);
+  lib.both = reinterpret_cast<decltype(lib.both)>(f[7]);
   Py_INCREF(args[8]);
-  Py_XSETREF(raw_stream_of, args[7]);
-  Py_XSETREF(current_device, args[8]);
+  Py_INCREF(args[9]);
+  Py_XSETREF(raw_stream_of, args[8]);
+  Py_XSETREF(current_device, args[9]);
   Py_RETURN_NONE;
 }
 
@@ -224,6 +226,8 @@ struct Bucket {
   size_t stride;
   int p_tag, g_tag;
   const uint32_t *salts;
+  int with = -1;               // kinds 1 and 2: a bucket of kind 0 of the same types that goes in the same call
+  bool taken = false;          // kind 0: goes in another one's call
 };
 
 // One param group's launches.  Every object here is borrowed: the Python plan that owns this one holds them.
@@ -303,6 +307,16 @@ PyObject *make_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
     b.salts = reinterpret_cast<const uint32_t *>((uintptr_t)salts);
     plan->buckets.push_back(std::move(b));
   }
+  // small tensors go with quantized ones of their types; refresh sees to it that a bucket has one step number,
+  // run that the two have the same one
+  for (Bucket &b : plan->buckets)
+    for (size_t k = 0; k < plan->buckets.size() && b.with < 0 && (b.kind == 1 || b.kind == 2); ++k) {
+      Bucket &o = plan->buckets[k];
+      if (o.kind == 0 && !o.taken && o.p_tag == b.p_tag && o.g_tag == b.g_tag) {
+        o.taken = true;
+        b.with = (int)k;
+      }
+    }
   plan->fresh.resize((size_t)plan->with_grad);
   PyObject *capsule = PyCapsule_New(plan.get(), kPlanName, drop_plan);
   if (capsule) plan.release();
@@ -350,6 +364,13 @@ PyObject *refresh(PyObject *, PyObject *const *args, Py_ssize_t n) {
   Py_RETURN_TRUE;
 }
 
+// whether a bucket of small tensors is at the step of the bucket in whose call it goes
+bool together(const Plan &plan, const Bucket &small) {
+  for (const Bucket &b : plan.buckets)
+    if (b.with >= 0 && &plan.buckets[(size_t)b.with] == &small) return plan.steps[b.idx[0]] == plan.steps[small.idx[0]];
+  return false;
+}
+
 // run(plan, beta1, beta2, lr, weight_decay, eps, options' address or 0, seed): advances the step counters and makes the
 // launches; the first status that is not 0 and its bucket's number, or (0, number of buckets), or None with nothing done
 PyObject *run(PyObject *, PyObject *const *args, Py_ssize_t n) {
@@ -370,6 +391,14 @@ PyObject *run(PyObject *, PyObject *const *args, Py_ssize_t n) {
     const Bucket &b = plan->buckets[k];
     const float step = plan->steps[b.idx[0]];
     const int count = (int)b.idx.size();
+    if (b.taken && together(*plan, b)) continue;
+    if (b.with >= 0 && together(*plan, plan->buckets[(size_t)b.with])) {
+      const Bucket &o = plan->buckets[(size_t)b.with];
+      rc = lib.both(reinterpret_cast<const q4adamw_tensor *>(b.arr), count, reinterpret_cast<const q4adamw_small_tensor *>(o.arr), (int)o.idx.size(),
+                    b.kind == 2, b.salts, seed, b.p_tag, b.g_tag, x[0], x[1], x[2], x[3], x[4], step, options, stream);
+      if (rc != 0) break;
+      continue;
+    }
     switch (b.kind) {
       case 0:
         rc = lib.small(reinterpret_cast<const q4adamw_small_tensor *>(b.arr), count, b.p_tag, b.g_tag, x[0], x[1], x[2], x[3], x[4], step, options, stream);

@@ -104,3 +104,49 @@ def test_refusals_are_the_python_codes(cuda):
     par.grad.as_strided_((n,), (2,))                              # re-strided in place: no longer dense
     with pytest.raises(AssertionError, match="grad must be contiguous"):
         opt.step()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p_dt,g_dt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)])
+@pytest.mark.parametrize("stochastic", [False, True])
+@pytest.mark.parametrize("quantized,small", [(1, 1), (5, 56), (5, 57), (0, 3), (3, 0)])
+def test_one_call_for_both_kinds(cuda, quantized, small, stochastic, p_dt, g_dt):
+    """q4adamw_fused_step_multi against the calls it stands for, bit for bit: 61 tensors, which are one launch, and 62;
+    small tensors of a part of a workgroup, of one, of more; a multiplier, cleared gradients, a cancelled step."""
+    L = _lib.load()
+    gen = torch.Generator(device=cuda).manual_seed(quantized * 100 + small)
+    q_sizes = [(5000, 128, 4097, 2048, 70001)[i % 5] + i for i in range(quantized)]
+    s_sizes = [(1, 255, 256, 1024, 1025, 2047, 2049, 4096, 9000)[i % 9] for i in range(small)]
+    tag = q._DTYPE_TAG
+    stream = q._stream(torch.device("cuda", torch.cuda.current_device()))
+    salts = q.make_salts([7 * i + 1 for i in range(quantized)]) if quantized else None
+    scale, skip = torch.full((1,), 0.5, device=cuda), torch.ones(1, device=cuda)
+    base = [(torch.randn(n, generator=gen, device=cuda) * 0.05).to(p_dt) for n in q_sizes + s_sizes]
+
+    def side():
+        ps = [b.clone() for b in base]
+        z = lambda n, dt=torch.float32: torch.zeros(n, dtype=dt, device=cuda)
+        qs = [(z(nb, torch.uint8), z(nb, torch.uint8), z(nk), z(nk)) for nb, nk in map(q.state_sizes, q_sizes)]
+        return ps, qs, [(z(n), z(n)) for n in s_sizes]
+
+    one, two = side(), side()
+    for step, opts in ((1, {}), (2, dict(grad_scale_dev=scale, zero_grad=True)), (3, dict(found_inf=skip, zero_grad=True)), (4, {})):
+        gs = [(torch.randn(n, generator=gen, device=cuda) * 1e-2).to(g_dt) for n in q_sizes + s_sizes]
+        kept = []
+        for k, (ps, qs, ss) in enumerate((one, two)):
+            g = [x.clone() for x in gs]
+            kept.append(g)
+            qt = q.make_table(ps[:quantized], g[:quantized], *([x[j] for x in qs] for j in range(4)))
+            st = q.make_small_table(ps[quantized:], g[quantized:], [x[0] for x in ss], [x[1] for x in ss])
+            o = q.grad_options(scale.device, **opts)
+            tail = (tag[p_dt], tag[g_dt], *HP[:5], float(step), o, stream)
+            if k == 0:
+                _lib.check(L.q4adamw_fused_step_multi(qt, quantized, st, small, int(stochastic), salts, 99, *tail), "fused_step_multi")
+            else:
+                _lib.check(L.q4adamw_fused_single_tensor_multi_ex(st, small, *tail), "small")
+                if stochastic:
+                    _lib.check(L.q4adamw_fused_4bit_multi_sr(qt, quantized, salts, 99, *tail), "sr")
+                else:
+                    _lib.check(L.q4adamw_fused_4bit_multi_ex(qt, quantized, *tail), "ex")
+        for a, b in zip(kept[0] + one[0] + [t for s in one[1] + one[2] for t in s], kept[1] + two[0] + [t for s in two[1] + two[2] for t in s]):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), f"step {step}"
