@@ -251,14 +251,17 @@ struct Plan {
   int64_t device, with_grad;
 };
 
+PyObject *state_keys[3];      // "step", "exp_avg", "exp_avg_sq"
+
 const char kPlanName[] = "quantfour_adamw_cuda_amd.plan";
 void drop_plan(PyObject *capsule) { delete static_cast<Plan *>(PyCapsule_GetPointer(capsule, kPlanName)); }
 Plan *plan_of(PyObject *o) { return static_cast<Plan *>(PyCapsule_GetPointer(o, kPlanName)); }
 
-// plan(parameters, step buffer, held [(dict, key, value)], buckets [(kind, [indices], address, stride, p tag, g tag, salts'
+// plan(parameters, step buffer, held [(state, step, exp_avg, exp_avg_sq)] and [(dict, key, value)], buckets [(kind, [indices], address, stride, p tag, g tag, salts'
 // address or 0)]): a capsule, or None if the group is not for the fast path.  All arguments are kept by the caller.
 PyObject *make_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
-  if (n != 4 || !PyTuple_CheckExact(args[0]) || !THPVariable_CheckExact(args[1]) || !PyList_CheckExact(args[2]) || !PyList_CheckExact(args[3]))
+  if (n != 5 || !PyTuple_CheckExact(args[0]) || !THPVariable_CheckExact(args[1]) || !PyList_CheckExact(args[2]) || !PyList_CheckExact(args[3]) ||
+      !PyList_CheckExact(args[4]))
     Py_RETURN_NONE;
   auto plan = std::make_unique<Plan>();
   try {
@@ -282,17 +285,19 @@ PyObject *make_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
   } catch (const std::exception &) {
     Py_RETURN_NONE;
   }
-  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[2]); ++i) {
-    PyObject *holder, *key, *value;
-    if (!PyArg_ParseTuple(PyList_GET_ITEM(args[2], i), "OOO", &holder, &key, &value)) return nullptr;
-    if (!PyDict_Check(holder)) Py_RETURN_NONE;
-    plan->held.push_back({holder, key, value});
-  }
-  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[3]); ++i) {
+  for (int list = 2; list < 4; ++list)
+    for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[list]); ++i) {
+      PyObject *t = PyList_GET_ITEM(args[list], i);
+      if (!PyTuple_CheckExact(t) || PyTuple_GET_SIZE(t) != (list == 2 ? 4 : 3) || !PyDict_Check(PyTuple_GET_ITEM(t, 0))) Py_RETURN_NONE;
+      if (list == 3) plan->held.push_back({PyTuple_GET_ITEM(t, 0), PyTuple_GET_ITEM(t, 1), PyTuple_GET_ITEM(t, 2)});
+      else
+        for (int k = 0; k < 3; ++k) plan->held.push_back({PyTuple_GET_ITEM(t, 0), state_keys[k], PyTuple_GET_ITEM(t, k + 1)});
+    }
+  for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[4]); ++i) {
     Bucket b;
     PyObject *idx;
     unsigned long long arr, stride, salts;
-    if (!PyArg_ParseTuple(PyList_GET_ITEM(args[3], i), "iO!KKiiK", &b.kind, &PyList_Type, &idx, &arr, &stride, &b.p_tag, &b.g_tag, &salts)) return nullptr;
+    if (!PyArg_ParseTuple(PyList_GET_ITEM(args[4], i), "iO!KKiiK", &b.kind, &PyList_Type, &idx, &arr, &stride, &b.p_tag, &b.g_tag, &salts)) return nullptr;
     for (Py_ssize_t k = 0; k < PyList_GET_SIZE(idx); ++k) {
       const long x = PyLong_AsLong(PyList_GET_ITEM(idx, k));
       if (x < 0 || x >= plan->with_grad) {
@@ -437,4 +442,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_q4host", nullptr, -1, kMethods, 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__q4host(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__q4host(void) {
+  const char *const names[3] = {"step", "exp_avg", "exp_avg_sq"};
+  for (int k = 0; k < 3; ++k)
+    if (!(state_keys[k] = PyUnicode_InternFromString(names[k]))) return nullptr;
+  return PyModule_Create(&kModule);
+}

@@ -671,12 +671,11 @@ class AdamWFused_QuantFour(torch.optim.Optimizer):
         """The plan in native code (csrc/q4host.cpp), where it is for it: plain tensors on one device.  It borrows
         every object that the plan holds."""
         core, extra = plan.held
-        held = [(st, key, value) for st, *values in core for key, value in zip(("step", "exp_avg", "exp_avg_sq"), values)] + extra
         buckets = [(_KINDS[b.kind], b.idx, ctypes.addressof(b.arr), ctypes.sizeof(b.arr._type_), b.p_tag, b.g_tag,
                     0 if b.salts is None else ctypes.addressof(b.salts)) for b in plan.buckets]
         buf = self._step_buffers[plan.gi][0]
-        plan.native_held = (held, buckets, buf)
-        plan.native = _lib.host.plan(plan.all_params, buf, held, buckets)
+        plan.native_held = (buckets, buf)
+        plan.native = _lib.host.plan(plan.all_params, buf, core, extra, buckets)
         if plan.native is not None:
             plan.grads = None        # native code looks at every gradient anew
 

@@ -23,7 +23,7 @@ def test_what_is_not_for_it_is_left_alone():
     par.grad = torch.zeros(4)
     table = (_lib.Q4Grad * 2)()
     assert h.gradients(([par],), ctypes.addressof(table), 2) is None and h.gradients(([],), ctypes.addressof(table), 2) is None
-    assert h.plan((par,), torch.zeros(1), [], []) is None
+    assert h.plan((par,), torch.zeros(1), [], [], []) is None
     with pytest.raises((TypeError, ValueError)):
         h.refresh(object(), [par], torch.zeros(1))
     with pytest.raises(TypeError):
