@@ -350,6 +350,32 @@ static ShortDesc short_desc(const q4adamw_rank1_tensor &t) {
   return d;
 }
 
+// The update kernels' descriptors; the last argument only says which.
+static ShortDesc update_desc(const q4adamw_rank1_tensor &t, int, int64_t, const ShortDesc &) { return short_desc(t); }
+
+static Rank1Desc update_desc(const q4adamw_rank1_tensor &t, int route, int64_t tile_elems, const Rank1Desc &) {
+  Rank1Desc d;
+  d.p = t.p;
+  d.g = t.g;
+  d.m = t.exp_avg;
+  d.v = t.exp_avg_sq;
+  d.sm = t.exp_avg_scale;
+  d.rmax = t.row_max;
+  d.cmax = t.col_max;
+  d.rmax_next = t.row_max_next;
+  d.cmax_next = t.col_max_next;
+  d.numel = t.rows * t.cols;
+  d.rows = t.rows;
+  d.cols = t.cols;
+  // the divisor the tensor's kernel needs: tiles per row, cols, or cols / 8
+  const FastDiv fd = make_fast_div(route == kShapeRows  ? (uint32_t)rank1_tiles_per_row(t, tile_elems)
+                                   : route == kShapeAny ? (uint32_t)t.cols
+                                                        : (uint32_t)(t.cols >> 3));
+  d.div_magic = fd.magic;
+  d.div_shift = fd.shift;
+  return d;
+}
+
 // Fills the kernels' view of the caller's gradient options; returns whether the
 // launch needs the EXT kernels (false: the options change nothing).
 static int make_grad_ops(const q4adamw_grad_options *opt, GradOps *go, bool *ext, int *update_form) {
@@ -692,7 +718,7 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t tile_elems = chunk_elems / kWaves;
   const bool exact = exact_update(update_form, p_dtype, sr, true);
-  ShortArgs ha;      // the batch, if it takes the kernel for short rows
+  ShortArgs ha;      // as `a`, for the kernel for short rows
   ha.sc = a.sc;
   ha.go = a.go;
   ha.seed_lo = a.seed_lo;
@@ -701,16 +727,16 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
   ra.go = a.go;
   CommitArgs ca;
   ca.go = a.go;
-  int leads = 0, route = 0;
-  Rank1Kernel kernel = nullptr;
-  ShortKernel short_kernel = nullptr;
+  // the batch: its tensors, their update kernels and noise salts
   const q4adamw_rank1_tensor *batch[kMaxRank1Tensors];
-  a.ntensors = 0;
+  int route_of[kMaxRank1Tensors];
+  uint32_t salt_of[kMaxRank1Tensors];
+  int ntensors = 0, shorts = 0, leads = 0;
   uint64_t chunks = 0, stat_chunks = 0, scale_chunks = 0, commit_chunks = 0;   // stat_chunks: an upper bound
   // statistics of the batch's tensors that take one kernel for them
   auto launch_stats = [&](Rank1StatForm form) -> int {
     uint64_t elements = 0, tallest = 0, tiles = 0;
-    for (int i = 0; i < a.ntensors; ++i) {
+    for (int i = 0; i < ntensors; ++i) {
       const q4adamw_rank1_tensor &t = *batch[i];
       if (rank1_stat_form(t) != form) continue;
       elements += (uint64_t)(t.rows * t.cols);
@@ -719,7 +745,7 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
     if (elements == 0) return 0;
     sa.stat_rows = form == kStatLead ? lead_stat_outer(elements, lead_run(g_dtype != Q4ADAMW_FP32)) : rank1_stat_rows(elements, tallest);
     int n = 0;
-    for (int i = 0; i < a.ntensors; ++i) {
+    for (int i = 0; i < ntensors; ++i) {
       const q4adamw_rank1_tensor &t = *batch[i];
       if (rank1_stat_form(t) != form) continue;
       Rank1StatArgs::Desc &sd = sa.desc[n];
@@ -752,9 +778,34 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       return 0;
     });
   };
+  // the update of the batch's tensors that take one kernel for it
+  auto launch_update = [&](auto &args, auto update, int route) -> int {
+    uint64_t tiles = 0;
+    int n = 0;
+    for (int i = 0; i < ntensors; ++i) {
+      if (route_of[i] != route) continue;
+      const q4adamw_rank1_tensor &t = *batch[i];
+      args.desc[n] = update_desc(t, route, tile_elems, args.desc[n]);
+      args.sr_salt[n] = salt_of[i];
+      args.first_chunk[n] = (uint32_t)tiles;
+      tiles += rank1_chunks(t, tile_elems);
+      ++n;
+    }
+    if (n == 0) return 0;
+    args.ntensors = n;
+    finish_prefix(args, n);
+    return for_each_grid(tiles, kThreads, [&](uint64_t base, uint64_t count) -> int {
+      args.chunk_base = (uint32_t)base;
+      args.runs = make_chunk_runs((uint32_t)count);
+      hipLaunchKernelGGL(update, dim3((unsigned)count), dim3(kThreads), 0, s, args);
+      Q4_HIP(hipGetLastError());
+      return 0;
+    });
+  };
   // statistics of every tensor of the batch (and its rows' scales, with several leading
-  // dimensions), then the update, then the commit
+  // dimensions), then the updates, then the commit
   auto launch = [&]() -> int {
+    if (ntensors == 0) return 0;
     for (int form = 0; form < kStatForms; ++form) {
       if (int rc = launch_stats((Rank1StatForm)form)) return rc;
     }
@@ -763,48 +814,36 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       hipLaunchKernelGGL(rank1_row_scale_kernel, dim3((unsigned)scale_chunks), dim3(256), 0, s, ra);
       Q4_HIP(hipGetLastError());
     }
-    auto launch_update = [&](auto &args, auto update) -> int {
-      finish_prefix(args, a.ntensors);
-      return for_each_grid(chunks, kThreads, [&](uint64_t base, uint64_t count) -> int {
-        args.chunk_base = (uint32_t)base;
-        args.runs = make_chunk_runs((uint32_t)count);
-        hipLaunchKernelGGL(update, dim3((unsigned)count), dim3(kThreads), 0, s, args);
-        Q4_HIP(hipGetLastError());
-        return 0;
-      });
-    };
-    if (int rc = route == kRouteShort ? launch_update(ha, short_kernel) : launch_update(a, kernel)) return rc;
-    finish_prefix(ca, a.ntensors);
+    // matrices whose rows are whole tiles take the kernel whose workgroups share the columns' maxima of four rows; other
+    // matrices with rows of at least a tile the one that finds a tile's row on the scalar unit; narrower ones the one
+    // whose lanes find their own; rows of any length the one whose lanes or elements do; short rows of tensors with
+    // several leading dimensions the one that makes their scales
+    if (int rc = launch_update(a, pick_rank1_rows(p_dtype, g_dtype, ext, sr, exact), kShapeRows)) return rc;
+    if (int rc = launch_update(a, pick_rank1_wide(p_dtype, g_dtype, ext, sr, exact), kShapeWide)) return rc;
+    if (int rc = launch_update(a, pick_rank1_narrow(p_dtype, g_dtype, ext, sr, exact), kShapeNarrow)) return rc;
+    if (int rc = launch_update(a, pick_rank1_any(p_dtype, g_dtype, ext, sr, exact), kShapeAny)) return rc;
+    if (int rc = launch_update(ha, pick_rank1_short(p_dtype, g_dtype, ext, sr, exact), kRouteShort)) return rc;
+    finish_prefix(ca, ntensors);
     hipLaunchKernelGGL(rank1_commit_kernel, dim3((unsigned)commit_chunks), dim3(256), 0, s, ca);
     Q4_HIP(hipGetLastError());
-    a.ntensors = leads = 0;
+    ntensors = shorts = leads = 0;
     chunks = stat_chunks = scale_chunks = commit_chunks = 0;
     return 0;
   };
-  // the batches of an update kernel: matrices whose rows are whole tiles take the
-  // one whose workgroups share the columns' maxima of four rows; other matrices with
-  // rows of at least a tile the one that finds a tile's row on the scalar unit; narrower ones
-  // the one whose lanes find their own; rows of any length the one whose elements do.  Tensors of one
-  // statistics kernel after another, and a batch may hold several kinds: a batch for each would repeat
-  // update and commit (bf16 matrices of 1000 x 64 and 1000 x 400: a step of 29 us, 34 with two batches)
+  // Batches in the order of the update kernels and, among a kernel's tensors, of the statistics kernels.  A batch holds
+  // tensors of any of them and makes a launch for each kind it has: a batch for each would repeat commit and, of
+  // tensors that differ in one kind only, the other's launch (bf16 matrices of 1000 x 64 and 1000 x 400: a step of 29 us,
+  // 34 with two batches; a residual network and its classifier, one commit and not two, 70.3 us, 73.2 with two).
   auto pass_of = [&](const q4adamw_rank1_tensor &t) { return rank1_route(t, tile_elems) * kStatForms + rank1_stat_form(t); };
   uint32_t present = 0u;   // a bit per pass
   for (int i = 0; i < count; ++i) {
     if (tensors[i].rows != 0 && tensors[i].cols != 0) present |= 1u << pass_of(tensors[i]);
   }
   for (int pass = 0; pass < kRoutes * kStatForms; ++pass) {
-    route = pass / kStatForms;
-    if (route == kRouteShort) short_kernel = pick_rank1_short(p_dtype, g_dtype, ext, sr, exact);
-    else
-      kernel = route == kShapeRows     ? pick_rank1_rows(p_dtype, g_dtype, ext, sr, exact)
-               : route == kShapeWide   ? pick_rank1_wide(p_dtype, g_dtype, ext, sr, exact)
-               : route == kShapeNarrow ? pick_rank1_narrow(p_dtype, g_dtype, ext, sr, exact)
-                                       : pick_rank1_any(p_dtype, g_dtype, ext, sr, exact);
-    const int capacity = route == kRouteShort ? kMaxShortTensors : kMaxRank1Tensors;
+    const int route = pass / kStatForms;
     for (int i = 0; i < count && (present >> pass & 1u) != 0u; ++i) {
       const q4adamw_rank1_tensor &t = tensors[i];
       if (t.rows == 0 || t.cols == 0 || pass_of(t) != pass) continue;
-      const int64_t numel = t.rows * t.cols;
       const uint64_t c = rank1_chunks(t, tile_elems), sc_ = rank1_stat_chunks(t, 32u, g_dtype);
       auto commit_chunks_of = [](int64_t size) { return ((uint64_t)size + kCommitChunk - 1) / kCommitChunk; };
       // the kernel for short rows writes the rows' scales itself
@@ -816,43 +855,16 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       const uint64_t rc_ = ((uint64_t)t.rows + kRowScaleChunk - 1) / kRowScaleChunk;
       // the row-scale and commit launches stay within one grid (one tensor's rows and columns
       // are fewer than 2^32, 2^21 chunks)
-      if (a.ntensors == capacity || chunks + c > kMaxChunksPerLaunch || stat_chunks + sc_ > kMaxChunksPerLaunch ||
-          commit_chunks + cc > kMaxStatWorkgroups || scale_chunks + rc_ > kMaxStatWorkgroups) {
+      if (ntensors == kMaxRank1Tensors || (rows_follow && shorts == kMaxShortTensors) || chunks + c > kMaxChunksPerLaunch ||
+          stat_chunks + sc_ > kMaxChunksPerLaunch || commit_chunks + cc > kMaxStatWorkgroups || scale_chunks + rc_ > kMaxStatWorkgroups) {
         if (int rc = launch()) return rc;
       }
-      const uint32_t salt = !sr ? 0u : a.go.sc_dev ? lowbias32(salts ? salts[i] : (uint32_t)i)
-                                                   : q4adamw_sr_tensor_salt(seed, step, salts ? salts[i] : (uint32_t)i);
-      if (route == kRouteShort) {
-        ShortDesc &d = ha.desc[a.ntensors];
-        d = short_desc(t);
-        ha.sr_salt[a.ntensors] = salt;
-        ha.first_chunk[a.ntensors] = (uint32_t)chunks;
-      } else {
-        Rank1Desc &d = a.desc[a.ntensors];
-        d.p = t.p;
-        d.g = t.g;
-        d.m = t.exp_avg;
-        d.v = t.exp_avg_sq;
-        d.sm = t.exp_avg_scale;
-        d.rmax = t.row_max;
-        d.cmax = t.col_max;
-        d.rmax_next = t.row_max_next;
-        d.cmax_next = t.col_max_next;
-        d.numel = numel;
-        d.rows = t.rows;
-        d.cols = t.cols;
-        // the divisor the tensor's kernel needs: tiles per row, cols, or cols / 8
-        const FastDiv fd = make_fast_div(route == kShapeRows  ? (uint32_t)rank1_tiles_per_row(t, tile_elems)
-                                         : route == kShapeAny ? (uint32_t)t.cols
-                                                              : (uint32_t)(t.cols >> 3));
-        d.div_magic = fd.magic;
-        d.div_shift = fd.shift;
-        a.sr_salt[a.ntensors] = salt;
-        a.first_chunk[a.ntensors] = (uint32_t)chunks;
-      }
-      batch[a.ntensors] = &t;
+      batch[ntensors] = &t;
+      route_of[ntensors] = route;
+      salt_of[ntensors] = !sr ? 0u : a.go.sc_dev ? lowbias32(salts ? salts[i] : (uint32_t)i)
+                                                 : q4adamw_sr_tensor_salt(seed, step, salts ? salts[i] : (uint32_t)i);
       const int lead_dims = rank1_has_leads(t) ? t.lead_dims : 0;
-      CommitArgs::Desc &cd = ca.desc[a.ntensors];
+      CommitArgs::Desc &cd = ca.desc[ntensors];
       cd.cur[0] = t.row_max;
       cd.next[0] = t.row_max_next;
       cd.size[0] = rows_follow ? 0u : (uint32_t)t.rows;
@@ -865,7 +877,7 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
         cd.next[2 + j] = there ? t.lead_max_next[j] : nullptr;
         cd.size[2 + j] = there ? (uint32_t)t.lead_shape[j] : 0u;
       }
-      ca.first_chunk[a.ntensors] = (uint32_t)commit_chunks;
+      ca.first_chunk[ntensors] = (uint32_t)commit_chunks;
       if (lead_dims != 0 && !rows_follow) {
         RowScaleArgs::Desc &rd = ra.desc[leads];
         rd.row_next = t.row_max_next;
@@ -879,16 +891,14 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
         ++leads;
         scale_chunks += rc_;
       }
-      ++a.ntensors;
+      ++ntensors;
+      shorts += rows_follow;
       chunks += c;
       stat_chunks += sc_;
       commit_chunks += cc;
     }
-    if (a.ntensors > 0 && pass % kStatForms == kStatForms - 1) {   // the next pass has another update kernel
-      if (int rc = launch()) return rc;
-    }
   }
-  return 0;
+  return launch();
 }
 
 // ---------------------------------------------------------------------------
