@@ -1,10 +1,12 @@
 """ctypes binding of libq4adamw.so (declarations: include/q4adamw.h).
 
 There is no fallback: if the library is missing, loading raises, and every
-optimizer step raises with it.
+optimizer step raises with it.  The host module _q4host, which only shortens the way to the library's calls, may be
+missing.
 """
 import ctypes
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libq4adamw.so")
@@ -123,16 +125,23 @@ EXPORTS = (
 )
 
 _lib = None
-host = None     # the module _q4host (csrc/q4host.cpp), once the library is loaded
+host = None     # the module _q4host (csrc/q4host.cpp) or PythonHost, once the library is loaded
+
+
+class PythonHost:
+    """In the place of the module _q4host where there is none: no call is for it, and the Python code takes them all."""
+    fused_4bit = fused_single_tensor = gradients = plan = staticmethod(lambda *args: None)
 
 
 def _bind_host(L):
-    """Hands the native host code the library's entry points."""
+    """The native host code with the library's entry points in hand.  It only makes the host part of a call
+    shorter, so without it the package works as well."""
     try:
         from . import _q4host
     except ImportError as e:
-        raise RuntimeError(f"{os.path.join(_HERE, '_q4host.so')} is missing or does not load ({e}): build it with "
-                           "`python -m quantfour_adamw_cuda_amd.build`") from None
+        warnings.warn(f"quantfour_adamw_cuda_amd: the host module _q4host is missing or does not load ({e}); steps and direct "
+                      "calls take the slower Python code.  `python -m quantfour_adamw_cuda_amd.build` builds it", stacklevel=3)
+        return PythonHost
     import torch
     address = lambda name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value
     c = torch._C
