@@ -490,7 +490,8 @@ int q4adamw_release(void);
 /* Message for the last non-zero status returned on this thread ("" if none). */
 const char *q4adamw_last_error(void);
 
-/* ABI version: major * 1000 + minor. */
+/* ABI version of this header, and of a built library: major * 1000 + minor. */
+#define Q4ADAMW_VERSION 1016
 int q4adamw_version(void);
 
 #ifdef __cplusplus

@@ -133,13 +133,35 @@ class PythonHost:
     fused_4bit = fused_single_tensor = gradients = plan = staticmethod(lambda *args: None)
 
 
+def host_module_tag():
+    """The builds of torch and of the interpreter that a host module is made for: it reads tensors through torch's
+    inline accessors, which belong to one build."""
+    import sysconfig
+
+    import torch
+    return f"torch {torch.__version__} {torch.version.git_version} {sysconfig.get_config_var('SOABI')}"
+
+
+def _why_not(module, L):
+    """Why a host module that was found is not for this process, or None."""
+    tag, version = getattr(module, "built_for", None), getattr(module, "library_version", None)
+    if tag != host_module_tag():
+        return f"was built for {tag}, and this is {host_module_tag()}"
+    if version != L.q4adamw_version():
+        return f"was built for version {version} of libq4adamw.so, and this one is {L.q4adamw_version()}"
+    return None
+
+
 def _bind_host(L):
     """The native host code with the library's entry points in hand.  It only makes the host part of a call
     shorter, so without it the package works as well."""
     try:
         from . import _q4host
+        reason = _why_not(_q4host, L)
     except ImportError as e:
-        warnings.warn(f"quantfour_adamw_cuda_amd: the host module _q4host is missing or does not load ({e}); steps and direct "
+        reason = f"is missing or does not load ({e})"
+    if reason is not None:
+        warnings.warn(f"quantfour_adamw_cuda_amd: the host module _q4host {reason}; steps and direct "
                       "calls take the slower Python code.  `python -m quantfour_adamw_cuda_amd.build` builds it", stacklevel=3)
         return PythonHost
     import torch

@@ -97,8 +97,10 @@ def compile_host_module(out=HOST_MODULE, verbose=False):
 
     import torch
     from torch.utils.cpp_extension import include_paths, library_paths
+
+    from ._lib import host_module_tag
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DQ4HOST_BUILT_FOR="{host_module_tag()}"']
     for path in [*include_paths(), sysconfig.get_paths()["include"]]:
         cmd += ["-isystem", path]
     cmd += ["-o", out, os.path.join(CSRC, "q4host.cpp")]

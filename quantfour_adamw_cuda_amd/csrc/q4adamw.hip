@@ -1289,6 +1289,6 @@ int q4adamw_release(void) { return 0; }
 
 const char *q4adamw_last_error(void) { return g_err.c_str(); }
 
-int q4adamw_version(void) { return 1016; }
+int q4adamw_version(void) { return Q4ADAMW_VERSION; }
 
 }  // extern "C"

@@ -20,6 +20,13 @@
 
 #include "../../include/q4adamw.h"
 
+// What the module was built for: torch's and the interpreter's builds, in words that the loader compares with the running
+// ones (the code below has torch's inline accessors of a tensor's fields in it, and a module of another build would
+// read them at that build's offsets).
+#ifndef Q4HOST_BUILT_FOR
+#error "define Q4HOST_BUILT_FOR: see compile_host_module in build.py"
+#endif
+
 namespace {
 
 // ---------------------------------------------------------------------------
@@ -446,5 +453,9 @@ PyMODINIT_FUNC PyInit__q4host(void) {
   const char *const names[3] = {"step", "exp_avg", "exp_avg_sq"};
   for (int k = 0; k < 3; ++k)
     if (!(state_keys[k] = PyUnicode_InternFromString(names[k]))) return nullptr;
-  return PyModule_Create(&kModule);
+  PyObject *module = PyModule_Create(&kModule);
+  if (module && (PyModule_AddStringConstant(module, "built_for", Q4HOST_BUILT_FOR) < 0 ||
+                 PyModule_AddIntConstant(module, "library_version", Q4ADAMW_VERSION) < 0))
+    Py_CLEAR(module);
+  return module;
 }

@@ -49,6 +49,27 @@ def test_the_package_works_without_the_module(tmp_path):
     assert out.returncode == 0 and "without: ok" in out.stdout, out.stdout[-3000:]
 
 
+@pytest.mark.parametrize("tag,version", [(None, None), ("torch 2.0.0 0 cpython-310", 0), ("torch 2.0.0 0 cpython-310", None), (None, 0)])
+def test_a_module_of_another_build_is_not_used(monkeypatch, tag, version):
+    """A module that reads tensors as another torch lays them out, or calls the library as another version declares it,
+    is never handed the library's entry points."""
+    L = _lib.load()
+    other = type("other", (), {"bind": staticmethod(lambda *a: pytest.fail("bound"))})
+    if tag is not None or version is not None:        # without either: a module that says nothing of its build
+        other.built_for = tag or _lib.host_module_tag()
+        other.library_version = L.q4adamw_version() + (1 if version is not None else 0)
+    monkeypatch.setattr(package, "_q4host", other, raising=False)
+    monkeypatch.setitem(sys.modules, "quantfour_adamw_cuda_amd._q4host", other)
+    with pytest.warns(UserWarning, match="_q4host was built for"):
+        assert _lib._bind_host(L) is _lib.PythonHost
+
+
+def test_the_built_module_is_used():
+    L = _lib.load()
+    assert _lib.host.built_for == _lib.host_module_tag() and _lib.host.library_version == L.q4adamw_version()
+    assert _lib.host.built_for.startswith("torch " + torch.__version__)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("p_dt,g_dt", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16)])
 def test_results_without_the_module(cuda, monkeypatch, p_dt, g_dt):
