@@ -91,8 +91,12 @@ def compile_library(out, sources, flags=None, verbose=False, check_output=True):
     return out
 
 
-def compile_host_module(out=HOST_MODULE, verbose=False):
-    """csrc/q4host.cpp against the running interpreter's and torch's headers."""
+def compile_host_module(out=None, verbose=False):
+    """csrc/q4host.cpp against the running interpreter's and torch's headers.  A build that fails leaves no module: one of
+    older sources would be loaded in its place."""
+    out = out or HOST_MODULE
+    if os.path.exists(out):
+        os.remove(out)
     import sysconfig
 
     import torch
@@ -116,10 +120,11 @@ def compile_host_module(out=HOST_MODULE, verbose=False):
 
 
 def build(verbose=False):
-    """Compile unconditionally; returns the path of the step library."""
-    compile_host_module(verbose=verbose)
+    """Compile unconditionally; returns the path of the step library.  The host module comes last: it needs a C++ compiler
+    and torch's headers, which the libraries do without."""
     compile_library(LIB, STEP_SOURCES, verbose=verbose)
     compile_library(PROBE_LIB, PROBE_SOURCES, verbose=verbose)
+    compile_host_module(verbose=verbose)
     return LIB
 
 
