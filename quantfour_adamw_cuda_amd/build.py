@@ -91,9 +91,9 @@ def compile_library(out, sources, flags=None, verbose=False, check_output=True):
     return out
 
 
-def compile_host_module(out=None, verbose=False):
+def compile_host_module(out=None, verbose=False, extra=()):
     """csrc/q4host.cpp against the running interpreter's and torch's headers.  A build that fails leaves no module: one of
-    older sources would be loaded in its place."""
+    older sources would be loaded in its place.  extra: further options and sources."""
     out = out or HOST_MODULE
     if os.path.exists(out):
         os.remove(out)
@@ -107,7 +107,7 @@ def compile_host_module(out=None, verbose=False):
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DQ4HOST_BUILT_FOR="{host_module_tag()}"']
     for path in [*include_paths(), sysconfig.get_paths()["include"]]:
         cmd += ["-isystem", path]
-    cmd += ["-o", out, os.path.join(CSRC, "q4host.cpp")]
+    cmd += ["-o", out, os.path.join(CSRC, "q4host.cpp"), *extra]
     for path in library_paths():
         cmd += ["-L" + path]
     cmd += ["-ltorch_python", "-ltorch_cpu", "-lc10"]

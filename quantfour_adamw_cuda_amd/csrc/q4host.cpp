@@ -266,32 +266,29 @@ Plan *plan_of(PyObject *o) { return static_cast<Plan *>(PyCapsule_GetPointer(o, 
 
 // plan(parameters, step buffer, held [(state, step, exp_avg, exp_avg_sq)] and [(dict, key, value)], buckets [(kind, [indices], address, stride, p tag, g tag, salts'
 // address or 0)]): a capsule, or None if the group is not for the fast path.  All arguments are kept by the caller.
-PyObject *make_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
+// May throw (torch's checks, or memory that is not there): make_plan takes that for None.
+PyObject *new_plan(PyObject *const *args, Py_ssize_t n) {
   if (n != 5 || !PyTuple_CheckExact(args[0]) || !THPVariable_CheckExact(args[1]) || !PyList_CheckExact(args[2]) || !PyList_CheckExact(args[3]) ||
       !PyList_CheckExact(args[4]))
     Py_RETURN_NONE;
   auto plan = std::make_unique<Plan>();
-  try {
-    plan->device = -1;
-    plan->with_grad = 0;
-    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(args[0]); ++i) {
-      PyObject *o = PyTuple_GET_ITEM(args[0], i);
-      Dense d, g;
-      if (!dense(o, &d)) Py_RETURN_NONE;
-      const at::Tensor &grad = THPVariable_Unpack(o).grad();
-      if (grad.defined() && !dense(grad, &g)) Py_RETURN_NONE;
-      if (plan->device == -1) plan->device = d.device;
-      if (d.device != plan->device) Py_RETURN_NONE;
-      plan->params.push_back({o, d.ptr, d.numel, grad.defined() ? g.type : d.type, grad.defined()});
-      plan->with_grad += grad.defined();
-    }
-    const at::Tensor &steps = THPVariable_Unpack(args[1]);
-    if (!steps.is_cpu() || steps.scalar_type() != c10::ScalarType::Float || !steps.is_contiguous() || steps.numel() != plan->with_grad) Py_RETURN_NONE;
-    plan->step_buffer = args[1];
-    plan->steps = static_cast<float *>(steps.data_ptr());
-  } catch (const std::exception &) {
-    Py_RETURN_NONE;
+  plan->device = -1;
+  plan->with_grad = 0;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(args[0]); ++i) {
+    PyObject *o = PyTuple_GET_ITEM(args[0], i);
+    Dense d, g;
+    if (!dense(o, &d)) Py_RETURN_NONE;
+    const at::Tensor &grad = THPVariable_Unpack(o).grad();
+    if (grad.defined() && !dense(grad, &g)) Py_RETURN_NONE;
+    if (plan->device == -1) plan->device = d.device;
+    if (d.device != plan->device) Py_RETURN_NONE;
+    plan->params.push_back({o, d.ptr, d.numel, grad.defined() ? g.type : d.type, grad.defined()});
+    plan->with_grad += grad.defined();
   }
+  const at::Tensor &steps = THPVariable_Unpack(args[1]);
+  if (!steps.is_cpu() || steps.scalar_type() != c10::ScalarType::Float || !steps.is_contiguous() || steps.numel() != plan->with_grad) Py_RETURN_NONE;
+  plan->step_buffer = args[1];
+  plan->steps = static_cast<float *>(steps.data_ptr());
   for (int list = 2; list < 4; ++list)
     for (Py_ssize_t i = 0; i < PyList_GET_SIZE(args[list]); ++i) {
       PyObject *t = PyList_GET_ITEM(args[list], i);
@@ -333,6 +330,14 @@ PyObject *make_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
   PyObject *capsule = PyCapsule_New(plan.get(), kPlanName, drop_plan);
   if (capsule) plan.release();
   return capsule;
+}
+
+PyObject *make_plan(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  try {
+    return new_plan(args, n);
+  } catch (const std::exception &) {
+    Py_RETURN_NONE;
+  }
 }
 
 // refresh(plan, the group's parameters, step buffer): True if the plan still describes the group -- the same parameters at
