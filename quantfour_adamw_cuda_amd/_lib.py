@@ -13,6 +13,7 @@ LIB_PATH = os.path.join(_HERE, "csrc", "libq4adamw.so")
 
 FP32, BF16, FP16 = 0, 1, 2
 BLOCK = 128
+MOST_IN_ONE_LAUNCH = 61     # tensors of both kinds that q4adamw_fused_step_multi takes in one launch
 
 
 class Q4Tensor(ctypes.Structure):

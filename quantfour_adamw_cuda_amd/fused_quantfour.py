@@ -167,8 +167,9 @@ class AdamWFused_QuantFour(torch.optim.Optimizer):
         # global gradient norm of the last step(max_grad_norm=...), a device scalar
         self.last_grad_norm = None
         self._norm_buffers: Dict[Any, Any] = {}
-        # set to a list to collect ("fused_4bit" | "fused_single_tensor" | "grad_norm", start, end)
-        # event triples around every launch, recorded on the launch stream
+        # set to a list to collect ("fused_4bit" | "fused_4bit_rank1" | "fused_single_tensor" | "grad_norm", start, end)
+        # event triples around every launch, recorded on the launch stream; small tensors that go in the quantized ones'
+        # launch are in its "fused_4bit"
         self.kernel_timing = None
 
     # -- state ------------------------------------------------------------
@@ -768,7 +769,18 @@ class AdamWFused_QuantFour(torch.optim.Optimizer):
             # one counter per device: advance it and derive the step's scalars there
             for device in {b.device for b in plan.buckets}:
                 step_consts[device] = self._device_step(gi, device, group, before, found_inf)
+        # timed steps make the launches that the native plan makes: small tensors with quantized ones of their types and step
+        joined = {}
+        if plan.native is not None:
+            for b in plan.buckets:
+                for o in plan.buckets:
+                    if (b.kind in (True, "sr") and o.kind is False and o not in joined.values() and b not in joined
+                            and (b.p_tag, b.g_tag, steps[b.idx[0]]) == (o.p_tag, o.g_tag, steps[o.idx[0]])
+                            and len(b.idx) + len(o.idx) <= _lib.MOST_IN_ONE_LAUNCH):
+                        joined[b] = o
         for b in plan.buckets:
+            if b in joined.values():
+                continue
             rank1 = b.kind in ("rank1", "rank1_sr")
             # lr and step of a capturable group enter through step_consts; the arguments only
             # pass the range check
@@ -776,7 +788,11 @@ class AdamWFused_QuantFour(torch.optim.Optimizer):
             options = _q.grad_options(b.device, host_mult, dev_mult, found_inf, zero_grad,
                                       step_consts.get(b.device), group.get("param_update", "auto"))
             hyper = (b.device, b.p_tag, b.g_tag, beta1, beta2, lr, weight_decay, eps, t_step, options)
-            if b.kind in ("sr", "rank1_sr"):
+            if b in joined:
+                launch = _q.launch_step_table
+                sr = b.kind == "sr"
+                args = (b.arr, joined[b].arr, b.salts if sr else None, int(group["seed"]) if sr else 0) + hyper
+            elif b.kind in ("sr", "rank1_sr"):
                 launch = _q.launch_rank1_table_sr if rank1 else _q.launch_table_sr
                 args = (b.arr, b.salts, group["seed"]) + hyper
             else:

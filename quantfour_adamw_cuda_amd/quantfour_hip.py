@@ -249,6 +249,16 @@ def launch_small_table(arr, device, p_tag, g_tag, beta1, beta2, lr, weight_decay
     _lib.check(rc, "fused_single_tensor_multi")
 
 
+def launch_step_table(arr, small_arr, salts, seed, device, p_tag, g_tag, beta1, beta2, lr, weight_decay, eps, step,
+                      options=None):
+    """Quantized tensors (stochastically rounded where salts are given) and small ones in one call."""
+    L = _lib.load()
+    with _on(device):
+        rc = L.q4adamw_fused_step_multi(arr, len(arr), small_arr, len(small_arr), int(salts is not None), salts, seed, p_tag, g_tag,
+                                        beta1, beta2, lr, weight_decay, eps, float(step), options, _stream(device))
+    _lib.check(rc, "fused_step_multi")
+
+
 def fused_4bit_multi(ps, gs, exps, sqs, exp_scales, sq_scales, beta1, beta2, lr, weight_decay,
                      eps, step, grad_scale=1.0, grad_scale_dev=None, found_inf=None, zero_grad=False,
                      step_consts=None, update_form="auto"):

@@ -77,6 +77,30 @@ def test_steps_equal_the_python_codes(cuda, kw, p_dt, g_dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("small,kinds", [(59, ["fused_4bit"]), (60, ["fused_4bit", "fused_single_tensor"])])
+@pytest.mark.parametrize("kw", [{}, dict(round_type="stochastic", seed=5)])
+def test_timed_steps_make_the_same_launches(cuda, kw, small, kinds):
+    """Steps with launch timing, which the Python code makes, against steps without: one launch for both kinds up to 61
+    tensors, and for tensors of one step number only; the same results."""
+    gen, ((pa, timed), (pb, plain)) = _twins(cuda, [(70, 129), (5000,)] + [(100 + i,) for i in range(small)], torch.float32, torch.float32, **kw)
+    plain._make_native, plain._one_norm = type(plain)._make_native.__get__(plain), type(plain)._one_norm.__get__(plain)
+    for step in range(4):
+        gs = [torch.randn(p.shape, generator=gen, device=cuda) * 1e-2 for p in pa]
+        timed.kernel_timing = []
+        for ps, opt in ((pa, timed), (pb, plain)):
+            for i, (p, g) in enumerate(zip(ps, gs)):
+                p.grad = None if step == 1 and i < 2 else g      # the quantized ones lag by a step from here on
+            opt.step(zero_grad=False)
+        seen = sorted(kind for kind, _, _ in timed.kernel_timing)
+        assert seen == (kinds if step == 0 else ["fused_single_tensor"] if step == 1 else ["fused_4bit", "fused_single_tensor"]), f"step {step}"
+        assert plain._plans[0].native is not None
+        for a, b in zip(pa, pb):
+            assert torch.equal(a, b), f"step {step}: {tuple(a.shape)}"
+            for key in ("exp_avg", "exp_avg_sq"):
+                assert torch.equal(timed.state[a][key], plain.state[b][key])
+
+
+@pytest.mark.gpu
 def test_refusals_are_the_python_codes(cuda):
     n = 5000
     nbytes, nblk = q.state_sizes(n)
