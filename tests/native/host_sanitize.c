@@ -163,6 +163,48 @@ static void refusals(void) {
   EXPECT(q4adamw_fused_single_tensor_multi(st, 1, F, F, B1, B2, LR, WD, EPS, 1.0f, NULL), Q4ADAMW_ERR_ARG);
   st[0].p = (char *)buf + 2; st[0].g = buf; st[0].exp_avg = buf; st[0].exp_avg_sq = buf;
   EXPECT(q4adamw_fused_single_tensor_multi(st, 1, F, F, B1, B2, LR, WD, EPS, 1.0f, NULL), Q4ADAMW_ERR_ALIGN);
+  /* both kinds in one call: refusals of either, and of the lists themselves */
+  {
+    q4adamw_tensor qt[1];
+    q4adamw_small_tensor s1[1];
+    const uint32_t salt[1] = {3};
+    memset(qt, 0, sizeof qt);
+    memset(s1, 0, sizeof s1);
+#define STEP(q_, nq, s_, ns, stochastic, opt_) \
+  q4adamw_fused_step_multi(q_, nq, s_, ns, stochastic, salt, 7, F, F, B1, B2, LR, WD, EPS, 1.0f, opt_, NULL)
+    EXPECT(STEP(NULL, 0, NULL, 0, 0, NULL), 0);
+    EXPECT(STEP(qt, 1, s1, 1, 1, NULL), 0);                       /* no elements */
+    EXPECT(STEP(NULL, 1, s1, 1, 0, NULL), Q4ADAMW_ERR_ARG);
+    EXPECT(STEP(qt, 1, NULL, 1, 0, NULL), Q4ADAMW_ERR_ARG);
+    EXPECT(STEP(qt, -1, s1, 1, 0, NULL), Q4ADAMW_ERR_ARG);
+    EXPECT(STEP(qt, 1, s1, -1, 0, NULL), Q4ADAMW_ERR_ARG);
+    s1[0].numel = 5;                                              /* null pointers, then misaligned ones */
+    EXPECT(STEP(qt, 1, s1, 1, 0, NULL), Q4ADAMW_ERR_ARG);
+    s1[0].p = buf; s1[0].g = (char *)buf + 2; s1[0].exp_avg = buf; s1[0].exp_avg_sq = buf;
+    EXPECT(STEP(qt, 1, s1, 1, 0, NULL), Q4ADAMW_ERR_ALIGN);
+    EXPECT(STEP(NULL, 0, s1, 1, 0, NULL), Q4ADAMW_ERR_ALIGN);
+    s1[0].g = buf; s1[0].exp_avg_sq = (float *)((char *)buf + 1);
+    EXPECT(STEP(qt, 1, s1, 1, 1, NULL), Q4ADAMW_ERR_ALIGN);
+    s1[0].exp_avg_sq = buf; s1[0].numel = -5;
+    EXPECT(STEP(qt, 1, s1, 1, 0, NULL), Q4ADAMW_ERR_ARG);
+    s1[0].numel = INT64_MAX;
+    EXPECT(STEP(qt, 1, s1, 1, 0, NULL), Q4ADAMW_ERR_TOO_LARGE);
+    s1[0].numel = 0;
+    qt[0].numel = -1;
+    EXPECT(STEP(qt, 1, s1, 1, 0, NULL), Q4ADAMW_ERR_ARG);
+    qt[0].numel = 10;
+    EXPECT(STEP(qt, 1, s1, 1, 0, NULL), Q4ADAMW_ERR_ARG);         /* null pointers */
+    qt[0].p = buf; qt[0].g = buf; qt[0].exp_avg = codes + 1; qt[0].exp_avg_sq = codes; qt[0].exp_avg_scale = scales; qt[0].exp_avg_sq_scale = scales;
+    EXPECT(STEP(qt, 1, s1, 1, 1, NULL), Q4ADAMW_ERR_ALIGN);
+    qt[0].exp_avg = codes; qt[0].numel = INT64_MAX;
+    EXPECT(STEP(qt, 1, NULL, 0, 0, NULL), Q4ADAMW_ERR_TOO_LARGE);
+    qt[0].numel = 0;
+    q4adamw_grad_options o = {1.0f, 0, (const float *)((const char *)buf + 2), NULL};
+    EXPECT(STEP(qt, 1, s1, 1, 0, &o), Q4ADAMW_ERR_ALIGN);
+    EXPECT(q4adamw_fused_step_multi(qt, 1, s1, 1, 0, salt, 7, F, 3, B1, B2, LR, WD, EPS, 1.0f, NULL, NULL), Q4ADAMW_ERR_ARG);
+    EXPECT(q4adamw_fused_step_multi(qt, 1, s1, 1, 0, salt, 7, F, F, 1.0f, B2, LR, WD, EPS, 1.0f, NULL, NULL), Q4ADAMW_ERR_HYPER);
+#undef STEP
+  }
   /* rank-1 */
   q4adamw_rank1_tensor r[1];
   memset(r, 0, sizeof r);

@@ -174,3 +174,60 @@ def test_one_call_for_both_kinds(cuda, quantized, small, stochastic, p_dt, g_dt)
                     _lib.check(L.q4adamw_fused_4bit_multi_ex(qt, quantized, *tail), "ex")
         for a, b in zip(kept[0] + one[0] + [t for s in one[1] + one[2] for t in s], kept[1] + two[0] + [t for s in two[1] + two[2] for t in s]):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), f"step {step}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("small", [2, 3])
+def test_one_call_at_the_most_workgroups(cuda, small):
+    """One launch takes both kinds up to 2^17 workgroups of 1024 elements; a list of one more takes two."""
+    L = _lib.load()
+    gen = torch.Generator(device=cuda).manual_seed(small)
+    n = ((1 << 17) - 2) * 1024 - 100                     # 2^17 - 2 workgroups, one more for every small tensor
+    z = lambda k, dt=torch.float32: torch.zeros(k, dtype=dt, device=cuda)
+    nb, nk = q.state_sizes(n)
+    stream = q._stream(torch.device("cuda", torch.cuda.current_device()))
+    base = [torch.randn(k, generator=gen, device=cuda) * 0.05 for k in [n] + [700] * small]
+    gs = [(torch.randn(b.numel(), generator=gen, device=cuda) * 1e-2).to(torch.bfloat16) for b in base]
+    sides = []
+    for one in (True, False):
+        ps = [b.clone() for b in base]
+        qs, ss = [z(nb, torch.uint8), z(nb, torch.uint8), z(nk), z(nk)], [(z(700), z(700)) for _ in range(small)]
+        qt = q.make_table(ps[:1], gs[:1], *([x] for x in qs))
+        st = q.make_small_table(ps[1:], gs[1:], [x[0] for x in ss], [x[1] for x in ss])
+        tail = (0, 1, *HP, 1.0, None, stream)
+        if one:
+            _lib.check(L.q4adamw_fused_step_multi(qt, 1, st, small, 0, None, 0, *tail), "fused_step_multi")
+        else:
+            _lib.check(L.q4adamw_fused_single_tensor_multi_ex(st, small, *tail), "small")
+            _lib.check(L.q4adamw_fused_4bit_multi_ex(qt, 1, *tail), "ex")
+        sides.append(ps + qs + [t for s in ss for t in s])
+    for a, b in zip(*sides):
+        assert torch.equal(a, b)
+    assert all(not torch.equal(p, b) for p, b in zip(sides[0], base))
+
+
+class _Named(torch.Tensor):
+    """A tensor subclass, as programs make them to carry a name along."""
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("where", ["parameter", "gradient"])
+def test_tensor_subclasses(cuda, where):
+    """A parameter of a subclass keeps its group on the Python path, a gradient of one is the memory that it is: the same
+    results as plain tensors."""
+    gen, ((pa, a), (pb, b)) = _twins(cuda, [(70, 129), (100,)], torch.float32, torch.float32)
+    if where == "parameter":
+        pa[0] = torch.nn.Parameter(pa[0].detach().as_subclass(_Named))
+        a = AdamWFused_QuantFour(pa, lr=1e-3, weight_decay=0.01)
+        assert isinstance(pa[0], _Named)
+    for step in range(3):
+        for x, y in zip(pa, pb):
+            g = torch.randn(y.shape, generator=gen, device=cuda) * 1e-2
+            x.grad = g.clone().as_subclass(_Named) if where == "gradient" else g.clone()
+            y.grad = g
+        a.step(max_grad_norm=0.5)
+        b.step(max_grad_norm=0.5)
+        if where == "parameter":
+            assert a._plans[0].native is None
+        for x, y in zip(pa, pb):
+            assert torch.equal(x.detach().as_subclass(torch.Tensor), y.detach()), f"step {step}"
