@@ -243,10 +243,13 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
   for (int qi = 1; qi < 4; ++qi) u = u > row_bits[qi][tid] ? u : row_bits[qi][tid];
   if (T.lead_dims == 0u) {
     if (tid < tile_rows && u != 0u) {
-      // A few rows of very many columns: what the launch waits for is the atomics on these rows' statistics, and
-      // nearly all of them find the maximum there.  us a step, atomics / with the look: 4 x 3000000 123 / 94, 3 x 5000001 and
-      // 5000001 others 198 / 133; but 20 x 600000 57 / 59, 100 x 200000 70 / 80.
-      if (T.rows <= 8u && groups > 256u) raise_max(T.rmax_next + tile_row0 + tid, u);
+      // A few rows of very many columns: what the launch waits for is the atomics on these rows' statistics, and once
+      // the first tiles are through, nearly all of them find the maximum there.  With few tiles most of them start together, find
+      // less and pay for the look as well.  us a step, atomics / with the look, in fp32 and bf16: 4 rows of 1024 tiles
+      // 29.1 / 34.7 and 31.8 / 32.7, 8 of 1536 49.8 / 55.0 and 49.5 / 51.5, 3 of 2560 54.9 / 57.0 and 58.1 / 63.5; 1 row of 3072
+      // 60.4 / 53.0 and 60.6 / 56.5, 3 of 3073 68.1 / 64.3 and 65.9 / 66.3, 8 of 3073 91.2 / 85.3 and 82.2 / 81.0, 4 of 9766
+      // 194 / 128 and 179 / 120.  More rows share fewer updates each: 24 rows of 1024 tiles 59 / 69 and 48 / 53.
+      if (T.rows <= 8u && groups > 3072u) raise_max(T.rmax_next + tile_row0 + tid, u);
       else atomic_max_bits(T.rmax_next + tile_row0 + tid, u);
     }
     return;
