@@ -92,6 +92,21 @@ __device__ __forceinline__ uint32_t load_part_codes(const void *run, uint32_t od
   return w;
 }
 
+// The codes of 4 elements in a matrix whose rows may begin at either nibble, in two steps: a load whose result nothing looks
+// at before all loads of a group of rows are under way, and their place in it.  With load_part_codes the byte after
+// an odd start is in a branch of its own, behind which every part of every odd row waited: a step of 97 x 511 fp32 elements took
+// 17.7 us (now 13.5), 15.8 before gradients were read in parts, of 30000 x 1001 123 (103).  The 4 bytes of the window end with the codes'
+// last byte; those of the matrix' first 4 elements, before which nothing may be read, begin with the first.
+__device__ __forceinline__ uint32_t load_window(const uint8_t *run, int64_t run_first, uint32_t elem) {
+  const uint32_t nibble = ((uint32_t)run_first & 1u) + elem, at_start = run_first == 0 && elem == 0u ? 2u : 0u;
+  return __builtin_amdgcn_raw_buffer_load_b32(tile_rsrc(run - 2), (nibble >> 1) + (nibble & 1u) + at_start, 0, kNtReadOnly);
+}
+
+__device__ __forceinline__ uint32_t window_codes(uint32_t window, int64_t run_first, uint32_t elem) {
+  const uint32_t odd = ((uint32_t)run_first + elem) & 1u;
+  return window >> (run_first == 0 && elem == 0u ? 0u : 16u - 4u * odd);
+}
+
 // New second moments of a tile of stat_rows x kStatCols elements, reduced to row and
 // column maxima (get_variance_tensor_statistics, adamw_fourbit_triton.py:738-746).  The
 // arithmetic is the update kernel's, operation for operation, so the maxima are maxima
@@ -117,6 +132,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
   // 14336 x 4096 elements 133 against 128, a step of 8000 x 9001 elements 327 against 314.
   constexpr int kParts = GT ? 1 : 2;
   constexpr uint32_t kPer = 8 / kParts;
+  constexpr bool kWindow = ANY && kPer == 4;
   __shared__ uint32_t row_bits[4][kStatRows];       // row maxima of each 16-lane quarter of the row's wave
   __shared__ uint32_t col_bits[kWaves][kStatCols];  // column maxima of each wave
   const uint32_t chunk = args.chunk_base + run_chunk(args.runs, blockIdx.x);
@@ -164,21 +180,23 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
     u32x4 gw[kAhead][kParts];
     uint32_t vw[kAhead][kParts];
     float r_old[kAhead];
+    int64_t run_first[kAhead];   // uniform
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
       const int r = r0 + i < nrows ? r0 + i : nrows - 1;
       const uint32_t row = tile_row0 + wave_row0 + r;
       r_old[i] = kAbs ? 0.0f : as_global<const float>(T.rmax)[row];
       // row bases are uniform; the lane's column is a 32-bit offset
-      const int64_t row_first = (int64_t)row * T.cols + col0;
+      const int64_t row_first = run_first[i] = (int64_t)row * T.cols + col0;
       const void *g_row = static_cast<const char *>(T.g) + row_first * (GT ? 2 : 4);
-      const void *v_row = T.v + (row_first >> 1);
+      const uint8_t *v_row = T.v + (row_first >> 1);
 #pragma unroll
       for (int h = 0; h < kParts; ++h) {
         vw[i][h] = 0u;
         gw[i][h] = u32x4{0u, 0u, 0u, 0u};
         if (active[h]) {
-          if (!kAbs) vw[i][h] = load_part_codes<kPer, ANY>(v_row, (uint32_t)row_first & 1u, part_elem[h]);
+          if (!kAbs)
+            vw[i][h] = kWindow ? load_window(v_row, row_first, part_elem[h]) : load_part_codes<kPer, ANY>(v_row, (uint32_t)row_first & 1u, part_elem[h]);
           gw[i][h] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_row), part_elem[h] * (GT ? 2u : 4u), 0, kNtReadOnly);
         }
       }
@@ -197,7 +215,8 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_kernel(const Rank1StatAr
         } else {
           g[4 * h] = bits2f(w.x); g[4 * h + 1] = bits2f(w.y); g[4 * h + 2] = bits2f(w.z); g[4 * h + 3] = bits2f(w.w);
         }
-        const uint32_t even = vw[i][h] & 0x0F0F0F0Fu, odd = (vw[i][h] >> 4) & 0x0F0F0F0Fu;  // one code per byte
+        const uint32_t codes = kWindow ? window_codes(vw[i][h], run_first[i], part_elem[h]) : vw[i][h];
+        const uint32_t even = codes & 0x0F0F0F0Fu, odd = (codes >> 4) & 0x0F0F0F0Fu;  // one code per byte
 #pragma unroll
         for (uint32_t k = 0; k < kPer; ++k) code[kPer * h + k] = (float)(((k & 1 ? odd : even) >> (8 * (k >> 1))) & 0xffu);
       }

@@ -24,6 +24,8 @@ TALL = [(6145, 50), (6144 + 63 * 5, 64), (6200, 255), (24577, 33), (24640, 88), 
 # either part, on its first and last columns and between them; 130 and 136 tiles, of which 128 are dealt in runs of 8
 PARTS = [(37, 258), (37, 259), (40, 260), (37, 261), (40, 504), (37, 507), (40, 508), (37, 510), (40, 512), (37, 515), (40, 520), (37, 767),
          (37, 770), (2080, 520), (1088, 1541),
+         # codes in windows of 4 bytes, which end the matrix' last byte and begin its first: rows that begin at either nibble
+         (1, 257), (2, 257), (3, 259), (2, 261), (1, 263), (2, 511), (1, 513), (3, 1031),
          # few rows and many tiles along them: more than 256, and on either side of the rule for their statistics (3072 tiles)
          (1, 131584), (8, 131073), (9, 131073), (3, 131585), (1, 1572864), (1, 1572865), (8, 1573380), (9, 1573376)]
 TENSORS = [(5, 300, 3, 3), (2, 700, 3), (1400, 1, 2), (300, 2, 7), (16, 16, 16), (3, 100, 260), (2, 130, 4, 257), (64, 3, 7, 7),
