@@ -211,11 +211,15 @@ __device__ __forceinline__ void process_tile(const Desc &T, int64_t tb, int lane
     // lie in one row, nearly every one of a matrix of hundreds of columns, takes one maximum of the row and the
     // columns' with 16-byte loads (at any element's address), old and new: 4 or 6 loads.  One of each kind per element
     // for every lane, 16 or 32, was what this form spent its time on.  Steps, us, then / now: 8000 x 9001
-    // (fp32 / bf16) 277 / 206, in bf16 352 / 169; 768 x 50257 in fp32 178 / 129; 300000 x 77 121 / 108.
+    // (fp32 / bf16) 277 / 206, in bf16 352 / 169; 768 x 50257 in fp32 178 / 129; 300000 x 77 121 / 108.  Lanes of 8 elements
+    // in rows shorter than two of them go both ways in nearly every wave, and the loads that start anywhere cost more than they
+    // save; the ones that start at 4 columns do not.  Steps of 20 million bf16 elements, us, per element / with the look-up: 9 columns
+    // 94.8 / 98.1, 11 95.7 / 100.9, 13 96.8 / 101.6, 14 97.0 / 99.5; 8 84.6 / 81.5, 12 97.2 / 91.9, 17 92.6 / 90.1, 19 93.9 / 95.7,
+    // 21 94.6 / 96.6, 22 97.9 / 93.7, 31 95.2 / 89.9.  Lanes of 4: 5 109.6 / 108.9, 7 107.3 / 106.4, 13 110.0 / 104.0.
     const uint32_t first = (uint32_t)tb + e0, cols = (uint32_t)T.cols, last = (uint32_t)T.rows - 1u;
     uint32_t row = fast_div(first, T.div_magic, T.div_shift);
     uint32_t col = first - row * cols;
-    if (col + N <= cols) {
+    if ((N == 4 || cols >= 16u || cols % 4u == 0u) && col + N <= cols) {
       const uint32_t there = row < last ? row : last;
       const float old_max = as_global<const float>(T.rmax)[there], new_max = as_global<const float>(T.rmax_next)[there];
 #pragma unroll
