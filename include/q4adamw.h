@@ -209,19 +209,23 @@ uint32_t q4adamw_sr_tensor_salt(uint64_t seed, float step, uint32_t tensor_salt)
  * sizes that must hold zeros on entry and holds zeros again afterwards.
  * rows x cols, row-major, cols >= 2; p and g aligned to their element type (see
  * q4adamw_tensor), col_max and col_max_next 16-byte aligned, the rest 4-byte aligned.  Rows of
- * a multiple of 8 elements (and at least 16) take the tuned kernels; any other row length is
- * taken element by element (matrices of fewer than 2^32 elements), as the draft scales every
- * tensor with dim() > 1 this way (optim/adamw_fourbit_triton.py:841-846).
+ * a multiple of 8 elements (and at least 16) have kernels whose lanes lie in one row each; rows of
+ * any other length take ones that find every element's row and column (matrices of fewer than 2^32
+ * elements), as the draft scales every tensor with dim() > 1 this way
+ * (optim/adamw_fourbit_triton.py:841-846).
  *
  * Tensors of three or four dimensions (lead_dims = 2 or 3): cols is the last dimension,
  * lead_shape the others, rows their product.  Every leading dimension has its own
  * statistic, the maximum over all other dimensions (the loop over x.dim() at
  * optim/adamw_fourbit_triton.py:741-745): lead_max[j] (lead_shape[j] floats, updated by the
  * call) with scratch lead_max_next[j] (zeros on entry and afterwards).  The scale of an
- * element is the minimum over all its dimensions' statistics (:749-755); row_max then holds,
- * for every flattened row, the minimum over its leading statistics -- derived state that the
- * call keeps up to date and the caller recomputes after loading a checkpoint.  lead_dims = 0
- * or 1: a matrix, the lead_* fields are not read.
+ * element is the minimum over all its dimensions' statistics (:749-755).  lead_max is what
+ * counts; row_max then holds, for every flattened row, the minimum over its leading statistics --
+ * derived state that the call keeps up to date and the caller recomputes after loading a
+ * checkpoint.  Which of the two a call reads depends on the shape (tensors with rows of up to 256
+ * elements take their statistics' old scales from lead_max, and those with rows of up to 64 that are
+ * no multiple of 8 or shorter than 16 the update's as well; row_max is then written only), so the two must
+ * agree on entry.  lead_dims = 0 or 1: a matrix, the lead_* fields are not read.
  */
 typedef struct q4adamw_rank1_tensor {
   void *p;
@@ -243,10 +247,13 @@ typedef struct q4adamw_rank1_tensor {
 } q4adamw_rank1_tensor;
 
 /*
- * The fused step with a rank-1-scaled second moment, per batch of up to 32 tensors
- * three launches: new second moments reduced to row and column maxima, the update
- * (dequantize with the old maxima, quantize with the new ones), and the commit of the
- * new maxima.  Everything else as q4adamw_fused_4bit_multi_ex (opt may be NULL).  The
+ * The fused step with a rank-1-scaled second moment, in batches of up to 32 tensors (of which up
+ * to 25 have several leading dimensions and short rows): new second moments reduced to row and
+ * column maxima, the update (dequantize with the old maxima, quantize with the new ones), and the
+ * commit of the new maxima.  A batch makes one launch for each of the four statistics kernels and
+ * the five update kernels that its tensors need, one for the commit and, with several leading
+ * dimensions and longer rows, one that makes the rows' scales: three launches where all its
+ * tensors are of one kind, eleven at most.  Everything else as q4adamw_fused_4bit_multi_ex (opt may be NULL).  The
  * device form of variance_quant / variance_dequant with scale_type "rank1"
  * (optim/adamw_fourbit_triton.py:498-527, :803-863) inside the fused step
  * (optim/cuda_adamw_kernels.cu:266-419).
@@ -293,8 +300,9 @@ int q4adamw_fused_single_tensor_multi_ex(const q4adamw_small_tensor *tensors, in
 
 /*
  * One step over both kinds of tensors: q4adamw_fused_4bit_multi_ex, or _sr with `stochastic`, for `tensors` and
- * q4adamw_fused_single_tensor_multi_ex for `small`, the same results; small models' lists, of up to 61 tensors
- * together, in one launch.  (optim/fused_quantfour.py:171-292 makes a launch per parameter.)
+ * q4adamw_fused_single_tensor_multi_ex for `small`, the same results; lists of both kinds with up to 61 tensors
+ * together and up to 2^17 workgroups (of 1024 elements, 2048 where parameters and gradients are 16-bit types) in one
+ * launch.  (optim/fused_quantfour.py:171-292 makes a launch per parameter.)
  */
 int q4adamw_fused_step_multi(const q4adamw_tensor *tensors, int count, const q4adamw_small_tensor *small,
                              int small_count, int stochastic, const uint32_t *salts, uint64_t seed,
@@ -461,10 +469,11 @@ int q4adamw_sr_affine_entry(uint32_t k, float *out2);
  * with a 32-bit element count (optim/cuda_adamw_kernels.cu:430-432) and stops at 2^31 elements.
  */
 int q4adamw_grid_plan(uint64_t chunks, int threads, uint64_t *bases, uint64_t *counts, int capacity);
-/* Host-only, for tests: which of its three update kernels q4adamw_fused_4bit_rank1_multi runs on
- * a rows x cols matrix: 0 = tiles aligned to the rows, 1 = tiles anywhere in rows of at least a
- * tile, 2 = rows shorter than a tile, 3 = rows of any length (no multiple of 8, or below 16).  both_16_bit: parameters and gradients are 16-bit types
- * (tiles of 512 elements instead of 256). */
+/* Host-only, for tests: which of its update kernels for matrices q4adamw_fused_4bit_rank1_multi
+ * runs on rows x cols elements: 0 = tiles aligned to the rows, 1 = tiles anywhere in rows of at
+ * least a tile, 2 = rows shorter than a tile, 3 = rows of any length (no multiple of 8, or below 16;
+ * with several leading dimensions and up to 64 columns a fifth kernel takes these).  both_16_bit:
+ * parameters and gradients are 16-bit types (tiles of 512 elements instead of 256). */
 int q4adamw_rank1_form(int64_t rows, int64_t cols, int both_16_bit);
 void q4adamw_set_grid_limit(uint64_t workgroups);
 

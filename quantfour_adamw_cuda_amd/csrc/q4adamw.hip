@@ -182,7 +182,7 @@ static SmallKernel pick_small(int p_dtype, int g_dtype, bool ext) {
   return ext ? pick_small_ext<true>(p_dtype, g_dtype) : pick_small_ext<false>(p_dtype, g_dtype);
 }
 
-// Which of the three update kernels a matrix takes, in the order of the launch passes.
+// Which of the four update kernels for matrices one takes, in the order of the launch passes.
 // Rows form: rows of a whole number of quantization blocks and at least two tiles, and enough
 // rows that the waves left idle in the last group of four do not matter.  The last tile of a
 // row may be a partial one as long as its idle lanes are at most a sixteenth of the row (they
@@ -213,9 +213,11 @@ static bool rank1_has_leads(const q4adamw_rank1_tensor &t) { return t.lead_dims 
 // Tensors with several leading dimensions whose elements would gather their scales one by one (kShapeAny) take a
 // kernel of their own if their rows are short, so that rows' scales are a good part of their bytes: it makes
 // them from the leading statistics, and no launches make and copy them around it.  us a step of [256, n, c], 41
-// million elements, in fp32 / in bf16, without and with it: c = 5 255 / 251 and 219 / 198, 8 239 / 188 and 209 / 188; the
-// form for multiples of 8 is the better one in bf16 from 16 columns on (213 / 168 and 208 / 185 at 16, 210 / 164 and 210 / 185
-// at 32).
+// million elements, without and with it: c = 3 fp32 222 / 162, bf16 189 / 122; 9 188 / 158, 154 / 118; 15 169 / 156, 142 / 118;
+// 17 166 / 153, 139 / 118; 33 169 / 159, 144 / 132; 49 166 / 157, 143 / 132; 63 179 / 170, 136 / 126.  It is the better one beyond
+// the line as well (c = 65 202 / 193, 156 / 148; 127 170 / 162, 134 / 126; 255 171 / 167, 141 / 134): there the line
+// is what its LDS was laid out for, 64 columns.  Multiples of 8 from 16 columns on have the better form in bf16 (bf16
+// without and with it, an earlier state of both, 168 / 185 at 16 and 164 / 185 at 32).
 constexpr int kRouteShort = 4, kRoutes = 5;   // the others: Rank1Shape
 
 static int rank1_route(const q4adamw_rank1_tensor &t, int64_t tile_elems) {
@@ -574,10 +576,12 @@ static int check_small(const q4adamw_small_tensor *tensors, int count, int p_dty
   return 0;
 }
 
-// One launch for both kinds of tensors up to this many workgroups and as many tensors as its arguments hold.  us a step
-// with two launches / one: tensors around the quantization threshold and two of 1 and 3 million elements 17.5 / 14.5, linear
-// layers 512 wide 16.9 / 14.0, 2048 wide in bf16 48.2 / 45.4, a table of 38 million elements and four layers in fp32 150.0 / 145.4; one
-// Llama-3-8B layer, beyond the limit, would gain under 1 per cent.
+// One launch for both kinds of tensors up to this many workgroups and as many tensors as its arguments hold.  What it
+// saves is a launch, 3 to 5 us whatever the list's size; the line is where that falls to about 1 %, and larger lists stay with the
+// kernel that knows one kind.  us a step with two launches / one, two quantized tensors of together 2^k workgroups and four small
+// ones, fp32 and bf16: k = 10 8.4 / 5.5 and 8.9 / 6.7, 14 41.5 / 37.4 and 46.5 / 43.6, 16 144.6 / 140.8 and 169.3 / 166.3, 17
+// 284.5 / 280.6 and 332.4 / 328.6, 18 565.8 / 560.4 and 656.7 / 652.5, 19 1177 / 1174 and 1340 / 1341; thirty of each, k = 17
+// 291.7 / 286.7 and 335.7 / 333.0.
 constexpr uint64_t kMixedMostChunks = 1ull << 17;
 
 static int fused_4bit_multi_impl(const q4adamw_tensor *tensors, int count, int p_dtype, int g_dtype,

@@ -34,8 +34,8 @@ FusedKernel pick_fused(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 FusedKernel pick_mixed(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 // the rank-1 update kernels: tiles anywhere in a matrix of rows at least a tile long
 // (pick_rank1_wide), matrices narrower than a tile (pick_rank1_narrow), tiles aligned to the
-// rows of a matrix (pick_rank1_rows), rows of any length (pick_rank1_any), rows shorter than a tile in tensors
-// of fewer than 2^32 elements (pick_rank1_short)
+// rows of a matrix (pick_rank1_rows), rows of any length (pick_rank1_any), such rows of up to 64
+// elements in tensors with several leading dimensions (pick_rank1_short); the last two: fewer than 2^32 elements
 Rank1Kernel pick_rank1_wide(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 Rank1Kernel pick_rank1_narrow(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);
 Rank1Kernel pick_rank1_rows(int p_dtype, int g_dtype, bool ext, bool sr, bool exact);

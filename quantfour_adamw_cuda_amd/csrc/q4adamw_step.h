@@ -40,8 +40,8 @@ struct Geometry {
 // (RowsTile).  kTileRowsLast is the same for the last tile of a row that is not a whole
 // number of tiles long: its first RowsTile::width elements are there (whole blocks), the
 // lanes of the others load nothing, work on zeros and store nothing.  kTileAny: rows of any
-// length (not a multiple of 8, or shorter than 16): every element finds its own row and column
-// (matrices of fewer than 2^32 elements).
+// length (not a multiple of 8, or shorter than 16): a lane finds its first element's row and column, and takes one row's
+// maxima where its elements lie in one row, else every element's (matrices of fewer than 2^32 elements).
 // kTileShort: short rows of a tensor with several leading dimensions; a workgroup's tiles are consecutive, and it lays
 // the scales of the rows they meet and those of all columns out in LDS (ShortTile).
 constexpr int kTileWide = 0, kTileNarrow = 1, kTileRows = 2, kTileRowsLast = 3, kTileAny = 4, kTileShort = 5;

@@ -386,7 +386,8 @@ def check_rank1(p, g, exp, sq, exp_scale, row_max, col_max, row_next, col_next, 
 def make_rank1_table(ps, gs, exps, sqs, exp_scales, row_maxes, col_maxes, row_nexts, col_nexts, leads=None):
     """leads: None, or per tensor None (a matrix) or (leading statistics, their scratch), two
     lists with one float32 tensor per leading dimension; row_maxes[i] then holds the flattened
-    rows' scales (rank1_row_scale)."""
+    rows' scales (rank1_row_scale), which must agree with the statistics: a step reads the one or
+    the other."""
     n = len(ps)
     arr = (_lib.Q4Rank1Tensor * n)()
     for i in range(n):
