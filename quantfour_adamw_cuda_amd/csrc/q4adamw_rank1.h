@@ -393,7 +393,9 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1S
 // their minimum once and the first dimension's is one number for the wave; the maxima stay in registers until the end.
 // With one element per lane, a load of each row's scale (4 bytes for every row of three elements) and 32 indices, steps
 // of residual networks took, us, 64 wide in fp32 88 (now 79), 96 wide in bf16 174 (133), of [256, n, 64] with 41 million
-// elements in fp32 213 (157), in bf16 166 (102).
+// elements in fp32 213 (157), in bf16 166 (102).  With fewer elements below an index than a lane's N, every lane takes one
+// (those past the end the first one again): all N of them in each lane, one load after another, made a step of [300000, 2, 3]
+// with bf16 gradients 119 us (now 76; 84 with one element per lane everywhere).
 constexpr uint32_t kLeadOuter = 32, kLeadMostOuter = 256;    // a round's indices; the most
 
 // elements of a run, at most (16 bytes of gradients per lane)
@@ -437,9 +439,9 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1S
   for (uint32_t i = tid; i < kSlots; i += kThreads) slots[0][i] = slots[1][i] = slots[2][i] = 0u;
 
   // this lane's elements, the same under every index of the first dimension: the last ones of the run for lanes
-  // that would reach past its end
+  // that would reach past its end, and of a run shorter than that a single one
   const bool whole = len >= N;
-  const uint32_t elem = !whole ? 0u : lane * N < len - N ? lane * N : len - N;
+  const uint32_t elem = !whole ? (lane < len ? lane : 0u) : lane * N < len - N ? lane * N : len - N;
   const uint32_t shape2 = T.lead_dims == 3u ? T.lead_shape[2] : 1u;
   const gptr<const float> before = as_global<const float>(T.lead_old[1]), last = as_global<const float>(T.lead_old[2]);
   float s_old[N], x_max[N];
@@ -449,7 +451,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1S
 #pragma unroll
     for (uint32_t k = 0; k < N; ++k) {
       float s = 0.0f;
-      if (whole || k < len) {
+      if (whole || k == 0u) {
         s = min_nonneg(as_global<const float>(T.cmax)[col], before[i1]);
         if (T.lead_dims == 3u) s = min_nonneg(s, last[i2]);
       }
@@ -478,19 +480,10 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1S
     if (whole) {
       gw[i] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_run), elem * (GT ? 2u : 4u), 0, 0);
       vw[i] = load_part_codes<N, true>(v_run, (uint32_t)e & 1u, elem);
-    } else {   // fewer elements below an index than a lane's
-      uint32_t w[4] = {0u, 0u, 0u, 0u};
-      vw[i] = 0u;
-#pragma unroll
-      for (uint32_t k = 0; k < N; ++k) {
-        if (k < len) {
-          if constexpr (GT != 0) w[k / 2] |= (uint32_t)as_global<const uint16_t>(g_run)[k] << (16 * (k & 1));
-          else w[k] = as_global<const uint32_t>(g_run)[k];
-          const uint32_t nibble = ((uint32_t)e & 1u) + k;
-          vw[i] |= ((as_global<const uint8_t>(v_run)[nibble >> 1] >> (4 * (nibble & 1u))) & 15u) << (4 * k);
-        }
-      }
-      gw[i] = u32x4{w[0], w[1], w[2], w[3]};
+    } else {
+      const uint32_t g_bits = GT != 0 ? (uint32_t)as_global<const uint16_t>(g_run)[elem] : as_global<const uint32_t>(g_run)[elem];
+      gw[i] = u32x4{g_bits, 0u, 0u, 0u};
+      vw[i] = as_global<const uint8_t>(v_run)[(((uint32_t)e & 1u) + elem) >> 1];
     }
   };
   auto reduce = [&](uint32_t base, int i) {
@@ -504,7 +497,10 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1S
     } else {
       g[0] = bits2f(w.x); g[1] = bits2f(w.y); g[2] = bits2f(w.z); g[3] = bits2f(w.w);
     }
-    const uint32_t even = vw[i] & 0x0F0F0F0Fu, odd = (vw[i] >> 4) & 0x0F0F0F0Fu;  // one code per byte
+    const uint32_t mine = base + wave + (uint32_t)i * kWaves, o = mine < no ? mine : no - 1u;
+    // a single element's code is the low or the high half of its byte
+    const uint32_t codes = whole ? vw[i] : vw[i] >> ((((uint32_t)(first + (int64_t)o * below) + elem) & 1u) * 4u);
+    const uint32_t even = codes & 0x0F0F0F0Fu, odd = (codes >> 4) & 0x0F0F0F0Fu;  // one code per byte
     float o_max = 0.0f;
 #pragma unroll
     for (uint32_t k = 0; k < N; ++k) {
@@ -513,10 +509,9 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1S
       const float v_old = code_value * min_nonneg(o_old[i], s_old[k]);
       const float v = args.b2 * v_old + args.r2 * (gk * gk);     // a NaN never becomes a maximum
       x_max[k] = __builtin_fmaxf(x_max[k], v);
-      if (whole || k < len) o_max = __builtin_fmaxf(o_max, v);
+      if (whole || k == 0u) o_max = __builtin_fmaxf(o_max, v);
     }
     o_max = row_max16(o_max);
-    const uint32_t mine = base + wave + (uint32_t)i * kWaves;
     if ((lane & 15u) == 0u) outer_bits[lane >> 4][mine] = f2bits(o_max);
   };
   for (uint32_t base = 0; base < no; base += kLeadOuter) {
@@ -534,7 +529,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1S
   }
 #pragma unroll
   for (uint32_t k = 0; k < N; ++k) {
-    if (whole || k < len) run_max[wave][elem + k] = x_max[k];
+    if (whole || k == 0u) run_max[wave][elem + k] = x_max[k];
   }
   __syncthreads();
   const uint32_t first1 = r0 / shape2;                         // the tile's first index of the second dimension
