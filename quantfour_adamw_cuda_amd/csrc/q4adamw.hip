@@ -293,17 +293,6 @@ static ChunkRuns stat_runs(Rank1StatForm form, int g_dtype, uint32_t tiles) {
   return grouped ? ChunkRuns{3u, tiles & ~63u} : ChunkRuns{0u, 0u};
 }
 
-// Indices of the first dimension whose statistics one workgroup of the lead form takes: as many as leave the launch
-// 768 workgroups, three per CU, because every workgroup updates the other dimensions' statistics, one update of an
-// address after another.  Steps, us, with at least 512 / 768 / 2048 / any number of workgroups of 32: residual networks,
-// 64 wide in fp32, three blocks a stage 104 / 94 / 104 / 104, 96 wide in bf16 139 / 133 / 142 / 140; [256, n, c] of 41 million fp32
-// elements, c = 5 166 / 155 / 172 / 197, c = 64 145 / 157 / 184 / 215.
-static uint32_t lead_stat_outer(uint64_t elements, uint32_t run) {
-  uint32_t most = kLeadMostOuter;
-  while (most > kLeadOuter && elements / ((uint64_t)run * most) < 768u) most /= 2u;
-  return most;
-}
-
 // tiles of the statistics launch of a matrix
 static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_rows, int g_dtype) {
   if (rank1_stat_form(t) == kStatFlat) {
@@ -315,6 +304,21 @@ static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_r
     return (uint64_t)((outer + stat_rows - 1) / stat_rows) * lead_tiles((uint32_t)t.rows, outer, (uint32_t)t.cols, lead_run(g_dtype != Q4ADAMW_FP32)).inner;
   }
   return (((uint64_t)t.rows + stat_rows - 1) / stat_rows) * (uint64_t)((t.cols + kStatCols - 1) / kStatCols);
+}
+
+// Indices of the first dimension whose statistics one workgroup of the lead form takes: as many as leave the launch
+// 768 workgroups, three per CU, because every workgroup updates the other dimensions' statistics, one update of an
+// address after another.  Steps, us, with at least 512 / 768 / 2048 / any number of workgroups of 32: residual networks,
+// 64 wide in fp32, three blocks a stage 104 / 94 / 104 / 104, 96 wide in bf16 139 / 133 / 142 / 140; [256, n, c] of 41 million fp32
+// elements, c = 5 166 / 155 / 172 / 197, c = 64 145 / 157 / 184 / 215.  They are counted and not estimated from the elements:
+// tensors with few elements below an index have short runs, and so many more workgroups.  Steps, us, bf16 gradients, by the estimate /
+// by the count: [200000, 3, 3] 74 / 69, [100000, 7, 7] 62 / 55, [50000, 1, 31] 41 / 34; fp32 58 / 53, 58 / 52, 39 / 32.
+// workgroups(most): of the launch's tensors that take this form
+template <typename F>
+static uint32_t lead_stat_outer(F workgroups) {
+  uint32_t most = kLeadOuter;
+  while (most < kLeadMostOuter && workgroups(2u * most) >= 768u) most *= 2u;
+  return most;
 }
 
 static FastDiv make_fast_div_any(uint32_t d) { return d == 1u ? FastDiv{0u, 0u} : make_fast_div(d); }
@@ -747,7 +751,12 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       tallest = (uint64_t)t.rows > tallest ? (uint64_t)t.rows : tallest;
     }
     if (elements == 0) return 0;
-    sa.stat_rows = form == kStatLead ? lead_stat_outer(elements, lead_run(g_dtype != Q4ADAMW_FP32)) : rank1_stat_rows(elements, tallest);
+    auto workgroups = [&](uint32_t stat_rows) {
+      uint64_t n = 0;
+      for (int i = 0; i < ntensors; ++i) n += rank1_stat_form(*batch[i]) == form ? rank1_stat_chunks(*batch[i], stat_rows, g_dtype) : 0u;
+      return n;
+    };
+    sa.stat_rows = form == kStatLead ? lead_stat_outer(workgroups) : rank1_stat_rows(elements, tallest);
     int n = 0;
     for (int i = 0; i < ntensors; ++i) {
       const q4adamw_rank1_tensor &t = *batch[i];

@@ -395,7 +395,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1S
 // of residual networks took, us, 64 wide in fp32 88 (now 79), 96 wide in bf16 174 (133), of [256, n, 64] with 41 million
 // elements in fp32 213 (157), in bf16 166 (102).  With fewer elements below an index than a lane's N, every lane takes one
 // (those past the end the first one again): all N of them in each lane, one load after another, made a step of [300000, 2, 3]
-// with bf16 gradients 119 us (now 76; 84 with one element per lane everywhere).
+// with bf16 gradients 119 us (now 69; 84 with one element per lane everywhere).
 constexpr uint32_t kLeadOuter = 32, kLeadMostOuter = 256;    // a round's indices; the most
 
 // elements of a run, at most (16 bytes of gradients per lane)

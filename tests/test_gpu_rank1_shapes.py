@@ -31,7 +31,9 @@ PARTS = [(37, 258), (37, 259), (40, 260), (37, 261), (40, 504), (37, 507), (40, 
 TENSORS = [(5, 300, 3, 3), (2, 700, 3), (1400, 1, 2), (300, 2, 7), (16, 16, 16), (3, 100, 260), (2, 130, 4, 257), (64, 3, 7, 7),
            # fewer elements below an index than a lane's; runs that end within a lane's; the most columns; half a round of
            # indices, a round and one more
-           (3, 1, 2), (70, 2, 3), (700, 1, 3), (40, 1, 1, 5), (33, 90, 256), (17, 5, 2, 255), (16, 30, 3, 3), (129, 57, 3, 3), (5, 171, 3)]
+           (3, 1, 2), (70, 2, 3), (700, 1, 3), (40, 1, 1, 5), (33, 90, 256), (17, 5, 2, 255), (16, 30, 3, 3), (129, 57, 3, 3), (5, 171, 3),
+           # many indices with few elements below them: 64, 128 and 256 of them in a workgroup, and one more
+           (49153, 1, 3), (98305, 1, 1, 7), (196609, 1, 2), (196609, 3, 3)]
 
 
 @pytest.mark.parametrize("p_dt,g_dt", [("fp32", "fp32"), ("bf16", "bf16"), ("fp32", "fp16")])
