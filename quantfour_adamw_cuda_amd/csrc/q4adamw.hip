@@ -253,18 +253,22 @@ static Rank1StatForm rank1_stat_form(const q4adamw_rank1_tensor &t) {
 }
 
 template <int GT, bool EXT>
-static Rank1StatKernel pick_rank1_stats_form(Rank1StatForm form) {
+static Rank1StatKernel pick_rank1_stats_form(Rank1StatForm form, bool runs = false) {
   if (form == kStatFlat) return rank1_stats_flat_kernel<GT, EXT>;
+  if constexpr (GT == Q4ADAMW_FP32) {
+    if (form == kStatLead && runs) return rank1_stats_lead_kernel<GT, EXT, true>;
+  }
   if constexpr (GT != kAbsValues) {
-    if (form == kStatLead) return rank1_stats_lead_kernel<GT, EXT>;
+    if (form == kStatLead) return rank1_stats_lead_kernel<GT, EXT, false>;
   }
   return form == kStatWide ? rank1_stats_kernel<GT, EXT, false> : rank1_stats_kernel<GT, EXT, true>;
 }
 
-static Rank1StatKernel pick_rank1_stats(Rank1StatForm form, int g_dtype, bool ext) {
+// runs: of fp32 gradients, several runs in a workgroup of the lead form
+static Rank1StatKernel pick_rank1_stats(Rank1StatForm form, int g_dtype, bool ext, bool runs) {
   if (g_dtype == Q4ADAMW_BF16) return ext ? pick_rank1_stats_form<Q4ADAMW_BF16, true>(form) : pick_rank1_stats_form<Q4ADAMW_BF16, false>(form);
   if (g_dtype == Q4ADAMW_FP16) return ext ? pick_rank1_stats_form<Q4ADAMW_FP16, true>(form) : pick_rank1_stats_form<Q4ADAMW_FP16, false>(form);
-  return ext ? pick_rank1_stats_form<Q4ADAMW_FP32, true>(form) : pick_rank1_stats_form<Q4ADAMW_FP32, false>(form);
+  return ext ? pick_rank1_stats_form<Q4ADAMW_FP32, true>(form, runs) : pick_rank1_stats_form<Q4ADAMW_FP32, false>(form, runs);
 }
 
 // Rows whose statistics one workgroup takes together, in a launch over `elements` elements of matrices
@@ -294,14 +298,14 @@ static ChunkRuns stat_runs(Rank1StatForm form, int g_dtype, uint32_t tiles) {
 }
 
 // tiles of the statistics launch of a matrix
-static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_rows, int g_dtype) {
+static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_rows, int g_dtype, uint32_t lead_runs = 1u) {
   if (rank1_stat_form(t) == kStatFlat) {
     const uint64_t rows = (uint64_t)flat_tile_rows((uint32_t)t.cols) * flat_tiles((uint32_t)t.cols, stat_rows);
     return ((uint64_t)t.rows + rows - 1) / rows;
   }
   if (rank1_stat_form(t) == kStatLead) {
     const uint32_t outer = (uint32_t)t.lead_shape[0];
-    return (uint64_t)((outer + stat_rows - 1) / stat_rows) * lead_tiles((uint32_t)t.rows, outer, (uint32_t)t.cols, lead_run(g_dtype != Q4ADAMW_FP32)).inner;
+    return (uint64_t)((outer + stat_rows - 1) / stat_rows) * lead_tiles((uint32_t)t.rows, outer, (uint32_t)t.cols, lead_run(g_dtype != Q4ADAMW_FP32), lead_runs).inner;
   }
   return (((uint64_t)t.rows + stat_rows - 1) / stat_rows) * (uint64_t)((t.cols + kStatCols - 1) / kStatCols);
 }
@@ -313,12 +317,22 @@ static uint64_t rank1_stat_chunks(const q4adamw_rank1_tensor &t, uint32_t stat_r
 // elements, c = 5 166 / 155 / 172 / 197, c = 64 145 / 157 / 184 / 215.  They are counted and not estimated from the elements:
 // tensors with few elements below an index have short runs, and so many more workgroups.  Steps, us, bf16 gradients, by the estimate /
 // by the count: [200000, 3, 3] 74 / 69, [100000, 7, 7] 62 / 55, [50000, 1, 31] 41 / 34; fp32 58 / 53, 58 / 52, 39 / 32.
-// workgroups(most): of the launch's tensors that take this form
+// Where the first dimension has no more indices to take, a workgroup takes several runs below them, down to the same number of
+// workgroups.  Steps, us, fp32, one run / several: [8, 4096, 128] 72 / 55, [8, 4096, 100] 73 / 52, [2, 40000, 64] 96 / 74, [16, 4096, 128]
+// 87 / 69, [33, 3000, 128] the same, [8, 64, 1000, 33] 164 / 110, [4, 300000, 7] 76 / 66; [8, 4096, 128] took 67 when lanes
+// kept one element.  16-bit gradients, whose runs are twice as long, keep one: several cost [4, 20000, 64] 56 / 61, [3, 40000, 64]
+// 77 / 81, [8, 100000, 12] 60 / 64, though [4, 65536, 128] took 213 / 188.
+// workgroups(indices, runs): of the launch's tensors that take this form
 template <typename F>
-static uint32_t lead_stat_outer(F workgroups) {
-  uint32_t most = kLeadOuter;
-  while (most < kLeadMostOuter && workgroups(2u * most) >= 768u) most *= 2u;
-  return most;
+static void lead_split(F workgroups, int g_dtype, uint32_t *most, uint32_t *runs) {
+  *most = kLeadOuter;
+  while (*most < kLeadMostOuter && workgroups(2u * *most, 1u) >= 768u) *most *= 2u;
+  *runs = 1u;
+  auto fewer = [&] {
+    const uint64_t n = workgroups(*most, 2u * *runs);
+    return n >= 768u && n < workgroups(*most, *runs);
+  };
+  while (g_dtype == Q4ADAMW_FP32 && *runs < kLeadMostRuns && fewer()) *runs *= 2u;
 }
 
 static FastDiv make_fast_div_any(uint32_t d) { return d == 1u ? FastDiv{0u, 0u} : make_fast_div(d); }
@@ -751,12 +765,16 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
       tallest = (uint64_t)t.rows > tallest ? (uint64_t)t.rows : tallest;
     }
     if (elements == 0) return 0;
-    auto workgroups = [&](uint32_t stat_rows) {
-      uint64_t n = 0;
-      for (int i = 0; i < ntensors; ++i) n += rank1_stat_form(*batch[i]) == form ? rank1_stat_chunks(*batch[i], stat_rows, g_dtype) : 0u;
-      return n;
-    };
-    sa.stat_rows = form == kStatLead ? lead_stat_outer(workgroups) : rank1_stat_rows(elements, tallest);
+    sa.lead_runs = 1u;
+    if (form == kStatLead) {
+      lead_split([&](uint32_t most, uint32_t runs) {
+        uint64_t n = 0;
+        for (int i = 0; i < ntensors; ++i) n += rank1_stat_form(*batch[i]) == form ? rank1_stat_chunks(*batch[i], most, g_dtype, runs) : 0u;
+        return n;
+      }, g_dtype, &sa.stat_rows, &sa.lead_runs);
+    } else {
+      sa.stat_rows = rank1_stat_rows(elements, tallest);
+    }
     int n = 0;
     for (int i = 0; i < ntensors; ++i) {
       const q4adamw_rank1_tensor &t = *batch[i];
@@ -778,11 +796,11 @@ static int fused_4bit_rank1_multi_impl(const q4adamw_rank1_tensor *tensors, int 
         sd.lead_shape[j] = there ? (uint32_t)t.lead_shape[j] : 1u;
       }
       sa.first_chunk[n] = (uint32_t)tiles;
-      tiles += rank1_stat_chunks(t, sa.stat_rows, g_dtype);
+      tiles += rank1_stat_chunks(t, sa.stat_rows, g_dtype, sa.lead_runs);
       ++n;
     }
     finish_prefix(sa, n);
-    const Rank1StatKernel stat_kernel = pick_rank1_stats(form, g_dtype, ext);
+    const Rank1StatKernel stat_kernel = pick_rank1_stats(form, g_dtype, ext, sa.lead_runs > 1u);
     return for_each_grid(tiles, kThreads, [&](uint64_t base, uint64_t count) -> int {
       sa.chunk_base = (uint32_t)base;
       sa.runs = stat_runs(form, g_dtype, (uint32_t)count);

@@ -268,6 +268,7 @@ struct Rank1StatArgs {
   ChunkRuns runs;          // wide forms: which tile a workgroup takes
   // rows of a workgroup (flat form: at most, but for one tile; lead form: indices of the first dimension): 32, 64, 128 or 256
   uint32_t stat_rows;
+  uint32_t lead_runs;      // lead form: runs of a workgroup, at most
   uint32_t pivot[kPivots];
   uint32_t first_chunk[kPivots * 8];
   struct Desc {  // 120 bytes

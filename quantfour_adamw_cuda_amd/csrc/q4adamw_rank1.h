@@ -397,28 +397,34 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_flat_kernel(const Rank1S
 // (those past the end the first one again): all N of them in each lane, one load after another, made a step of [300000, 2, 3]
 // with bf16 gradients 119 us (now 69; 84 with one element per lane everywhere).
 constexpr uint32_t kLeadOuter = 32, kLeadMostOuter = 256;    // a round's indices; the most
+constexpr uint32_t kLeadMostRows = 256, kLeadMostRuns = 16;  // rows and runs of a workgroup, at most
 
 // elements of a run, at most (16 bytes of gradients per lane)
 __host__ __device__ __forceinline__ constexpr uint32_t lead_run(bool half) { return half ? 512u : 256u; }
 
 struct LeadTiles {
   uint32_t inner_rows;   // rows below one index of the first dimension
-  uint32_t rows;         // of them in a tile; the last tile begins early enough to have as many
-  uint32_t inner;        // tiles along them
+  uint32_t rows;         // of them in a run; the last run begins early enough to have as many
+  uint32_t runs;         // along them
+  uint32_t each;         // of a workgroup, one after another: so many that their rows are at most 256
+  uint32_t inner;        // workgroups along them
 };
 
-__host__ __device__ __forceinline__ LeadTiles lead_tiles(uint32_t rows, uint32_t outer, uint32_t cols, uint32_t run) {
+__host__ __device__ __forceinline__ LeadTiles lead_tiles(uint32_t rows, uint32_t outer, uint32_t cols, uint32_t run, uint32_t each) {
   LeadTiles l;
   l.inner_rows = rows / outer;
   const uint32_t most = run / cols;
-  l.inner = (l.inner_rows + most - 1u) / most;
-  l.rows = (l.inner_rows + l.inner - 1u) / l.inner;   // evenly
+  l.runs = (l.inner_rows + most - 1u) / most;
+  l.rows = (l.inner_rows + l.runs - 1u) / l.runs;   // evenly
+  l.each = each == 1u || each * l.rows <= kLeadMostRows ? each : kLeadMostRows / l.rows;
+  l.inner = (l.runs + l.each - 1u) / l.each;
   return l;
 }
 
-template <int GT, bool EXT>
+// RUNS: a workgroup takes several runs (lead_split), which cost the form with one of them 3 to 10 %.
+template <int GT, bool EXT, bool RUNS>
 __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1StatArgs args) {
-  constexpr uint32_t N = GT ? 8 : 4, kRun = lead_run(GT != 0), kSlots = 258;   // more than a run's rows, and than columns
+  constexpr uint32_t N = GT ? 8 : 4, kRun = lead_run(GT != 0), kSlots = 258;   // more than the rows, and than columns
   constexpr int kPerWave = kLeadOuter / kWaves;                // indices of the first dimension, all in flight together
   __shared__ uint32_t outer_bits[4][kLeadMostOuter];           // first dimension: each 16 lanes' maxima
   __shared__ float run_max[kWaves][kRun];                      // the run's elements
@@ -430,11 +436,12 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1S
   const auto &T = args.desc[t];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, cols = T.cols, outer = T.lead_shape[0];
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-  const LeadTiles L = lead_tiles(T.rows, outer, cols, kRun);
-  const uint32_t local = chunk - args.first_chunk[t], ot = local / L.inner, it = local - ot * L.inner;
+  const LeadTiles L = lead_tiles(T.rows, outer, cols, kRun, RUNS ? args.lead_runs : 1u);
+  const uint32_t local = chunk - args.first_chunk[t], ot = local / L.inner, run0 = (local - ot * L.inner) * L.each;
   const uint32_t o0 = ot * args.stat_rows, no = outer - o0 < args.stat_rows ? outer - o0 : args.stat_rows;
+  const uint32_t nruns = !RUNS ? 1u : L.runs - run0 < L.each ? L.runs - run0 : L.each;
   // maxima do not mind rows seen twice
-  const uint32_t r0 = it * L.rows < L.inner_rows - L.rows ? it * L.rows : L.inner_rows - L.rows;
+  auto first_row = [&](uint32_t run) { return run * L.rows < L.inner_rows - L.rows ? run * L.rows : L.inner_rows - L.rows; };
   const uint32_t len = L.rows * cols;                          // elements of the run
   for (uint32_t i = tid; i < kSlots; i += kThreads) slots[0][i] = slots[1][i] = slots[2][i] = 0u;
 
@@ -444,110 +451,116 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1S
   const uint32_t elem = !whole ? (lane < len ? lane : 0u) : lane * N < len - N ? lane * N : len - N;
   const uint32_t shape2 = T.lead_dims == 3u ? T.lead_shape[2] : 1u;
   const gptr<const float> before = as_global<const float>(T.lead_old[1]), last = as_global<const float>(T.lead_old[2]);
-  float s_old[N], x_max[N];
-  {
-    const uint32_t row = elem / cols;
-    uint32_t col = elem - row * cols, i1 = (r0 + row) / shape2, i2 = r0 + row - i1 * shape2;
+  const uint32_t row0 = first_row(run0), first1 = row0 / shape2;   // the workgroup's first row and index of the second dimension
+  for (uint32_t run = 0; run < nruns; ++run) {
+    const uint32_t r0 = first_row(run0 + run);
+    float s_old[N], x_max[N];
+    {
+      const uint32_t row = elem / cols;
+      uint32_t col = elem - row * cols, i1 = (r0 + row) / shape2, i2 = r0 + row - i1 * shape2;
 #pragma unroll
-    for (uint32_t k = 0; k < N; ++k) {
-      float s = 0.0f;
-      if (whole || k == 0u) {
-        s = min_nonneg(as_global<const float>(T.cmax)[col], before[i1]);
-        if (T.lead_dims == 3u) s = min_nonneg(s, last[i2]);
+      for (uint32_t k = 0; k < N; ++k) {
+        float s = 0.0f;
+        if (whole || k == 0u) {
+          s = min_nonneg(as_global<const float>(T.cmax)[col], before[i1]);
+          if (T.lead_dims == 3u) s = min_nonneg(s, last[i2]);
+        }
+        s_old[k] = s;
+        x_max[k] = 0.0f;
+        const bool row_ends = ++col == cols;
+        col = row_ends ? 0u : col;
+        i2 += row_ends ? 1u : 0u;
+        const bool wraps = i2 == shape2;
+        i2 = wraps ? 0u : i2;
+        i1 += wraps ? 1u : 0u;
       }
-      s_old[k] = s;
-      x_max[k] = 0.0f;
-      const bool row_ends = ++col == cols;
-      col = row_ends ? 0u : col;
-      i2 += row_ends ? 1u : 0u;
-      const bool wraps = i2 == shape2;
-      i2 = wraps ? 0u : i2;
-      i1 += wraps ? 1u : 0u;
     }
-  }
-  const int64_t below = (int64_t)L.inner_rows * cols;          // elements below one index
-  const int64_t first = (int64_t)o0 * below + (int64_t)r0 * cols;
-  u32x4 gw[kPerWave];
-  uint32_t vw[kPerWave];
-  float o_old[kPerWave];
-  auto load = [&](uint32_t base, int i) {
-    // past the first dimension's end: its last index once more
-    const uint32_t mine = base + wave + (uint32_t)i * kWaves, o = mine < no ? mine : no - 1u;
-    const int64_t e = first + (int64_t)o * below;              // uniform
-    const void *g_run = static_cast<const char *>(T.g) + e * (GT ? 2 : 4);
-    const void *v_run = T.v + (e >> 1);
-    o_old[i] = as_constant<const float>(T.lead_old[0])[o0 + o];
-    if (whole) {
-      gw[i] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_run), elem * (GT ? 2u : 4u), 0, 0);
-      vw[i] = load_part_codes<N, true>(v_run, (uint32_t)e & 1u, elem);
-    } else {
-      const uint32_t g_bits = GT != 0 ? (uint32_t)as_global<const uint16_t>(g_run)[elem] : as_global<const uint32_t>(g_run)[elem];
-      gw[i] = u32x4{g_bits, 0u, 0u, 0u};
-      vw[i] = as_global<const uint8_t>(v_run)[(((uint32_t)e & 1u) + elem) >> 1];
+    const int64_t below = (int64_t)L.inner_rows * cols;          // elements below one index
+    const int64_t first = (int64_t)o0 * below + (int64_t)r0 * cols;
+    u32x4 gw[kPerWave];
+    uint32_t vw[kPerWave];
+    float o_old[kPerWave];
+    auto load = [&](uint32_t base, int i) {
+      // past the first dimension's end: its last index once more
+      const uint32_t mine = base + wave + (uint32_t)i * kWaves, o = mine < no ? mine : no - 1u;
+      const int64_t e = first + (int64_t)o * below;              // uniform
+      const void *g_run = static_cast<const char *>(T.g) + e * (GT ? 2 : 4);
+      const void *v_run = T.v + (e >> 1);
+      o_old[i] = as_constant<const float>(T.lead_old[0])[o0 + o];
+      if (whole) {
+        gw[i] = __builtin_amdgcn_raw_buffer_load_b128(tile_rsrc(g_run), elem * (GT ? 2u : 4u), 0, 0);
+        vw[i] = load_part_codes<N, true>(v_run, (uint32_t)e & 1u, elem);
+      } else {
+        const uint32_t g_bits = GT != 0 ? (uint32_t)as_global<const uint16_t>(g_run)[elem] : as_global<const uint32_t>(g_run)[elem];
+        gw[i] = u32x4{g_bits, 0u, 0u, 0u};
+        vw[i] = as_global<const uint8_t>(v_run)[(((uint32_t)e & 1u) + elem) >> 1];
+      }
+    };
+    auto reduce = [&](uint32_t base, int i) {
+      float g[8];
+      const u32x4 w = gw[i];
+      if constexpr (GT != 0) {
+        widen_pair<GT>(w.x, g[0], g[1]);
+        widen_pair<GT>(w.y, g[2], g[3]);
+        widen_pair<GT>(w.z, g[4], g[5]);
+        widen_pair<GT>(w.w, g[6], g[7]);
+      } else {
+        g[0] = bits2f(w.x); g[1] = bits2f(w.y); g[2] = bits2f(w.z); g[3] = bits2f(w.w);
+      }
+      const uint32_t mine = base + wave + (uint32_t)i * kWaves, o = mine < no ? mine : no - 1u;
+      // a single element's code is the low or the high half of its byte
+      const uint32_t codes = whole ? vw[i] : vw[i] >> ((((uint32_t)(first + (int64_t)o * below) + elem) & 1u) * 4u);
+      const uint32_t even = codes & 0x0F0F0F0Fu, odd = (codes >> 4) & 0x0F0F0F0Fu;  // one code per byte
+      float o_max = 0.0f;
+#pragma unroll
+      for (uint32_t k = 0; k < N; ++k) {
+        const float gk = EXT ? g[k] * gscale : g[k];
+        const float code_value = __builtin_fmaf((float)(((k & 1 ? odd : even) >> (8 * (k >> 1))) & 0xffu), 0.0625f, 0.0625f);  // (code + 1) / 16, exact
+        const float v_old = code_value * min_nonneg(o_old[i], s_old[k]);
+        const float v = args.b2 * v_old + args.r2 * (gk * gk);     // a NaN never becomes a maximum
+        x_max[k] = __builtin_fmaxf(x_max[k], v);
+        if (whole || k == 0u) o_max = __builtin_fmaxf(o_max, v);
+      }
+      o_max = row_max16(o_max);
+      if ((lane & 15u) == 0u) {
+        uint32_t &slot = outer_bits[lane >> 4][mine];   // this lane's in every run
+        slot = run != 0u && slot > f2bits(o_max) ? slot : f2bits(o_max);
+      }
+    };
+    for (uint32_t base = 0; base < no; base += kLeadOuter) {
+      if (no - base > kLeadOuter / 2) {
+#pragma unroll
+        for (int i = 0; i < kPerWave; ++i) load(base, i);
+#pragma unroll
+        for (int i = 0; i < kPerWave; ++i) reduce(base, i);
+      } else {   // few indices are left: half as many rounds
+#pragma unroll
+        for (int i = 0; i < kPerWave / 2; ++i) load(base, i);
+#pragma unroll
+        for (int i = 0; i < kPerWave / 2; ++i) reduce(base, i);
+      }
     }
-  };
-  auto reduce = [&](uint32_t base, int i) {
-    float g[8];
-    const u32x4 w = gw[i];
-    if constexpr (GT != 0) {
-      widen_pair<GT>(w.x, g[0], g[1]);
-      widen_pair<GT>(w.y, g[2], g[3]);
-      widen_pair<GT>(w.z, g[4], g[5]);
-      widen_pair<GT>(w.w, g[6], g[7]);
-    } else {
-      g[0] = bits2f(w.x); g[1] = bits2f(w.y); g[2] = bits2f(w.z); g[3] = bits2f(w.w);
-    }
-    const uint32_t mine = base + wave + (uint32_t)i * kWaves, o = mine < no ? mine : no - 1u;
-    // a single element's code is the low or the high half of its byte
-    const uint32_t codes = whole ? vw[i] : vw[i] >> ((((uint32_t)(first + (int64_t)o * below) + elem) & 1u) * 4u);
-    const uint32_t even = codes & 0x0F0F0F0Fu, odd = (codes >> 4) & 0x0F0F0F0Fu;  // one code per byte
-    float o_max = 0.0f;
 #pragma unroll
     for (uint32_t k = 0; k < N; ++k) {
-      const float gk = EXT ? g[k] * gscale : g[k];
-      const float code_value = __builtin_fmaf((float)(((k & 1 ? odd : even) >> (8 * (k >> 1))) & 0xffu), 0.0625f, 0.0625f);  // (code + 1) / 16, exact
-      const float v_old = code_value * min_nonneg(o_old[i], s_old[k]);
-      const float v = args.b2 * v_old + args.r2 * (gk * gk);     // a NaN never becomes a maximum
-      x_max[k] = __builtin_fmaxf(x_max[k], v);
-      if (whole || k == 0u) o_max = __builtin_fmaxf(o_max, v);
+      if (whole || k == 0u) run_max[wave][elem + k] = x_max[k];
     }
-    o_max = row_max16(o_max);
-    if ((lane & 15u) == 0u) outer_bits[lane >> 4][mine] = f2bits(o_max);
-  };
-  for (uint32_t base = 0; base < no; base += kLeadOuter) {
-    if (no - base > kLeadOuter / 2) {
+    __syncthreads();
+    for (uint32_t x = tid; x < len; x += kThreads) {
+      float u = run_max[0][x];
 #pragma unroll
-      for (int i = 0; i < kPerWave; ++i) load(base, i);
-#pragma unroll
-      for (int i = 0; i < kPerWave; ++i) reduce(base, i);
-    } else {   // few indices are left: half as many rounds
-#pragma unroll
-      for (int i = 0; i < kPerWave / 2; ++i) load(base, i);
-#pragma unroll
-      for (int i = 0; i < kPerWave / 2; ++i) reduce(base, i);
+      for (int w = 1; w < kWaves; ++w) u = __builtin_fmaxf(u, run_max[w][x]);
+      const uint32_t row = x / cols, i1 = (r0 + row) / shape2, i2 = r0 + row - i1 * shape2;
+      auto raise_slot = [&](uint32_t &slot) {
+        if (f2bits(u) > slot) atomicMax(&slot, f2bits(u));
+      };
+      raise_slot(slots[0][i1 - first1]);
+      // the third dimension's indices of consecutive rows: there are fewer rows than slots, so rows that
+      // share a slot share the index
+      if (T.lead_dims == 3u) raise_slot(slots[1][shape2 < kSlots ? i2 : r0 - row0 + row]);
+      raise_slot(slots[2][x - row * cols]);
     }
+    __syncthreads();
   }
-#pragma unroll
-  for (uint32_t k = 0; k < N; ++k) {
-    if (whole || k == 0u) run_max[wave][elem + k] = x_max[k];
-  }
-  __syncthreads();
-  const uint32_t first1 = r0 / shape2;                         // the tile's first index of the second dimension
-  for (uint32_t x = tid; x < len; x += kThreads) {
-    float u = run_max[0][x];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) u = __builtin_fmaxf(u, run_max[w][x]);
-    const uint32_t row = x / cols, i1 = (r0 + row) / shape2, i2 = r0 + row - i1 * shape2;
-    auto raise_slot = [&](uint32_t &slot) {
-      if (f2bits(u) > slot) atomicMax(&slot, f2bits(u));
-    };
-    raise_slot(slots[0][i1 - first1]);
-    // the third dimension's indices of consecutive rows: a run has fewer rows than slots, so rows that
-    // share a slot share the index
-    if (T.lead_dims == 3u) raise_slot(slots[1][shape2 < kSlots ? i2 : row]);
-    raise_slot(slots[2][x - row * cols]);
-  }
-  __syncthreads();
   static_assert(kLeadMostOuter <= kThreads, "one index per thread below");
   if (tid < no) {
     uint32_t u = outer_bits[0][tid];
@@ -557,7 +570,7 @@ __global__ __launch_bounds__(kThreads) void rank1_stats_lead_kernel(const Rank1S
   }
   for (uint32_t i = tid; i < kSlots; i += kThreads) {
     if (slots[0][i] != 0u) raise_max(T.lead_next[1] + first1 + i, slots[0][i]);
-    if (slots[1][i] != 0u) raise_max(T.lead_next[2] + (shape2 < kSlots ? i : (r0 + i) % shape2), slots[1][i]);
+    if (slots[1][i] != 0u) raise_max(T.lead_next[2] + (shape2 < kSlots ? i : (row0 + i) % shape2), slots[1][i]);
     if (slots[2][i] != 0u) raise_max(T.cmax_next + i, slots[2][i]);
   }
 }

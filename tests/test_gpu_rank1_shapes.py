@@ -33,7 +33,11 @@ TENSORS = [(5, 300, 3, 3), (2, 700, 3), (1400, 1, 2), (300, 2, 7), (16, 16, 16),
            # indices, a round and one more
            (3, 1, 2), (70, 2, 3), (700, 1, 3), (40, 1, 1, 5), (33, 90, 256), (17, 5, 2, 255), (16, 30, 3, 3), (129, 57, 3, 3), (5, 171, 3),
            # many indices with few elements below them: 64, 128 and 256 of them in a workgroup, and one more
-           (49153, 1, 3), (98305, 1, 1, 7), (196609, 1, 2), (196609, 3, 3)]
+           (49153, 1, 3), (98305, 1, 1, 7), (196609, 1, 2), (196609, 3, 3),
+           # fp32 gradients, few indices: two, four and sixteen runs in a workgroup, the last of which end early; so many rows in a
+           # run that the workgroup's 256 stop it at two; a third dimension with fewer and with more indices than rows; two
+           # workgroups along the first dimension
+           (2, 3073, 128), (1, 12517, 64), (5, 197000, 2), (1, 1025, 3, 130), (1, 11, 300, 129), (33, 800, 255)]
 
 
 @pytest.mark.parametrize("p_dt,g_dt", [("fp32", "fp32"), ("bf16", "bf16"), ("fp32", "fp16")])
@@ -175,7 +179,8 @@ def test_short_rows_of_several_dimensions(cuda, shape, p_dt, g_dt, stochastic):
 @pytest.mark.parametrize("stochastic", [False, True])
 @pytest.mark.parametrize("g_dt", ["fp32", "bf16", "fp16"])
 @pytest.mark.parametrize("shape", [(300, 3), (77, 50), (1000, 88), (6200, 41), (64, 264), (33, 301),
-                                   (5, 40, 3, 3), (33, 7, 5), (20, 3, 64), (3, 9, 264), (2, 5, 300), (2, 3, 300, 3), (3, 2, 270, 40)])
+                                   (5, 40, 3, 3), (33, 7, 5), (20, 3, 64), (3, 9, 264), (2, 5, 300), (2, 3, 300, 3), (3, 2, 270, 40),
+                                   (2, 3073, 128)])
 def test_multiplier_and_non_finite_gradients(cuda, shape, g_dt, stochastic):
     """Every statistics kernel with a device multiplier (gradients scaled up by it, so that the product is
     exact) and cleared gradients; NaN and infinities in the second step: maxima are taken over the

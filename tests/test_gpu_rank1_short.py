@@ -36,7 +36,8 @@ def _step(ts, gs, step, **kw):
 
 @pytest.mark.parametrize("p_dt,g_dt", [("fp32", "fp32"), ("bf16", "bf16")])
 @pytest.mark.parametrize("shape", [(5, 40, 3, 3), (6, 70, 1, 5), (33, 7, 5),
-                                   (4, 30, 96), (3, 20, 264)])      # scales from vectors; leading statistics of the wide form
+                                   (4, 30, 96), (3, 20, 264),       # scales from vectors; leading statistics of the wide form
+                                   (2, 3073, 128)])                 # several runs in a workgroup of the leading statistics
 def test_cancelled_steps_leave_everything(cuda, shape, p_dt, g_dt):
     """An overflow flag after a step: parameters, codes, statistics and the rows' scales, which the kernel for short rows
     writes itself, stay; the gradients are cleared only where that is asked for."""
